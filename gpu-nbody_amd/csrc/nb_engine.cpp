@@ -168,8 +168,6 @@ nb::Ctl initial_ctl(const nb_sim *s, uint32_t epoch)
     c.n_cells = 1;
     c.max_depth = 1; // GPUBarnesHutNBodySimulation.java:170
     c.error = 0;
-    c.interactions = 0;
-    c.cell_interactions = 0;
     (void)s;
     return c;
 }
@@ -196,10 +194,16 @@ int check_device_error(nb_sim *s)
     int r = read_ctl(s, &c);
     if (r) return r;
     update_hint(s, c);
-    s->last_interactions = (long long)(c.interactions - s->inter_before);
-    s->inter_before = c.interactions;
-    s->last_cell_interactions = (long long)(c.cell_interactions - s->cell_inter_before);
-    s->cell_inter_before = c.cell_interactions;
+    unsigned long long all = 0;
+    long long cells = 0;
+    for (const nb::Tally &t : c.tally) {
+        all += t.all;
+        cells += (long long)t.cells;
+    }
+    s->last_interactions = (long long)(all - s->inter_before);
+    s->inter_before = all;
+    s->last_cell_interactions = cells - s->cell_inter_before;
+    s->cell_inter_before = cells;
     switch (c.error) {
     case nb::kErrNone: return NB_OK;
     case nb::kErrPool: return fail(s, NB_E_POOL, "octree cell pool exhausted (%d cells)", s->d.cap);

@@ -1,159 +1,214 @@
 // nb_force.hip -- force traversal (calculateforce.cl:25-188) for gfx950, and
 // the FP64 direct sum used to measure force errors.
 //
-// A block is one wave: 64 consecutive sorted positions. A vote group
-// is G consecutive lanes (G = 16, 32 or 64; 16 is the reference's work-group
-// vote of calculateforce.cl:145 and 64 is one wave). Every group owns one
-// stack in LDS; entries are (cell << 6 | depth). Popping a cell tests all of
-// its (at most 8, compacted) children: bodies always interact, a child cell is
-// accepted only if every lane of the group has d^2 + eps^2 >= dq[depth], and an
-// opened cell is pushed. Which nodes interact therefore matches the reference
-// exactly; only the order of the terms differs.
+// A wave takes 64 consecutive sorted positions. A vote group is G consecutive
+// lanes (G = 16, 32 or 64; 16 is the reference's work-group vote of
+// calculateforce.cl:145 and 64 is one wave). Visiting a cell tests all of its
+// (at most 8, compacted) children: bodies always interact, a child cell is
+// accepted by a group only if every lane of the group has d^2 + eps^2 >=
+// dq[depth], and a child that a group does not accept is opened by that group.
+// Which nodes interact therefore matches the reference exactly; only the order
+// of the terms differs.
 //
-// A popped cell's children indices and their (x, y, z, m) are contiguous
-// (cchild, cdata: 32 + 128 bytes). With G = 64 the whole traversal state is
-// wave-uniform: the cell comes off the LDS stack into a scalar register and
-// its 160 bytes arrive through scalar loads, so the vector ALU only does the
-// per-body arithmetic and the opening vote is one ballot.
+// The wave walks the union of its groups' traversals: a stack entry is a cell
+// (cell << 6 | depth) and the groups that opened it, and a cell is visited once
+// for all of them. The cell is wave-uniform, so its children's indices and
+// their (x, y, z, m) (contiguous in cchild and cdata: 32 + 128 bytes) arrive
+// through scalar loads whatever G is, and the vector ALU only does the per-body
+// arithmetic. Lanes whose group did not open the cell take an infinite
+// softening: their 1 / sqrt(d^2) is 0, so they add nothing and accept every
+// child. The groups of a wave are neighbours in the tree's order and open
+// nearly the same cells, and never more than one 64-lane group would: a cell
+// is opened when some lane of some group that reached it rejects it. With a
+// stack per 16-lane group the four groups of a wave were at different cells,
+// each child came through vector loads, and three quarters of the lanes idled
+// in most of the branches: 25.5 -> 8.4 ms at 4M clustered bodies (theta 0.4,
+// vote 16), 6.03 -> 2.38 ms at 1M Plummer bodies (theta 0.5, vote 16).
 //
-// Accumulation: the terms of one popped cell (<= 8) are summed in FP32 and the
-// batch sum is added into a Kahan-compensated FP32 accumulator.
+// Bound: vector issue. Of the 14 issue slots of a term (3 sub, 3 fma, rsq =
+// 2, 3 mul, 3 fma), 3,690 terms per body at 1M Plummer bodies (theta 0.5,
+// vote 64) are 52k of the 69k slots that a wave takes; 1.89 ms (2.37 ms before
+// the scalar side was cut and the FP64 sums), 98 % of vector issue.
+//
+// Accumulation: the terms of one visited cell (<= 8) are summed in FP32 and
+// added into FP64 sums. An FP64 add issues at the rate of an FP32 add here, so
+// convert and add (6 instructions per cell) cost half of a compensated FP32
+// sum (12) and keep more bits.
 #include "nb_device.h"
 
 namespace nb {
 
+constexpr uint64_t kAllLanes = ~0ull;
 
-// ---------------------------------------------------------------------------
-// Vote width 64: one wave, one group, uniform traversal. kForceWaves waves
-// (groups) per block: they share nothing, and a block of one wave frees its
-// slot as soon as its group is done, where a block of four holds its CU's
-// share until its slowest group ends (8.97 -> 8.67 ms at 4M clustered bodies).
-// ---------------------------------------------------------------------------
-constexpr int kForceWaves = 1;
-
-__global__ __launch_bounds__(64 * kForceWaves) void k_force64(Dev d, const int *__restrict__ cchild,
-                                                 const float4 *__restrict__ cdata, int mode)
+// Groups as bits: bit f stands for the 16 lanes of field f, and a vote group of
+// 32 or 64 lanes is two or four fields. group_bits: the groups in which a lane
+// of r is set; field_lanes: the lanes of the fields f. (s_quadmask ors each
+// four bits into one, s_bitreplicate doubles each bit; neither has a builtin.)
+template <int G> __device__ __forceinline__ unsigned group_bits(uint64_t r)
 {
-    __shared__ unsigned stk[kForceWaves][kStack];
-    __shared__ float dq_s[kMaxDepth];
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wv = tid >> 6;
-    const int n = d.n;
-    Ctl *ctl = d.ctl;
-    if (ctl->error) return;
-    if (ctl->max_depth > kMaxDepth) { // calculateforce.cl:69-73
-        if (tid == 0) flag_error(ctl, kErrDepth);
-        return;
-    }
-    for (int i = tid; i < kMaxDepth; i += 64 * kForceWaves) dq_s[i] = ctl->dq[i];
-    const int step = ctl->step;
-    __syncthreads();
-
-    const int pos = blockIdx.x * (64 * kForceWaves) + tid;
-    const bool valid = pos < n;
-    // a lane past the last body sits at infinity: its d^2 is infinite, so it
-    // accepts every cell and never holds up the vote (its sums are discarded)
-    const float4 me = valid ? d.pm4[d.sorted[pos]] : make_float4(kFar, kFar, kFar, 0.f);
-    const float eps2 = d.eps2;
-    const int cap = d.cap;
-
-    if (lane == 0) stk[wv][0] = 0; // root cell 0 at depth 0
-    int sp = 1;
-    float sx = 0.f, sy = 0.f, sz = 0.f, kx = 0.f, ky = 0.f, kz = 0.f;
-    long long ninter = 0; // per wave: every lane meets the same nodes
-    bool bad = false;
-    while (sp > 0) {
-        __builtin_amdgcn_wave_barrier();
-        --sp;
-        const unsigned e = __builtin_amdgcn_readfirstlane(stk[wv][sp]);
-        const int c = (int)(e >> 6);
-        const int dep = (int)(e & 63u);
-        const float thr = dq_s[dep];
-        const int *chp = cchild + (size_t)c * 8;
-        const float4 *cdp = cdata + (size_t)c * 8;
-        int ch[8];
-        float4 q[8];
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            ch[k] = __builtin_amdgcn_readfirstlane(chp[k]);
-            q[k] = cdp[k];
-        }
-        float px = 0.f, py = 0.f, pz = 0.f;
-        int cnt = 0;
-        int npush = 0;
-        bool badv = false;
-        unsigned push = 0;
-        // Every branch in this loop is wave-uniform and none leaves it early
-        // (children are compacted to the front: past the first negative entry
-        // every one is negative). An opened cell's stack entry goes into lane
-        // `npush` of `push` by a lane write, and the opened children are stored
-        // after the loop in one go: no lane-divergent store inside the loop,
-        // which otherwise makes the compiler copy the running sums at every
-        // child.
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const int v = ch[k];
-            if (v < 0) continue;
-            const float dx = q[k].x - me.x, dy = q[k].y - me.y, dz = q[k].z - me.z;
-            const float d2 = fmaf(dx, dx, fmaf(dy, dy, fmaf(dz, dz, eps2)));
-            bool acc = v < n;
-            if (!acc) acc = wave_all(d2 >= thr);
-            if (acc) {
-                const float ri = __builtin_amdgcn_rsqf(d2);
-                const float f = q[k].w * (ri * ri * ri);
-                px = fmaf(dx, f, px);
-                py = fmaf(dy, f, py);
-                pz = fmaf(dz, f, pz);
-                ++cnt;
-            } else {
-                push = lane_write(push, ((unsigned)(v - n) << 6) | (unsigned)(dep + 1), npush);
-                ++npush;
-                badv |= v - n >= cap;
-            }
-        }
-        // the opened children in child order (the last one is popped first);
-        // the tree is at most kMaxDepth deep and the pool holds `cap` cells:
-        // anything else is corrupt
-        if (npush) {
-            if (sp + npush > kStack || badv || dep + 1 >= kMaxDepth) {
-                bad = true;
-            } else {
-                if (lane < npush) stk[wv][sp + lane] = push;
-                sp += npush;
-            }
-        }
-        kahan_add(sx, kx, px);
-        kahan_add(sy, ky, py);
-        kahan_add(sz, kz, pz);
-        ninter += cnt;
-        if (bad) break;
-    }
-    if (bad && lane == 0) flag_error(ctl, kErrStack);
-    if (valid) finish_body(d, pos, me, sx - kx, sy - ky, sz - kz, mode, step);
-    // device interaction counter: one atomic per wave
-    const unsigned long long nvalid = (unsigned long long)__popcll(__ballot(valid));
-    if (lane == 0 && ninter && nvalid)
-        __hip_atomic_fetch_add(&ctl->interactions, (unsigned long long)ninter * nvalid, __ATOMIC_RELAXED, AGENT);
+    static_assert(G == 16 || G == 32 || G == 64, "vote width");
+    if constexpr (G == 64) return r ? 15u : 0u;
+    uint64_t quads;
+    asm("s_quadmask_b64 %0, %1" : "=s"(quads) : "s"(r) : "scc");
+    unsigned f;
+    asm("s_quadmask_b32 %0, %1" : "=s"(f) : "s"((unsigned)quads) : "scc");
+    if constexpr (G == 32) f |= ((f >> 1) & 5u) | ((f << 1) & 10u);
+    return f;
 }
 
-// ---------------------------------------------------------------------------
-// Vote width 16 or 32: several groups per wave, each with its own stack.
-// ---------------------------------------------------------------------------
-// threads per block of the vote-16/32 traversal: one wave (its groups share
-// nothing; blocks of 256 held a CU's share until their slowest group ended:
-// vote 16 27.6 -> 25.6 ms, vote 32 18.6 -> 18.0 ms at 4M clustered bodies)
-constexpr int kGThreads = 64;
-
-template <int G>
-__global__ __launch_bounds__(kGThreads) void k_force_g(Dev d, int mode)
+__device__ __forceinline__ uint64_t field_lanes(unsigned f)
 {
-    constexpr int kGroups = kGThreads / G;
-    __shared__ unsigned stk[kGroups][kStack];
+    uint64_t x = f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const unsigned lo = (unsigned)x;
+        asm("s_bitreplicate_b64_b32 %0, %1" : "=s"(x) : "s"(lo));
+    }
+    return x;
+}
+
+typedef int i32x8 __attribute__((ext_vector_type(8)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+// the softened monopole term of mass m at (dx, dy, dz), d2 = |d|^2 + eps^2
+__device__ __forceinline__ void add_term(float dx, float dy, float dz, float d2, float m, float &px, float &py,
+                                         float &pz)
+{
+    const float ri = __builtin_amdgcn_rsqf(d2);
+    const float f = m * (ri * ri * ri);
+    px = fmaf(dx, f, px);
+    py = fmaf(dy, f, py);
+    pz = fmaf(dz, f, pz);
+}
+
+// One visit: the children of cell `e >> 6` (on level e & 63) against the
+// wave's bodies. act: the lanes whose groups opened the cell. The terms'
+// sum goes to (px, py, pz), the number of children is returned;
+// opened(entry, lanes) is called for every child that some group opens. Every
+// branch is wave-uniform. Child cells sit at the front of the cell's record and
+// bodies at its back, and their counts in the first two index words
+// (nb_internal.h): a body costs a compare and a branch on the scalar side, a
+// cell two more for its vote. The scalar unit issues one instruction per SIMD
+// and four cycles like the vector one, and with a test of each child's kind
+// it was the busier of the two (72k scalar against 64k vector instructions
+// per wave at 1M Plummer bodies, theta 0.5).
+template <int G, bool SPLIT, class Opened>
+__device__ __forceinline__ int visit_cell(unsigned e, unsigned fields, uint64_t act, float thr, float4 me,
+                                          float eps2, const int *__restrict__ cchild,
+                                          const float4 *__restrict__ cdata, float &px, float &py, float &pz,
+                                          bool &bad, Opened &&opened)
+{
+    const size_t c = e >> 6;
+    const i32x8 ch = *reinterpret_cast<const i32x8 *>(cchild + c * 8);
+    const f32x16 q0 = *reinterpret_cast<const f32x16 *>(cdata + c * 8);
+    const f32x16 q1 = *reinterpret_cast<const f32x16 *>(cdata + c * 8 + 4);
+    // all loads issued together (the compiler would put the second half
+    // behind the first children's work, one more round trip per visit)
+    if constexpr (SPLIT) asm volatile("" ::"s"(ch), "s"(q0), "s"(q1));
+    const int nbody = (int)((unsigned)ch[0] >> kCountShift);
+    int ncell = (int)((unsigned)ch[1] >> kCountShift);
+    // cells live on kMaxDepth levels: child cells below the last are corrupt
+    // (and not followed, so a visit never descends past it)
+    if ((e & 63u) == kMaxDepth - 1 && ncell > 0) {
+        bad = true;
+        ncell = 0;
+    }
+    float e2 = eps2;
+    if constexpr (G < 64) e2 = __builtin_amdgcn_inverse_ballot_w64(act) ? eps2 : kFar;
+    px = py = pz = 0.f;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        if (k >= ncell) break;
+        const f32x16 &q = k < 4 ? q0 : q1;
+        const float dx = q[4 * (k & 3)] - me.x, dy = q[4 * (k & 3) + 1] - me.y, dz = q[4 * (k & 3) + 2] - me.z;
+        const float d2 = fmaf(dx, dx, fmaf(dy, dy, fmaf(dz, dz, e2)));
+        const uint64_t r = act & ~__builtin_amdgcn_fcmpf(d2, thr, 3); // 3 = ordered >=
+        const float m = q[4 * (k & 3) + 3];
+        if (r) {
+            const unsigned rej = group_bits<G>(r); // the groups that open this child
+            opened(((unsigned)ch[k] << 6) | ((e & 63u) + 1u), rej);
+            // some groups accept, some open: the latter add nothing (the asm
+            // keeps the compiler from joining this arm's sums with the
+            // other's behind a flag: 2480 -> 2380 us at 1M Plummer bodies,
+            // theta 0.5, vote 16)
+            if constexpr (G < 64) {
+                if (rej != fields) {
+                    add_term(dx, dy, dz, d2, __builtin_amdgcn_inverse_ballot_w64(field_lanes(rej)) ? 0.f : m, px, py, pz);
+                    asm volatile("" : "+v"(px), "+v"(py), "+v"(pz));
+                }
+            }
+        } else {
+            add_term(dx, dy, dz, d2, m, px, py, pz);
+        }
+    }
+#pragma unroll
+    for (int k = 7; k >= 0; --k) {
+        if (7 - k >= nbody) break;
+        const f32x16 &q = k < 4 ? q0 : q1;
+        const float dx = q[4 * (k & 3)] - me.x, dy = q[4 * (k & 3) + 1] - me.y, dz = q[4 * (k & 3) + 2] - me.z;
+        const float d2 = fmaf(dx, dx, fmaf(dy, dy, fmaf(dz, dz, e2)));
+        add_term(dx, dy, dz, d2, q[4 * (k & 3) + 3], px, py, pz);
+    }
+    return nbody + ncell;
+}
+
+// Entries of a block's stack. One wave (K = 1) walks depth first: at most 7
+// siblings wait per level. K waves take the K top entries together; the limit
+// kSplitTop above which they take one entry at a time (depth first from there,
+// again at most 7 per level) bounds the stack for every tree of kMaxDepth
+// levels: kSplitTop + the children of one round + 7 per level.
+constexpr int kSplitTop = 512;
+template <int K> constexpr int force_stack() { return K == 1 ? kStack : kSplitTop + 8 * K + kStack; }
+
+template <int G> struct StackEntry {
+    using type = uint2;
+};
+template <> struct StackEntry<64> {
+    using type = unsigned;
+};
+
+// The epilogue's per-wave sums overlay the stack.
+template <int G, int K> constexpr int force_lds()
+{
+    const int stack = force_stack<K>() * (int)sizeof(typename StackEntry<G>::type), red = K == 1 ? 0 : K * 3 * 64 * 8;
+    return ((stack > red ? stack : red) + 15) & ~15;
+}
+
+// K waves share the group of 64 positions (K > 1: few groups, so that one
+// wave per group would leave the chip idle). They take the stack's top K
+// entries in rounds: wave w visits the w-th from the top, and after a barrier
+// pushes what it opened behind the lower waves' entries. The order depends on
+// nothing but the tree, and so do the sums. (Eight waves per SIMD by the
+// attribute: the scalar registers would otherwise allow seven, 1.90 against
+// 2.19 ms at 1M Plummer bodies, theta 0.5, vote 64.)
+template <int G, int K>
+__global__ __launch_bounds__(64 * K) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_force(
+    Dev d, const int *__restrict__ cchild, const float4 *__restrict__ cdata, int mode)
+{
+    constexpr int kCap = force_stack<K>();
+    __shared__ __attribute__((aligned(16))) unsigned char lds[force_lds<G, K>()];
     __shared__ float dq_s[kMaxDepth];
+    __shared__ unsigned pushed[K]; // per wave: entries pushed this round, | kBad on a corrupt tree
+    __shared__ unsigned long long wint[K];
+    constexpr unsigned kBad = 1u << 16;
+    // (cell << 6 | depth), with narrow votes beside the groups that opened it
+    using Entry = typename StackEntry<G>::type;
+    Entry *stk = reinterpret_cast<Entry *>(lds);
+    auto entry = [](unsigned e, unsigned f) {
+        if constexpr (G < 64) return make_uint2(e, f);
+        else return e;
+    };
+    auto take_entry = [](Entry v, unsigned &e, unsigned &f) {
+        if constexpr (G < 64) {
+            e = __builtin_amdgcn_readfirstlane(v.x);
+            f = __builtin_amdgcn_readfirstlane(v.y);
+        } else {
+            e = __builtin_amdgcn_readfirstlane(v);
+        }
+    };
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const int gl = tid / G;
+    const int wv = K == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = d.n;
     Ctl *ctl = d.ctl;
     if (ctl->error) return;
@@ -161,97 +216,155 @@ __global__ __launch_bounds__(kGThreads) void k_force_g(Dev d, int mode)
         if (tid == 0) flag_error(ctl, kErrDepth);
         return;
     }
-    for (int i = tid; i < kMaxDepth; i += kGThreads) dq_s[i] = ctl->dq[i];
+    for (int i = tid; i < kMaxDepth; i += 64 * K) dq_s[i] = ctl->dq[i];
     const int step = ctl->step;
-    __syncthreads();
 
-    const int pos = blockIdx.x * kGThreads + tid;
+    const int pos = blockIdx.x * 64 + lane;
     const bool valid = pos < n;
     // a lane past the last body sits at infinity: its d^2 is infinite, so it
     // accepts every cell and never holds up the vote (its sums are discarded)
     const float4 me = valid ? d.pm4[d.sorted[pos]] : make_float4(kFar, kFar, kFar, 0.f);
+    const uint64_t vmask = __ballot(valid);
     const float eps2 = d.eps2;
-    const unsigned long long gmask = ((1ull << G) - 1ull) << ((lane / G) * G);
-    const int glane = lane % G; // this lane's place in its group
-    const bool leader = glane == 0;
-
-    if (leader) stk[gl][0] = 0; // root cell 0 at depth 0
-    int sp = 1;
-    float sx = 0.f, sy = 0.f, sz = 0.f, kx = 0.f, ky = 0.f, kz = 0.f;
-    int ninter = 0;
+    const unsigned cap = (unsigned)d.cap;
+    double sx = 0.0, sy = 0.0, sz = 0.0;
+    // Interactions: every child of a visited cell meets the lanes that opened
+    // it, except where it is opened in turn, which is a visit of its own: the
+    // sum over the visits of (children - 1) x lanes, plus the root's lanes.
+    unsigned long long inter = 0;
     bool bad = false;
-    while (sp > 0) {
-        __builtin_amdgcn_wave_barrier();
-        const unsigned e = stk[gl][--sp];
-        const int c = (int)(e >> 6);
-        const int dep = (int)(e & 63u);
-        const float thr = dq_s[dep];
-        const int4 c0 = *reinterpret_cast<const int4 *>(d.cchild + (size_t)c * 8);
-        const int4 c1 = *reinterpret_cast<const int4 *>(d.cchild + (size_t)c * 8 + 4);
-        const int ch[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
-        const float4 *cdp = d.cdata + (size_t)c * 8;
-        float px = 0.f, py = 0.f, pz = 0.f;
-        int cnt = 0;
-        int npush = 0;
-        bool badv = false;
-        unsigned push = 0;
-        // as in k_force64: no early exit, and the opened children's stack
-        // entries gathered in lanes 0 .. npush-1 of the group by a select and
-        // stored after the loop
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const int v = ch[k];
-            if (v < 0) continue;
-            const float4 q = cdp[k];
-            const float dx = q.x - me.x, dy = q.y - me.y, dz = q.z - me.z;
-            const float d2 = fmaf(dx, dx, fmaf(dy, dy, fmaf(dz, dz, eps2)));
-            bool acc = v < n;
-            if (!acc) acc = (__builtin_amdgcn_ballot_w64(d2 >= thr) & gmask) == gmask;
-            if (acc) {
-                const float ri = __builtin_amdgcn_rsqf(d2);
-                const float f = q.w * (ri * ri * ri);
-                px = fmaf(dx, f, px);
-                py = fmaf(dy, f, py);
-                pz = fmaf(dz, f, pz);
-                ++cnt;
-            } else {
-                push = glane == npush ? ((unsigned)(v - n) << 6) | (unsigned)(dep + 1) : push;
-                ++npush;
-                badv |= v - n >= d.cap;
-            }
-        }
-        if (npush) {
-            if (sp + npush > kStack || badv || dep + 1 >= kMaxDepth) {
+
+    if constexpr (K == 1) {
+        __syncthreads();
+        unsigned cur = 0, fields = 15u; // root cell 0 at depth 0, opened by every group
+        int sp = 0;
+        for (;;) {
+            const uint64_t act = G < 64 ? field_lanes(fields) : kAllLanes;
+            float px, py, pz;
+            const int children = visit_cell<G, false>(cur, fields, act, dq_s[cur & 63u], me, eps2, cchild, cdata, px, py, pz, bad,
+                                               [&](unsigned e, unsigned f) {
+                                                   stk[sp] = entry(e, f); // every lane, one address
+                                                   ++sp;
+                                               });
+            sx += (double)px;
+            sy += (double)py;
+            sz += (double)pz;
+            inter += (G < 64 ? (unsigned long long)(unsigned)__popcll(act & vmask) : 1ull) * (unsigned)(children - 1);
+            if (sp == 0) break;
+            --sp;
+            take_entry(stk[sp], cur, fields);
+            if ((cur >> 6) >= cap) { // the pool holds `cap` cells: corrupt
                 bad = true;
-            } else {
-                if (glane < npush) stk[gl][sp + glane] = push;
-                sp += npush;
+                break;
             }
         }
-        kahan_add(sx, kx, px);
-        kahan_add(sy, ky, py);
-        kahan_add(sz, kz, pz);
-        ninter += cnt;
-        if (bad) break;
-    }
-    if (bad && leader) flag_error(ctl, kErrStack);
-    if (valid) finish_body(d, pos, me, sx - kx, sy - ky, sz - kz, mode, step);
-    unsigned long long tot = valid ? (unsigned long long)ninter : 0ull;
+    } else {
+        if (tid == 0) stk[0] = entry(0, 15u); // root cell 0 at depth 0
+        int sp = 1;                           // the same in every wave
+        __syncthreads();
+        for (;;) {
+            const int take = sp > kSplitTop ? 1 : min(sp, K);
+            int npush = 0;
+            unsigned push = 0, pushf = 0; // entry j of this wave's children in lane j
+            if (wv < take) {
+                unsigned cur, fields = 15u;
+                take_entry(stk[sp - 1 - wv], cur, fields);
+                if ((cur >> 6) >= cap) { // the pool holds `cap` cells: corrupt
+                    bad = true;
+                } else {
+                    const uint64_t act = G < 64 ? field_lanes(fields) : kAllLanes;
+                    float px, py, pz;
+                    const int children = visit_cell<G, true>(cur, fields, act, dq_s[cur & 63u], me, eps2, cchild,
+                                                             cdata, px, py, pz, bad, [&](unsigned e, unsigned f) {
+                                                                 push = lane_write(push, e, npush);
+                                                                 if constexpr (G < 64) pushf = lane_write(pushf, f, npush);
+                                                                 ++npush;
+                                                             });
+                    sx += (double)px;
+                    sy += (double)py;
+                    sz += (double)pz;
+                    inter += (G < 64 ? (unsigned long long)(unsigned)__popcll(act & vmask) : 1ull) *
+                             (unsigned)(children - 1);
+                }
+            }
+            if (lane == 0) pushed[wv] = (unsigned)npush | (bad ? kBad : 0u);
+            __syncthreads(); // the entries of this round are read, the counts are in
+            unsigned before = 0, total = 0;
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) tot += __shfl_xor(tot, o);
-    if (lane == 0 && tot) __hip_atomic_fetch_add(&ctl->interactions, tot, __ATOMIC_RELAXED, AGENT);
+            for (int w = 0; w < K; ++w) {
+                const unsigned c = pushed[w];
+                before += w < wv ? c : 0u;
+                total += c;
+            }
+            total = __builtin_amdgcn_readfirstlane(total);
+            bad = total >= kBad || sp - take + (int)total > kCap; // the same in every wave
+            if (bad) break;
+            if (lane < npush) stk[sp - take + (int)before + lane] = entry(push, pushf);
+            sp += (int)total - take;
+            if (sp == 0) break;
+            __syncthreads();
+        }
+        // the waves' sums in wave order
+        __syncthreads();
+        double *red = reinterpret_cast<double *>(lds);
+        red[(wv * 3 + 0) * 64 + lane] = sx;
+        red[(wv * 3 + 1) * 64 + lane] = sy;
+        red[(wv * 3 + 2) * 64 + lane] = sz;
+        if (lane == 0) wint[wv] = inter;
+        __syncthreads();
+        if (wv > 0) return;
+#pragma unroll 1
+        for (int w = 1; w < K; ++w) {
+            sx += red[(w * 3 + 0) * 64 + lane];
+            sy += red[(w * 3 + 1) * 64 + lane];
+            sz += red[(w * 3 + 2) * 64 + lane];
+            inter += wint[w];
+        }
+    }
+    if (bad && lane == 0) flag_error(ctl, kErrStack);
+    if (valid) finish_body(d, pos, me, (float)sx, (float)sy, (float)sz, mode, step);
+    // device interaction counters: one atomic per block
+    if (lane == 0) {
+        const unsigned nv = (unsigned)__popcll(vmask);
+        __hip_atomic_fetch_add(&ctl->tally[blockIdx.x % kTallies].all, G < 64 ? inter + nv : (inter + 1) * nv,
+                               __ATOMIC_RELAXED, AGENT);
+    }
+}
+
+// Waves per group, by the number of groups g. One wave per group leaves the
+// 1,024 SIMDs (8 waves each) short of waves below about 8,192 groups, and a
+// visit is a chain of a stack read and scalar loads; more waves shorten the
+// chain of visits but wait for each other every round (a fifth to a third of
+// the time once the chip is full). us of the force stage, 1 / 4 / 8 / 16 waves:
+//   16,384 bodies (256), ball, theta 0.5, vote 16          307 / 149 / 94 / 71
+//   32,768 bodies (512), disk, theta 1.22, vote 16         110 / 74 / 46 / 36
+//   65,536 bodies (1,024), ball, theta 0.5, vote 64        402 / 189 / 147 / 167
+//   100,003 bodies (1,563), two spheres, theta 0.4, 64     890 / 440 / 431 / 470
+//   131,072 bodies (2,048), Plummer, theta 1.22, vote 16   140 / 98 / 106 / 148
+//   262,144 bodies (4,096), two spheres, theta 0.4, 64     1156 / 913 / 1014 / 1216
+//   524,288 bodies (8,192), two spheres, theta 0.4, 64     1635 / 1740 / 1996 / 2452
+static int waves_per_group(int groups) { return groups <= 640 ? 16 : groups <= 1792 ? 8 : groups <= 5120 ? 4 : 1; }
+
+template <int G> static void launch_force_g(const Dev &d, int mode, hipStream_t st)
+{
+    const int groups = (d.n + 63) / 64;
+    const dim3 grid(groups);
+    const int *cc = d.cchild;
+    const float4 *cd = d.cdata;
+    switch (waves_per_group(groups)) {
+    case 16: hipLaunchKernelGGL((k_force<G, 16>), grid, dim3(1024), 0, st, d, cc, cd, mode); break;
+    case 8: hipLaunchKernelGGL((k_force<G, 8>), grid, dim3(512), 0, st, d, cc, cd, mode); break;
+    case 4: hipLaunchKernelGGL((k_force<G, 4>), grid, dim3(256), 0, st, d, cc, cd, mode); break;
+    default: hipLaunchKernelGGL((k_force<G, 1>), grid, dim3(64), 0, st, d, cc, cd, mode); break;
+    }
 }
 
 hipError_t launch_force(const Dev &d, int vote, int mode, hipStream_t st)
 {
-    const dim3 grid((d.n + kGThreads - 1) / kGThreads), block(kGThreads);
     switch (vote) {
-    case 16: hipLaunchKernelGGL(k_force_g<16>, grid, block, 0, st, d, mode); break;
-    case 32: hipLaunchKernelGGL(k_force_g<32>, grid, block, 0, st, d, mode); break;
-    case 64:
-        hipLaunchKernelGGL(k_force64, dim3((d.n + 64 * kForceWaves - 1) / (64 * kForceWaves)), dim3(64 * kForceWaves),
-                           0, st, d, (const int *)d.cchild, (const float4 *)d.cdata, mode);
-        break;
+    case 16: launch_force_g<16>(d, mode, st); break;
+    case 32: launch_force_g<32>(d, mode, st); break;
+    case 64: launch_force_g<64>(d, mode, st); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();

@@ -10,13 +10,18 @@
 //                                   the cell is published
 //            count : int32[cap]     bodies in the cell's subtree
 //            com64 : double4[cap]   FP64 centre of mass (x, y, z) and mass (w)
-//            cchild: int32[8*cap]   children compacted to the front; cells as
-//                                   N + cell, bodies by index (-1 after the last)
-//            cdata : float4[8*cap]  (x, y, z, m) of those children: body position
-//                                   and mass, or the child cell's FP32 centre of
-//                                   mass and mass -- a popped cell is one
-//                                   contiguous 160-byte read in the traversal;
-//                                   slots past the last child are not written
+//            cchild: int32[8*cap]   a cell's child cells, packed to the front in
+//                                   octant order; above kCountShift word 0
+//                                   holds the number of bodies among the
+//                                   children and word 1 the number of cells
+//            cdata : float4[8*cap]  (x, y, z, m): the child cells' FP32 centres of
+//                                   mass and masses at the front (as cchild),
+//                                   the bodies' positions and masses at the
+//                                   back in reverse octant order -- a visited
+//                                   cell is one contiguous 160-byte read in
+//                                   the traversal, and a child's place says
+//                                   what it is; the places between are not
+//                                   written
 //            cq64  : double[8*cap]  second moments about the centre of mass, learned
 //                                   mode only: traceless Q (xx, yy, zz, xy, xz, yz),
 //                                   trace T, 0
@@ -65,6 +70,7 @@ constexpr int kTailThreads = 512;    // the single block of the deepest summariz
 constexpr unsigned char kNotLive = 0xff; // clvl of a cell that is not in the tree
 constexpr int kCostKeys = 32;        // cost classes of the coarse traversal's launch order
 constexpr uint32_t kEmpty = 0xffffffffu;
+constexpr int kCountShift = 26;      // child counts above the cell numbers in cchild (the pool holds at most 2^26)
 
 enum DevError : int {
     kErrNone = 0,
@@ -72,6 +78,18 @@ enum DevError : int {
     kErrDepth = 2, // tree too deep
     kErrSync = 3,  // inconsistent tree detected
     kErrStack = 4, // traversal stack overflow
+};
+
+// Interaction counters, a cache line each. A traversal block adds its count to
+// one of kTallies (the host sums them): one counter for all blocks made the
+// adds the longest part of short traversals, whose blocks also read the rest
+// of Ctl through the line the counter kept moving (1M bodies at theta 1.22,
+// vote 16: 650 -> 420 us).
+constexpr int kTallies = 32;
+struct Tally {
+    unsigned long long all;   // cumulative body-node interactions
+    unsigned long long cells; // of those, cell interactions of the coarse traversal
+    unsigned long long pad[14];
 };
 
 // Device-resident scalars of one simulation (the reference keeps these in
@@ -87,12 +105,11 @@ struct Ctl {
     float radius;        // reference _radius
     float root[3];
     float dq[kMaxDepth]; // opening thresholds (calculateforce.cl:52-67)
-    unsigned long long interactions; // cumulative body-node interactions
     int levels;          // number of non-empty cell levels of the last tree
     int live_cells;      // cells linked into the tree by the last build
-    unsigned long long cell_interactions; // cumulative cell interactions of the coarse traversal
     int lvl_start[kMaxDepth + 2]; // first lvl_list entry of each level
     int large_buckets;   // buckets of warm builds sorted through device memory, cumulative
+    alignas(128) Tally tally[kTallies]; // interactions by block number modulo kTallies
 };
 
 struct Dev {

@@ -315,6 +315,8 @@ template <int OUT> __device__ __forceinline__ void coarse_traverse(NB_COARSE_PAR
             q[k] = cdp[k];
             if (!kGeo) mc[k] = cmac[(size_t)c * 8 + k];
         }
+        // child cells at the front of the record, bodies at its back
+        const int nbody = (int)((unsigned)ch[0] >> kCountShift), ncellc = (int)((unsigned)ch[1] >> kCountShift);
         // the children's quadrupole records, child k in lanes k, k + 8, ...:
         // two vector loads issued now, waited for at the first accepted cell
         // (which reads them from the wave's LDS), so their latency hides
@@ -326,9 +328,8 @@ template <int OUT> __device__ __forceinline__ void coarse_traverse(NB_COARSE_PAR
             qav = (cqa + (size_t)c * 8)[(unsigned)lane & 7u];
             qbv = (cqb + (size_t)c * 8)[(unsigned)lane & 7u];
         }
-        // First the opening decisions, wave-uniform bit masks of the children
-        // (children are compacted to the front: past the first negative entry
-        // every one is negative). A cell: the opening test of this traversal.
+        // First the opening decisions, a wave-uniform bit mask of the child
+        // cells: the opening test of this traversal.
         // The coarse one takes the extent test first (threshold b^2 /
         // theta_c^2 + eps^2 from summarize) and the relative test (threshold
         // the product of the cell's and the body's factors) only when every
@@ -338,18 +339,14 @@ template <int OUT> __device__ __forceinline__ void coarse_traverse(NB_COARSE_PAR
         // ordered <=). An opened cell's stack entry goes into lane `npush` of
         // `push` (v_writelane: no compare, no branch on the lane); all of them
         // are stored after the loop.
-        unsigned bodies = 0, cells = 0;
+        unsigned cells = 0;
         int npush = 0;
         bool badv = false;
         unsigned push = 0;
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
-            const int v = ch[k];
-            if (v < 0) continue;
-            if (v < n) {
-                bodies |= 1u << k;
-                continue;
-            }
+            if (k >= ncellc) continue;
+            const int v = ch[k] & ((1 << kCountShift) - 1);
             const float dx = q[k].x - me.x, dy = q[k].y - me.y, dz = q[k].z - me.z;
             const float d2 = fmaf(dx, dx, fmaf(dy, dy, fmaf(dz, dz, eps2)));
             const uint64_t exec = __builtin_amdgcn_read_exec();
@@ -358,9 +355,9 @@ template <int OUT> __device__ __forceinline__ void coarse_traverse(NB_COARSE_PAR
             if (take) {
                 cells |= 1u << k;
             } else {
-                push = lane_write(push, ((unsigned)(v - n) << 6) | (unsigned)(dep + 1), npush);
+                push = lane_write(push, ((unsigned)v << 6) | (unsigned)(dep + 1), npush);
                 ++npush;
-                badv |= v - n >= cap;
+                badv |= v >= cap;
             }
         }
         // Then the interactions, each kind in child order, each branch only
@@ -389,8 +386,8 @@ template <int OUT> __device__ __forceinline__ void coarse_traverse(NB_COARSE_PAR
             pqz = qz;
         }
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            if (!((bodies >> k) & 1u)) continue;
+        for (int k = 7; k >= 0; --k) {
+            if (7 - k >= nbody) continue;
             const float4 qk = q[k];
             const float dx = qk.x - me.x, dy = qk.y - me.y, dz = qk.z - me.z;
             const float d2 = fmaf(dx, dx, fmaf(dy, dy, fmaf(dz, dz, eps2)));
@@ -454,7 +451,7 @@ template <int OUT> __device__ __forceinline__ void coarse_traverse(NB_COARSE_PAR
                 pmz = fmaf(dz, h, fmaf(-r5, Qz, pmz));
             }
         }
-        const int nb_here = __popc(bodies), nc_here = __popc(cells);
+        const int nb_here = nbody, nc_here = __popc(cells);
         const int cnt = nb_here + nc_here;
         ncell += nc_here;
         if (kFeatOn) {
@@ -661,13 +658,12 @@ template <int OUT> __device__ __forceinline__ void coarse_traverse(NB_COARSE_PAR
             if (valid) finish_body(d, pos, me, rx, ry, rz, fmode, step);
         }
     }
-    // device interaction counter: one atomic per wave
+    // device interaction counters: one atomic each per wave
     const unsigned long long nvalid = (unsigned long long)__popcll(__ballot(valid));
     if (lane == 0 && ninter && nvalid) {
-        __hip_atomic_fetch_add(&ctl->interactions, (unsigned long long)ninter * nvalid, __ATOMIC_RELAXED,
-                               AGENT);
-        __hip_atomic_fetch_add(&ctl->cell_interactions, (unsigned long long)ncell * nvalid, __ATOMIC_RELAXED,
-                               AGENT);
+        Tally *t = &ctl->tally[blockIdx.x % kTallies];
+        __hip_atomic_fetch_add(&t->all, (unsigned long long)ninter * nvalid, __ATOMIC_RELAXED, AGENT);
+        __hip_atomic_fetch_add(&t->cells, (unsigned long long)ncell * nvalid, __ATOMIC_RELAXED, AGENT);
     }
 }
 

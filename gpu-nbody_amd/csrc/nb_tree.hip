@@ -273,8 +273,9 @@ __global__ __launch_bounds__(256) void k_level_scatter(Dev d)
 // from its children's results of the previous launch, over the eight slots
 // (an empty slot adds 0) in the fixed pairwise order
 // ((s0 + s1) + (s2 + s3)) + ((s4 + s5) + (s6 + s7)), which the xor-shuffle
-// reduction produces identically on every lane. Children are compacted to
-// the front (summarizetree.cl:75-81) into the traversal list.
+// reduction produces identically on every lane. Children are compacted
+// (summarizetree.cl:75-81) into the traversal list: cells to its front,
+// bodies to its back.
 // ---------------------------------------------------------------------------
 // Lane exchanges inside each group of 8 lanes as DPP moves (no LDS):
 // quad_perm [1,0,3,2] = lane ^ 1, quad_perm [2,3,0,1] = lane ^ 2, and
@@ -348,12 +349,14 @@ __device__ __forceinline__ void summarize_cell(const Dev &d, int first, int i, i
             bc = q1.w;
         }
     }
-    // compaction: position of this child among the cell's non-empty slots;
-    // empty slots fill the tail
+    // places: child cells from the front, bodies from the back, the empty
+    // slots between them
     const int gl = (int)(threadIdx.x & 63) & ~7;
-    const unsigned gm = (unsigned)((__ballot(v >= 0) >> gl) & 0xffull);
-    const int used = __popc(gm), below = __popc(gm & ((1u << k) - 1u));
-    const int at = v >= 0 ? below : used + (k - below);
+    const unsigned gc = (unsigned)((__ballot(v >= n) >> gl) & 0xffull);
+    const unsigned gb = (unsigned)((__ballot(v >= 0 && v < n) >> gl) & 0xffull);
+    const unsigned lower = (1u << k) - 1u;
+    const int ncell = __popc(gc), nbody = __popc(gb);
+    const int at = v >= n ? __popc(gc & lower) : v >= 0 ? 7 - __popc(gb & lower) : ncell + __popc(~(gc | gb) & lower);
     const double sm = sum8(m), sx = sum8(m * x), sy = sum8(m * y), sz = sum8(m * z);
     int scnt = cnt;
     scnt += dpp_i<kDppXor1>(scnt);
@@ -363,11 +366,12 @@ __device__ __forceinline__ void summarize_cell(const Dev &d, int first, int i, i
     // reference's 0 * inf = NaN (summarizetree.cl:161-167)
     const double inv = sm > 0.0 ? 1.0 / sm : 0.0;
     const double4 com = make_double4(sx * inv, sy * inv, sz * inv, sm);
-    // the traversals and the sort read a slot's record only up to the first
-    // empty slot: the empty ones keep stale records (a cell has 3 children on
+    // the traversals read the records of the children only: the places
+    // between cells and bodies keep stale ones (a cell has 3 children on
     // average, so this skips well over half of the record writes)
     if (live) {
-        d.cchild[(size_t)c * 8 + at] = v;
+        const int counts = at == 0 ? nbody << kCountShift : at == 1 ? ncell << kCountShift : 0;
+        d.cchild[(size_t)c * 8 + at] = (v >= n ? v - n : 0) | counts;
         if (v >= 0) d.cdata[(size_t)c * 8 + at] = rec;
         if (k == 0) {
             d.com64[c] = com;
