@@ -580,11 +580,8 @@ int train_buffers(Scratch &m, nb::Train &t, int S, int B, int iters)
     int r = NB_OK;
     for (float **f : {&t.P, &t.G, &t.M, &t.V})
         if (!r) r = m.get(f, (size_t)nb::kMlpParams);
-    for (float **f : {&t.Z1, &t.H1, &t.Z2, &t.H2, &t.dZ1, &t.dZ2})
-        if (!r) r = m.get(f, (size_t)B * nb::kHid);
-    if (!r) r = m.get(&t.dY, (size_t)B * nb::kOut);
-    if (!r) r = m.get(&t.gpart, (size_t)nb::kGradChunks * (nb::kHid + 1) * nb::kHid);
-    if (!r) r = m.get(&t.loss_part, (size_t)(B + 255) / 256);
+    if (!r) r = m.get(&t.gpart, (size_t)nb::train_parts(B) * nb::kMlpParams);
+    if (!r) r = m.get(&t.loss_part, (size_t)nb::train_parts(B));
     if (!r) r = m.get(&t.loss_hist, (size_t)std::max(iters, 1));
     t.S = S;
     return r;

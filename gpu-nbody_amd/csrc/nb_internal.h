@@ -223,7 +223,13 @@ constexpr int kW1Frag = 4 * 64 * 8, kW2Frag = 4 * 2 * 64 * 8, kW3Frag = 2 * 64 *
 // both have rare tails of tens of standard deviations (bodies whose coarse
 // acceleration nearly cancels), which would otherwise dominate the squared loss
 constexpr float kClipZ = 8.0f;
-constexpr int kGradChunks = 16; // row chunks of the weight-gradient reduction
+// training: rows of the batch per tile (one block), and the most blocks an iteration runs
+constexpr int kTrainTile = 64, kGradBlocks = 256;
+inline int train_parts(int batch)
+{
+    const int tiles = (batch + kTrainTile - 1) / kTrainTile;
+    return tiles < kGradBlocks ? tiles : kGradBlocks;
+}
 constexpr size_t kMlpBufBytes = (size_t)(kW1Frag + kW2Frag + kW3Frag) * 2 + (64 + 64 + 16 + 24 + 24) * 4;
 
 struct Learn {
@@ -260,9 +266,8 @@ struct Train {
     float *P, *G, *M, *V;  // parameters, gradient, Adam moments (kMlpParams each)
     const float *X, *T;    // dataset: normalized features [S][24], targets [S][3]
     int S;
-    float *Z1, *H1, *Z2, *H2, *dZ1, *dZ2, *dY; // [B][64] (dY [B][3])
-    float *gpart;          // weight-gradient partial sums: kGradChunks x (kHid + 1) x kHid
-    float *loss_part;      // one per 256 rows of the batch
+    float *gpart;          // partial gradients: train_parts(B) x kMlpParams
+    float *loss_part;      // train_parts(B)
     float *loss_hist;      // one per iteration
 };
 // forward + backward of one minibatch (rows drawn with `seed`, or rows 0..B-1

@@ -85,19 +85,6 @@ __device__ __forceinline__ float tanh_fast(float y)
 constexpr float kGeluC = 0.7978845608028654f; // sqrt(2 / pi)
 constexpr float kGeluA = 0.044715f;
 
-__device__ __forceinline__ float gelu(float x)
-{
-    const float t = tanh_fast(kGeluC * (x + kGeluA * x * x * x));
-    return 0.5f * x * (1.0f + t);
-}
-
-__device__ __forceinline__ float gelu_grad(float x)
-{
-    const float x2 = x * x;
-    const float t = tanh_fast(kGeluC * (x + kGeluA * x2 * x));
-    return 0.5f * (1.0f + t) + 0.5f * x * (1.0f - t * t) * kGeluC * (1.0f + 3.0f * kGeluA * x2);
-}
-
 __device__ __forceinline__ float clipz(float z) { return fminf(fmaxf(z, -kClipZ), kClipZ); }
 
 // Inference GELU in the logistic form of the same function,
@@ -938,204 +925,267 @@ __device__ __forceinline__ int batch_row(uint64_t seed, int it, int r, int S)
     return (int)(z % (uint64_t)S);
 }
 
-constexpr int kRowsPerBlock = 16;
+// ---------------------------------------------------------------------------
+// One training iteration: forward, backward and weight gradients of the batch
+// in one kernel, the gradient's sum over the blocks and the Adam step in a
+// second.
+//
+// The products run on the FP32 matrix instruction v_mfma_f32_16x16x4_f32 (FP32
+// operands, products and sums). Operand layout, lane l with m = l % 16 and
+// g = l / 16: A row m, k = g; B column m, k = g; D column m, rows 4 g .. 4 g + 3.
+// The order of k is free as long as A and B agree, so a group of 16 k's is
+// taken as k = 4 g + s in step s = 0 .. 3.
+//
+// A wave takes 16 rows of the batch through the network in the transposed
+// form Z^T = W^T X^T, the rows being the columns: a lane's D registers (four
+// hidden units of one row) are then its B operands of the next layer, forward
+// and backward, and activations never leave the registers. The weights come
+// straight from the parameters (they sit in the caches: every wave reads the
+// same 24 KB). The weight gradients contract over the rows, which are spread
+// over the lanes: activations and their gradients go to LDS once, as [unit][row]
+// with rows of kTrainLd floats (a 16-byte read is conflict-free and holds four
+// steps of an operand), and after a barrier the block's four waves each take a
+// quarter of the gradient's tiles. A block loops over tiles of 64 rows and
+// keeps its gradient in accumulators; there are at most kGradBlocks blocks, so
+// the partial gradients stay within 6 MB. All sums have a fixed order.
+//
+// Bound: latency (a batch of 4,096 rows is 64 blocks; about 300 matrix
+// instructions of 32 cycles per wave). An iteration of 4,096 rows takes 17.6 +
+// 4.8 us; as twelve launches that passed every layer's activations through
+// memory and re-read the batch for each row of weights it took 130 us.
+// ---------------------------------------------------------------------------
+constexpr int kTrainRows = kTrainTile;     // rows per tile: four waves of 16
+constexpr int kTrainLd = kTrainRows + 4;   // LDS row length
+static_assert(kFeat == 24 && kHid == 64 && kOut == 3, "the tiling below");
 
-// Z = X W + b, H = gelu(Z) for 16 rows per block; K inputs (24 or 64), 64 outputs.
-// gather: X rows come from the dataset through batch_row.
-template <int K, bool GATHER>
-__global__ __launch_bounds__(256) void k_fwd_hidden(const float *__restrict__ X, uint64_t seed, int it, int S,
-                                                    const float *__restrict__ W, const float *__restrict__ b,
-                                                    int B, float *__restrict__ Z, float *__restrict__ H)
+__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c)
 {
-    __shared__ float w[K * 64];
-    __shared__ float xin[kRowsPerBlock][K];
-    const int t = threadIdx.x;
-    for (int i = t; i < K * 64; i += 256) w[i] = W[i];
-    const int r0 = blockIdx.x * kRowsPerBlock;
-    for (int i = t; i < kRowsPerBlock * K; i += 256) {
-        const int rl = i / K, k = i % K;
-        const int r = r0 + rl;
-        float v = 0.f;
-        if (r < B) v = GATHER ? X[(size_t)batch_row(seed, it, r, S) * K + k] : X[(size_t)r * K + k];
-        xin[rl][k] = v;
-    }
-    __syncthreads();
-    const int j = t & 63;
-    const float bj = b[j];
-    for (int rl = t >> 6; rl < kRowsPerBlock; rl += 4) {
-        const int r = r0 + rl;
-        if (r >= B) break;
-        float z = bj;
-#pragma unroll 8
-        for (int k = 0; k < K; ++k) z = fmaf(xin[rl][k], w[k * 64 + j], z);
-        Z[(size_t)r * 64 + j] = z;
-        H[(size_t)r * 64 + j] = gelu(z);
-    }
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-// Y = H2 W3 + b3; dY = 2 (Y - T) / (3 B); per-block sum of (Y - T)^2
-__global__ __launch_bounds__(256) void k_fwd_out(const float *__restrict__ H2, const float *__restrict__ W3,
-                                                 const float *__restrict__ b3, const float *__restrict__ T,
-                                                 uint64_t seed, int it, int S, int B, float *__restrict__ dY,
-                                                 float *__restrict__ loss_part)
+// gelu and its derivative from one tanh
+__device__ __forceinline__ float gelu_both(float x, float &grad)
 {
-    __shared__ float w[64 * 3];
-    __shared__ float red[256];
-    const int t = threadIdx.x;
-    if (t < 64 * 3) w[t] = W3[t];
-    __syncthreads();
-    const int r = blockIdx.x * 256 + t;
-    float l = 0.f;
-    if (r < B) {
-        float y0 = b3[0], y1 = b3[1], y2 = b3[2];
-        const float *h = H2 + (size_t)r * 64;
-        for (int k = 0; k < 64; ++k) {
-            const float hk = h[k];
-            y0 = fmaf(hk, w[k * 3 + 0], y0);
-            y1 = fmaf(hk, w[k * 3 + 1], y1);
-            y2 = fmaf(hk, w[k * 3 + 2], y2);
+    const float x2 = x * x;
+    const float t = tanh_fast(kGeluC * (x + kGeluA * x2 * x));
+    grad = 0.5f * (1.0f + t) + 0.5f * x * (1.0f - t * t) * kGeluC * (1.0f + 3.0f * kGeluA * x2);
+    return 0.5f * x * (1.0f + t);
+}
+
+__global__ __launch_bounds__(256) void k_train_grad(const float *__restrict__ P, const float *__restrict__ X,
+                                                    const float *__restrict__ T, uint64_t seed, int it, int S, int B,
+                                                    float *__restrict__ gpart, float *__restrict__ loss_part)
+{
+    __shared__ __attribute__((aligned(16))) float xs[kFeat][kTrainLd], h1s[kHid][kTrainLd], d1s[kHid][kTrainLd];
+    __shared__ __attribute__((aligned(16))) float h2s[kHid][kTrainLd], d2s[kHid][kTrainLd], dys[kOut][kTrainLd];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int m = lane & 15, g = lane >> 4;
+    const float *W1 = P, *b1 = P + kOffB1, *W2 = P + kOffW2, *b2 = P + kOffB2, *W3 = P + kOffW3, *b3 = P + kOffB3;
+    const f32x4 z4 = {0.f, 0.f, 0.f, 0.f};
+    // this wave's gradient tiles: dW2 rows 16 w .., all columns; dW1 all rows
+    // (two tiles of 16, the second half empty), columns 16 w ..; dW3 rows 16 w ..;
+    // the biases' columns 16 w .. (b3: wave 0)
+    f32x4 gw2[4] = {z4, z4, z4, z4}, gw1[2] = {z4, z4}, gw3 = z4;
+    float gb1 = 0.f, gb2 = 0.f, gb3 = 0.f, loss = 0.f;
+    const float sc = 2.0f / (3.0f * (float)B);
+    const int ntiles = (B + kTrainRows - 1) / kTrainRows;
+    for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+        const int rl = 16 * w + m, r = tile * kTrainRows + rl; // this lane's row (column of the products)
+        const bool in = r < B;
+        const size_t row = in ? (size_t)batch_row(seed, it, r, S) : 0;
+        f32x4 x0 = z4, x1 = z4; // features 4 g .., and 16 + 4 g .. (g < 2)
+        if (in) {
+            x0 = *reinterpret_cast<const f32x4 *>(X + row * kFeat + 4 * g);
+            if (g < 2) x1 = *reinterpret_cast<const f32x4 *>(X + row * kFeat + 16 + 4 * g);
         }
-        const float *tt = T + (size_t)batch_row(seed, it, r, S) * 3;
-        const float e0 = y0 - tt[0], e1 = y1 - tt[1], e2 = y2 - tt[2];
-        const float sc = 2.0f / (3.0f * (float)B);
-        dY[(size_t)r * 3 + 0] = sc * e0;
-        dY[(size_t)r * 3 + 1] = sc * e1;
-        dY[(size_t)r * 3 + 2] = sc * e2;
-        l = e0 * e0 + e1 * e1 + e2 * e2;
-    }
-    red[t] = l;
-    __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if (t < o) red[t] += red[t + o];
+        float t0 = 0.f, t1 = 0.f, t2 = 0.f;
+        if (in && g == 0) {
+            t0 = T[row * kOut];
+            t1 = T[row * kOut + 1];
+            t2 = T[row * kOut + 2];
+        }
+        f32x4 h1[4], p1[4], h2[4], p2[4]; // activations and their derivatives, units 16 t + 4 g + v
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            f32x4 z = *reinterpret_cast<const f32x4 *>(b1 + 16 * t + 4 * g);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) z = mfma4(W1[(4 * g + q) * kHid + 16 * t + m], x0[q], z);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) z = mfma4(g < 2 ? W1[(16 + 4 * g + q) * kHid + 16 * t + m] : 0.f, x1[q], z);
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                float d;
+                h1[t][v] = gelu_both(z[v], d);
+                p1[t][v] = d;
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            f32x4 z = *reinterpret_cast<const f32x4 *>(b2 + 16 * t + 4 * g);
+#pragma unroll
+            for (int rb = 0; rb < 4; ++rb)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) z = mfma4(W2[(16 * rb + 4 * g + q) * kHid + 16 * t + m], h1[rb][q], z);
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                float d;
+                h2[t][v] = gelu_both(z[v], d);
+                p2[t][v] = d;
+            }
+        }
+        // outputs 0 .. 2 of row r in lane m (g = 0)
+        f32x4 y = z4;
+        if (g == 0) y = f32x4{b3[0], b3[1], b3[2], 0.f};
+#pragma unroll
+        for (int rb = 0; rb < 4; ++rb)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) y = mfma4(m < kOut ? W3[(16 * rb + 4 * g + q) * kOut + m] : 0.f, h2[rb][q], y);
+        float e0 = 0.f, e1 = 0.f, e2 = 0.f;
+        if (in && g == 0) {
+            e0 = y[0] - t0;
+            e1 = y[1] - t1;
+            e2 = y[2] - t2;
+            loss += e0 * e0 + e1 * e1 + e2 * e2;
+        }
+        e0 *= sc;
+        e1 *= sc;
+        e2 *= sc;
+        // output g's gradient of row r in lane (m, g)
+        const float s0 = __shfl(e0, m), s1 = __shfl(e1, m), s2 = __shfl(e2, m);
+        const float dy = g == 0 ? s0 : g == 1 ? s1 : g == 2 ? s2 : 0.f;
+        f32x4 d2[4], d1[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) d2[t] = mfma4(g < kOut ? W3[(16 * t + m) * kOut + g] : 0.f, dy, z4) * p2[t];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            f32x4 z = z4;
+#pragma unroll
+            for (int rb = 0; rb < 4; ++rb) {
+                const f32x4 a = *reinterpret_cast<const f32x4 *>(W2 + (16 * t + m) * kHid + 16 * rb + 4 * g);
+#pragma unroll
+                for (int q = 0; q < 4; ++q) z = mfma4(a[q], d2[rb][q], z);
+            }
+            d1[t] = z * p1[t];
+        }
+        __syncthreads(); // the last tile's gradients have been read
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            xs[4 * g + v][rl] = x0[v];
+            if (g < 2) xs[16 + 4 * g + v][rl] = x1[v];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                h1s[16 * t + 4 * g + v][rl] = h1[t][v];
+                d1s[16 * t + 4 * g + v][rl] = d1[t][v];
+                h2s[16 * t + 4 * g + v][rl] = h2[t][v];
+                d2s[16 * t + 4 * g + v][rl] = d2[t][v];
+            }
+        }
+        if (g < kOut) dys[g][rl] = dy;
         __syncthreads();
+#pragma unroll
+        for (int c = 0; c < kTrainRows / 16; ++c) {
+            const int k0 = 16 * c + 4 * g; // this lane's rows of the chunk
+            auto frag = [&](float (*u)[kTrainLd], int unit) { return *reinterpret_cast<const f32x4 *>(&u[unit][k0]); };
+            const f32x4 a2 = frag(h1s, 16 * w + m), a3 = frag(h2s, 16 * w + m);
+            const f32x4 a1 = frag(xs, m), a1b = m < 8 ? frag(xs, 16 + (m & 7)) : z4;
+            const f32x4 c1 = frag(d1s, 16 * w + m), c3 = m < kOut ? frag(dys, m < kOut ? m : 0) : z4;
+            gb1 += (c1[0] + c1[1]) + (c1[2] + c1[3]);
+            gb3 += (c3[0] + c3[1]) + (c3[2] + c3[3]);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const f32x4 c2 = frag(d2s, 16 * t + m);
+                if (t == w) gb2 += (c2[0] + c2[1]) + (c2[2] + c2[3]);
+#pragma unroll
+                for (int q = 0; q < 4; ++q) gw2[t] = mfma4(a2[q], c2[q], gw2[t]);
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                gw1[0] = mfma4(a1[q], c1[q], gw1[0]);
+                gw1[1] = mfma4(a1b[q], c1[q], gw1[1]);
+                gw3 = mfma4(a3[q], c3[q], gw3);
+            }
+        }
     }
-    if (t == 0) loss_part[blockIdx.x] = red[0];
-}
-
-// dZ = (dNext W^T) * gelu'(Z): W is [64][N] (N = 3 or 64); 16 rows per block
-template <int N>
-__global__ __launch_bounds__(256) void k_back_hidden(const float *__restrict__ dNext, const float *__restrict__ W,
-                                                     const float *__restrict__ Z, int B, float *__restrict__ dZ)
-{
-    __shared__ float wt[N][65]; // wt[j][k] = W[k][j], padded
-    __shared__ float dn[kRowsPerBlock][N];
-    const int t = threadIdx.x;
-    for (int i = t; i < 64 * N; i += 256) {
-        const int k = i / N, j = i % N;
-        wt[j][k] = W[i];
+    float *o = gpart + (size_t)blockIdx.x * kMlpParams;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        const int i = 4 * g + v;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) o[kOffW2 + (16 * w + i) * kHid + 16 * t + m] = gw2[t][v];
+        o[i * kHid + 16 * w + m] = gw1[0][v];
+        if (i < 8) o[(16 + i) * kHid + 16 * w + m] = gw1[1][v];
+        if (m < kOut) o[kOffW3 + (16 * w + i) * kOut + m] = gw3[v];
     }
-    const int r0 = blockIdx.x * kRowsPerBlock;
-    for (int i = t; i < kRowsPerBlock * N; i += 256) {
-        const int rl = i / N, j = i % N;
-        const int r = r0 + rl;
-        dn[rl][j] = r < B ? dNext[(size_t)r * N + j] : 0.f;
+    // the biases: the four lanes of a column hold a quarter of the rows each
+    auto over_g = [](float v) {
+        v += __shfl_xor(v, 16);
+        return v + __shfl_xor(v, 32);
+    };
+    gb1 = over_g(gb1);
+    gb2 = over_g(gb2);
+    gb3 = over_g(gb3);
+    if (g == 0) {
+        o[kOffB1 + 16 * w + m] = gb1;
+        o[kOffB2 + 16 * w + m] = gb2;
+        if (w == 0 && m < kOut) o[kOffB3 + m] = gb3;
     }
+#pragma unroll
+    for (int k = 1; k < 16; k <<= 1) loss += __shfl_xor(loss, k);
     __syncthreads();
-    const int k = t & 63;
-    for (int rl = t >> 6; rl < kRowsPerBlock; rl += 4) {
-        const int r = r0 + rl;
-        if (r >= B) break;
-        float s = 0.f;
-#pragma unroll 8
-        for (int j = 0; j < N; ++j) s = fmaf(dn[rl][j], wt[j][k], s);
-        dZ[(size_t)r * 64 + k] = s * gelu_grad(Z[(size_t)r * 64 + k]);
-    }
+    if (lane == 0) xs[0][w] = loss;
+    __syncthreads();
+    if (threadIdx.x == 0) loss_part[blockIdx.x] = (xs[0][0] + xs[0][1]) + (xs[0][2] + xs[0][3]);
 }
 
-// Partial weight gradients: block (k, ch) sums rows [ch B / C, (ch + 1) B / C)
-// of A[r][k] dZ[r][j] (k < K), or of dZ[r][j] for the bias (k = K); each
-// thread takes every 4th row and the 4 partial sums are added in a fixed
-// order. k_wgrad_reduce then adds the C chunks in order: deterministic.
-template <bool GATHER>
-__global__ __launch_bounds__(256) void k_wgrad(const float *__restrict__ A, int lda, uint64_t seed, int it, int S,
-                                               const float *__restrict__ dZ, int N, int B, int K,
-                                               float *__restrict__ part)
+// The gradient: the blocks' partial gradients added in order (four threads per
+// parameter, a quarter of the blocks each), then the Adam step. Block 0 also
+// adds the loss.
+__global__ __launch_bounds__(256) void k_train_adam(float *__restrict__ P, float *__restrict__ G,
+                                                    float *__restrict__ M, float *__restrict__ V,
+                                                    const float *__restrict__ gpart, int nparts, float lr, float b1,
+                                                    float b2, float eps, float c1, float c2,
+                                                    const float *__restrict__ loss_part, int B,
+                                                    float *__restrict__ loss_out, bool step)
 {
     __shared__ float red[4][64];
-    const int t = threadIdx.x;
-    const int j = t & 63, rq = t >> 6;
-    const int k = blockIdx.x, ch = blockIdx.y;
-    const int r0 = (int)((long long)B * ch / kGradChunks), r1 = (int)((long long)B * (ch + 1) / kGradChunks);
-    float acc = 0.f;
-    if (j < N) {
-        for (int r = r0 + rq; r < r1; r += 4) {
-            float a = 1.0f;
-            if (k < K) a = GATHER ? A[(size_t)batch_row(seed, it, r, S) * lda + k] : A[(size_t)r * lda + k];
-            acc = fmaf(a, dZ[(size_t)r * N + j], acc);
-        }
-    }
-    red[rq][j] = acc;
-    __syncthreads();
-    if (rq == 0 && j < N)
-        part[((size_t)ch * (K + 1) + k) * N + j] = ((red[0][j] + red[1][j]) + red[2][j]) + red[3][j];
-}
-
-__global__ void k_wgrad_reduce(const float *__restrict__ part, int K, int N, float *__restrict__ gW,
-                               float *__restrict__ gb)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (K + 1) * N) return;
+    const int j = threadIdx.x & 63, q = threadIdx.x >> 6;
+    const int i = blockIdx.x * 64 + j;
     float v = 0.f;
-    for (int ch = 0; ch < kGradChunks; ++ch) v += part[(size_t)ch * (K + 1) * N + i];
-    const int k = i / N, j = i % N;
-    if (k < K)
-        gW[k * N + j] = v;
-    else
-        gb[j] = v;
-}
-
-__global__ void k_adam(float *__restrict__ P, const float *__restrict__ G, float *__restrict__ M,
-                       float *__restrict__ V, int np, float lr, float b1, float b2, float eps, float c1, float c2,
-                       const float *__restrict__ loss_part, int nparts, int B, float *__restrict__ loss_out,
-                       bool step)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i == 0) {
-        float s = 0.f;
-        for (int p = 0; p < nparts; ++p) s += loss_part[p];
-        *loss_out = s / (3.0f * (float)B);
+    if (i < kMlpParams) {
+        const int k0 = nparts * q / 4, k1 = nparts * (q + 1) / 4;
+#pragma unroll 8
+        for (int k = k0; k < k1; ++k) v += gpart[(size_t)k * kMlpParams + i];
     }
-    if (!step || i >= np) return;
-    const float g = G[i];
-    const float m = b1 * M[i] + (1.0f - b1) * g;
-    const float v = b2 * V[i] + (1.0f - b2) * g * g;
-    M[i] = m;
-    V[i] = v;
-    P[i] -= lr * (m * c1) / (sqrtf(v * c2) + eps);
+    red[q][j] = v;
+    if (blockIdx.x == 0 && q == 3) {
+        // lane j the parts j, j + 64, ..., then the lanes in order of a tree
+        float s = 0.f;
+        for (int k = j; k < nparts; k += 64) s += loss_part[k];
+#pragma unroll
+        for (int k = 1; k < 64; k <<= 1) s += __shfl_xor(s, k);
+        if (j == 0) *loss_out = s / (3.0f * (float)B);
+    }
+    __syncthreads();
+    if (q != 0 || i >= kMlpParams) return;
+    const float grad = (red[0][j] + red[1][j]) + (red[2][j] + red[3][j]);
+    G[i] = grad;
+    if (!step) return;
+    const float mm = b1 * M[i] + (1.0f - b1) * grad;
+    const float vv = b2 * V[i] + (1.0f - b2) * grad * grad;
+    M[i] = mm;
+    V[i] = vv;
+    P[i] -= lr * (mm * c1) / (sqrtf(vv * c2) + eps);
 }
 
 hipError_t launch_train_iter(const Train &t, int B, int it, uint64_t seed, bool adam, float lr, float beta1,
                              float beta2, float eps, float c1, float c2, hipStream_t st)
 {
     if (B <= 0) return hipErrorInvalidValue;
-    const dim3 blk(256);
-    const dim3 gh((B + kRowsPerBlock - 1) / kRowsPerBlock);
-    const int nparts = (B + 255) / 256;
-    const float *P = t.P;
-    float *G = t.G;
-    hipLaunchKernelGGL((k_fwd_hidden<kFeat, true>), gh, blk, 0, st, t.X, seed, it, t.S, P, P + kOffB1, B, t.Z1, t.H1);
-    hipLaunchKernelGGL((k_fwd_hidden<kHid, false>), gh, blk, 0, st, (const float *)t.H1, seed, it, t.S,
-                       P + kOffW2, P + kOffB2, B, t.Z2, t.H2);
-    hipLaunchKernelGGL(k_fwd_out, dim3(nparts), blk, 0, st, (const float *)t.H2, P + kOffW3, P + kOffB3, t.T, seed,
-                       it, t.S, B, t.dY, t.loss_part);
-    hipLaunchKernelGGL(k_back_hidden<kOut>, gh, blk, 0, st, (const float *)t.dY, P + kOffW3,
-                       (const float *)t.Z2, B, t.dZ2);
-    hipLaunchKernelGGL(k_wgrad<false>, dim3(kHid + 1, kGradChunks), blk, 0, st, (const float *)t.H2, kHid, seed, it,
-                       t.S, (const float *)t.dY, kOut, B, kHid, t.gpart);
-    hipLaunchKernelGGL(k_wgrad_reduce, dim3(((kHid + 1) * kOut + 255) / 256), blk, 0, st, (const float *)t.gpart,
-                       kHid, kOut, G + kOffW3, G + kOffB3);
-    hipLaunchKernelGGL(k_back_hidden<kHid>, gh, blk, 0, st, (const float *)t.dZ2, P + kOffW2,
-                       (const float *)t.Z1, B, t.dZ1);
-    hipLaunchKernelGGL(k_wgrad<false>, dim3(kHid + 1, kGradChunks), blk, 0, st, (const float *)t.H1, kHid, seed, it,
-                       t.S, (const float *)t.dZ2, kHid, B, kHid, t.gpart);
-    hipLaunchKernelGGL(k_wgrad_reduce, dim3(((kHid + 1) * kHid + 255) / 256), blk, 0, st, (const float *)t.gpart,
-                       kHid, kHid, G + kOffW2, G + kOffB2);
-    hipLaunchKernelGGL(k_wgrad<true>, dim3(kFeat + 1, kGradChunks), blk, 0, st, t.X, kFeat, seed, it, t.S,
-                       (const float *)t.dZ1, kHid, B, kFeat, t.gpart);
-    hipLaunchKernelGGL(k_wgrad_reduce, dim3(((kFeat + 1) * kHid + 255) / 256), blk, 0, st, (const float *)t.gpart,
-                       kFeat, kHid, G, G + kOffB1);
-    hipLaunchKernelGGL(k_adam, dim3((kMlpParams + 255) / 256), blk, 0, st, t.P, (const float *)G, t.M, t.V,
-                       kMlpParams, lr, beta1, beta2, eps, c1, c2, (const float *)t.loss_part, nparts, B,
+    const int nparts = train_parts(B);
+    hipLaunchKernelGGL(k_train_grad, dim3(nparts), dim3(256), 0, st, (const float *)t.P, t.X, t.T, seed, it, t.S, B,
+                       t.gpart, t.loss_part);
+    hipLaunchKernelGGL(k_train_adam, dim3((kMlpParams + 63) / 64), dim3(256), 0, st, t.P, t.G, t.M, t.V,
+                       (const float *)t.gpart, nparts, lr, beta1, beta2, eps, c1, c2, (const float *)t.loss_part, B,
                        t.loss_hist + it, adam);
     return hipGetLastError();
 }
