@@ -9,6 +9,20 @@ namespace nb {
 
 constexpr float kFar = __builtin_huge_valf();
 constexpr int kStack = 512; // >= 7 * 64 + 8 entries: the deepest possible push pattern
+constexpr uint64_t kAllLanes = ~0ull;
+
+// Entries of the stack of K waves that share a vote group. One wave (K = 1)
+// walks depth first: at most 7 siblings wait per level. K waves take the K
+// top entries together; the limit kSplitTop above which they take one entry at
+// a time (depth first from there, again at most 7 per level) bounds the stack
+// for every tree of kMaxDepth levels: kSplitTop + the children of one round +
+// 7 per level.
+constexpr int kSplitTop = 512;
+template <int K> constexpr int split_stack() { return K == 1 ? kStack : kSplitTop + 8 * K + kStack; }
+constexpr unsigned kSplitBad = 1u << 16; // a wave's report of a corrupt tree, above its push count
+
+typedef int i32x8 __attribute__((ext_vector_type(8)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 // v_writelane_b32: `old` with lane `lane` (wave-uniform) set to the
 // wave-uniform value v; one instruction (LLVM's amdgcn.writelane intrinsic,
@@ -20,11 +34,31 @@ __device__ __forceinline__ unsigned lane_write(unsigned old, unsigned v, int lan
     return (unsigned)amdgcn_writelane_i32((int)v, lane, (int)old);
 }
 
-// The opening vote of a wave: true when every active lane's predicate holds.
-// The compare result goes straight into the lane mask (no bool round trip).
-__device__ __forceinline__ bool wave_all(bool pred)
+// End of a round of K waves that took `take` entries off the top of the shared
+// stack of sp entries, this wave having opened npush cells (entry j in lane j
+// of `push`): after the barrier every wave knows the others' counts, the new
+// entries go behind those of the lower waves, and sp becomes the new count.
+// False when the tree is corrupt (some wave says so, or the stack would
+// overflow). Every wave of the block calls it; `pushed` holds K words.
+template <int K, class Entry>
+__device__ __forceinline__ bool end_round(Entry *stk, unsigned *pushed, int wv, int lane, int take, int npush, Entry push,
+                                          bool bad, int &sp)
 {
-    return __builtin_amdgcn_ballot_w64(pred) == __builtin_amdgcn_read_exec();
+    if (lane == 0) pushed[wv] = (unsigned)npush | (bad ? kSplitBad : 0u);
+    __syncthreads(); // the entries of this round are read, the counts are in
+    unsigned before = 0, total = 0;
+#pragma unroll
+    for (int w = 0; w < K; ++w) {
+        const unsigned c = pushed[w];
+        before += w < wv ? c : 0u;
+        total += c;
+    }
+    total = __builtin_amdgcn_readfirstlane(total);
+    if (total >= kSplitBad || sp - take + (int)total > split_stack<K>()) return false; // the same in every wave
+    if (lane < npush) stk[sp - take + (int)before + lane] = push;
+    sp += (int)total - take;
+    if (sp) __syncthreads();
+    return true;
 }
 
 __device__ __forceinline__ void kahan_add(float &sum, float &comp, float x)

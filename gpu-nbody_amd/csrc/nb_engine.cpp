@@ -65,6 +65,7 @@ struct nb_sim {
     // priority) beside the step's tree stages and traversal
     hipStream_t side = nullptr;
     hipEvent_t chk_go = nullptr; // the step's positions are final (recorded on stream)
+    hipEvent_t pair_ev[2] = {nullptr, nullptr}; // a training step's pairs: records copied, pairs done
     int32_t *chk_host = nullptr; // pinned sample indices, so the upload never blocks the host
     int chk_host_cap = 0, chk_ns = 0;
     // the coarse traversal's group order for the next pass is worked out on a
@@ -274,8 +275,7 @@ int launch_coarse_ordered(nb_sim *s, int out, int fmode)
         HIP_TRY(s, hipStreamWaitEvent(s->stream, s->ord_out, 0));
     else
         HIP_TRY(s, nb::launch_group_order(d, s->stream));
-    HIP_TRY(s, nb::launch_coarse(d, s->L, out, nullptr, d.gorder, (d.n + 63) / 64, nullptr, nullptr, nullptr, fmode,
-                                 s->stream));
+    HIP_TRY(s, nb::launch_coarse(d, s->L, out, d.gorder, (d.n + 63) / 64, nullptr, nullptr, fmode, s->stream));
     HIP_TRY(s, hipEventRecord(s->ord_in, s->stream));
     HIP_TRY(s, hipStreamWaitEvent(s->ord, s->ord_in, 0));
     HIP_TRY(s, nb::launch_group_order(d, s->ord));
@@ -519,6 +519,8 @@ void free_all(nb_sim *s)
     for (auto &e : s->chk_ev)
         if (e) (void)hipEventDestroy(e);
     if (s->chk_go) (void)hipEventDestroy(s->chk_go);
+    for (auto &e : s->pair_ev)
+        if (e) (void)hipEventDestroy(e);
     if (s->chk_host) (void)hipHostFree(s->chk_host);
     if (s->side) (void)hipStreamDestroy(s->side);
     if (s->ord_in) (void)hipEventDestroy(s->ord_in);
@@ -561,7 +563,7 @@ struct Scratch {
     explicit Scratch(nb_sim *sim) : s(sim) {}
     ~Scratch()
     {
-        (void)hipStreamSynchronize(s->stream);
+        drain(s); // the training pairs' stream too, when a launch failed halfway
         for (void *p : ptrs) (void)hipFree(p);
     }
     template <class T> int get(T **p, size_t count)
@@ -760,6 +762,7 @@ int nb_create(const nb_params *p, nb_sim **out)
     }
     d.fp64 = (p->flags & NB_FP64_POSITIONS) ? 1 : 0;
     d.quad = p->mode != NB_MODE_PLAIN ? 1 : 0;
+    d.narrow = p->vote_width < 64 ? 1 : 0;
     const size_t cap = (size_t)d.cap;
     bool ok = dalloc(&d.ctl, 1) == hipSuccess;
     for (float4 **f : {&d.pm4, &d.vel4, &d.acc4}) ok = ok && dalloc(f, (size_t)n) == hipSuccess;
@@ -1315,13 +1318,14 @@ int nb_train(nb_sim *s, const nb_train_params *tp_in, nb_train_report *rep)
     Scratch m(s);
     nb::Train t{};
     float *X = nullptr, *T = nullptr, *stats = nullptr;
-    float4 *frame = nullptr, *afine = nullptr;
+    float4 *frame = nullptr, *afine = nullptr, *rec = nullptr;
     int *gdev = nullptr;
     r = train_buffers(m, t, S, B, tp.iters);
     if (!r) r = m.get(&X, (size_t)S * nb::kFeat);
     if (!r) r = m.get(&T, (size_t)S * nb::kOut);
     if (!r) r = m.get(&stats, (size_t)2 * (nb::kFeat + nb::kOut));
     if (!r) r = m.get(&frame, (size_t)2 * rows);
+    if (!r) r = m.get(&rec, (size_t)2 * rows);
     if (!r) r = m.get(&afine, (size_t)rows);
     if (!r) r = m.get(&gdev, (size_t)G * tp.steps);
     if (r) return r;
@@ -1339,6 +1343,10 @@ int nb_train(nb_sim *s, const nb_train_params *tp_in, nb_train_report *rep)
     }
     r = upload(s, gdev, groups.data(), groups.size() * sizeof(int));
     if (r) return r;
+    if (!s->side) HIP_TRY(s, hipStreamCreateWithFlags(&s->side, hipStreamNonBlocking));
+    for (auto &ev : s->pair_ev)
+        if (!ev) HIP_TRY(s, hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+    const hipEvent_t pairs_in = s->pair_ev[0], pairs_out = s->pair_ev[1];
 
     const auto t0 = std::chrono::steady_clock::now();
     const int fused = (s->p.flags & NB_FUSED_UPDATE) ? 1 : 0;
@@ -1347,17 +1355,24 @@ int nb_train(nb_sim *s, const nb_train_params *tp_in, nb_train_report *rep)
             r = launch_stage(s, st);
             if (r) return r;
         }
-        hipError_t e = nb::launch_coarse(d, s->L, nb::kOutRaw, nullptr, gdev + (size_t)k * G, G,
-                                         X + (size_t)k * rows * nb::kFeat, frame, nullptr, 0, s->stream);
+        // the pairs of this step's tree on the second stream, on copies of the
+        // bodies' records, beside the force pass that advances the bodies;
+        // the next step rebuilds the tree only when they are done
+        hipError_t e = nb::launch_pair_records(d, gdev + (size_t)k * G, G, rec, s->stream);
+        if (e == hipSuccess) e = hipEventRecord(pairs_in, s->stream);
+        if (e == hipSuccess) e = hipStreamWaitEvent(s->side, pairs_in, 0);
         if (e == hipSuccess)
-            e = nb::launch_coarse(d, s->L, nb::kOutAccel, dq_plain_ptr(s), gdev + (size_t)k * G, G, nullptr,
-                                  nullptr, afine, 0, s->stream);
-        if (e == hipSuccess) e = nb::launch_make_target(frame, afine, rows, T + (size_t)k * rows * nb::kOut, s->stream);
+            e = nb::launch_pairs(d, s->L, dq_plain_ptr(s), gdev + (size_t)k * G, G, rec,
+                                 X + (size_t)k * rows * nb::kFeat, frame, afine, s->side);
+        if (e == hipSuccess)
+            e = nb::launch_make_target(frame, afine, rows, T + (size_t)k * rows * nb::kOut, s->side);
+        if (e == hipSuccess) e = hipEventRecord(pairs_out, s->side);
         if (e != hipSuccess) return fail(s, NB_E_HIP, "training pair launch: %s", hipGetErrorString(e));
         // the bodies advance with plain theta
         r = launch_force_method(s, NB_MODE_PLAIN, fused);
         if (!r) r = launch_stage(s, NB_STAGE_INTEGRATE);
         if (r) return r;
+        HIP_TRY(s, hipStreamWaitEvent(s->stream, pairs_out, 0));
     }
     r = check_device_error(s);
     if (r) return r;
@@ -1446,7 +1461,7 @@ int nb_coarse_features(nb_sim *s, float *feat, float *acc3, float *e2)
         r = launch_stage(s, st);
         if (r) return r;
     }
-    hipError_t e = nb::launch_coarse(d, s->L, nb::kOutRaw, nullptr, nullptr, 0, xr, fr, nullptr, 0, s->stream);
+    hipError_t e = nb::launch_coarse(d, s->L, nb::kOutRaw, nullptr, 0, xr, fr, 0, s->stream);
     if (e != hipSuccess) return fail(s, NB_E_HIP, "coarse launch: %s", hipGetErrorString(e));
     HIP_TRY(s, hipMemcpyAsync(&d.ctl->step, &c0.step, sizeof(int), hipMemcpyHostToDevice, s->stream));
     r = check_device_error(s);

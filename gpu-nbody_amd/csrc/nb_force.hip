@@ -22,8 +22,8 @@
 // is opened when some lane of some group that reached it rejects it. With a
 // stack per 16-lane group the four groups of a wave were at different cells,
 // each child came through vector loads, and three quarters of the lanes idled
-// in most of the branches: 25.5 -> 8.4 ms at 4M clustered bodies (theta 0.4,
-// vote 16), 6.03 -> 2.38 ms at 1M Plummer bodies (theta 0.5, vote 16).
+// in most of the branches: 25.5 -> 10.0 ms at 4M clustered bodies (theta 0.4,
+// vote 16), 6.03 -> 2.76 ms at 1M Plummer bodies (theta 0.5, vote 16).
 //
 // Bound: vector issue. Of the 14 issue slots of a term (3 sub, 3 fma, rsq =
 // 2, 3 mul, 3 fma), 3,690 terms per body at 1M Plummer bodies (theta 0.5,
@@ -33,12 +33,11 @@
 // Accumulation: the terms of one visited cell (<= 8) are summed in FP32 and
 // added into FP64 sums. An FP64 add issues at the rate of an FP32 add here, so
 // convert and add (6 instructions per cell) cost half of a compensated FP32
-// sum (12) and keep more bits.
+// sum (12) and keep more bits. A wave that walks narrow groups alone keeps the
+// compensated sums (see waves_per_group).
 #include "nb_device.h"
 
 namespace nb {
-
-constexpr uint64_t kAllLanes = ~0ull;
 
 // Groups as bits: bit f stands for the 16 lanes of field f, and a vote group of
 // 32 or 64 lanes is two or four fields. group_bits: the groups in which a lane
@@ -67,9 +66,6 @@ __device__ __forceinline__ uint64_t field_lanes(unsigned f)
     return x;
 }
 
-typedef int i32x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-
 // the softened monopole term of mass m at (dx, dy, dz), d2 = |d|^2 + eps^2
 __device__ __forceinline__ void add_term(float dx, float dy, float dz, float d2, float m, float &px, float &py,
                                          float &pz)
@@ -81,20 +77,18 @@ __device__ __forceinline__ void add_term(float dx, float dy, float dz, float d2,
     pz = fmaf(dz, f, pz);
 }
 
-// One visit: the children of cell `e >> 6` (on level e & 63) against the
-// wave's bodies. act: the lanes whose groups opened the cell. The terms'
-// sum goes to (px, py, pz), the number of children is returned;
-// opened(entry, lanes) is called for every child that some group opens. Every
-// branch is wave-uniform. Child cells sit at the front of the cell's record and
-// bodies at its back, and their counts in the first two index words
-// (nb_internal.h): a body costs a compare and a branch on the scalar side, a
-// cell two more for its vote. The scalar unit issues one instruction per SIMD
-// and four cycles like the vector one, and with a test of each child's kind
-// it was the busier of the two (72k scalar against 64k vector instructions
-// per wave at 1M Plummer bodies, theta 0.5).
-template <int G, bool SPLIT, class Opened>
-__device__ __forceinline__ int visit_cell(unsigned e, unsigned fields, uint64_t act, float thr, float4 me,
-                                          float eps2, const int *__restrict__ cchild,
+// One visit at vote width 64: the children of cell `e >> 6` (on level e & 63)
+// against the wave's bodies. The terms' sum goes to (px, py, pz), the number of
+// children is returned; opened(entry) is called for every child that is
+// opened. Every branch is wave-uniform. Child cells sit at the front of the
+// cell's record and bodies at its back, and their counts in the first two index
+// words (nb_internal.h): a body costs a compare and a branch on the scalar
+// side, a cell two more for its vote. The scalar unit issues one instruction
+// per SIMD and four cycles like the vector one, and with a test of each child's
+// kind it is the busier of the two: 1.92 against 2.65 ms at 1M Plummer bodies,
+// theta 0.5.
+template <bool SPLIT, class Opened>
+__device__ __forceinline__ int visit_wide(unsigned e, float thr, float4 me, float eps2, const int *__restrict__ cchild,
                                           const float4 *__restrict__ cdata, float &px, float &py, float &pz,
                                           bool &bad, Opened &&opened)
 {
@@ -113,52 +107,86 @@ __device__ __forceinline__ int visit_cell(unsigned e, unsigned fields, uint64_t 
         bad = true;
         ncell = 0;
     }
-    float e2 = eps2;
-    if constexpr (G < 64) e2 = __builtin_amdgcn_inverse_ballot_w64(act) ? eps2 : kFar;
     px = py = pz = 0.f;
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
         if (k >= ncell) break;
         const f32x16 &q = k < 4 ? q0 : q1;
         const float dx = q[4 * (k & 3)] - me.x, dy = q[4 * (k & 3) + 1] - me.y, dz = q[4 * (k & 3) + 2] - me.z;
-        const float d2 = fmaf(dx, dx, fmaf(dy, dy, fmaf(dz, dz, e2)));
-        const uint64_t r = act & ~__builtin_amdgcn_fcmpf(d2, thr, 3); // 3 = ordered >=
-        const float m = q[4 * (k & 3) + 3];
-        if (r) {
-            const unsigned rej = group_bits<G>(r); // the groups that open this child
-            opened(((unsigned)ch[k] << 6) | ((e & 63u) + 1u), rej);
-            // some groups accept, some open: the latter add nothing (the asm
-            // keeps the compiler from joining this arm's sums with the
-            // other's behind a flag: 2480 -> 2380 us at 1M Plummer bodies,
-            // theta 0.5, vote 16)
-            if constexpr (G < 64) {
-                if (rej != fields) {
-                    add_term(dx, dy, dz, d2, __builtin_amdgcn_inverse_ballot_w64(field_lanes(rej)) ? 0.f : m, px, py, pz);
-                    asm volatile("" : "+v"(px), "+v"(py), "+v"(pz));
-                }
-            }
-        } else {
-            add_term(dx, dy, dz, d2, m, px, py, pz);
-        }
+        const float d2 = fmaf(dx, dx, fmaf(dy, dy, fmaf(dz, dz, eps2)));
+        // 3 = ordered >=
+        if (__builtin_amdgcn_fcmpf(d2, thr, 3) != kAllLanes)
+            opened(((unsigned)ch[k] << 6) | ((e & 63u) + 1u));
+        else
+            add_term(dx, dy, dz, d2, q[4 * (k & 3) + 3], px, py, pz);
     }
 #pragma unroll
     for (int k = 7; k >= 0; --k) {
         if (7 - k >= nbody) break;
         const f32x16 &q = k < 4 ? q0 : q1;
         const float dx = q[4 * (k & 3)] - me.x, dy = q[4 * (k & 3) + 1] - me.y, dz = q[4 * (k & 3) + 2] - me.z;
-        const float d2 = fmaf(dx, dx, fmaf(dy, dy, fmaf(dz, dz, e2)));
+        const float d2 = fmaf(dx, dx, fmaf(dy, dy, fmaf(dz, dz, eps2)));
         add_term(dx, dy, dz, d2, q[4 * (k & 3) + 3], px, py, pz);
     }
     return nbody + ncell;
 }
 
-// Entries of a block's stack. One wave (K = 1) walks depth first: at most 7
-// siblings wait per level. K waves take the K top entries together; the limit
-// kSplitTop above which they take one entry at a time (depth first from there,
-// again at most 7 per level) bounds the stack for every tree of kMaxDepth
-// levels: kSplitTop + the children of one round + 7 per level.
-constexpr int kSplitTop = 512;
-template <int K> constexpr int force_stack() { return K == 1 ? kStack : kSplitTop + 8 * K + kStack; }
+// The same for narrower votes. fields: the groups that opened the cell; act:
+// their lanes; opened(entry, groups) for every child that some group opens.
+// The children come in octant order, each with its kind: with the order of the
+// cells' walk and the compensated sums of the kernel below, a wave alone then
+// adds every body's terms exactly as its group by itself would.
+template <int G, bool SPLIT, class Opened>
+__device__ __forceinline__ int visit_narrow(unsigned e, unsigned fields, uint64_t act, float thr, float4 me,
+                                          float eps2, const int *__restrict__ cchild,
+                                          const float4 *__restrict__ cdata, float &px, float &py, float &pz,
+                                          bool &bad, Opened &&opened)
+{
+    const size_t c = e >> 6;
+    const i32x8 ch = *reinterpret_cast<const i32x8 *>(cchild + c * 8);
+    const f32x16 q0 = *reinterpret_cast<const f32x16 *>(cdata + c * 8);
+    const f32x16 q1 = *reinterpret_cast<const f32x16 *>(cdata + c * 8 + 4);
+    // all loads issued together (the compiler would put the second half
+    // behind the first children's work, one more round trip per visit)
+    if constexpr (SPLIT) asm volatile("" ::"s"(ch), "s"(q0), "s"(q1));
+    const int nchild = (int)((unsigned)ch[0] >> kCountShift) & 15;
+    const unsigned below = (e & 63u) + 1u;
+    const float e2 = __builtin_amdgcn_inverse_ballot_w64(act) ? eps2 : kFar;
+    px = py = pz = 0.f;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        if (k >= nchild) break;
+        const f32x16 &q = k < 4 ? q0 : q1;
+        const float dx = q[4 * (k & 3)] - me.x, dy = q[4 * (k & 3) + 1] - me.y, dz = q[4 * (k & 3) + 2] - me.z;
+        const float d2 = fmaf(dx, dx, fmaf(dy, dy, fmaf(dz, dz, e2)));
+        const float m = q[4 * (k & 3) + 3];
+        // the lanes that reject the child, a cell (the asm keeps the vote in
+        // a branch of its own: 2.94 -> 2.76 ms at 1M Plummer bodies, theta
+        // 0.5, vote 16, against an arm of its own for bodies)
+        uint64_t r = 0;
+        if (ch[k] >= 0) {
+            r = act & ~__builtin_amdgcn_fcmpf(d2, thr, 3); // 3 = ordered >=
+            asm volatile("");
+        }
+        if (r) {
+            const unsigned rej = group_bits<G>(r); // the groups that open this child
+            // cells live on kMaxDepth levels: one below the last is corrupt
+            // (and not followed)
+            if (below < (unsigned)kMaxDepth) opened(((unsigned)ch[k] << 6) | below, rej);
+            else bad = true;
+            // some groups accept, some open: the latter add nothing (the asm
+            // keeps the compiler from joining this arm's sums with the
+            // other's behind a flag: 4 % of the kernel)
+            if (rej != fields) {
+                add_term(dx, dy, dz, d2, __builtin_amdgcn_inverse_ballot_w64(field_lanes(rej)) ? 0.f : m, px, py, pz);
+                asm volatile("" : "+v"(px), "+v"(py), "+v"(pz));
+            }
+        } else {
+            add_term(dx, dy, dz, d2, m, px, py, pz);
+        }
+    }
+    return nchild;
+}
 
 template <int G> struct StackEntry {
     using type = uint2;
@@ -170,7 +198,7 @@ template <> struct StackEntry<64> {
 // The epilogue's per-wave sums overlay the stack.
 template <int G, int K> constexpr int force_lds()
 {
-    const int stack = force_stack<K>() * (int)sizeof(typename StackEntry<G>::type), red = K == 1 ? 0 : K * 3 * 64 * 8;
+    const int stack = split_stack<K>() * (int)sizeof(typename StackEntry<G>::type), red = K == 1 ? 0 : K * 3 * 64 * 8;
     return ((stack > red ? stack : red) + 15) & ~15;
 }
 
@@ -185,12 +213,10 @@ template <int G, int K>
 __global__ __launch_bounds__(64 * K) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_force(
     Dev d, const int *__restrict__ cchild, const float4 *__restrict__ cdata, int mode)
 {
-    constexpr int kCap = force_stack<K>();
     __shared__ __attribute__((aligned(16))) unsigned char lds[force_lds<G, K>()];
     __shared__ float dq_s[kMaxDepth];
-    __shared__ unsigned pushed[K]; // per wave: entries pushed this round, | kBad on a corrupt tree
+    __shared__ unsigned pushed[K];
     __shared__ unsigned long long wint[K];
-    constexpr unsigned kBad = 1u << 16;
     // (cell << 6 | depth), with narrow votes beside the groups that opened it
     using Entry = typename StackEntry<G>::type;
     Entry *stk = reinterpret_cast<Entry *>(lds);
@@ -228,6 +254,7 @@ __global__ __launch_bounds__(64 * K) __attribute__((amdgpu_waves_per_eu(8, 8))) 
     const float eps2 = d.eps2;
     const unsigned cap = (unsigned)d.cap;
     double sx = 0.0, sy = 0.0, sz = 0.0;
+    float fx = 0.f, fy = 0.f, fz = 0.f, kx = 0.f, ky = 0.f, kz = 0.f; // narrow votes, K = 1
     // Interactions: every child of a visited cell meets the lanes that opened
     // it, except where it is opened in turn, which is a visit of its own: the
     // sum over the visits of (children - 1) x lanes, plus the root's lanes.
@@ -241,14 +268,29 @@ __global__ __launch_bounds__(64 * K) __attribute__((amdgpu_waves_per_eu(8, 8))) 
         for (;;) {
             const uint64_t act = G < 64 ? field_lanes(fields) : kAllLanes;
             float px, py, pz;
-            const int children = visit_cell<G, false>(cur, fields, act, dq_s[cur & 63u], me, eps2, cchild, cdata, px, py, pz, bad,
-                                               [&](unsigned e, unsigned f) {
-                                                   stk[sp] = entry(e, f); // every lane, one address
-                                                   ++sp;
-                                               });
-            sx += (double)px;
-            sy += (double)py;
-            sz += (double)pz;
+            auto opened = [&](unsigned e, unsigned f = 15u) {
+                stk[sp] = entry(e, f); // every lane, one address
+                ++sp;
+            };
+            const float thr = dq_s[cur & 63u];
+            int children;
+            if constexpr (G < 64)
+                children = visit_narrow<G, false>(cur, fields, act, thr, me, eps2, cchild, cdata, px, py, pz, bad, opened);
+            else
+                children = visit_wide<false>(cur, thr, me, eps2, cchild, cdata, px, py, pz, bad, opened);
+            if constexpr (G < 64) {
+                // only the lanes that opened the cell, as each group alone
+                // would sum
+                if (__builtin_amdgcn_inverse_ballot_w64(act)) {
+                    kahan_add(fx, kx, px);
+                    kahan_add(fy, ky, py);
+                    kahan_add(fz, kz, pz);
+                }
+            } else {
+                sx += (double)px;
+                sy += (double)py;
+                sz += (double)pz;
+            }
             inter += (G < 64 ? (unsigned long long)(unsigned)__popcll(act & vmask) : 1ull) * (unsigned)(children - 1);
             if (sp == 0) break;
             --sp;
@@ -274,12 +316,17 @@ __global__ __launch_bounds__(64 * K) __attribute__((amdgpu_waves_per_eu(8, 8))) 
                 } else {
                     const uint64_t act = G < 64 ? field_lanes(fields) : kAllLanes;
                     float px, py, pz;
-                    const int children = visit_cell<G, true>(cur, fields, act, dq_s[cur & 63u], me, eps2, cchild,
-                                                             cdata, px, py, pz, bad, [&](unsigned e, unsigned f) {
-                                                                 push = lane_write(push, e, npush);
-                                                                 if constexpr (G < 64) pushf = lane_write(pushf, f, npush);
-                                                                 ++npush;
-                                                             });
+                    auto opened = [&](unsigned e, unsigned f = 15u) {
+                        push = lane_write(push, e, npush);
+                        if constexpr (G < 64) pushf = lane_write(pushf, f, npush);
+                        ++npush;
+                    };
+                    const float thr = dq_s[cur & 63u];
+                    int children;
+                    if constexpr (G < 64)
+                        children = visit_narrow<G, true>(cur, fields, act, thr, me, eps2, cchild, cdata, px, py, pz, bad, opened);
+                    else
+                        children = visit_wide<true>(cur, thr, me, eps2, cchild, cdata, px, py, pz, bad, opened);
                     sx += (double)px;
                     sy += (double)py;
                     sz += (double)pz;
@@ -287,22 +334,11 @@ __global__ __launch_bounds__(64 * K) __attribute__((amdgpu_waves_per_eu(8, 8))) 
                              (unsigned)(children - 1);
                 }
             }
-            if (lane == 0) pushed[wv] = (unsigned)npush | (bad ? kBad : 0u);
-            __syncthreads(); // the entries of this round are read, the counts are in
-            unsigned before = 0, total = 0;
-#pragma unroll
-            for (int w = 0; w < K; ++w) {
-                const unsigned c = pushed[w];
-                before += w < wv ? c : 0u;
-                total += c;
+            if (!end_round<K>(stk, pushed, wv, lane, take, npush, entry(push, pushf), bad, sp)) {
+                bad = true;
+                break;
             }
-            total = __builtin_amdgcn_readfirstlane(total);
-            bad = total >= kBad || sp - take + (int)total > kCap; // the same in every wave
-            if (bad) break;
-            if (lane < npush) stk[sp - take + (int)before + lane] = entry(push, pushf);
-            sp += (int)total - take;
             if (sp == 0) break;
-            __syncthreads();
         }
         // the waves' sums in wave order
         __syncthreads();
@@ -322,7 +358,11 @@ __global__ __launch_bounds__(64 * K) __attribute__((amdgpu_waves_per_eu(8, 8))) 
         }
     }
     if (bad && lane == 0) flag_error(ctl, kErrStack);
-    if (valid) finish_body(d, pos, me, (float)sx, (float)sy, (float)sz, mode, step);
+    if constexpr (G < 64 && K == 1) {
+        if (valid) finish_body(d, pos, me, fx - kx, fy - ky, fz - kz, mode, step);
+    } else {
+        if (valid) finish_body(d, pos, me, (float)sx, (float)sy, (float)sz, mode, step);
+    }
     // device interaction counters: one atomic per block
     if (lane == 0) {
         const unsigned nv = (unsigned)__popcll(vmask);
@@ -331,19 +371,28 @@ __global__ __launch_bounds__(64 * K) __attribute__((amdgpu_waves_per_eu(8, 8))) 
     }
 }
 
-// Waves per group, by the number of groups g. One wave per group leaves the
+// Waves per group, by the number of groups. One wave per group leaves the
 // 1,024 SIMDs (8 waves each) short of waves below about 8,192 groups, and a
 // visit is a chain of a stack read and scalar loads; more waves shorten the
 // chain of visits but wait for each other every round (a fifth to a third of
 // the time once the chip is full). us of the force stage, 1 / 4 / 8 / 16 waves:
-//   16,384 bodies (256), ball, theta 0.5, vote 16          307 / 149 / 94 / 71
+//   16,384 bodies (256), ball, theta 0.5, vote 16          307 / 149 / 94 / 73
 //   32,768 bodies (512), disk, theta 1.22, vote 16         110 / 74 / 46 / 36
 //   65,536 bodies (1,024), ball, theta 0.5, vote 64        402 / 189 / 147 / 167
 //   100,003 bodies (1,563), two spheres, theta 0.4, 64     890 / 440 / 431 / 470
 //   131,072 bodies (2,048), Plummer, theta 1.22, vote 16   140 / 98 / 106 / 148
 //   262,144 bodies (4,096), two spheres, theta 0.4, 64     1156 / 913 / 1014 / 1216
 //   524,288 bodies (8,192), two spheres, theta 0.4, 64     1635 / 1740 / 1996 / 2452
-static int waves_per_group(int groups) { return groups <= 640 ? 16 : groups <= 1792 ? 8 : groups <= 5120 ? 4 : 1; }
+// Narrow votes split only where it gains most (three times and more). A wave
+// alone adds every body's terms in the order of its group's own depth-first
+// walk, bit for bit what a walk per group gives, and the reference's vote and
+// time step can make a run chaotic: a rotating disk (dt 0.025) carries a
+// last-bit difference to 1e-3 of the velocities in 20 steps.
+static int waves_per_group(int groups, bool narrow)
+{
+    if (narrow) return groups <= 640 ? 16 : 1;
+    return groups <= 640 ? 16 : groups <= 1792 ? 8 : groups <= 5120 ? 4 : 1;
+}
 
 template <int G> static void launch_force_g(const Dev &d, int mode, hipStream_t st)
 {
@@ -351,7 +400,7 @@ template <int G> static void launch_force_g(const Dev &d, int mode, hipStream_t 
     const dim3 grid(groups);
     const int *cc = d.cchild;
     const float4 *cd = d.cdata;
-    switch (waves_per_group(groups)) {
+    switch (waves_per_group(groups, G < 64)) {
     case 16: hipLaunchKernelGGL((k_force<G, 16>), grid, dim3(1024), 0, st, d, cc, cd, mode); break;
     case 8: hipLaunchKernelGGL((k_force<G, 8>), grid, dim3(512), 0, st, d, cc, cd, mode); break;
     case 4: hipLaunchKernelGGL((k_force<G, 4>), grid, dim3(256), 0, st, d, cc, cd, mode); break;

@@ -10,17 +10,24 @@
 //                                   the cell is published
 //            count : int32[cap]     bodies in the cell's subtree
 //            com64 : double4[cap]   FP64 centre of mass (x, y, z) and mass (w)
-//            cchild: int32[8*cap]   a cell's child cells, packed to the front in
+//            cchild: int32[8*cap]   a cell's children. Vote width 64: the child
+//                                   cells' numbers, packed to the front in
 //                                   octant order; above kCountShift word 0
 //                                   holds the number of bodies among the
-//                                   children and word 1 the number of cells
-//            cdata : float4[8*cap]  (x, y, z, m): the child cells' FP32 centres of
-//                                   mass and masses at the front (as cchild),
-//                                   the bodies' positions and masses at the
-//                                   back in reverse octant order -- a visited
-//                                   cell is one contiguous 160-byte read in
-//                                   the traversal, and a child's place says
-//                                   what it is; the places between are not
+//                                   children and word 1 the number of cells.
+//                                   Narrower votes (d.narrow): all children
+//                                   packed to the front in octant order, a
+//                                   cell as its number and a body as
+//                                   kChildBody; word 0 also holds the number
+//                                   of children, from bit kCountShift
+//            cdata : float4[8*cap]  (x, y, z, m): a child cell's FP32 centre of
+//                                   mass and mass at its place in cchild, a
+//                                   body's position and mass at its place
+//                                   there (narrow) or, from the back in
+//                                   octant order, in the record's last places
+//                                   (width 64) -- a visited cell is one
+//                                   contiguous 160-byte read in the
+//                                   traversal; places of no child are not
 //                                   written
 //            cq64  : double[8*cap]  second moments about the centre of mass, learned
 //                                   mode only: traceless Q (xx, yy, zz, xy, xz, yz),
@@ -70,7 +77,8 @@ constexpr int kTailThreads = 512;    // the single block of the deepest summariz
 constexpr unsigned char kNotLive = 0xff; // clvl of a cell that is not in the tree
 constexpr int kCostKeys = 32;        // cost classes of the coarse traversal's launch order
 constexpr uint32_t kEmpty = 0xffffffffu;
-constexpr int kCountShift = 26;      // child counts above the cell numbers in cchild (the pool holds at most 2^26)
+constexpr int kCountShift = 26;      // child count above the cell number in cchild (the pool holds at most 2^26)
+constexpr int kChildBody = (int)0x80000000u; // cchild of a body: negative
 
 enum DevError : int {
     kErrNone = 0,
@@ -120,6 +128,7 @@ struct Dev {
     float alpha2_coarse; // learned mode: coarse_alpha^2 (the relative test; 0 = off)
     int fp64;
     int quad;            // summarize also computes quadrupole moments
+    int narrow;          // vote width below 64: the children's layout
     Ctl *ctl;
     float4 *pm4, *vel4, *acc4;
     double4 *pos64;
@@ -238,16 +247,21 @@ struct Learn {
 
 // What the coarse traversal does with its result: the learned step (features
 // through the network, corrected acceleration, body update), raw FP32
-// features and frames of listed groups (training pairs), accelerations of
-// listed groups (training targets), or the body update with the coarse
-// acceleration alone.
+// features and frames (of listed groups, or of all when `groups` is null),
+// accelerations of listed groups (training targets), or the body update with
+// the coarse acceleration alone.
 // kOutAccel opens cells with the force stage's table `dqtab` (the fine
 // traversal of the training targets); the others with the extent and
-// relative tests of the coarse traversal (dqtab unused).
+// relative tests of the coarse traversal.
 enum CoarseOut { kOutLearned = 0, kOutRaw = 1, kOutAccel = 2, kOutFinish = 3 };
-hipError_t launch_coarse(const Dev &d, const Learn &L, int out, const float *dqtab, const int *groups,
-                         int ngroups, float *xraw, float4 *frame_out, float4 *acc_out, int fmode,
-                         hipStream_t st);
+hipError_t launch_coarse(const Dev &d, const Learn &L, int out, const int *groups, int ngroups, float *xraw,
+                         float4 *frame_out, int fmode, hipStream_t st);
+// a step's training pairs: the listed groups' records and accelerations
+// (rec: 2 * 64 per group), then kOutRaw and kOutAccel over the groups, which
+// read the bodies from rec only
+hipError_t launch_pair_records(const Dev &d, const int *groups, int ngroups, float4 *rec, hipStream_t st);
+hipError_t launch_pairs(const Dev &d, const Learn &L, const float *dqtab, const int *groups, int ngroups,
+                        const float4 *rec, float *xraw, float4 *frame_out, float4 *acc_out, hipStream_t st);
 // The network alone on raw FP32 features x[rows][24] -> residual y[rows][3]
 // (the same matrix-core code as the learned step)
 hipError_t launch_mlp_rows(const Learn &L, const float *xraw, int rows, float *y, hipStream_t st);

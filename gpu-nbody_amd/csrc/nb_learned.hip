@@ -23,6 +23,12 @@
 // sit within a few softening lengths.) Bodies interact as point masses. The
 // training targets use the same kernel with the force stage's opening table
 // (kOutAccel).
+// A visited cell's bodies come first (its quadrupole records are on their way
+// from memory meanwhile), then each child cell is tested and, when taken,
+// added at once: with all tests before all terms the squared distance of a taken
+// cell was worked out twice (3.27 -> 2.97 ms at 4M clustered bodies, alpha
+// 0.0175; the bodies' and cells' places in the record make each loop a run of
+// one kind, so no branch has three ways). Bound: vector issue.
 //
 // Features. Per body, 24 numbers in a frame built from the body's own coarse
 // acceleration a: e1 = a / |a|, e2 = the part of the quadrupole acceleration
@@ -113,9 +119,6 @@ __device__ __forceinline__ bf16x8 load_bf16x8(const uint16_t *p)
     return __builtin_bit_cast(bf16x8, *reinterpret_cast<const u16x8 *>(p));
 }
 
-constexpr int kStackC = 768; // >= kStack; 768 words = 64 rows of 24 BF16 features
-static_assert(kStackC >= kStack && kStackC * 4 >= 64 * kFeat * 2, "coarse stack doubles as the feature rows");
-
 // ---------------------------------------------------------------------------
 // BF16 matrix-core network (shared by the learned step and the test path)
 //
@@ -196,40 +199,44 @@ __device__ __forceinline__ void mlp_wave(const uint16_t *fs, const Mlp &m, int l
 // ---------------------------------------------------------------------------
 // Coarse traversal
 // ---------------------------------------------------------------------------
-// lane k's value of x (k wave-uniform)
-__device__ __forceinline__ float lane_read(float x, int k)
-{
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), k));
-}
-
 #define NB_COARSE_PARAMS                                                                                     \
     Dev d, Learn L, const int *__restrict__ cchild, const float4 *__restrict__ cdata,                        \
         const float4 *__restrict__ cqa, const float4 *__restrict__ cqb, const float2 *__restrict__ cmac,     \
-        const float *__restrict__ dqtab, const int *__restrict__ groups, int ngroups, float *__restrict__ xraw, \
-        float4 *__restrict__ frame_out, float4 *__restrict__ acc_out, int fmode
-#define NB_COARSE_PASS d, L, cchild, cdata, cqa, cqb, cmac, dqtab, groups, ngroups, xraw, frame_out, acc_out, fmode
+        const float *__restrict__ dqtab, const int *__restrict__ groups, int ngroups,                        \
+        const float4 *__restrict__ rec, float *__restrict__ xraw, float4 *__restrict__ frame_out,            \
+        float4 *__restrict__ acc_out, int fmode
+#define NB_COARSE_PASS \
+    d, L, cchild, cdata, cqa, cqb, cmac, dqtab, groups, ngroups, rec, xraw, frame_out, acc_out, fmode
 
-// waves (vote groups) per block of the coarse traversal. The waves share
-// nothing, and a block of one wave frees its slot as soon as its group is
-// done, where a block of four holds a CU's share until its slowest group
-// ends (learned force 3.48 -> 3.42 ms at 4M against four, 3.44 with two)
-constexpr int kCoarseWaves = 1;
-
-template <int OUT> __device__ __forceinline__ void coarse_traverse(NB_COARSE_PARAMS)
+// K waves share a vote group, as in k_force (nb_force.hip): one wave walks depth
+// first; K take the stack's top K entries in rounds, and their sums are added in
+// wave order.
+template <int OUT, int K, bool REC> __device__ __forceinline__ void coarse_traverse(int gslot, NB_COARSE_PARAMS)
 {
     constexpr bool kFeatOn = OUT == kOutLearned || OUT == kOutRaw;
     constexpr bool kGeo = OUT == kOutAccel; // the fine traversal: the force stage's opening table
-    constexpr bool kLaneQ = true; // quadrupole records by vector loads, read back from LDS
-    // a wave's traversal stack; after the traversal the learned step reuses it
-    // for the wave's 64 rows of BF16 features (64 x 24 x 2 bytes)
-    __shared__ __attribute__((aligned(16))) unsigned stk[kCoarseWaves][kStackC];
-    // a popped cell's children's quadrupole records, (qa, qb) per child, for
+    // the stack; after the traversal the waves' sums overlay it, and the
+    // learned step's 64 rows of BF16 features (64 x 24 x 2 bytes)
+    constexpr int kRedBytes = K == 1 ? 0 : K * 64 * (kFeatOn ? 9 * 4 : 3 * 8);
+    constexpr int kFeatBytes = OUT == kOutLearned ? 64 * kFeat * 2 : 0;
+    constexpr int kStackBytes = split_stack<K>() * 4;
+    constexpr int kLds = kStackBytes > kRedBytes ? (kStackBytes > kFeatBytes ? kStackBytes : kFeatBytes)
+                                                 : (kRedBytes > kFeatBytes ? kRedBytes : kFeatBytes);
+    struct WaveTotals {
+        float smb;
+        int bodies, cells, visits;
+    };
+    __shared__ __attribute__((aligned(16))) unsigned char lds[kLds];
+    // a visited cell's children's quadrupole records, (qa, qb) per child, for
     // the accepted cells' uniform LDS reads
-    __shared__ float4 qst[kCoarseWaves][16];
+    __shared__ float4 qst[K][16];
     __shared__ float dq_s[kMaxDepth];
+    __shared__ unsigned pushed[K];
+    __shared__ WaveTotals totals[K];
+    unsigned *stk = reinterpret_cast<unsigned *>(lds); // (cell << 6 | depth)
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const int wv = tid >> 6;
+    const int wv = K == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = d.n;
     Ctl *ctl = d.ctl;
     if (ctl->error) return;
@@ -238,12 +245,10 @@ template <int OUT> __device__ __forceinline__ void coarse_traverse(NB_COARSE_PAR
         return;
     }
     if (kGeo)
-        for (int i = tid; i < kMaxDepth; i += 64 * kCoarseWaves) dq_s[i] = dqtab[i];
+        for (int i = tid; i < kMaxDepth; i += 64 * K) dq_s[i] = dqtab[i];
     const int step = ctl->step;
     const float root_r = ctl->radius;
-    __syncthreads();
 
-    const int gslot = blockIdx.x * kCoarseWaves + wv;
     int g = gslot;
     if (groups) {
         if (gslot >= ngroups) return;
@@ -251,170 +256,117 @@ template <int OUT> __device__ __forceinline__ void coarse_traverse(NB_COARSE_PAR
     }
     const int pos = g * 64 + lane;
     const bool valid = pos >= 0 && pos < n;
-    if (__ballot(valid) == 0ull) return; // wave-uniform
+    if (__ballot(valid) == 0ull) return; // the same in every wave of the block
     // a lane past the last body sits at infinity: its d^2 is infinite, so it
     // accepts every cell and never holds up the vote (its sums are discarded)
-    const float4 me = valid ? d.pm4[d.sorted[pos]] : make_float4(kFar, kFar, kFar, 0.f);
+    // REC: the groups' records and accelerations as k_pair_records copied them
+    float4 me = make_float4(kFar, kFar, kFar, 0.f);
+    if (valid) me = REC ? rec[2 * ((size_t)gslot * 64 + lane)] : d.pm4[d.sorted[pos]];
     const float eps2 = d.eps2;
-    const int cap = d.cap;
+    const unsigned cap = (unsigned)d.cap;
     // the body's factor (alpha^2 |a_old|^2)^(-1/5) of the relative test's
     // threshold; 0 switches it off (no previous acceleration yet, as in the
     // force stage's kick, or alpha = 0)
     float a5 = 0.f;
     if (!kGeo && valid && step > 0 && d.alpha2_coarse > 0.f) {
-        const float4 a0 = d.acc4[d.sorted[pos]];
+        const float4 a0 = REC ? rec[2 * ((size_t)gslot * 64 + lane) + 1] : d.acc4[d.sorted[pos]];
         const float a2 = fmaf(a0.x, a0.x, fmaf(a0.y, a0.y, a0.z * a0.z));
         if (a2 > 0.f) a5 = (float)pow((double)(d.alpha2_coarse * a2), -0.2);
     }
 
-    if (lane == 0) stk[wv][0] = 0; // root cell 0 at depth 0
-    int sp = 1;
-    // The fine traversal (training targets) sums each popped cell's terms into
-    // a compensated total (s, k). The coarse one keeps three running sums --
-    // bodies (b), cell monopoles (s; with the quadrupole when no features are
-    // made) and cell quadrupoles (q) -- and adds them at the end: its error
-    // bound is 1e-3, and the compensation cost 12 of its 27 instructions per
-    // popped cell.
-    float sx = 0.f, sy = 0.f, sz = 0.f, kx = 0.f, ky = 0.f, kz = 0.f;
+    // The learned step and the features keep three FP32 running sums --
+    // bodies (b), cell monopoles (s) and cell quadrupoles (q): the features
+    // need them apart, and the step's error bound is 1e-3. The coarse force
+    // alone sums a visited cell's terms in FP32 and adds them into FP64 sums
+    // (t; convert and add issue like two FP32 adds), the fine pass into
+    // compensated FP32 sums (s, k), in the order of its walk.
+    double tx = 0.0, ty = 0.0, tz = 0.0;
+    float kx = 0.f, ky = 0.f, kz = 0.f;
+    float sx = 0.f, sy = 0.f, sz = 0.f;
     float bx = 0.f, by = 0.f, bz = 0.f;
     float qx = 0.f, qy = 0.f, qz = 0.f;
     float smb = 0.f; // mass of the bodies met (the accepted cells hold the rest)
-    int nc = 0, nbod = 0;
-    long long ninter = 0, ncell = 0;
-    int npop = 0;
+    // children met so far: every child cell of a visited cell is accepted or
+    // visited in turn
+    int nbod = 0, nchild = 0, nvisit = 0;
     bool bad = false;
-    while (sp > 0) {
-        __builtin_amdgcn_wave_barrier();
-        --sp;
-        ++npop;
-        const unsigned e = __builtin_amdgcn_readfirstlane(stk[wv][sp]);
-        const int c = (int)(e >> 6);
-        const int dep = (int)(e & 63u);
-        const float thr_geo = kGeo ? dq_s[dep] : 0.f;
-        const int *chp = cchild + (size_t)c * 8;
-        const float4 *cdp = cdata + (size_t)c * 8;
-        int ch[8];
-        float4 q[8];
-        float2 mc[8];
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            ch[k] = __builtin_amdgcn_readfirstlane(chp[k]);
-            q[k] = cdp[k];
-            if (!kGeo) mc[k] = cmac[(size_t)c * 8 + k];
-        }
-        // child cells at the front of the record, bodies at its back
-        const int nbody = (int)((unsigned)ch[0] >> kCountShift), ncellc = (int)((unsigned)ch[1] >> kCountShift);
+
+    // One visit of cell e >> 6 on level e & 63; opened(entry) for the
+    // children to visit. Every branch is wave-uniform.
+    auto visit = [&](unsigned e, auto &&opened) {
+        const size_t c = e >> 6;
+        const i32x8 ch = *reinterpret_cast<const i32x8 *>(cchild + c * 8);
+        const f32x16 q0 = *reinterpret_cast<const f32x16 *>(cdata + c * 8);
+        const f32x16 q1 = *reinterpret_cast<const f32x16 *>(cdata + c * 8 + 4);
+        f32x16 mc;
+        if constexpr (!kGeo) mc = *reinterpret_cast<const f32x16 *>(cmac + c * 8);
+        float thr = 0.f;
+        if constexpr (kGeo) thr = dq_s[e & 63u];
         // the children's quadrupole records, child k in lanes k, k + 8, ...:
-        // two vector loads issued now, waited for at the first accepted cell
-        // (which reads them from the wave's LDS), so their latency hides
-        // behind the decisions and the bodies; each from the popped cell's
-        // uniform base plus an unsigned lane offset (fewer 64-bit address
-        // adds per pop)
-        float4 qav, qbv;
-        if constexpr (kLaneQ) {
-            qav = (cqa + (size_t)c * 8)[(unsigned)lane & 7u];
-            qbv = (cqb + (size_t)c * 8)[(unsigned)lane & 7u];
+        // two vector loads issued now, waited for after the bodies; each from
+        // the cell's uniform base plus an unsigned lane offset (no 64-bit
+        // address adds per lane)
+        const float4 qav = (cqa + c * 8)[(unsigned)lane & 7u];
+        const float4 qbv = (cqb + c * 8)[(unsigned)lane & 7u];
+        // child cells at the front of the record, bodies at its back
+        const int nbody = (int)((unsigned)ch[0] >> kCountShift);
+        int ncell = (int)((unsigned)ch[1] >> kCountShift);
+        if ((e & 63u) == kMaxDepth - 1 && ncell > 0) { // no level below: corrupt
+            bad = true;
+            ncell = 0;
         }
-        // First the opening decisions, a wave-uniform bit mask of the child
-        // cells: the opening test of this traversal.
-        // The coarse one takes the extent test first (threshold b^2 /
-        // theta_c^2 + eps^2 from summarize) and the relative test (threshold
-        // the product of the cell's and the body's factors) only when every
-        // lane passed it: both votes are wave-uniform, so the short circuit is
-        // a scalar branch.
-        // Lane masks come straight from the compares (3 = ordered >=, 5 =
-        // ordered <=). An opened cell's stack entry goes into lane `npush` of
-        // `push` (v_writelane: no compare, no branch on the lane); all of them
-        // are stored after the loop.
-        unsigned cells = 0;
-        int npush = 0;
-        bool badv = false;
-        unsigned push = 0;
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            if (k >= ncellc) continue;
-            const int v = ch[k] & ((1 << kCountShift) - 1);
-            const float dx = q[k].x - me.x, dy = q[k].y - me.y, dz = q[k].z - me.z;
-            const float d2 = fmaf(dx, dx, fmaf(dy, dy, fmaf(dz, dz, eps2)));
-            const uint64_t exec = __builtin_amdgcn_read_exec();
-            bool take = __builtin_amdgcn_fcmpf(d2, kGeo ? thr_geo : mc[k].x, 3) == exec;
-            if (!kGeo && take) take = __builtin_amdgcn_fcmpf(mc[k].y * a5, d2, 5) == exec;
-            if (take) {
-                cells |= 1u << k;
-            } else {
-                push = lane_write(push, ((unsigned)v << 6) | (unsigned)(dep + 1), npush);
-                ++npush;
-                badv |= v >= cap;
-            }
-        }
-        // Then the interactions, each kind in child order, each branch only
-        // around its own work, so the running sums are updated in place (a
-        // branch that both accumulates and pushes makes the compiler copy
-        // them at every child): bodies, cell monopoles and cell quadrupoles
-        // summed separately (the features need the parts). The learned step
-        // adds its terms to its three running sums directly; the fine
-        // traversal sums a popped cell's terms from zero for its compensated
-        // add, and the coarse one without features (one sum of monopole and
-        // quadrupole) from zero for its running sums, which keeps it within
-        // 1e-5 of the oracle's FP64 sums. d is worked out again, with the
-        // same operations as for the test.
-        float pbx, pby, pbz, pmx, pmy, pmz, pqx, pqy, pqz;
-        if constexpr (kGeo || !kFeatOn) {
-            pbx = pby = pbz = pmx = pmy = pmz = pqx = pqy = pqz = 0.f;
-        } else {
-            pbx = bx;
-            pby = by;
-            pbz = bz;
-            pmx = sx;
-            pmy = sy;
-            pmz = sz;
-            pqx = qx;
-            pqy = qy;
-            pqz = qz;
-        }
+        nbod += nbody;
+        nchild += ncell;
+        ++nvisit;
+        float px = 0.f, py = 0.f, pz = 0.f, cx = 0.f, cy = 0.f, cz = 0.f; // this cell's bodies and child cells
+        float &bpx = kFeatOn ? bx : px, &bpy = kFeatOn ? by : py, &bpz = kFeatOn ? bz : pz;
+        float &mpx = kFeatOn ? sx : kGeo ? cx : px, &mpy = kFeatOn ? sy : kGeo ? cy : py, &mpz = kFeatOn ? sz : kGeo ? cz : pz;
 #pragma unroll
         for (int k = 7; k >= 0; --k) {
-            if (7 - k >= nbody) continue;
-            const float4 qk = q[k];
-            const float dx = qk.x - me.x, dy = qk.y - me.y, dz = qk.z - me.z;
+            if (7 - k >= nbody) break;
+            const f32x16 &q = k < 4 ? q0 : q1;
+            const int o = 4 * (k & 3);
+            const float dx = q[o] - me.x, dy = q[o + 1] - me.y, dz = q[o + 2] - me.z;
             const float d2 = fmaf(dx, dx, fmaf(dy, dy, fmaf(dz, dz, eps2)));
             const float ri = __builtin_amdgcn_rsqf(d2);
-            const float f = qk.w * (ri * ri * ri);
-            pbx = fmaf(dx, f, pbx);
-            pby = fmaf(dy, f, pby);
-            pbz = fmaf(dz, f, pbz);
-            if (kFeatOn) smb += qk.w;
+            const float f = q[o + 3] * (ri * ri * ri);
+            bpx = fmaf(dx, f, bpx);
+            bpy = fmaf(dy, f, bpy);
+            bpz = fmaf(dz, f, bpz);
+            if (kFeatOn) smb += q[o + 3];
         }
-        // the children's quadrupole records into this wave's LDS rows (the
-        // vector loads have had the decisions and the bodies to arrive): an
-        // accepted cell reads its two with uniform LDS reads, no VALU
-        if constexpr (kLaneQ) {
-            if (cells) {
-                if (lane < 8) {
-                    qst[wv][2 * lane] = qav;
-                    qst[wv][2 * lane + 1] = qbv;
-                }
-                __builtin_amdgcn_wave_barrier();
+        // the records into this wave's LDS rows: an accepted cell reads its two
+        // with uniform LDS reads, no VALU
+        if (ncell) {
+            if (lane < 8) {
+                qst[wv][2 * lane] = qav;
+                qst[wv][2 * lane + 1] = qbv;
             }
+            __builtin_amdgcn_wave_barrier();
         }
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
-            if (!((cells >> k) & 1u)) continue;
-            const float4 qk = q[k];
-            const float dx = qk.x - me.x, dy = qk.y - me.y, dz = qk.z - me.z;
+            if (k >= ncell) break;
+            const f32x16 &q = k < 4 ? q0 : q1;
+            const int o = 4 * (k & 3);
+            const float dx = q[o] - me.x, dy = q[o + 1] - me.y, dz = q[o + 2] - me.z;
             const float d2 = fmaf(dx, dx, fmaf(dy, dy, fmaf(dz, dz, eps2)));
-            float4 qa, qb; // (Qxx, Qyy, Qzz, T eps^2), (Qxy, Qxz, Qyz, 0)
-            if constexpr (kLaneQ) {
-                qa = qst[wv][2 * k];
-                qb = qst[wv][2 * k + 1];
-            } else {
-                qa = cqa[(size_t)c * 8 + k];
-                qb = cqb[(size_t)c * 8 + k];
+            // The coarse test: the extent (threshold b^2 / theta_c^2 + eps^2
+            // from summarize), then the relative test (threshold the product
+            // of the cell's and the body's factors) only when every lane
+            // passed it. Lane masks come straight from the compares (3 =
+            // ordered >=, 5 = ordered <=).
+            bool take = __builtin_amdgcn_fcmpf(d2, kGeo ? thr : mc[2 * k], 3) == kAllLanes;
+            if (!kGeo && take) take = __builtin_amdgcn_fcmpf(mc[2 * k + 1] * a5, d2, 5) == kAllLanes;
+            if (!take) {
+                opened(((unsigned)ch[k] << 6) | ((e & 63u) + 1u));
+                continue;
             }
+            const float4 qa = qst[wv][2 * k], qb = qst[wv][2 * k + 1]; // (Qxx, Qyy, Qzz, T eps^2), (Qxy, Qxz, Qyz, 0)
             const float ri = __builtin_amdgcn_rsqf(d2);
             const float r2i = ri * ri;
             const float r3 = r2i * ri;
-            const float f = qk.w * r3;
+            const float f = q[o + 3] * r3;
             const float Qx = fmaf(qa.x, dx, fmaf(qb.x, dy, qb.y * dz));
             const float Qy = fmaf(qb.x, dx, fmaf(qa.y, dy, qb.z * dz));
             const float Qz = fmaf(qb.y, dx, fmaf(qb.z, dy, qa.z * dz));
@@ -423,76 +375,121 @@ template <int OUT> __device__ __forceinline__ void coarse_traverse(NB_COARSE_PAR
             if (kFeatOn) {
                 // the quadrupole part as r5 (u d - Q d), u = 5/2 (d.Q.d - T eps^2) / s^2
                 const float u = (dQd - qa.w) * (2.5f * r2i);
-                pmx = fmaf(dx, f, pmx);
-                pmy = fmaf(dy, f, pmy);
-                pmz = fmaf(dz, f, pmz);
-                pqx = fmaf(r5, fmaf(u, dx, -Qx), pqx);
-                pqy = fmaf(r5, fmaf(u, dy, -Qy), pqy);
-                pqz = fmaf(r5, fmaf(u, dz, -Qz), pqz);
+                mpx = fmaf(dx, f, mpx);
+                mpy = fmaf(dy, f, mpy);
+                mpz = fmaf(dz, f, mpz);
+                qx = fmaf(r5, fmaf(u, dx, -Qx), qx);
+                qy = fmaf(r5, fmaf(u, dy, -Qy), qy);
+                qz = fmaf(r5, fmaf(u, dz, -Qz), qz);
             } else {
                 const float c2 = (dQd - qa.w) * ((2.5f * r5) * r2i);
                 // monopole and quadrupole radial terms share one factor
                 const float h = f + c2;
-                pmx = fmaf(dx, h, fmaf(-r5, Qx, pmx));
-                pmy = fmaf(dy, h, fmaf(-r5, Qy, pmy));
-                pmz = fmaf(dz, h, fmaf(-r5, Qz, pmz));
+                mpx = fmaf(dx, h, fmaf(-r5, Qx, mpx));
+                mpy = fmaf(dy, h, fmaf(-r5, Qy, mpy));
+                mpz = fmaf(dz, h, fmaf(-r5, Qz, mpz));
             }
         }
-        const int nb_here = nbody, nc_here = __popc(cells);
-        const int cnt = nb_here + nc_here;
-        ncell += nc_here;
-        if (kFeatOn) {
-            nbod += nb_here;
-            nc += nc_here;
-        }
-        // the opened children in one store, in child order (the last one is
-        // popped first); the tree is at most kMaxDepth deep and the pool holds
-        // `cap` cells: anything else is corrupt
-        if (npush) {
-            if (sp + npush > kStackC || badv || dep + 1 >= kMaxDepth) {
-                bad = true;
+        if constexpr (!kFeatOn) {
+            if constexpr (kGeo) {
+                kahan_add(sx, kx, px + cx);
+                kahan_add(sy, ky, py + cy);
+                kahan_add(sz, kz, pz + cz);
             } else {
-                if (lane < npush) stk[wv][sp + lane] = push;
-                sp += npush;
+                tx += (double)px;
+                ty += (double)py;
+                tz += (double)pz;
             }
         }
-        if constexpr (kGeo) {
-            // the training targets: compensated
-            kahan_add(sx, kx, (pbx + pmx) + pqx);
-            kahan_add(sy, ky, (pby + pmy) + pqy);
-            kahan_add(sz, kz, (pbz + pmz) + pqz);
-        } else if constexpr (!kFeatOn) {
-            sx += pmx;
-            sy += pmy;
-            sz += pmz;
-            bx += pbx;
-            by += pby;
-            bz += pbz;
-        } else {
-            // the coarse force: its parts summed apart (the features need them)
-            sx = pmx;
-            sy = pmy;
-            sz = pmz;
-            bx = pbx;
-            by = pby;
-            bz = pbz;
-            qx = pqx;
-            qy = pqy;
-            qz = pqz;
+    };
+
+    if constexpr (K == 1) {
+        if (kGeo) __syncthreads();
+        unsigned cur = 0; // root cell 0 at depth 0
+        int sp = 0;
+        for (;;) {
+            visit(cur, [&](unsigned e) {
+                stk[sp] = e; // every lane, one address
+                ++sp;
+            });
+            if (sp == 0) break;
+            --sp;
+            cur = __builtin_amdgcn_readfirstlane(stk[sp]);
+            if ((cur >> 6) >= cap) { // the pool holds `cap` cells: corrupt
+                bad = true;
+                break;
+            }
         }
-        ninter += cnt;
-        if (bad) break;
+    } else {
+        if (tid == 0) stk[0] = 0; // root cell 0 at depth 0
+        int sp = 1;               // the same in every wave
+        __syncthreads();
+        for (;;) {
+            const int take = sp > kSplitTop ? 1 : min(sp, K);
+            int npush = 0;
+            unsigned push = 0; // entry j of this wave's children in lane j
+            if (wv < take) {
+                const unsigned cur = __builtin_amdgcn_readfirstlane(stk[sp - 1 - wv]);
+                if ((cur >> 6) >= cap) { // the pool holds `cap` cells: corrupt
+                    bad = true;
+                } else {
+                    visit(cur, [&](unsigned e) {
+                        push = lane_write(push, e, npush);
+                        ++npush;
+                    });
+                }
+            }
+            if (!end_round<K>(stk, pushed, wv, lane, take, npush, push, bad, sp)) {
+                bad = true;
+                break;
+            }
+            if (sp == 0) break;
+        }
+        // the waves' sums in wave order
+        __syncthreads();
+        if (lane == 0) totals[wv] = WaveTotals{smb, nbod, nchild, nvisit};
+        float *rf = reinterpret_cast<float *>(lds);
+        double *rd = reinterpret_cast<double *>(lds);
+        if constexpr (kFeatOn) {
+            const float v[9] = {bx, by, bz, sx, sy, sz, qx, qy, qz};
+#pragma unroll
+            for (int i = 0; i < 9; ++i) rf[(wv * 9 + i) * 64 + lane] = v[i];
+        } else {
+            rd[(wv * 3 + 0) * 64 + lane] = tx;
+            rd[(wv * 3 + 1) * 64 + lane] = ty;
+            rd[(wv * 3 + 2) * 64 + lane] = tz;
+        }
+        __syncthreads();
+        if (wv > 0) return;
+#pragma unroll 1
+        for (int w = 1; w < K; ++w) {
+            if constexpr (kFeatOn) {
+                const float *o = rf + w * 9 * 64 + lane;
+                bx += o[0 * 64]; by += o[1 * 64]; bz += o[2 * 64];
+                sx += o[3 * 64]; sy += o[4 * 64]; sz += o[5 * 64];
+                qx += o[6 * 64]; qy += o[7 * 64]; qz += o[8 * 64];
+            } else {
+                tx += rd[(w * 3 + 0) * 64 + lane];
+                ty += rd[(w * 3 + 1) * 64 + lane];
+                tz += rd[(w * 3 + 2) * 64 + lane];
+            }
+            smb += totals[w].smb;
+            nbod += totals[w].bodies;
+            nchild += totals[w].cells;
+            nvisit += totals[w].visits;
+        }
     }
+    const int nc = nchild - (nvisit - 1); // accepted cells
     if (bad && lane == 0) flag_error(ctl, kErrStack);
     if constexpr (OUT == kOutLearned || OUT == kOutFinish) {
         // the group's cost for the next launch order, in interactions: a
-        // popped cell (its loads and up to eight tests) weighs about three
-        const long long cost = ninter + 3ll * npop;
+        // visited cell (its loads and up to eight tests) weighs about three
+        const long long cost = (long long)nbod + nc + 3ll * nvisit;
         if (lane == 0) d.gcost[g] = cost < 0x7fffffffll ? (int)cost : 0x7fffffff;
     }
-    const float ax = kGeo ? sx - kx : (bx + sx) + qx;
-    const float ay = kGeo ? sy - ky : (by + sy) + qy;
-    const float az = kGeo ? sz - kz : (bz + sz) + qz;
+    const float ax = kFeatOn ? (bx + sx) + qx : kGeo ? sx - kx : (float)tx;
+    const float ay = kFeatOn ? (by + sy) + qy : kGeo ? sy - ky : (float)ty;
+    const float az = kFeatOn ? (bz + sz) + qz : kGeo ? sz - kz : (float)tz;
     const int slot = gslot * 64 + lane;
     if constexpr (OUT == kOutAccel) {
         if (valid) acc_out[slot] = make_float4(ax, ay, az, 0.f);
@@ -616,7 +613,7 @@ template <int OUT> __device__ __forceinline__ void coarse_traverse(NB_COARSE_PAR
         } else {
             // the learned step: normalized BF16 features into this wave's LDS
             // rows, the network, the correction, the body update
-            uint16_t *fs = reinterpret_cast<uint16_t *>(stk[wv]);
+            uint16_t *fs = reinterpret_cast<uint16_t *>(lds);
             uint32_t w[kFeat / 2];
 #pragma unroll
             for (int i = 0; i < kFeat; i += 2) {
@@ -645,30 +642,56 @@ template <int OUT> __device__ __forceinline__ void coarse_traverse(NB_COARSE_PAR
             if (valid) finish_body(d, pos, me, rx, ry, rz, fmode, step);
         }
     }
-    // device interaction counters: one atomic each per wave
+    // device interaction counters: one atomic each per block
     const unsigned long long nvalid = (unsigned long long)__popcll(__ballot(valid));
-    if (lane == 0 && ninter && nvalid) {
+    if (lane == 0) {
         Tally *t = &ctl->tally[blockIdx.x % kTallies];
-        __hip_atomic_fetch_add(&t->all, (unsigned long long)ninter * nvalid, __ATOMIC_RELAXED, AGENT);
-        __hip_atomic_fetch_add(&t->cells, (unsigned long long)ncell * nvalid, __ATOMIC_RELAXED, AGENT);
+        __hip_atomic_fetch_add(&t->all, (unsigned long long)(unsigned)(nbod + nc) * nvalid, __ATOMIC_RELAXED, AGENT);
+        __hip_atomic_fetch_add(&t->cells, (unsigned long long)(unsigned)nc * nvalid, __ATOMIC_RELAXED, AGENT);
     }
 }
 
-// The kernels. Six waves per SIMD at least for the network's epilogue (80
-// registers); the coarse force without it asks for seven, which its 68
-// registers allow and which changes its scalar register budget and code
-// (0.12-0.17 ms less at 4M; the learned kernel at seven spills in its
-// epilogue and is slower).
-template <int OUT>
-__global__ __launch_bounds__(64 * kCoarseWaves) __attribute__((amdgpu_waves_per_eu(6, 8))) void k_coarse64(NB_COARSE_PARAMS)
+// The kernels. Seven waves per SIMD at least, by the attribute (learned step
+// at 4M clustered bodies 2.97 ms at six, 2.87 ms at seven, where 14 registers
+// of its epilogue spill; the coarse force at eight would spill scalar
+// registers in the loop, 0.85 -> 1.29 ms at 700,001 bodies).
+template <int OUT, int K>
+__global__ __launch_bounds__(64 * K) __attribute__((amdgpu_waves_per_eu(7, 8))) void k_coarse64(
+    NB_COARSE_PARAMS)
 {
-    coarse_traverse<OUT>(NB_COARSE_PASS);
+    coarse_traverse<OUT, K, false>((int)blockIdx.x, NB_COARSE_PASS);
 }
 
-template <>
-__global__ __launch_bounds__(64 * kCoarseWaves) __attribute__((amdgpu_waves_per_eu(7, 8))) void k_coarse64<kOutFinish>(NB_COARSE_PARAMS)
+// A step's training pairs, both passes over the listed groups in one launch: the
+// fine pass (targets) in the blocks 0 .. ngroups - 1, the raw one (features)
+// after them. One wave per group, in the order of its walk: some features are
+// ill-conditioned (the direction of the part of the quadrupole acceleration
+// across a, where that part is small), targets are the small difference of two
+// accelerations, and Adam turns rounding into full steps where a parameter's
+// gradient nearly cancels. With waves sharing a group (978 + 270 -> 247 us for
+// 256 groups of a 262,144-body run) equally exact sums moved trained weights
+// by up to 4e-3. The few long chains run beside the step's force pass instead
+// (the engine puts them on a stream of their own, on copies of the bodies'
+// records).
+__global__ __launch_bounds__(64) void k_pairs(NB_COARSE_PARAMS)
 {
-    coarse_traverse<kOutFinish>(NB_COARSE_PASS);
+    if ((int)blockIdx.x < ngroups)
+        coarse_traverse<kOutAccel, 1, true>((int)blockIdx.x, NB_COARSE_PASS);
+    else
+        coarse_traverse<kOutRaw, 1, true>((int)blockIdx.x - ngroups, NB_COARSE_PASS);
+}
+
+// The records and accelerations of the listed groups' bodies, 64 slots a group
+__global__ __launch_bounds__(256) void k_pair_records(Dev d, const int *__restrict__ groups, int slots,
+                                                      float4 *__restrict__ rec)
+{
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= slots) return;
+    const int pos = groups[i >> 6] * 64 + (i & 63);
+    if (pos < 0 || pos >= d.n) return;
+    const int b = d.sorted[pos];
+    rec[2 * (size_t)i] = d.pm4[b];
+    rec[2 * (size_t)i + 1] = d.acc4[b];
 }
 
 // One block: a histogram of the groups' cost classes (1 + floor(log2 cost),
@@ -765,23 +788,61 @@ hipError_t launch_group_order(const Dev &d, hipStream_t st)
     return hipGetLastError();
 }
 
-hipError_t launch_coarse(const Dev &d, const Learn &L, int out, const float *dqtab, const int *groups,
-                         int ngroups, float *xraw, float4 *frame_out, float4 *acc_out, int fmode,
-                         hipStream_t st)
+// Waves per group, by the number of groups (see waves_per_group in
+// nb_force.hip). us of the force stage, 1 / 4 / 8 / 16 waves, coarse and
+// learned (theta_c 0.9, alpha 0.02):
+//   16,384 bodies (256 groups), Plummer      299 / 157 / 101 / 81     311 / 157 / 89 / 92
+//   40,960 (640), Plummer                    368 / 175 / 131 / 165    377 / 174 / 109 / 181
+//   65,536 (1,024), halo and disk            383 / 199 / 168 / 232    387 / 187 / 140 / 251
+//   131,072 (2,048), Plummer                 443 / 303 / 308 / 451    469 / 275 / 235 / 484
+//   262,144 (4,096), clusters                358 / 333 / 411 / 726    368 / 320 / 348 / 782
+//   524,288 (8,192), halo and disk           670 / 953 / 1105 / 1723  691 / 811 / 826 / 1803
+static int coarse_waves_per_group(int groups)
+{
+    return groups <= 320 ? 16 : groups <= 1536 ? 8 : groups <= 5120 ? 4 : 1;
+}
+
+hipError_t launch_coarse(const Dev &d, const Learn &L, int out, const int *groups, int ngroups, float *xraw,
+                         float4 *frame_out, int fmode, hipStream_t st)
 {
     const int waves = groups ? ngroups : (d.n + 63) / 64;
     if (waves <= 0) return hipSuccess;
-    const dim3 grid((waves + kCoarseWaves - 1) / kCoarseWaves), block(64 * kCoarseWaves);
+    const float *dqtab = nullptr;
+    const float4 *rec = nullptr;
+    float4 *acc_out = nullptr;
 #define NB_COARSE_ARGS                                                                             \
     d, L, (const int *)d.cchild, (const float4 *)d.cdata, (const float4 *)d.cqa, (const float4 *)d.cqb, \
-        (const float2 *)d.cmac, dqtab, groups, ngroups, xraw, frame_out, acc_out, fmode
+        (const float2 *)d.cmac, dqtab, groups, ngroups, rec, xraw, frame_out, acc_out, fmode
+#define NB_COARSE_LAUNCH(OUT)                                                                                  \
+    switch (coarse_waves_per_group(waves)) {                                                                   \
+    case 16: hipLaunchKernelGGL((k_coarse64<OUT, 16>), dim3(waves), dim3(1024), 0, st, NB_COARSE_ARGS); break; \
+    case 8: hipLaunchKernelGGL((k_coarse64<OUT, 8>), dim3(waves), dim3(512), 0, st, NB_COARSE_ARGS); break;    \
+    case 4: hipLaunchKernelGGL((k_coarse64<OUT, 4>), dim3(waves), dim3(256), 0, st, NB_COARSE_ARGS); break;    \
+    default: hipLaunchKernelGGL((k_coarse64<OUT, 1>), dim3(waves), dim3(64), 0, st, NB_COARSE_ARGS); break;    \
+    }
     switch (out) {
-    case kOutLearned: hipLaunchKernelGGL(k_coarse64<kOutLearned>, grid, block, 0, st, NB_COARSE_ARGS); break;
-    case kOutRaw: hipLaunchKernelGGL(k_coarse64<kOutRaw>, grid, block, 0, st, NB_COARSE_ARGS); break;
-    case kOutAccel: hipLaunchKernelGGL(k_coarse64<kOutAccel>, grid, block, 0, st, NB_COARSE_ARGS); break;
-    case kOutFinish: hipLaunchKernelGGL(k_coarse64<kOutFinish>, grid, block, 0, st, NB_COARSE_ARGS); break;
+    case kOutLearned: NB_COARSE_LAUNCH(kOutLearned); break;
+    case kOutRaw: hipLaunchKernelGGL((k_coarse64<kOutRaw, 1>), dim3(waves), dim3(64), 0, st, NB_COARSE_ARGS); break;
+    case kOutFinish: NB_COARSE_LAUNCH(kOutFinish); break;
     default: return hipErrorInvalidValue;
     }
+#undef NB_COARSE_LAUNCH
+    return hipGetLastError();
+}
+
+hipError_t launch_pair_records(const Dev &d, const int *groups, int ngroups, float4 *rec, hipStream_t st)
+{
+    if (ngroups <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_pair_records, dim3((ngroups * 64 + 255) / 256), dim3(256), 0, st, d, groups, ngroups * 64, rec);
+    return hipGetLastError();
+}
+
+hipError_t launch_pairs(const Dev &d, const Learn &L, const float *dqtab, const int *groups, int ngroups,
+                        const float4 *rec, float *xraw, float4 *frame_out, float4 *acc_out, hipStream_t st)
+{
+    if (ngroups <= 0) return hipSuccess;
+    const int fmode = 0;
+    hipLaunchKernelGGL(k_pairs, dim3(2 * ngroups), dim3(64), 0, st, NB_COARSE_ARGS);
 #undef NB_COARSE_ARGS
     return hipGetLastError();
 }

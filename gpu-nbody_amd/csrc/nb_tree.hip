@@ -274,8 +274,7 @@ __global__ __launch_bounds__(256) void k_level_scatter(Dev d)
 // (an empty slot adds 0) in the fixed pairwise order
 // ((s0 + s1) + (s2 + s3)) + ((s4 + s5) + (s6 + s7)), which the xor-shuffle
 // reduction produces identically on every lane. Children are compacted
-// (summarizetree.cl:75-81) into the traversal list: cells to its front,
-// bodies to its back.
+// (summarizetree.cl:75-81) into the traversal list.
 // ---------------------------------------------------------------------------
 // Lane exchanges inside each group of 8 lanes as DPP moves (no LDS):
 // quad_perm [1,0,3,2] = lane ^ 1, quad_perm [2,3,0,1] = lane ^ 2, and
@@ -349,14 +348,22 @@ __device__ __forceinline__ void summarize_cell(const Dev &d, int first, int i, i
             bc = q1.w;
         }
     }
-    // places: child cells from the front, bodies from the back, the empty
-    // slots between them
+    // compaction (nb_internal.h, cchild). Narrow: the children from the front.
+    // Width 64: child cells from the front, bodies from the back, the empty
+    // slots between them (words 0 and 1 hold the counts whoever's they are).
     const int gl = (int)(threadIdx.x & 63) & ~7;
     const unsigned gc = (unsigned)((__ballot(v >= n) >> gl) & 0xffull);
     const unsigned gb = (unsigned)((__ballot(v >= 0 && v < n) >> gl) & 0xffull);
     const unsigned lower = (1u << k) - 1u;
     const int ncell = __popc(gc), nbody = __popc(gb);
-    const int at = v >= n ? __popc(gc & lower) : v >= 0 ? 7 - __popc(gb & lower) : ncell + __popc(~(gc | gb) & lower);
+    int at, word;
+    if (d.narrow) {
+        at = __popc((gc | gb) & lower);
+        word = (v >= n ? v - n : kChildBody) | (at == 0 ? (ncell + nbody) << kCountShift : 0);
+    } else {
+        at = v >= n ? __popc(gc & lower) : v >= 0 ? 7 - __popc(gb & lower) : ncell + __popc(~(gc | gb) & lower);
+        word = (v >= n ? v - n : 0) | (at == 0 ? nbody << kCountShift : at == 1 ? ncell << kCountShift : 0);
+    }
     const double sm = sum8(m), sx = sum8(m * x), sy = sum8(m * y), sz = sum8(m * z);
     int scnt = cnt;
     scnt += dpp_i<kDppXor1>(scnt);
@@ -366,12 +373,11 @@ __device__ __forceinline__ void summarize_cell(const Dev &d, int first, int i, i
     // reference's 0 * inf = NaN (summarizetree.cl:161-167)
     const double inv = sm > 0.0 ? 1.0 / sm : 0.0;
     const double4 com = make_double4(sx * inv, sy * inv, sz * inv, sm);
-    // the traversals read the records of the children only: the places
-    // between cells and bodies keep stale ones (a cell has 3 children on
-    // average, so this skips well over half of the record writes)
+    // the traversals read the records of the children only: the other places
+    // keep stale ones (a cell has 3 children on average, so this skips well
+    // over half of the record writes)
     if (live) {
-        const int counts = at == 0 ? nbody << kCountShift : at == 1 ? ncell << kCountShift : 0;
-        d.cchild[(size_t)c * 8 + at] = (v >= n ? v - n : 0) | counts;
+        if (v >= 0 || !d.narrow) d.cchild[(size_t)c * 8 + at] = word;
         if (v >= 0) d.cdata[(size_t)c * 8 + at] = rec;
         if (k == 0) {
             d.com64[c] = com;
