@@ -625,7 +625,7 @@ int start_check(nb_sim *s)
     HIP_TRY(s, hipStreamWaitEvent(s->side, s->chk_go, 0));
     HIP_TRY(s, hipMemcpyAsync(s->chk_idx, s->chk_host, (size_t)ns * sizeof(int32_t), hipMemcpyHostToDevice, s->side));
     HIP_TRY(s, hipEventRecord(s->chk_ev[0], s->side));
-    hipError_t e = nb::launch_direct64(s->d, s->chk_idx, ns, s->chk_part, s->chk_out, false, s->side);
+    hipError_t e = nb::launch_direct64(s->d, s->chk_idx, ns, s->chk_part, s->chk_out, nb::kDirectAcc, s->side);
     if (e == hipSuccess) e = hipEventRecord(s->chk_ev[1], s->side);
     if (e != hipSuccess) return fail(s, NB_E_HIP, "sampled check launch: %s", hipGetErrorString(e));
     s->chk_ns = ns;
@@ -1160,7 +1160,7 @@ static int direct_accel(nb_sim *s, const int32_t *idx, int32_t ns, std::vector<d
     int r = ensure_check_buffers(s, ns);
     if (r) return r;
     HIP_TRY(s, hipMemcpyAsync(s->chk_idx, idx, (size_t)ns * sizeof(int), hipMemcpyHostToDevice, s->stream));
-    hipError_t e = nb::launch_direct64(s->d, s->chk_idx, ns, s->chk_part, s->chk_out, false, s->stream);
+    hipError_t e = nb::launch_direct64(s->d, s->chk_idx, ns, s->chk_part, s->chk_out, nb::kDirectAcc, s->stream);
     if (e != hipSuccess) return fail(s, NB_E_HIP, "direct-sum launch: %s", hipGetErrorString(e));
     return fetch(s, out, (const double4 *)s->chk_out, (size_t)ns);
 }
@@ -1608,13 +1608,15 @@ int nb_diagnostics(nb_sim *s, int32_t pe_samples, uint64_t seed, double *out)
         std::vector<double4> res;
         HIP_TRY(s, hipMemcpyAsync(s->chk_idx, idx.data() + b0, (size_t)nb_ * sizeof(int), hipMemcpyHostToDevice,
                                   s->stream));
-        e = nb::launch_direct64(s->d, s->chk_idx, nb_, s->chk_part, s->chk_out, true, s->stream);
+        e = nb::launch_direct64(s->d, s->chk_idx, nb_, s->chk_part, s->chk_out,
+                                exact ? nb::kDirectPhiAfter : nb::kDirectPhi, s->stream);
         if (e != hipSuccess) return fail(s, NB_E_HIP, "direct-sum launch: %s", hipGetErrorString(e));
         r = fetch(s, res, (const double4 *)s->chk_out, (size_t)nb_);
         if (r) return r;
         for (int i = 0; i < nb_; ++i) pe += (double)pm[idx[b0 + i]].w * res[i].w;
     }
-    pe *= -0.5 * (double)n / (double)ns;
+    // every pair once, or the sampled bodies' pairs, scaled and halved
+    pe *= exact ? -1.0 : -0.5 * (double)n / (double)ns;
     out[0] = sum[4];
     out[1] = pe;
     out[2] = sum[1];

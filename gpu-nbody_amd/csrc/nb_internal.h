@@ -190,10 +190,12 @@ hipError_t launch_summarize_block(const Dev &d, int lo, int hi, hipStream_t st);
 // mode: 0 = store accelerations (reference semantics), 1 = also integrate
 // (fused kick-drift-kick), 2 = probe: write accelerations to d.probe only
 hipError_t launch_force(const Dev &d, int vote, int mode, hipStream_t st);
-// FP64 direct-sum accelerations of the bodies idx[0..ns) (G = 1), into out;
-// out[i].w = sum_{j != idx[i]} m_j / sqrt(r^2 + eps^2) (the softened potential, negated)
-// when phi, else 0
-hipError_t launch_direct64(const Dev &d, const int *idx, int ns, double4 *part, double4 *out, bool phi,
+// FP64 direct sums of the bodies idx[0..ns) (G = 1), into out: accelerations
+// (x, y, z), or in w the softened potential (negated)
+// sum_{j != idx[i]} m_j / sqrt(r^2 + eps^2), or the part of it from the bodies
+// j > idx[i] (idx then holds consecutive bodies)
+enum DirectSum { kDirectAcc, kDirectPhi, kDirectPhiAfter };
+hipError_t launch_direct64(const Dev &d, const int *idx, int ns, double4 *part, double4 *out, DirectSum sum,
                            hipStream_t st);
 hipError_t launch_integrate(const Dev &d, hipStream_t st);
 // FP64 per-block sums of m, m v, m v^2 / 2, m x cross v, m x (11 doubles per block)
