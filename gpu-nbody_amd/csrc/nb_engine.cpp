@@ -511,7 +511,7 @@ void free_all(nb_sim *s)
                     s->chk_idx, s->chk_part, s->chk_out, d.cq64, d.cqa, d.cqb, d.cmac,
                     s->mlpbuf, s->chk_acc, s->vtx, d.kb_key[0], d.kb_key[1], d.kb_val[0], d.kb_val[1],
                     d.kb_deep, d.kb_hist, d.kb_offs, d.kb_tot, d.kb_ipar, d.kb_lpar, d.kb_lo,
-                    d.kb_own, d.kb_ktop, d.kb_obase, d.kb_scan, d.kb_tdep, d.kb_spl, d.kb_bcnt, d.kb_bfill, d.kb_bstart, d.kb_big};
+                    d.kb_own, d.kb_ktop, d.kb_obase, d.kb_scan, d.kb_tdep, d.kb_spl, d.kb_bcnt, d.kb_bfill, d.kb_bstart};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     for (auto &e : s->tev)
@@ -793,8 +793,7 @@ int nb_create(const nb_params *p, nb_sim **out)
         ok = ok && dalloc(&d.kb_scan, stiles) == hipSuccess && dalloc(&d.kb_tdep, stiles) == hipSuccess;
         const size_t S = (size_t)nb::bucket_samples(n);
         ok = ok && dalloc(&d.kb_spl, S) == hipSuccess && dalloc(&d.kb_bcnt, S + 1) == hipSuccess &&
-             dalloc(&d.kb_bfill, S + 1) == hipSuccess && dalloc(&d.kb_bstart, S + 2) == hipSuccess &&
-             dalloc(&d.kb_big, S + 2) == hipSuccess;
+             dalloc(&d.kb_bfill, S + 1) == hipSuccess && dalloc(&d.kb_bstart, S + 2) == hipSuccess;
     }
     if (!ok) {
         fail(s, NB_E_HIP, "device allocation failed for %d bodies / %d cells", n, d.cap);

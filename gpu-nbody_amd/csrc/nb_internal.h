@@ -165,7 +165,6 @@ struct Dev {
     // counters (S + 1 each) and starts (S + 2)
     unsigned long long *kb_spl;
     unsigned *kb_bcnt, *kb_bfill, *kb_bstart;
-    int *kb_big; // S + 2: the count of buckets above kBucketCap, then their numbers
 };
 
 // ---- launchers (nb_tree.hip, nb_force.hip) ---------------------------------
@@ -177,7 +176,7 @@ hipError_t launch_build_keys(const Dev &d, bool warm, bool staged, hipStream_t s
 constexpr int kKeyTile = 2048;     // keys per radix-sort tile (first build)
 constexpr int kKeyScanTile = 1024; // cell counts per scan tile
 constexpr int kBucketT = 256;      // warm builds: one splitter per kBucketT bodies
-constexpr int kBucketCap = 512;    // buckets sorted by one wave up to this size
+constexpr int kBucketCap = 512;    // buckets sorted in LDS up to this size
 inline int bucket_samples(int n) { return (n + kBucketT - 1) / kBucketT; }
 hipError_t launch_levels(const Dev &d, hipStream_t st); // group live cells by level
 // Summarize and sort read each level's cell count on the device; the host's

@@ -257,25 +257,26 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_scatter(const unsigned long l
 //     bucket and block (k_keys_warm, with the keys); the counts' exclusive
 //     scan (k_bucket_scan); then each body takes the next place of its
 //     bucket the same way (k_bucket_scatter);
-//   * each bucket is sorted by one wave (k_bucket_sort): up to kBucketCap
-//     bodies held in registers, stable radix passes over the key bits that
-//     vary inside it, permuted through LDS; a larger bucket (stale order) is
-//     listed and sorted by a block through device memory (k_bucket_sort_big).
+//   * each bucket is sorted by one block (k_bucket_sort): up to kBucketCap
+//     bodies in LDS, a larger bucket (stale order) by radix passes through
+//     device memory.
 // The order inside a bucket before its sort depends on the atomics; the keys
 // are distinct after the run ordering below (equal keys are ordered by their
 // deeper levels), so the result does not.
 // ---------------------------------------------------------------------------
-constexpr int kBsThreads = 512; // blocks of the large-bucket sort
+constexpr int kBsThreads = 256; // blocks of the bucket sort
 constexpr int kBsWaves = kBsThreads / 64;
-static_assert(kBucketCap % 64 == 0, "whole rows of a wave");
+constexpr int kBsPerThread = kBucketCap / kBsThreads;
+static_assert(kBucketCap % kBsThreads == 0, "whole rows of the block");
+static_assert(kBsThreads == kRsBins, "a thread per digit");
 
 // Splitters spl[0 .. S-1]: the keys at positions j * kBucketT of `key` (the
 // last tree's sorted keys, so non-decreasing: a decrease means the buffer does
-// not hold them and stops the build with an error); the bucket counters and
-// the list of large buckets cleared.
+// not hold them and stops the build with an error); the bucket counters
+// cleared.
 __global__ __launch_bounds__(256) void k_splitters(Ctl *ctl, const unsigned long long *__restrict__ key, int S,
                                                    unsigned long long *__restrict__ spl, unsigned *__restrict__ bcnt,
-                                                   unsigned *__restrict__ bfill, int *__restrict__ big)
+                                                   unsigned *__restrict__ bfill)
 {
     const int j = blockIdx.x * blockDim.x + threadIdx.x;
     if (ctl->error || j > S) return;
@@ -286,7 +287,6 @@ __global__ __launch_bounds__(256) void k_splitters(Ctl *ctl, const unsigned long
     }
     bcnt[j] = 0;
     bfill[j] = 0;
-    if (j == 0) big[0] = 0;
 }
 
 // the first j with spl[j] > k (S if none): spl is non-decreasing; searched
@@ -660,161 +660,11 @@ __device__ int varying_top_bit(SK key, int m, unsigned long long *red)
     return all ? 63 - __clzll((long long)all) : -1;
 }
 
-// Bucket blockIdx.x of the S + 1 (blocks of one wave), in place in (key,
-// val): lane l holds elements r * 64 + l (r < kSortPer) in registers. A pass
-// by the 8 bits at `shift`: digit counts (LDS atomics) and their exclusive
-// scan give each digit's first place; then row by row, in element order, a
-// key's place is its digit's next free place plus its rank among the lanes
-// of the row with its digit (eight ballots); the row's lanes move their
-// digit's next place on. The keys go to those places in LDS and come back to
-// the registers in element order. A bucket above kBucketCap is listed in
-// big[1 ..] (big[0] counts them) for k_bucket_sort_big.
-constexpr int kSortPer = kBucketCap / 64;
-
-__global__ __launch_bounds__(64) void k_bucket_sort(const Ctl *ctl, unsigned long long *__restrict__ key,
-                                                    int *__restrict__ val, const unsigned *__restrict__ bstart,
-                                                    int *__restrict__ big)
-{
-    __shared__ unsigned long long sk[kBucketCap];
-    __shared__ int sv[kBucketCap];
-    __shared__ unsigned next[kRsBins];
-    if (ctl->error) return;
-    const int b = blockIdx.x, lane = threadIdx.x;
-    const int base = (int)bstart[b], m = (int)bstart[b + 1] - base;
-    if (m <= 1) return;
-    if (m > kBucketCap) {
-        if (lane == 0) big[1 + atomicAdd(&big[0], 1)] = b;
-        return;
-    }
-    unsigned long long k[kSortPer];
-    int v[kSortPer];
-    unsigned long long diff = 0;
-    const unsigned long long k0 = key[base];
-#pragma unroll
-    for (int r = 0; r < kSortPer; ++r) {
-        const int idx = r * 64 + lane;
-        k[r] = idx < m ? key[base + idx] : k0;
-        v[r] = idx < m ? val[base + idx] : 0;
-        diff |= k[r] ^ k0;
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) diff |= __shfl_xor(diff, o);
-    const int top = diff ? 63 - __clzll((long long)diff) : -1;
-    const unsigned long long below = lane ? (~0ull >> (64 - lane)) : 0ull;
-    for (int shift = 0; shift <= top; shift += 8) {
-#pragma unroll
-        for (int q = 0; q < kRsBins / 64; ++q) next[q * 64 + lane] = 0;
-        __syncthreads();
-#pragma unroll
-        for (int r = 0; r < kSortPer; ++r) {
-            if (r * 64 >= m) break;
-            if (r * 64 + lane < m) atomicAdd(&next[(unsigned)(k[r] >> shift) & 255u], 1u);
-        }
-        __syncthreads();
-        {
-            // lane l scans digits 4l .. 4l+3
-            unsigned c[4], sum = 0;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                c[q] = next[lane * 4 + q];
-                sum += c[q];
-            }
-            unsigned x = sum;
-#pragma unroll
-            for (int o = 1; o < 64; o <<= 1) {
-                const unsigned y = __shfl_up(x, o);
-                if (lane >= o) x += y;
-            }
-            unsigned run = x - sum;
-            __syncthreads();
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                next[lane * 4 + q] = run;
-                run += c[q];
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int r = 0; r < kSortPer; ++r) {
-            if (r * 64 >= m) break; // rows past the bucket: no key
-            const bool valid = r * 64 + lane < m;
-            const unsigned dg = (unsigned)(k[r] >> shift) & 255u;
-            unsigned long long peers = __ballot(valid);
-#pragma unroll
-            for (int bit = 0; bit < 8; ++bit) {
-                const unsigned long long bal = __ballot((dg >> bit) & 1u);
-                peers &= ((dg >> bit) & 1u) ? bal : ~bal;
-            }
-            const unsigned rank = (unsigned)__popcll(peers & below);
-            const unsigned at = valid ? next[dg] + rank : 0u;
-            __syncthreads();
-            if (valid) {
-                if (rank == 0) next[dg] += (unsigned)__popcll(peers);
-                sk[at] = k[r];
-                sv[at] = v[r];
-            }
-            __syncthreads();
-        }
-#pragma unroll
-        for (int r = 0; r < kSortPer; ++r) {
-            const int idx = r * 64 + lane;
-            if (idx < m) {
-                k[r] = sk[idx];
-                v[r] = sv[idx];
-            }
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int r = 0; r < kSortPer; ++r) {
-        const int idx = r * 64 + lane;
-        if (idx < m) {
-            key[base + idx] = k[r];
-            val[base + idx] = v[r];
-        }
-    }
-}
-
-// The listed buckets (more than kBucketCap bodies), one block each, in place
-// in (key, val) through (tkey, tval), free n-element buffers.
-constexpr int kBigBlocks = 64;
-
-__global__ __launch_bounds__(kBsThreads) void k_bucket_sort_big(Ctl *ctl, unsigned long long *__restrict__ key,
-                                                                int *__restrict__ val, unsigned long long *__restrict__ tkey,
-                                                                int *__restrict__ tval, const unsigned *__restrict__ bstart,
-                                                                const int *__restrict__ big)
-{
-    __shared__ RankLds R;
-    __shared__ unsigned long long red;
-    if (ctl->error) return;
-    const int t = threadIdx.x, nbig = big[0];
-    for (int q = blockIdx.x; q < nbig; q += gridDim.x) {
-        const int b = big[1 + q];
-        const int base = (int)bstart[b], m = (int)bstart[b + 1] - base;
-        if (t == 0) atomicAdd(&ctl->large_buckets, 1);
-        unsigned long long *k0 = key + base, *k1 = tkey + base;
-        int *v0 = val + base, *v1 = tval + base;
-        const int top = varying_top_bit(k0, m, &red);
-        bool in_tmp = false;
-        for (int shift = 0; shift <= top; shift += 8) {
-            if (in_tmp) rank_pass(k1, v1, k0, v0, m, shift, R);
-            else rank_pass(k0, v0, k1, v1, m, shift, R);
-            in_tmp = !in_tmp;
-        }
-        if (in_tmp) {
-            for (int j = t; j < m; j += kBsThreads) {
-                k0[j] = k1[j];
-                v0[j] = v1[j];
-            }
-        }
-        __syncthreads();
-    }
-}
-
 // ---------------------------------------------------------------------------
 // Runs of equal 21-level keys: their bodies' paths extended to 84 levels
-// (deep[0..2][pos], levels 21 .. 83), each run ordered by them, one thread
-// per run.
+// (deep[0..2][pos], levels 21 .. 83), each run ordered by them: by the bucket
+// sort in a warm build, by one thread per run (k_deep_runs) after the radix
+// sort.
 // ---------------------------------------------------------------------------
 // levels 21 .. 83 of body p's path, three words of 21 levels
 __device__ __forceinline__ void deep_words(float rx, float ry, float rz, float rr, float4 p,
@@ -884,6 +734,199 @@ __device__ void order_long_run(const Dev &d, int i, int m, int *val, unsigned lo
     }
     for (int a = 1; a < m; ++a)
         if (!deep_less(base, n, a - 1, a)) flag_error(d.ctl, kErrDepth); // one 84-level path
+}
+
+// Bucket blockIdx.x of the S + 1, in place in (key, val), and the runs of equal
+// keys in it (a run is never split: its keys fall into one bucket).
+//
+// A bucket of up to kBucketCap bodies stays in LDS: one distribution by the 8
+// highest key bits that vary inside it, whose order inside a digit is free,
+// then every key counts the smaller keys of its digit, which gives its place.
+// A digit holds a few keys (a bucket covers about a cell of 256 bodies, 8 bits
+// are two to three levels below it), so the counts are short; a digit that
+// holds them all costs kBucketCap reads, no more. Five barriers and about 40
+// dependent LDS accesses in all, where radix passes over every varying digit
+// took some 30 of each per pass (one wave per bucket, 5 or 6 passes):
+// bound by that latency, not by bandwidth or the adds. One launch instead of
+// three (buckets, large buckets, runs): 16,384 bodies 29 -> 6.3 us, 1M 42 ->
+// 22.7 us, 4M 85 -> 54 us.
+// Keys that meet an equal key get their levels 21 .. 83 here too, and their
+// place among the equals by counting the smaller of those.
+//
+// A larger bucket goes through device memory by stable radix passes ((tkey,
+// tval) are free n-element buffers), and one thread orders each of its runs.
+constexpr int kCountStep = 4; // keys a count reads at once
+struct BucketLds {
+    unsigned long long sk[kBucketCap + kCountStep]; // past the bucket: ~0 (keys use 63 bits)
+    unsigned long long dw[kDeepWords][kBucketCap]; // deep words of the keys that have equals
+    int sv[kBucketCap];
+    unsigned start[kRsBins + 1];
+    unsigned cnt[kRsBins];
+    unsigned wsum[kBsWaves];
+    unsigned long long diff[kBsWaves];
+};
+
+__device__ void sort_large_bucket(const Dev &d, unsigned long long *key, int *val, unsigned long long *deep,
+                                  unsigned long long *tkey, int *tval, int *perm, int *tmp, int base, int m,
+                                  RankLds &R, unsigned long long *red)
+{
+    const int t = threadIdx.x;
+    if (t == 0) atomicAdd(&d.ctl->large_buckets, 1);
+    unsigned long long *k0 = key + base, *k1 = tkey + base;
+    int *v0 = val + base, *v1 = tval + base;
+    const int top = varying_top_bit(k0, m, red);
+    bool in_tmp = false;
+    for (int shift = 0; shift <= top; shift += 8) {
+        if (in_tmp) rank_pass(k1, v1, k0, v0, m, shift, R);
+        else rank_pass(k0, v0, k1, v1, m, shift, R);
+        in_tmp = !in_tmp;
+    }
+    if (in_tmp) {
+        for (int j = t; j < m; j += kBsThreads) {
+            k0[j] = k1[j];
+            v0[j] = v1[j];
+        }
+    }
+    __syncthreads();
+    for (int j = t; j + 1 < m; j += kBsThreads) {
+        const unsigned long long k = k0[j];
+        if (k0[j + 1] != k || (j > 0 && k0[j - 1] == k)) continue; // not the start of a run
+        int run = 2;
+        while (j + run < m && k0[j + run] == k) ++run;
+        order_long_run(d, base + j, run, val, deep, perm, tmp, tkey, tval);
+    }
+}
+
+__global__ __launch_bounds__(kBsThreads) void k_bucket_sort(Dev d, unsigned long long *__restrict__ key,
+                                                            int *__restrict__ val,
+                                                            unsigned long long *__restrict__ deep,
+                                                            unsigned long long *__restrict__ tkey,
+                                                            int *__restrict__ tval, int *__restrict__ perm,
+                                                            int *__restrict__ tmp,
+                                                            const unsigned *__restrict__ bstart)
+{
+    __shared__ union {
+        BucketLds b;
+        struct {
+            RankLds rank;
+            unsigned long long red;
+        } large;
+    } lds;
+    const Ctl *ctl = d.ctl;
+    const int t = threadIdx.x, w = t >> 6;
+    const int base = (int)bstart[blockIdx.x], m = (int)bstart[blockIdx.x + 1] - base;
+    if (ctl->error || m <= 1) return;
+    if (m > kBucketCap) {
+        sort_large_bucket(d, key, val, deep, tkey, tval, perm, tmp, base, m, lds.large.rank, &lds.large.red);
+        return;
+    }
+    BucketLds &s = lds.b;
+    const size_t n = (size_t)d.n;
+    unsigned long long k[kBsPerThread], diff = 0;
+    int v[kBsPerThread];
+    const unsigned long long k0 = key[base];
+#pragma unroll
+    for (int r = 0; r < kBsPerThread; ++r) {
+        const int i = r * kBsThreads + t;
+        k[r] = i < m ? key[base + i] : k0;
+        v[r] = i < m ? val[base + i] : 0;
+        diff |= k[r] ^ k0;
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) diff |= __shfl_xor(diff, o);
+    if ((t & 63) == 0) s.diff[w] = diff;
+    s.cnt[t] = 0;
+    __syncthreads();
+    diff = s.diff[0] | s.diff[1] | s.diff[2] | s.diff[3];
+    const int top = diff ? 63 - __clzll((long long)diff) : 0;
+    const int shift = max(0, top - 7);
+    unsigned at[kBsPerThread];
+#pragma unroll
+    for (int r = 0; r < kBsPerThread; ++r)
+        if (r * kBsThreads + t < m) at[r] = atomicAdd(&s.cnt[(unsigned)(k[r] >> shift) & 255u], 1u);
+    __syncthreads();
+    const unsigned mine = s.cnt[t];
+    s.start[t] = scan256_excl(mine, s.wsum);
+    if (t == 0) s.start[kRsBins] = (unsigned)m;
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kBsPerThread; ++r) {
+        if (r * kBsThreads + t >= m) continue;
+        const unsigned p = s.start[(unsigned)(k[r] >> shift) & 255u] + at[r];
+        s.sk[p] = k[r];
+        s.sv[p] = v[r];
+    }
+    if (t < kCountStep) s.sk[m + t] = ~0ull;
+    __syncthreads();
+    // from here a thread's elements are the places i of the distributed order
+    bool run = false;
+    int place[kBsPerThread];
+#pragma unroll
+    for (int r = 0; r < kBsPerThread; ++r) {
+        const int i = r * kBsThreads + t;
+        place[r] = -1;
+        if (i >= m) continue;
+        const unsigned long long kk = s.sk[i];
+        const unsigned dg = (unsigned)(kk >> shift) & 255u;
+        const int lo = (int)s.start[dg], hi = (int)s.start[dg + 1];
+        int less = 0, same = 0;
+        for (int j = lo; j < hi; j += kCountStep) { // the keys past hi are larger
+#pragma unroll
+            for (int q = 0; q < kCountStep; ++q) {
+                const unsigned long long kj = s.sk[j + q];
+                less += kj < kk ? 1 : 0;
+                same += kj == kk ? 1 : 0;
+            }
+        }
+        k[r] = kk;
+        v[r] = s.sv[i];
+        place[r] = lo + less;
+        at[r] = (unsigned)same;
+        run |= same > 1;
+    }
+    if (__syncthreads_or(run)) {
+        const float rx = ctl->root[0], ry = ctl->root[1], rz = ctl->root[2], rr = ctl->radius;
+#pragma unroll
+        for (int r = 0; r < kBsPerThread; ++r) {
+            if (place[r] < 0 || at[r] < 2) continue;
+            unsigned long long w3[kDeepWords];
+            deep_words(rx, ry, rz, rr, d.pm4[v[r]], w3);
+#pragma unroll
+            for (int q = 0; q < kDeepWords; ++q) s.dw[q][r * kBsThreads + t] = w3[q];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < kBsPerThread; ++r) {
+            if (place[r] < 0 || at[r] < 2) continue;
+            const int i = r * kBsThreads + t;
+            const unsigned dg = (unsigned)(k[r] >> shift) & 255u;
+            const int lo = (int)s.start[dg], hi = (int)s.start[dg + 1];
+            const unsigned long long a0 = s.dw[0][i], a1 = s.dw[1][i], a2 = s.dw[2][i];
+            int before = 0;
+            for (int j = lo; j < hi; ++j) {
+                if (s.sk[j] != k[r] || j == i) continue;
+                const unsigned long long b0 = s.dw[0][j], b1 = s.dw[1][j], b2 = s.dw[2][j];
+                if (b0 == a0 && b1 == a1 && b2 == a2) {
+                    // two bodies on one 84-level path are closer than the tree can separate
+                    flag_error(d.ctl, kErrDepth);
+                    before += j < i ? 1 : 0;
+                } else {
+                    before += b0 < a0 || (b0 == a0 && (b1 < a1 || (b1 == a1 && b2 < a2))) ? 1 : 0;
+                }
+            }
+            place[r] += before;
+            const size_t o = (size_t)(base + place[r]);
+            deep[o] = a0;
+            deep[n + o] = a1;
+            deep[2 * n + o] = a2;
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < kBsPerThread; ++r) {
+        if (place[r] < 0) continue;
+        key[base + place[r]] = k[r];
+        val[base + place[r]] = v[r];
+    }
 }
 
 __global__ __launch_bounds__(256) void k_deep_runs(Dev d, const unsigned long long *__restrict__ key, int *val,
@@ -1362,15 +1405,15 @@ hipError_t launch_build_keys(const Dev &d, bool warm, bool staged, hipStream_t s
         const int S = bucket_samples(n);
         const dim3 gw((n + kWinBodies - 1) / kWinBodies);
         hipLaunchKernelGGL(k_splitters, dim3((S + 1 + 255) / 256), b256, 0, st, d.ctl, ka, S, d.kb_spl, d.kb_bcnt,
-                           d.kb_bfill, d.kb_big);
+                           d.kb_bfill);
         hipLaunchKernelGGL(k_keys_warm, dim3((n + kWarmBodies - 1) / kWarmBodies), b256, 0, st, d, d.sorted,
                            staged ? d.bnode : nullptr, d.kb_spl, S, kb, vb, d.kb_lo, d.kb_bcnt);
         hipLaunchKernelGGL(k_bucket_scan, dim3(1), dim3(1024), 0, st, d.ctl, d.kb_bcnt, S, d.kb_bstart);
         hipLaunchKernelGGL(k_bucket_scatter, gw, b256, 0, st, d.ctl, kb, vb, d.kb_lo, ka, va, n, d.kb_bstart,
                            d.kb_bfill);
-        hipLaunchKernelGGL(k_bucket_sort, dim3(S + 1), dim3(64), 0, st, d.ctl, ka, va, d.kb_bstart, d.kb_big);
-        hipLaunchKernelGGL(k_bucket_sort_big, dim3(kBigBlocks), dim3(kBsThreads), 0, st, d.ctl, ka, va, kb, vb,
-                           d.kb_bstart, d.kb_big);
+        // (the binary tree's arrays, written later, serve the runs of large buckets)
+        hipLaunchKernelGGL(k_bucket_sort, dim3(S + 1), dim3(kBsThreads), 0, st, d, ka, va, d.kb_deep, kb, vb, d.kb_ipar,
+                           d.kb_lpar, d.kb_bstart);
     } else {
         const int ntiles = (n + kRsTile - 1) / kRsTile;
         hipLaunchKernelGGL(k_keys, g256, b256, 0, st, d, nullptr, ka, va);
@@ -1387,10 +1430,10 @@ hipError_t launch_build_keys(const Dev &d, bool warm, bool staged, hipStream_t s
             va = vb;
             vb = tv;
         }
-        // eight passes: the sorted keys are back in kb_key[0] / kb_val[0]
+        // eight passes: the sorted keys are back in kb_key[0] / kb_val[0]; the
+        // other pair and the binary tree's arrays (written later) serve long runs
+        hipLaunchKernelGGL(k_deep_runs, g256, b256, 0, st, d, ka, va, d.kb_deep, d.kb_ipar, d.kb_lpar, kb, vb);
     }
-    // the other pair and the binary tree's arrays (written later) serve long runs
-    hipLaunchKernelGGL(k_deep_runs, g256, b256, 0, st, d, ka, va, d.kb_deep, d.kb_ipar, d.kb_lpar, kb, vb);
     KeyTree kt{ka, d.kb_deep, va, d.kb_ipar, d.kb_lpar, d.kb_lo, d.kb_own, d.kb_ktop, d.kb_obase, d.kb_scan};
     if (n >= 2) {
         const dim3 gi((n - 1 + kBtThreads - 1) / kBtThreads);
