@@ -749,7 +749,7 @@ __device__ void order_long_run(const Dev &d, int i, int m, int *val, unsigned lo
 // took some 30 of each per pass (one wave per bucket, 5 or 6 passes):
 // bound by that latency, not by bandwidth or the adds. One launch instead of
 // three (buckets, large buckets, runs): 16,384 bodies 29 -> 6.3 us, 1M 42 ->
-// 22.7 us, 4M 85 -> 54 us.
+// 24 us, 4M 85 -> 58 us.
 // Keys that meet an equal key get their levels 21 .. 83 here too, and their
 // place among the equals by counting the smaller of those.
 //
@@ -815,7 +815,9 @@ __global__ __launch_bounds__(kBsThreads) void k_bucket_sort(Dev d, unsigned long
     const Ctl *ctl = d.ctl;
     const int t = threadIdx.x, w = t >> 6;
     const int base = (int)bstart[blockIdx.x], m = (int)bstart[blockIdx.x + 1] - base;
-    if (ctl->error || m <= 1) return;
+    // the same decision in every wave: a bucket sorted at the same time may flag
+    // an error, and a wave that left then would leave its keys out of the counts
+    if (__syncthreads_or(ctl->error) || m <= 1) return;
     if (m > kBucketCap) {
         sort_large_bucket(d, key, val, deep, tkey, tval, perm, tmp, base, m, lds.large.rank, &lds.large.red);
         return;
