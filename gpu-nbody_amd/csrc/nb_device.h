@@ -76,6 +76,23 @@ __device__ __forceinline__ void flag_error(Ctl *ctl, int code)
                                          __ATOMIC_RELAXED, AGENT);
 }
 
+// Splitter j of a warm build (j < S = bucket_samples(n)): the key at position
+// j * kBucketT of the last tree's sorted keys, so non-decreasing (a decrease
+// means the buffer does not hold them and stops the build with an error), and
+// the counters of bucket j (j <= S) cleared.
+__device__ __forceinline__ void make_splitter(const Dev &d, int j, int S)
+{
+    if (j > S) return;
+    if (j < S) {
+        const unsigned long long *key = d.kb_key[0];
+        const unsigned long long k = key[(size_t)j * kBucketT];
+        d.kb_spl[j] = k;
+        if (j > 0 && key[(size_t)(j - 1) * kBucketT] > k) flag_error(d.ctl, kErrSync);
+    }
+    d.kb_bcnt[j] = 0;
+    d.kb_bfill[j] = 0;
+}
+
 // Epilogue for one body: velocity correction and store (calculateforce.cl:
 // 174-185), optionally the kick-drift-kick of integrate.cl:29-43 (mode 1), or
 // only the acceleration into the probe buffer (mode 2).

@@ -76,6 +76,7 @@ struct nb_sim {
     bool ord_ready = false; // d.gorder holds an order once ord_out has passed
     bool keys_warm = false; // d.sorted holds the last tree's body order (the build starts from it)
     bool staged = false;    // d.bnode holds pm4 in d.sorted order (the last fused update wrote it)
+    bool splitters = false; // the last bounding box worked out the next warm build's splitters
     bool sort_pending = false; // d.kb_val[0] holds the order of a build the sort stage has not taken yet
     // copyVertices staging: 2 N float4 (positions, then velocities), allocated
     // by the first nb_copy_vertices call and kept until nb_destroy
@@ -225,12 +226,12 @@ int hint_cells(const nb_sim *s, int level)
 // first larger level, and from the top down to the first larger level.
 constexpr int kTailCells = 2 * nb::kTailThreads / 8;
 
-// Groups the live cells by level. Without level sizes of an earlier tree (the
+// The live cells grouped by level, if the build has not done it. Without level sizes of an earlier tree (the
 // first step of a state) it reads this tree's back, the only host wait inside
 // a step; later steps size their launches from the last sizes read.
 int prepare_levels(nb_sim *s)
 {
-    hipError_t e = nb::launch_levels(s->d, s->stream);
+    const hipError_t e = nb::build_levels(s->d.n) ? hipSuccess : nb::launch_levels(s->d, s->stream);
     if (e != hipSuccess) return fail(s, NB_E_HIP, "level grouping launch: %s", hipGetErrorString(e));
     if (!s->hint_valid) {
         nb::Ctl c;
@@ -312,9 +313,13 @@ int launch_stage(nb_sim *s, int stage)
     hipError_t e = hipSuccess;
     const int fused = (s->p.flags & NB_FUSED_UPDATE) ? 1 : 0;
     switch (stage) {
-    case NB_STAGE_BBOX: e = nb::launch_bbox(d, s->bbox_blocks, s->stream); break;
+    case NB_STAGE_BBOX:
+        e = nb::launch_bbox(d, s->bbox_blocks, s->keys_warm, s->stream);
+        s->splitters = s->keys_warm;
+        break;
     case NB_STAGE_BUILD:
-        e = nb::launch_build_keys(d, s->keys_warm, s->keys_warm && s->staged, s->stream);
+        e = nb::launch_build_keys(d, s->keys_warm, s->keys_warm && s->staged, s->splitters, s->stream);
+        s->splitters = false; // the build replaces the keys they were taken from
         s->sort_pending = e == hipSuccess;
         break;
     case NB_STAGE_SUMMARIZE: {
@@ -507,7 +512,7 @@ void free_all(nb_sim *s)
     if (s->ord) (void)hipStreamSynchronize(s->ord); // it may still be writing d.gorder
     void *ptrs[] = {d.ctl,   d.pm4,   d.vel4,   d.acc4,          d.pos64,    d.slot,
                     d.cinfo, d.count, d.com64,         d.cchild,   d.lvl_list, d.clvl,
-                    d.lvl_blockhist,  d.cdata,  d.bnode,  d.sorted, d.probe, d.bbox_part, d.gcost, d.gorder,
+                    d.lvl_blockhist, d.lvl_count, d.cdata,  d.bnode,  d.sorted, d.probe, d.bbox_part, d.gcost, d.gorder,
                     s->chk_idx, s->chk_part, s->chk_out, d.cq64, d.cqa, d.cqb, d.cmac,
                     s->mlpbuf, s->chk_acc, s->vtx, d.kb_key[0], d.kb_key[1], d.kb_val[0], d.kb_val[1],
                     d.kb_deep, d.kb_hist, d.kb_offs, d.kb_tot, d.kb_ipar, d.kb_lpar, d.kb_lo,
@@ -774,6 +779,7 @@ int nb_create(const nb_params *p, nb_sim **out)
     ok = ok && dalloc(&d.cchild, 8 * cap) == hipSuccess;
     ok = ok && dalloc(&d.lvl_list, cap) == hipSuccess && dalloc(&d.clvl, cap) == hipSuccess;
     ok = ok && dalloc(&d.lvl_blockhist, (size_t)nb::kLevelBlocks * nb::kMaxDepth) == hipSuccess;
+    ok = ok && dalloc(&d.lvl_count, (size_t)2 * nb::kMaxDepth * nb::kLevelLine) == hipSuccess;
     ok = ok && dalloc(&d.cdata, 8 * cap) == hipSuccess;
     ok = ok && dalloc(&d.bnode, (size_t)n) == hipSuccess && dalloc(&d.probe, (size_t)n) == hipSuccess;
     ok = ok && dalloc(&d.sorted, (size_t)n) == hipSuccess;
@@ -873,6 +879,7 @@ int nb_set_state(nb_sim *s, const float *x, const float *y, const float *z, cons
     s->ord_ready = false;  // the launch order of the coarse traversal belongs to the old bodies
     s->keys_warm = false;  // and so does sorted[]: the next build sorts from scratch
     s->staged = false;
+    s->splitters = false;
     s->sort_pending = false;
     reset_control(s);
     s->have_state = true;

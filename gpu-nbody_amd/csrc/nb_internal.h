@@ -145,6 +145,7 @@ struct Dev {
     int *lvl_list;
     unsigned char *clvl; // cap: each cell's level, or kNotLive (level histogram -> scatter)
     int *lvl_blockhist; // kLevelBlocks * kMaxDepth
+    int *lvl_count;     // cells per level of the tree in the build, then how many k_link has placed (kLevelLine apart)
     float4 *bnode;
     int *sorted;
     float4 *probe;      // accelerations of a probe force pass (error checks)
@@ -168,16 +169,27 @@ struct Dev {
 };
 
 // ---- launchers (nb_tree.hip, nb_force.hip) ---------------------------------
-hipError_t launch_bbox(const Dev &d, int blocks, hipStream_t st);
+// splitters: also those of a warm build, from the last tree's sorted keys
+hipError_t launch_bbox(const Dev &d, int blocks, bool splitters, hipStream_t st);
 // the build from sorted octant-path keys (the same child slots and cell records)
 // warm: start from sorted[] and the last sorted keys; staged: bnode[] holds
-// the records in sorted[] order
-hipError_t launch_build_keys(const Dev &d, bool warm, bool staged, hipStream_t st);
+// the records in sorted[] order; splitters: launch_bbox has worked them out
+hipError_t launch_build_keys(const Dev &d, bool warm, bool staged, bool splitters, hipStream_t st);
 constexpr int kKeyTile = 2048;     // keys per radix-sort tile (first build)
-constexpr int kKeyScanTile = 1024; // cell counts per scan tile
+constexpr int kKeyScanTile = 512;  // binary nodes per scan tile (at least)
 constexpr int kBucketT = 256;      // warm builds: one splitter per kBucketT bodies
 constexpr int kBucketCap = 512;    // buckets sorted in LDS up to this size
 inline int bucket_samples(int n) { return (n + kBucketT - 1) / kBucketT; }
+// The cells grouped by level: up to kBuildLevels bodies the build's last two
+// kernels scan the cell counts and group the cells themselves, by counters of
+// the levels in device memory; for more, two launches scan and launch_levels'
+// three group. A step (Plummer, theta 1.2) with the five launches less: 16,384
+// bodies 150 -> 133 us, 262,144 309 -> 297, 524,288 404 -> 397; at 1M the two
+// ways are equal, and at 4M the waits inside the build's blocks cost 22 us more
+// than the launches they save.
+constexpr int kBuildLevels = 524288;
+inline bool build_levels(int n) { return n <= kBuildLevels; }
+constexpr int kLevelLine = 32; // a level's counters, a cache line each
 hipError_t launch_levels(const Dev &d, hipStream_t st); // group live cells by level
 // Summarize and sort read each level's cell count on the device; the host's
 // cells_hint (the level's size in an earlier tree) only sizes the grid. The

@@ -64,6 +64,19 @@ __device__ __forceinline__ void key_descend(float &cx, float &cy, float &cz, flo
     r = rh;
 }
 
+// The level counters of the tree to be built, and no levels until it is there
+// (one block of at least kMaxDepth threads): a build that an error stops leaves
+// none to summarize.
+__device__ __forceinline__ void clear_levels(const Dev &d)
+{
+    const int t = threadIdx.x;
+    if (t < kMaxDepth) d.lvl_count[t * kLevelLine] = d.lvl_count[(kMaxDepth + t) * kLevelLine] = 0;
+    if (t == 0) {
+        d.ctl->levels = 0;
+        d.ctl->live_cells = 0;
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Keys: 21 levels of each body's octant path, level 0 in bits 62..60, for the
 // bodies in the order `order` (the identity when null).
@@ -72,6 +85,7 @@ __global__ __launch_bounds__(256) void k_keys(Dev d, const int *__restrict__ ord
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     const Ctl *ctl = d.ctl;
+    if (blockIdx.x == 0) clear_levels(d);
     if (i >= d.n || ctl->error) return;
     const int b = order ? order[i] : i;
     const float4 p = d.pm4[b];
@@ -249,7 +263,8 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_scatter(const unsigned long l
 // (sorted[]), which the new keys nearly keep, and the last tree's sorted keys
 // are still in kb_key[0]. Bucketing by splitters taken from those keys then
 // moves most bodies a short way and every bucket is small:
-//   * splitters: every kBucketT-th of the last tree's sorted keys;
+//   * splitters: every kBucketT-th of the last tree's sorted keys (with the
+//     bounding box, make_splitter);
 //   * a body's bucket: the number of splitters <= its key. A block's bodies
 //     are consecutive in the last order, so their buckets are nearly all in
 //     a window of kWin around the one their places suggest: searched in an
@@ -270,23 +285,11 @@ constexpr int kBsPerThread = kBucketCap / kBsThreads;
 static_assert(kBucketCap % kBsThreads == 0, "whole rows of the block");
 static_assert(kBsThreads == kRsBins, "a thread per digit");
 
-// Splitters spl[0 .. S-1]: the keys at positions j * kBucketT of `key` (the
-// last tree's sorted keys, so non-decreasing: a decrease means the buffer does
-// not hold them and stops the build with an error); the bucket counters
-// cleared.
-__global__ __launch_bounds__(256) void k_splitters(Ctl *ctl, const unsigned long long *__restrict__ key, int S,
-                                                   unsigned long long *__restrict__ spl, unsigned *__restrict__ bcnt,
-                                                   unsigned *__restrict__ bfill)
+// the splitters of the next warm build alone (launch_bbox does it otherwise)
+__global__ __launch_bounds__(256) void k_splitters(Dev d, int S)
 {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (ctl->error || j > S) return;
-    if (j < S) {
-        const unsigned long long k = key[(size_t)j * kBucketT];
-        spl[j] = k;
-        if (j > 0 && key[(size_t)(j - 1) * kBucketT] > k) flag_error(ctl, kErrSync);
-    }
-    bcnt[j] = 0;
-    bfill[j] = 0;
+    if (d.ctl->error) return;
+    make_splitter(d, blockIdx.x * blockDim.x + threadIdx.x, S);
 }
 
 // the first j with spl[j] > k (S if none): spl is non-decreasing; searched
@@ -399,6 +402,7 @@ __global__ __launch_bounds__(256) void k_keys_warm(Dev d, const int *__restrict_
     const int t = threadIdx.x, first = blockIdx.x * kWarmBodies;
     const int n = d.n;
     const Ctl *ctl = d.ctl;
+    if (blockIdx.x == 0) clear_levels(d);
     if (ctl->error) return;
     const int w0 = first / kBucketT + 1 - kWin / 4;
     if (t < kWin) h[t] = 0;
@@ -507,15 +511,40 @@ __global__ __launch_bounds__(1024) void k_bucket_scan(const Ctl *ctl, const unsi
 
 // Each body takes the next place of its bucket: LDS counters for the buckets
 // of the block's window (one global atomic per bucket and block), a global
-// atomic for a bucket outside it.
+// atomic for a bucket outside it. SCAN (S < kScatterScan): every block works out
+// the buckets' starts from their counts by itself, and the first block keeps
+// them for the sort; a launch less (4.5 us) for about 1 us of it.
+constexpr int kScatterScan = 1024;
+
+// exclusive scan of v over 256 threads, wave by wave; wsum: 4 words of LDS.
+// Ends with wsum[3] = the total.
+__device__ __forceinline__ unsigned scan256_total(unsigned v, unsigned *wsum)
+{
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    unsigned x = v;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const unsigned y = __shfl_up(x, o);
+        if (lane >= o) x += y;
+    }
+    if (lane == 63) wsum[w] = x;
+    __syncthreads();
+    const unsigned w0 = wsum[0], w1 = wsum[1], w2 = wsum[2], w3 = wsum[3];
+    __syncthreads();
+    if (t == 0) wsum[3] = w0 + w1 + w2 + w3;
+    return x - v + (w > 0 ? w0 : 0u) + (w > 1 ? w1 : 0u) + (w > 2 ? w2 : 0u);
+}
+
+template <bool SCAN>
 __global__ __launch_bounds__(256) void k_bucket_scatter(const Ctl *ctl, const unsigned long long *__restrict__ kin,
                                                         const int *__restrict__ vin, const int *__restrict__ bid,
                                                         unsigned long long *__restrict__ kout, int *__restrict__ vout,
-                                                        int n, const unsigned *__restrict__ bstart,
-                                                        unsigned *__restrict__ bfill)
+                                                        int n, const unsigned *__restrict__ bcnt, int S,
+                                                        unsigned *__restrict__ bstart, unsigned *__restrict__ bfill)
 {
     __shared__ unsigned h[kWin], hb[kWin];
-    if (ctl->error) return;
+    __shared__ unsigned starts[SCAN ? kScatterScan : 1], wsum[4];
+    const int err = ctl->error;
     const int t = threadIdx.x, first = blockIdx.x * kWinBodies;
     const int w0 = first / kBucketT + 1 - kWin / 4;
     if (t < kWin) h[t] = 0;
@@ -528,7 +557,26 @@ __global__ __launch_bounds__(256) void k_bucket_scatter(const Ctl *ctl, const un
         v[j] = vin[i];
         b[j] = bid[i];
     }
-    __syncthreads();
+    if (SCAN) {
+        unsigned c[4], sum = 0;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int i = 4 * t + q;
+            c[q] = i <= S ? bcnt[i] : 0u;
+            sum += c[q];
+        }
+        unsigned run = scan256_total(sum, wsum);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int i = 4 * t + q;
+            starts[i] = run;
+            if (blockIdx.x == 0 && i <= S) bstart[i] = run;
+            run += c[q];
+        }
+        if (blockIdx.x == 0 && t == 0) bstart[S + 1] = (unsigned)n;
+    }
+    if (__syncthreads_or(err)) return;
+    const auto start = [&](int bk) { return SCAN ? starts[bk] : bstart[bk]; };
     unsigned at[kWinPer];
 #pragma unroll
     for (int j = 0; j < kWinPer; ++j) {
@@ -536,10 +584,10 @@ __global__ __launch_bounds__(256) void k_bucket_scatter(const Ctl *ctl, const un
         const unsigned o = (unsigned)(b[j] - w0);
         const bool inwin = valid && o < (unsigned)kWin;
         at[j] = claim_bin(h, inwin ? (int)o : 0, inwin);
-        if (valid && !inwin) at[j] = bstart[b[j]] + atomicAdd(&bfill[b[j]], 1u);
+        if (valid && !inwin) at[j] = start(b[j]) + atomicAdd(&bfill[b[j]], 1u);
     }
     __syncthreads();
-    if (t < kWin) hb[t] = h[t] ? bstart[w0 + t] + atomicAdd(&bfill[w0 + t], h[t]) : 0u;
+    if (t < kWin) hb[t] = h[t] ? start(w0 + t) + atomicAdd(&bfill[w0 + t], h[t]) : 0u;
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < kWinPer; ++j) {
@@ -1069,13 +1117,14 @@ __device__ __forceinline__ int delta_at(const K &ka, const unsigned long long *_
 
 struct BinOut {
     int *__restrict__ iparent, *__restrict__ lparent, *__restrict__ lo, *__restrict__ own, *__restrict__ ktop;
+    int *__restrict__ obase, *__restrict__ tsum, *__restrict__ tdep;
 };
 
-// Internal node i: its searches, then its outputs. dir and dmin come from
-// the neighbours i - 1 and i + 1. n <= 2^26 (the pool limit), so every probe
-// fits an int.
+// Internal node i: its searches, then its outputs (own and top also returned).
+// dir and dmin come from the neighbours i - 1 and i + 1. n <= 2^26 (the pool
+// limit), so every probe fits an int.
 template <class K>
-__device__ __forceinline__ void bintree_node(const Dev &d, const K &ka, const unsigned long long *__restrict__ deep,
+__device__ __forceinline__ int2 bintree_node(const Dev &d, const K &ka, const unsigned long long *__restrict__ deep,
                                              int n, int i, const BinOut &o)
 {
     const unsigned long long ki = ka(i);
@@ -1110,39 +1159,99 @@ __device__ __forceinline__ void bintree_node(const Dev &d, const K &ka, const un
         flag_error(d.ctl, kErrDepth);
         kb = kBuildLevelLimit - 1;
     }
-    o.own[i] = max(0, kb - kt + 1);
+    const int own = max(0, kb - kt + 1);
+    o.own[i] = own;
     o.ktop[i] = kt;
+    return make_int2(own, kt);
 }
 
+// SCAN: a block's nodes are also a tile of the scan of the cells that the nodes
+// hold (-> their first cells): obase = the cells of the tile's earlier nodes,
+// tsum = the tile's cells, tdep = the tile's depth (the deepest cell's level +
+// 1: its children are bodies); and the cells of each level are counted.
+template <bool SCAN>
 __global__ __launch_bounds__(kBtThreads) void k_bintree(Dev d, const unsigned long long *__restrict__ key,
                                                         const unsigned long long *__restrict__ deep, BinOut o)
 {
     __shared__ unsigned long long ks[kBtSpan];
-    const int n = d.n;
+    __shared__ int wsum[SCAN ? kBtThreads / 64 : 1], wdep[SCAN ? kBtThreads / 64 : 1];
+    __shared__ int h[SCAN ? kMaxDepth : 1];
+    const int n = d.n, t = threadIdx.x, lane = t & 63, w = t >> 6;
     Ctl *ctl = d.ctl;
     if (ctl->error) return; // block-uniform
     const int base = (int)blockIdx.x * kBtThreads - kBtHalo;
-    for (int t = threadIdx.x; t < kBtSpan; t += kBtThreads) {
-        const int g = base + t;
-        ks[t] = g >= 0 && g < n ? key[g] : 0ull;
+    if (SCAN && t < kMaxDepth) h[t] = 0;
+    for (int u = t; u < kBtSpan; u += kBtThreads) {
+        const int g = base + u;
+        ks[u] = g >= 0 && g < n ? key[g] : 0ull;
     }
     __syncthreads();
-    const int i = (int)blockIdx.x * kBtThreads + (int)threadIdx.x;
-    if (i >= n - 1) return;
-    bintree_node(d, KeysAny{ks, key, base}, deep, n, i, o);
+    const int i = (int)blockIdx.x * kBtThreads + t;
+    int2 node = make_int2(0, 0); // cells held, level of the first
+    if (i < n - 1) node = bintree_node(d, KeysAny{ks, key, base}, deep, n, i, o);
+    if (!SCAN) return;
+    for (int k = 0; k < node.x; ++k) atomicAdd(&h[node.y + k], 1);
+    int dep = node.x > 0 ? node.y + node.x : 0;
+#pragma unroll
+    for (int q = 32; q > 0; q >>= 1) dep = max(dep, __shfl_xor(dep, q));
+    int x = node.x; // inclusive scan over the wave
+#pragma unroll
+    for (int q = 1; q < 64; q <<= 1) {
+        const int y = __shfl_up(x, q);
+        if (lane >= q) x += y;
+    }
+    if (lane == 63) {
+        wsum[w] = x;
+        wdep[w] = dep;
+    }
+    __syncthreads();
+    int before = 0, all = 0, deepest = 0;
+#pragma unroll
+    for (int q = 0; q < kBtThreads / 64; ++q) {
+        before += q < w ? wsum[q] : 0;
+        all += wsum[q];
+        deepest = max(deepest, wdep[q]);
+    }
+    if (i < n - 1) o.obase[i] = before + x - node.x;
+    if (t == 0) {
+        o.tsum[blockIdx.x] = all;
+        o.tdep[blockIdx.x] = deepest;
+    }
+    if (t < kMaxDepth && h[t]) atomicAdd(&d.lvl_count[t * kLevelLine], h[t]);
+}
+
+// the running maximum of the depths (buildtree.cl:199)
+__device__ __forceinline__ void raise_depth(Ctl *ctl, int dep)
+{
+    if (dep > 0) __hip_atomic_fetch_max(&ctl->max_depth, dep, __ATOMIC_RELAXED, AGENT);
+}
+
+// The cell count C (the total of the scan), the pool check and the root's
+// record: by one thread.
+__device__ __forceinline__ void finish_count(const Dev &d, int C)
+{
+    Ctl *ctl = d.ctl;
+    if (C > d.cap) {
+        flag_error(ctl, kErrPool);
+    } else {
+        ctl->n_cells = C;
+        d.cinfo[0] = make_int4(-1, 0, (int)ctl->epoch, 0);
+    }
 }
 
 // ---------------------------------------------------------------------------
 // Exclusive scan of the cells each internal node holds (-> its first cell):
 // tiles of kScanTile scanned with their sums kept (k_scan_tiles), the sums
-// scanned by one block (k_scan_sums); readers add the two (first_cell).
-// The same passes find the tree's depth: the deepest cell's level + 1 (its
-// children are bodies), per tile and then over the tiles, into the running
-// maximum (buildtree.cl:199) with one atomic.
+// scanned by one block (k_scan_sums); readers add the two.
+// The same passes find the tree's depth: the deepest cell's level + 1, per tile
+// and then over the tiles, into the running maximum with one atomic.
+// This is the way of large trees (build_levels): the binary tree's blocks would
+// wait for their slowest node to scan, which costs more than these launches.
 // ---------------------------------------------------------------------------
 constexpr int kScanPer = 4; // one int4 per thread: coalesced
 constexpr int kScanTile = 256 * kScanPer;
-static_assert(kScanTile == kKeyScanTile, "the engine sizes the tile sums with kKeyScanTile");
+static_assert(kScanTile >= kKeyScanTile && kBtThreads >= kKeyScanTile,
+              "the engine sizes the tile sums with kKeyScanTile");
 
 __device__ __forceinline__ int4 load4(const int *__restrict__ a, int i0, int m)
 {
@@ -1193,7 +1302,7 @@ __global__ __launch_bounds__(256) void k_scan_tiles(const Ctl *ctl, const int *_
 }
 
 // one block: exclusive scan of the tile sums in place (each thread a run of
-// them); the tiles' depths into the running maximum
+// them)
 __global__ __launch_bounds__(1024) void k_scan_sums(Dev d, int *__restrict__ sums, int ntiles,
                                                    const int *__restrict__ tdepth)
 {
@@ -1233,17 +1342,8 @@ __global__ __launch_bounds__(1024) void k_scan_sums(Dev d, int *__restrict__ sum
     }
     if (t == 0) {
         for (int k = 0; k < 16; ++k) dep = max(dep, wdep[k]);
-        if (dep > 0) __hip_atomic_fetch_max(&ctl->max_depth, dep, __ATOMIC_RELAXED, AGENT);
-    }
-    // the cell count (the total of the scan), the pool check, and the root's record
-    if (t == 1023) {
-        const int C = s[1023];
-        if (C > d.cap) {
-            flag_error(ctl, kErrPool);
-        } else {
-            ctl->n_cells = C;
-            d.cinfo[0] = make_int4(-1, 0, (int)ctl->epoch, 0);
-        }
+        raise_depth(ctl, dep);
+        finish_count(d, s[1023]);
     }
 }
 
@@ -1256,29 +1356,31 @@ struct KeyTree {
     const int *val, *iparent, *lparent, *lo, *own, *ktop, *obase, *tsum;
 };
 
-__device__ __forceinline__ int first_cell(const KeyTree &kt, int i) { return kt.obase[i] + kt.tsum[i / kScanTile]; }
-
 // The deepest cell of the nearest binary ancestor (p itself included) that
 // holds a cell, or -1 (an inconsistent tree; the caller flags it). A node that
 // holds none shares its level with its parent, so the walk is at most a few
 // steps; it is bounded anyway.
-__device__ __forceinline__ int holding_cell(const KeyTree &kt, int p)
+template <class T> __device__ __forceinline__ int holding_cell(const KeyTree &kt, const T &tile, int p)
 {
     for (int steps = 0; steps < 4 * kBuildLevelLimit * 3 && p >= 0; ++steps) {
         const int o = kt.own[p];
-        if (o != 0) return first_cell(kt, p) + o - 1;
+        if (o != 0) return kt.obase[p] + tile(p) + o - 1;
         p = kt.iparent[p];
     }
     return -1;
 }
 
-// one body: the root is the one cell (k_scan_sums counts the cells otherwise)
+// one body: the root is the one cell
 __global__ void k_one_cell(Dev d)
 {
     Ctl *ctl = d.ctl;
     if (ctl->error) return;
     ctl->n_cells = 1;
     d.cinfo[0] = make_int4(-1, 0, (int)ctl->epoch, 0);
+    d.lvl_list[0] = 0;
+    for (int k = 0; k <= kMaxDepth; ++k) ctl->lvl_start[k] = k > 0 ? 1 : 0;
+    ctl->levels = 1;
+    ctl->live_cells = 1;
 }
 
 // Position g: the cells of internal node g (g < n - 1) -- each in the slot of
@@ -1292,26 +1394,41 @@ __global__ void k_one_cell(Dev d)
 constexpr int kLinkPer = 2;
 constexpr int kLinkSpan = 256 * kLinkPer;
 
-__device__ __forceinline__ int deepest_of(const KeyTree &kt, int own, int ob, int ts, int p)
+template <class T>
+__device__ __forceinline__ int deepest_of(const KeyTree &kt, const T &tile, int own, int ob, int p)
 {
-    // the holding cell of binary node p, given p's own, obase and tile sum:
-    // p itself when it holds cells, else the walk up from its parent
-    return own != 0 ? ob + ts + own - 1 : (p >= 0 ? holding_cell(kt, kt.iparent[p]) : -1);
+    // the holding cell of binary node p, given the cells it holds and the
+    // first of them: p itself when it holds any, else the walk up from its parent
+    return own != 0 ? ob + own - 1 : (p >= 0 ? holding_cell(kt, tile, kt.iparent[p]) : -1);
 }
 
-__global__ __launch_bounds__(256) void k_link(Dev d, KeyTree kt)
+// SCAN (after k_bintree<true>, at most kLinkSums tiles): every block scans the
+// tile sums by itself, and the first block does what k_scan_sums does with
+// their total; a block also puts its cells into the lists of their levels
+// (lvl_list): it counts them by level, takes that many places of each level
+// with one atomic, and places them as it writes the cells.
+constexpr int kLinkSums = 1024;
+static_assert(kBuildLevels <= kLinkSums * kBtThreads, "k_link scans the tiles of every tree it groups by level");
+
+template <bool SCAN>
+__global__ __launch_bounds__(256) void k_link(Dev d, KeyTree kt, int ntiles, const int *__restrict__ tdep)
 {
-    const int n = d.n;
+    constexpr int kTile = SCAN ? kBtThreads : kScanTile;
+    __shared__ int sums[SCAN ? kLinkSums : 1];
+    __shared__ unsigned wsum[4];
+    __shared__ int h[SCAN ? kMaxDepth : 1], at[SCAN ? kMaxDepth : 1];
+    const int n = d.n, t = threadIdx.x;
     Ctl *ctl = d.ctl;
-    if (ctl->error) return;
+    const int err = ctl->error;
     const uint32_t ep = ctl->epoch;
-    const int g0 = blockIdx.x * kLinkSpan + threadIdx.x;
+    const int g0 = blockIdx.x * kLinkSpan + t;
     if (n < 2) { // the root holds the one body
-        if (g0 == 0) d.slot[key_digit(kt.key, kt.deep, n, 0, 0)] = slot_tag(ep, kt.val[0]);
+        if (g0 == 0 && !err) d.slot[key_digit(kt.key, kt.deep, n, 0, 0)] = slot_tag(ep, kt.val[0]);
         return;
     }
+    if (SCAN && t < kMaxDepth) h[t] = 0;
     // round 1: each position's node and leaf records and the keys around it
-    int own[kLinkPer], top[kLinkPer], lo[kLinkPer], ip[kLinkPer], ob[kLinkPer], ts[kLinkPer], lp[kLinkPer];
+    int own[kLinkPer], top[kLinkPer], lo[kLinkPer], ip[kLinkPer], ob[kLinkPer], lp[kLinkPer];
     int body[kLinkPer];
     unsigned long long kg[kLinkPer], km[kLinkPer], kq[kLinkPer];
 #pragma unroll
@@ -1323,26 +1440,81 @@ __global__ __launch_bounds__(256) void k_link(Dev d, KeyTree kt)
         lo[u] = kt.lo[gi];
         ip[u] = kt.iparent[gi];
         ob[u] = kt.obase[gi];
-        ts[u] = kt.tsum[gi / kScanTile];
         lp[u] = kt.lparent[g];
         body[u] = kt.val[g];
         kg[u] = kt.key[g];
         km[u] = kt.key[max(g - 1, 0)];
         kq[u] = kt.key[min(g + 1, n - 1)];
     }
+    if (SCAN) {
+        constexpr int per = kLinkSums / 256;
+        unsigned c[per], sum = 0;
+#pragma unroll
+        for (int q = 0; q < per; ++q) {
+            const int j = per * t + q;
+            c[q] = j < ntiles ? (unsigned)kt.tsum[j] : 0u;
+            sum += c[q];
+        }
+        unsigned run = scan256_total(sum, wsum);
+#pragma unroll
+        for (int q = 0; q < per; ++q) {
+            sums[per * t + q] = (int)run;
+            run += c[q];
+        }
+    }
+    // the same decision in every wave: another block may flag an error meanwhile
+    if (__syncthreads_or(err)) return;
+    if (SCAN) {
+        const int C = (int)wsum[3];
+        if (blockIdx.x == 0) {
+            int dep = 0;
+            for (int j = t; j < ntiles; j += 256) dep = max(dep, tdep[j]);
+#pragma unroll
+            for (int q = 32; q > 0; q >>= 1) dep = max(dep, __shfl_xor(dep, q));
+            if ((t & 63) == 0) raise_depth(ctl, dep);
+            if (t == 0) finish_count(d, C);
+        }
+        if (C > d.cap) return; // every block sees it: no cell is written
+    }
+    const auto tile = [&](int i) { return SCAN ? sums[i / kTile] : kt.tsum[i / kTile]; };
     // round 2: the parents' records, and the key of each node's first body
-    int own_ip[kLinkPer], ob_ip[kLinkPer], ts_ip[kLinkPer], own_lp[kLinkPer], ob_lp[kLinkPer], ts_lp[kLinkPer];
+    int own_ip[kLinkPer], ob_ip[kLinkPer], own_lp[kLinkPer], ob_lp[kLinkPer];
     unsigned long long klo[kLinkPer];
 #pragma unroll
     for (int u = 0; u < kLinkPer; ++u) {
         const int ipc = max(ip[u], 0);
         own_ip[u] = kt.own[ipc];
-        ob_ip[u] = kt.obase[ipc];
-        ts_ip[u] = kt.tsum[ipc / kScanTile];
+        ob_ip[u] = kt.obase[ipc] + tile(ipc);
         own_lp[u] = kt.own[lp[u]];
-        ob_lp[u] = kt.obase[lp[u]];
-        ts_lp[u] = kt.tsum[lp[u] / kScanTile];
+        ob_lp[u] = kt.obase[lp[u]] + tile(lp[u]);
         klo[u] = kt.key[lo[u]];
+    }
+    if (SCAN) {
+#pragma unroll
+        for (int u = 0; u < kLinkPer; ++u)
+            if (g0 + u * 256 < n - 1)
+                for (int k = 0; k < own[u]; ++k) atomicAdd(&h[top[u] + k], 1);
+        __syncthreads();
+        if (t < kMaxDepth) { // the first wave
+            const int cells = d.lvl_count[t * kLevelLine];
+            int x = cells;
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const int y = __shfl_up(x, o);
+                if (t >= o) x += y;
+            }
+            at[t] = x - cells + (h[t] ? atomicAdd(&d.lvl_count[(kMaxDepth + t) * kLevelLine], h[t]) : 0);
+            if (blockIdx.x == 0) {
+                const unsigned long long some = __ballot(cells > 0);
+                ctl->lvl_start[t] = x - cells;
+                if (t == kMaxDepth - 1) {
+                    ctl->lvl_start[kMaxDepth] = x;
+                    ctl->live_cells = x;
+                    ctl->levels = 64 - __clzll((long long)some);
+                }
+            }
+        }
+        __syncthreads();
     }
 #pragma unroll
     for (int u = 0; u < kLinkPer; ++u) {
@@ -1351,13 +1523,13 @@ __global__ __launch_bounds__(256) void k_link(Dev d, KeyTree kt)
         if (g < n - 1 && own[u] > 0) {
             int par = -1;
             if (top[u] > 0) {
-                par = deepest_of(kt, own_ip[u], ob_ip[u], ts_ip[u], ip[u]);
+                par = deepest_of(kt, tile, own_ip[u], ob_ip[u], ip[u]);
                 if (par < 0) {
                     flag_error(ctl, kErrSync);
                     return;
                 }
             }
-            const int base = ob[u] + ts[u];
+            const int base = ob[u] + tile(g);
             for (int k = top[u]; k < top[u] + own[u]; ++k) {
                 const int cid = base + (k - top[u]);
                 if (k > 0) {
@@ -1367,10 +1539,11 @@ __global__ __launch_bounds__(256) void k_link(Dev d, KeyTree kt)
                     d.slot[(size_t)par * 8 + dg] = slot_tag(ep, n + cid);
                     d.cinfo[cid] = make_int4(par, k | (dg << 8), (int)ep, 0);
                 }
+                if (SCAN) d.lvl_list[atomicAdd(&at[k], 1)] = cid;
                 par = cid;
             }
         }
-        const int par = deepest_of(kt, own_lp[u], ob_lp[u], ts_lp[u], lp[u]);
+        const int par = deepest_of(kt, tile, own_lp[u], ob_lp[u], lp[u]);
         if (par < 0) {
             flag_error(ctl, kErrSync);
             return;
@@ -1393,7 +1566,7 @@ __global__ __launch_bounds__(256) void k_link(Dev d, KeyTree kt)
 // ---------------------------------------------------------------------------
 // launcher
 // ---------------------------------------------------------------------------
-hipError_t launch_build_keys(const Dev &d, bool warm, bool staged, hipStream_t st)
+hipError_t launch_build_keys(const Dev &d, bool warm, bool staged, bool splitters, hipStream_t st)
 {
     const int n = d.n;
     const dim3 b256(256), g256((n + 255) / 256);
@@ -1406,13 +1579,17 @@ hipError_t launch_build_keys(const Dev &d, bool warm, bool staged, hipStream_t s
         // (the buckets of the bodies go to kb_lo, which the binary tree fills later)
         const int S = bucket_samples(n);
         const dim3 gw((n + kWinBodies - 1) / kWinBodies);
-        hipLaunchKernelGGL(k_splitters, dim3((S + 1 + 255) / 256), b256, 0, st, d.ctl, ka, S, d.kb_spl, d.kb_bcnt,
-                           d.kb_bfill);
+        if (!splitters) hipLaunchKernelGGL(k_splitters, dim3((S + 1 + 255) / 256), b256, 0, st, d, S);
         hipLaunchKernelGGL(k_keys_warm, dim3((n + kWarmBodies - 1) / kWarmBodies), b256, 0, st, d, d.sorted,
                            staged ? d.bnode : nullptr, d.kb_spl, S, kb, vb, d.kb_lo, d.kb_bcnt);
-        hipLaunchKernelGGL(k_bucket_scan, dim3(1), dim3(1024), 0, st, d.ctl, d.kb_bcnt, S, d.kb_bstart);
-        hipLaunchKernelGGL(k_bucket_scatter, gw, b256, 0, st, d.ctl, kb, vb, d.kb_lo, ka, va, n, d.kb_bstart,
-                           d.kb_bfill);
+        if (S < kScatterScan) {
+            hipLaunchKernelGGL(k_bucket_scatter<true>, gw, b256, 0, st, d.ctl, kb, vb, d.kb_lo, ka, va, n, d.kb_bcnt, S,
+                               d.kb_bstart, d.kb_bfill);
+        } else {
+            hipLaunchKernelGGL(k_bucket_scan, dim3(1), dim3(1024), 0, st, d.ctl, d.kb_bcnt, S, d.kb_bstart);
+            hipLaunchKernelGGL(k_bucket_scatter<false>, gw, b256, 0, st, d.ctl, kb, vb, d.kb_lo, ka, va, n, d.kb_bcnt,
+                               S, d.kb_bstart, d.kb_bfill);
+        }
         // (the binary tree's arrays, written later, serve the runs of large buckets)
         hipLaunchKernelGGL(k_bucket_sort, dim3(S + 1), dim3(kBsThreads), 0, st, d, ka, va, d.kb_deep, kb, vb, d.kb_ipar,
                            d.kb_lpar, d.kb_bstart);
@@ -1437,18 +1614,22 @@ hipError_t launch_build_keys(const Dev &d, bool warm, bool staged, hipStream_t s
         hipLaunchKernelGGL(k_deep_runs, g256, b256, 0, st, d, ka, va, d.kb_deep, d.kb_ipar, d.kb_lpar, kb, vb);
     }
     KeyTree kt{ka, d.kb_deep, va, d.kb_ipar, d.kb_lpar, d.kb_lo, d.kb_own, d.kb_ktop, d.kb_obase, d.kb_scan};
-    if (n >= 2) {
-        const dim3 gi((n - 1 + kBtThreads - 1) / kBtThreads);
-        const BinOut bo{d.kb_ipar, d.kb_lpar, d.kb_lo, d.kb_own, d.kb_ktop};
-        hipLaunchKernelGGL(k_bintree, gi, dim3(kBtThreads), 0, st, d, ka, d.kb_deep, bo);
+    const dim3 gl((n + kLinkSpan - 1) / kLinkSpan), gi((n + kBtThreads - 2) / kBtThreads);
+    const BinOut bo{d.kb_ipar, d.kb_lpar, d.kb_lo, d.kb_own, d.kb_ktop, d.kb_obase, d.kb_scan, d.kb_tdep};
+    if (n < 2) {
+        hipLaunchKernelGGL(k_one_cell, dim3(1), dim3(1), 0, st, d);
+        hipLaunchKernelGGL(k_link<false>, gl, b256, 0, st, d, kt, 0, d.kb_tdep);
+    } else if (build_levels(n)) {
+        hipLaunchKernelGGL(k_bintree<true>, gi, dim3(kBtThreads), 0, st, d, ka, d.kb_deep, bo);
+        hipLaunchKernelGGL(k_link<true>, gl, b256, 0, st, d, kt, (int)gi.x, d.kb_tdep);
+    } else {
         const int m = n - 1, nt = (m + kScanTile - 1) / kScanTile;
+        hipLaunchKernelGGL(k_bintree<false>, gi, dim3(kBtThreads), 0, st, d, ka, d.kb_deep, bo);
         hipLaunchKernelGGL(k_scan_tiles, dim3(nt), dim3(256), 0, st, d.ctl, d.kb_own, d.kb_ktop, d.kb_obase, m,
                            d.kb_scan, d.kb_tdep);
         hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(1024), 0, st, d, d.kb_scan, nt, d.kb_tdep);
-    } else {
-        hipLaunchKernelGGL(k_one_cell, dim3(1), dim3(1), 0, st, d);
+        hipLaunchKernelGGL(k_link<false>, gl, b256, 0, st, d, kt, nt, d.kb_tdep);
     }
-    hipLaunchKernelGGL(k_link, dim3((n + kLinkSpan - 1) / kLinkSpan), b256, 0, st, d, kt);
     return hipGetLastError();
 }
 

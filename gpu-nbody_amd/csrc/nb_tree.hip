@@ -8,11 +8,9 @@
 // (On MI355X each XCD has its own L2; an agent-scope acquire/release costs an
 // L2 invalidate / write-back, which is why the per-cell hand-offs of the
 // reference's summarize are replaced by level launches.)
-#include "nb_internal.h"
+#include "nb_device.h"
 
 namespace nb {
-
-#define AGENT __HIP_MEMORY_SCOPE_AGENT
 
 __device__ __forceinline__ int dec_slot(unsigned long long w, uint32_t ep)
 {
@@ -24,13 +22,6 @@ __device__ __forceinline__ int dec_slot(unsigned long long w, uint32_t ep)
 __device__ __forceinline__ int octant(float cx, float cy, float cz, float bx, float by, float bz)
 {
     return (cx < bx ? 1 : 0) | (cy < by ? 2 : 0) | (cz < bz ? 4 : 0);
-}
-
-__device__ __forceinline__ void set_error(Ctl *ctl, int code)
-{
-    int expected = 0;
-    __hip_atomic_compare_exchange_strong(&ctl->error, &expected, code, __ATOMIC_RELAXED,
-                                         __ATOMIC_RELAXED, AGENT);
 }
 
 // A cell is in the tree when its record carries this tree's epoch: the build
@@ -47,14 +38,23 @@ __device__ __forceinline__ bool cell_live(const Dev &d, int c, uint32_t ep, int 
 }
 
 // ---------------------------------------------------------------------------
-// Stage 1: bounding box (boundingbox.cl:20-199). Two launches: min/max per
-// block (wave64 shuffle reduction, one partial per block), then one block
-// combines the partials and sets up the root, the opening table and the
-// per-step counters. The launch boundary orders the two, where the
-// reference's last-block hand-off (boundingbox.cl:133-196) needs an
-// agent-scope release per block: on MI355X an L2 write-back each, which cost
-// about 40 us per step at 4M bodies against 11 us for the reads.
+// Stage 1: bounding box (boundingbox.cl:20-199): min/max per block (wave64
+// shuffle reduction), then the root, the opening table and the per-step
+// counters. Up to kBoxOne bodies one block of 1024 threads does it all: it
+// reads 512 KiB in about the time of one launch, which it saves (16,384
+// bodies: 9.1 us of two launches -> 6.7 us). More bodies take two launches,
+// one partial per block and one block that combines them; the launch boundary
+// orders the two, where the reference's last-block hand-off
+// (boundingbox.cl:133-196) needs an agent-scope release per block: on MI355X
+// an L2 write-back each, which cost about 40 us per step at 4M bodies against
+// 11 us for the reads.
+//
+// The splitters of a warm build (S >= 0: there are S) go with the box: neither
+// needs the other, and alone they were a launch of 4.6 us.
 // ---------------------------------------------------------------------------
+constexpr int kBoxOne = 32768;
+constexpr int kBoxOneThreads = 1024;
+
 __device__ __forceinline__ float wave_min(float v)
 {
 #pragma unroll
@@ -68,7 +68,7 @@ __device__ __forceinline__ float wave_max(float v)
     return v;
 }
 
-__device__ void block_minmax(float v[6], float (*part)[6])
+template <int T> __device__ __forceinline__ void block_minmax(float v[6], float (*part)[6])
 {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
 #pragma unroll
@@ -81,7 +81,7 @@ __device__ void block_minmax(float v[6], float (*part)[6])
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-        for (int j = 1; j < (int)(blockDim.x >> 6); ++j) {
+        for (int j = 1; j < T / 64; ++j) {
 #pragma unroll
             for (int k = 0; k < 3; ++k) v[k] = fminf(v[k], part[j][k]);
 #pragma unroll
@@ -96,9 +96,32 @@ __device__ __forceinline__ void minmax_into(float v[6], float4 q)
     v[3] = fmaxf(v[3], q.x); v[4] = fmaxf(v[4], q.y); v[5] = fmaxf(v[5], q.z);
 }
 
-__global__ __launch_bounds__(256) void k_bbox(Dev d)
+// by one thread: the box w of all bodies
+__device__ __forceinline__ void finish_box(const Dev &d, const float w[6])
 {
-    __shared__ float part[4][6];
+    Ctl *c = d.ctl;
+    // root cell, boundingbox.cl:171-189
+    c->root[0] = 0.5f * (w[0] + w[3]);
+    c->root[1] = 0.5f * (w[1] + w[4]);
+    c->root[2] = 0.5f * (w[2] + w[5]);
+    const float radius = 0.5f * fmaxf(fmaxf(w[3] - w[0], w[4] - w[1]), w[5] - w[2]);
+    c->radius = radius;
+    // opening thresholds, calculateforce.cl:52-67 (FP32 quotient via a
+    // double division rounded once = the correctly rounded FP32 quotient)
+    float raw = radius * radius;
+    if (d.theta2 > 0.0f) raw = (float)((double)raw / (double)d.theta2);
+    for (int i = 0; i < kMaxDepth; ++i) {
+        c->dq[i] = raw + d.eps2;
+        raw = 0.25f * raw;
+    }
+    c->n_cells = 1; // the root is cell 0 (reference: _bottom = NUMBER_OF_NODES, :180)
+    c->epoch += 1;  // every child slot of the last tree turns stale
+    c->step += 1;   // boundingbox.cl:195
+}
+
+template <int T, bool ONE> __global__ __launch_bounds__(T) void k_bbox(Dev d, int S)
+{
+    __shared__ float part[T / 64][6];
     // a device error stops the pipeline until the host has seen it: the steps
     // that were already queued behind it change nothing
     if (d.ctl->error) return;
@@ -110,8 +133,8 @@ __global__ __launch_bounds__(256) void k_bbox(Dev d)
     // span per wave and iteration: body j is read by wave (j / 256) mod W at
     // element j mod 256.
     const int lane = threadIdx.x & 63;
-    const long long nwaves = ((long long)gridDim.x * blockDim.x) >> 6;
-    long long i = (((long long)blockIdx.x * blockDim.x + threadIdx.x) >> 6) * 256 + lane;
+    const long long nwaves = ((long long)gridDim.x * T) >> 6;
+    long long i = (((long long)blockIdx.x * T + threadIdx.x) >> 6) * 256 + lane;
     for (; i + 192 < n; i += nwaves * 256) {
         float4 q[4];
 #pragma unroll
@@ -124,10 +147,15 @@ __global__ __launch_bounds__(256) void k_bbox(Dev d)
         if (i + 64 * u >= n) break;
         minmax_into(v, d.pm4[i + 64 * u]);
     }
-    block_minmax(v, part);
+    for (int j = blockIdx.x * T + threadIdx.x; j <= S; j += gridDim.x * T) make_splitter(d, j, S);
+    block_minmax<T>(v, part);
     if (threadIdx.x == 0) {
+        if (ONE) {
+            finish_box(d, v);
+        } else {
 #pragma unroll
-        for (int k = 0; k < 6; ++k) d.bbox_part[6 * blockIdx.x + k] = v[k];
+            for (int k = 0; k < 6; ++k) d.bbox_part[6 * blockIdx.x + k] = v[k];
+        }
     }
 }
 
@@ -135,8 +163,7 @@ __global__ __launch_bounds__(256) void k_bbox(Dev d)
 __global__ __launch_bounds__(256) void k_bbox_final(Dev d, int blocks)
 {
     __shared__ float part[4][6];
-    Ctl *c = d.ctl;
-    if (c->error) return;
+    if (d.ctl->error) return;
     float w[6] = {d.bbox_part[0], d.bbox_part[1], d.bbox_part[2], d.bbox_part[3], d.bbox_part[4],
                   d.bbox_part[5]};
     for (int b = threadIdx.x; b < blocks; b += blockDim.x) {
@@ -144,26 +171,8 @@ __global__ __launch_bounds__(256) void k_bbox_final(Dev d, int blocks)
         w[0] = fminf(w[0], q[0]); w[1] = fminf(w[1], q[1]); w[2] = fminf(w[2], q[2]);
         w[3] = fmaxf(w[3], q[3]); w[4] = fmaxf(w[4], q[4]); w[5] = fmaxf(w[5], q[5]);
     }
-    block_minmax(w, part);
-    if (threadIdx.x == 0) {
-        // root cell, boundingbox.cl:171-189
-        c->root[0] = 0.5f * (w[0] + w[3]);
-        c->root[1] = 0.5f * (w[1] + w[4]);
-        c->root[2] = 0.5f * (w[2] + w[5]);
-        const float radius = 0.5f * fmaxf(fmaxf(w[3] - w[0], w[4] - w[1]), w[5] - w[2]);
-        c->radius = radius;
-        // opening thresholds, calculateforce.cl:52-67 (FP32 quotient via a
-        // double division rounded once = the correctly rounded FP32 quotient)
-        float raw = radius * radius;
-        if (d.theta2 > 0.0f) raw = (float)((double)raw / (double)d.theta2);
-        for (int i = 0; i < kMaxDepth; ++i) {
-            c->dq[i] = raw + d.eps2;
-            raw = 0.25f * raw;
-        }
-        c->n_cells = 1; // the root is cell 0 (reference: _bottom = NUMBER_OF_NODES, :180)
-        c->epoch += 1;  // every child slot of the last tree turns stale
-        c->step += 1;   // boundingbox.cl:195
-    }
+    block_minmax<256>(w, part);
+    if (threadIdx.x == 0) finish_box(d, w);
 }
 
 // ---------------------------------------------------------------------------
@@ -551,9 +560,14 @@ __global__ __launch_bounds__(256) void k_paths(Dev d, unsigned long long *paths3
 }
 
 // ---- launchers ---------------------------------------------------------------
-hipError_t launch_bbox(const Dev &d, int blocks, hipStream_t st)
+hipError_t launch_bbox(const Dev &d, int blocks, bool splitters, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_bbox, dim3(blocks), dim3(256), 0, st, d);
+    const int S = splitters ? bucket_samples(d.n) : -1;
+    if (d.n <= kBoxOne) {
+        hipLaunchKernelGGL((k_bbox<kBoxOneThreads, true>), dim3(1), dim3(kBoxOneThreads), 0, st, d, S);
+        return hipGetLastError();
+    }
+    hipLaunchKernelGGL((k_bbox<256, false>), dim3(blocks), dim3(256), 0, st, d, S);
     hipLaunchKernelGGL(k_bbox_final, dim3(1), dim3(256), 0, st, d, blocks);
     return hipGetLastError();
 }
