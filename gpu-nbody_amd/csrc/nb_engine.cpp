@@ -8,6 +8,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <cstddef>
 #include <cmath>
@@ -16,10 +17,14 @@
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "../../include/nbody.h"
 #include "nb_internal.h"
+
+constexpr int kMaxSlots = 16;
+constexpr size_t kKeepBytes = (size_t)64 << 20;
 
 struct nb_sim {
     nb_params p;
@@ -78,9 +83,17 @@ struct nb_sim {
     bool staged = false;    // d.bnode holds pm4 in d.sorted order (the last fused update wrote it)
     bool splitters = false; // the last bounding box worked out the next warm build's splitters
     bool sort_pending = false; // d.kb_val[0] holds the order of a build the sort stage has not taken yet
-    // copyVertices staging: 2 N float4 (positions, then velocities), allocated
-    // by the first nb_copy_vertices call and kept until nb_destroy
-    float4 *vtx = nullptr;
+    // pinned staging of the copies to and from the caller's arrays (through_slots),
+    // and a pinned copy of Ctl
+    char *slot = nullptr;
+    int slots = 0;
+    size_t slot_bytes = 0;
+    hipEvent_t slot_ev[kMaxSlots] = {};
+    bool slot_busy[kMaxSlots] = {}; // a copy to the device that slot_ev ends may still read it
+    nb::Ctl *ctl_host = nullptr;
+    // device blocks of earlier calls' Scratch, at most kKeepBytes in all
+    std::vector<std::pair<void *, size_t>> kept;
+    size_t kept_bytes = 0;
     std::string err;
 };
 
@@ -176,9 +189,124 @@ nb::Ctl initial_ctl(const nb_sim *s, uint32_t epoch)
 
 int read_ctl(nb_sim *s, nb::Ctl *out)
 {
-    HIP_TRY(s, hipMemcpyAsync(out, s->d.ctl, sizeof(nb::Ctl), hipMemcpyDeviceToHost, s->stream));
+    HIP_TRY(s, nb::launch_copy(s->ctl_host, s->d.ctl, sizeof(nb::Ctl), s->stream));
     HIP_TRY(s, hipStreamSynchronize(s->stream));
+    *out = *s->ctl_host;
     return NB_OK;
+}
+
+// ---- copies between the caller's arrays and the device ------------------------
+//
+// hipMemcpyAsync of pageable memory goes through the runtime's own staging, one
+// piece after the other on the calling thread: 4M bodies' vertices (134 MB) came
+// back at 17 GB/s, each small array cost 40 to 80 us, and the columns of a state
+// were first woven into records on one core. Here a chunk goes through a pinned
+// slot of the handle: a kernel on the stream moves it across the bus between the
+// device and the slot (without the hand-over to a copy engine and back), a host
+// copy between the slot and the caller's array. A worker has two slots, so that
+// its next chunk crosses the bus while it copies the last; large transfers have
+// several workers, which take chunks as they come free. New state of 16,384
+// bodies 446 -> 48 us, of 1M 12.7 -> 0.80 ms; vertices of 1000 bodies 55 -> 17
+// us, of 4M 7.5 -> 3.1 ms (43 GB/s).
+constexpr size_t kWorkerBytes = (size_t)4 << 20; // one worker more for each of these (helpers for 1 MiB cost more than they copy)
+
+// How a transfer's chunks are cut: `per` items of `bytes` each fill a slot.
+size_t slot_items(const nb_sim *s, size_t bytes) { return s->slot_bytes / bytes & ~(size_t)63; }
+
+// Items 0 .. items-1 in chunks of `per`. To the host (out): issue(first, count,
+// slot) queues the chunk's way into the slot on the stream, host(first, count,
+// slot) takes it from there. To the device: host fills the slot, issue queues
+// its way out of it. On return the caller's arrays are done with, and a copy to
+// the device is queued on the stream. Both may run on several threads at once.
+template <class Issue, class Host>
+int through_slots(nb_sim *s, bool out, size_t items, size_t per, size_t bytes, const Issue &issue, const Host &host)
+{
+    const size_t chunks = (items + per - 1) / per;
+    std::atomic<size_t> next{0};
+    std::atomic<int> bad{(int)hipSuccess};
+    const auto work = [&](int worker) {
+        hipError_t e = hipSetDevice(s->device);
+        size_t held = chunks; // the chunk on its way into the other slot
+        for (int turn = 0; e == hipSuccess && bad.load() == (int)hipSuccess; ++turn) {
+            const int k = 2 * worker + (turn & 1), other = 2 * worker + (~turn & 1);
+            char *const slot = s->slot + (size_t)k * s->slot_bytes;
+            const size_t c = next.fetch_add(1), first = c * per;
+            if (c < chunks) {
+                const size_t count = std::min(per, items - first);
+                if (s->slot_busy[k]) e = hipEventSynchronize(s->slot_ev[k]);
+                s->slot_busy[k] = false;
+                if (e == hipSuccess && !out) host(first, count, slot);
+                if (e == hipSuccess) e = issue(first, count, slot);
+                if (e == hipSuccess) e = hipEventRecord(s->slot_ev[k], s->stream);
+                s->slot_busy[k] = true;
+            }
+            if (out && held < chunks && e == hipSuccess) {
+                e = hipEventSynchronize(s->slot_ev[other]);
+                s->slot_busy[other] = false;
+                const size_t from = held * per;
+                if (e == hipSuccess) host(from, std::min(per, items - from), s->slot + (size_t)other * s->slot_bytes);
+            }
+            if (c >= chunks) break;
+            held = c;
+        }
+        if (e != hipSuccess) bad.store((int)e);
+    };
+    const size_t want = std::min<size_t>({chunks, (size_t)s->slots / 2, 1 + items * bytes / kWorkerBytes});
+    std::thread helper[kMaxSlots / 2];
+    for (size_t w = 1; w < want; ++w) {
+        try {
+            helper[w] = std::thread(work, (int)w);
+        } catch (const std::exception &) {
+            break; // the workers that there are take all chunks
+        }
+    }
+    work(0);
+    for (std::thread &t : helper)
+        if (t.joinable()) t.join();
+    const hipError_t e = (hipError_t)bad.load();
+    if (e != hipSuccess) {
+        (void)hipStreamSynchronize(s->stream);
+        return fail(s, NB_E_HIP, "copy: %s", hipGetErrorString(e));
+    }
+    return NB_OK;
+}
+
+// Device memory to the host, complete on return; host memory to the device,
+// queued on the stream.
+int receive(nb_sim *s, void *dst, const void *src, size_t bytes)
+{
+    return through_slots(
+        s, true, bytes, s->slot_bytes, 1,
+        [&](size_t first, size_t count, char *slot) {
+            return nb::launch_copy(slot, (const char *)src + first, count, s->stream);
+        },
+        [&](size_t first, size_t count, char *slot) { std::memcpy((char *)dst + first, slot, count); });
+}
+
+int send(nb_sim *s, void *dst, const void *src, size_t bytes)
+{
+    return through_slots(
+        s, false, bytes, s->slot_bytes, 1,
+        [&](size_t first, size_t count, char *slot) {
+            return nb::launch_copy((char *)dst + first, slot, count, s->stream);
+        },
+        [&](size_t first, size_t count, char *slot) { std::memcpy(slot, (const char *)src + first, count); });
+}
+
+// x, y and z of the records src[0 .. n) into the caller's arrays, of which some
+// may be null
+int receive_columns(nb_sim *s, const float4 *src, float *const (&col)[3])
+{
+    if (!col[0] && !col[1] && !col[2]) return NB_OK;
+    return through_slots(
+        s, true, (size_t)s->d.n, slot_items(s, 3 * sizeof(float)), 3 * sizeof(float),
+        [&](size_t first, size_t count, char *slot) {
+            return nb::launch_columns(src + first, (int)count, (float *)slot, s->stream);
+        },
+        [&](size_t first, size_t count, char *slot) {
+            for (int k = 0; k < 3; ++k)
+                if (col[k]) std::memcpy(col[k] + first, (const float *)slot + k * count, count * sizeof(float));
+        });
 }
 
 // Keeps the level sizes of a tree read back to size later launches.
@@ -415,7 +543,8 @@ void drain(nb_sim *s)
 // Host -> device copy ordered on the handle's stream, complete on return.
 int upload(nb_sim *s, void *dst, const void *src, size_t bytes)
 {
-    HIP_TRY(s, hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s->stream));
+    const int r = send(s, dst, src, bytes);
+    if (r) return r;
     HIP_TRY(s, hipStreamSynchronize(s->stream));
     return NB_OK;
 }
@@ -520,7 +649,7 @@ void free_all(nb_sim *s)
                     d.cinfo, d.count, d.com64,         d.cchild,   d.lvl_list, d.clvl,
                     d.lvl_blockhist, d.lvl_count, d.cdata,  d.bnode,  d.sorted, d.probe, d.bbox_part, d.gcost, d.gorder,
                     s->chk_idx, s->chk_part, s->chk_out, d.cq64, d.cqa, d.cqb, d.cmac,
-                    s->mlpbuf, s->chk_acc, s->vtx, d.kb_key[0], d.kb_key[1], d.kb_val[0], d.kb_val[1],
+                    s->mlpbuf, s->chk_acc, d.kb_key[0], d.kb_key[1], d.kb_val[0], d.kb_val[1],
                     d.kb_deep, d.kb_hist, d.kb_offs, d.kb_tot, d.kb_ipar, d.kb_lpar, d.kb_lo,
                     d.kb_own, d.kb_ktop, d.kb_obase, d.kb_scan, d.kb_tdep, d.kb_spl, d.kb_bcnt, d.kb_bfill, d.kb_bstart};
     for (void *p : ptrs)
@@ -533,6 +662,11 @@ void free_all(nb_sim *s)
     for (auto &e : s->pair_ev)
         if (e) (void)hipEventDestroy(e);
     if (s->chk_host) (void)hipHostFree(s->chk_host);
+    for (auto &e : s->slot_ev)
+        if (e) (void)hipEventDestroy(e);
+    if (s->slot) (void)hipHostFree(s->slot);
+    if (s->ctl_host) (void)hipHostFree(s->ctl_host);
+    for (const auto &b : s->kept) (void)hipFree(b.first);
     if (s->side) (void)hipStreamDestroy(s->side);
     if (s->ord_in) (void)hipEventDestroy(s->ord_in);
     if (s->ord_out) (void)hipEventDestroy(s->ord_out);
@@ -543,9 +677,7 @@ void free_all(nb_sim *s)
 template <class T> int fetch(nb_sim *s, std::vector<T> &out, const T *src, size_t count)
 {
     out.resize(count);
-    HIP_TRY(s, hipMemcpyAsync(out.data(), src, count * sizeof(T), hipMemcpyDeviceToHost, s->stream));
-    HIP_TRY(s, hipStreamSynchronize(s->stream));
-    return NB_OK;
+    return receive(s, out.data(), src, count * sizeof(T));
 }
 
 int ensure_check_buffers(nb_sim *s, int ns)
@@ -568,34 +700,67 @@ int ensure_check_buffers(nb_sim *s, int ns)
 }
 
 // Device allocations that live for one API call; freed after the stream drains.
+// Device memory of one call. The blocks stay with the handle for its next call
+// (a gradient of 4096 rows spent half its time on hipMalloc and hipFree), up to
+// kKeepBytes; more is freed.
 struct Scratch {
     nb_sim *s;
-    std::vector<void *> ptrs;
+    std::vector<std::pair<void *, size_t>> blocks;
     explicit Scratch(nb_sim *sim) : s(sim) {}
     ~Scratch()
     {
         drain(s); // the training pairs' stream too, when a launch failed halfway
-        for (void *p : ptrs) (void)hipFree(p);
+        for (const auto &b : blocks) {
+            if (s->kept_bytes + b.second <= kKeepBytes) {
+                s->kept.push_back(b);
+                s->kept_bytes += b.second;
+            } else {
+                (void)hipFree(b.first);
+            }
+        }
     }
     template <class T> int get(T **p, size_t count)
     {
+        const size_t bytes = (count * sizeof(T) + 64 + 255) & ~(size_t)255;
         *p = nullptr;
-        hipError_t e = hipMalloc((void **)p, count * sizeof(T) + 64);
+        auto best = s->kept.end();
+        for (auto it = s->kept.begin(); it != s->kept.end(); ++it)
+            if (it->second >= bytes && it->second <= 2 * bytes && (best == s->kept.end() || it->second < best->second))
+                best = it;
+        if (best != s->kept.end()) {
+            *p = (T *)best->first;
+            blocks.push_back(*best);
+            s->kept_bytes -= best->second;
+            s->kept.erase(best);
+            return NB_OK;
+        }
+        hipError_t e = hipMalloc((void **)p, bytes);
+        if (e != hipSuccess) {
+            // what is kept may be in the way
+            for (const auto &b : s->kept) (void)hipFree(b.first);
+            s->kept.clear();
+            s->kept_bytes = 0;
+            e = hipMalloc((void **)p, bytes);
+        }
         if (e != hipSuccess) return fail(s, NB_E_HIP, "hipMalloc(%zu): %s", count * sizeof(T), hipGetErrorString(e));
-        ptrs.push_back(*p);
+        blocks.push_back({*p, bytes});
         return NB_OK;
     }
 };
+
+constexpr size_t kLossAt = (nb::kMlpParams + 3) & ~3; // whole 16 bytes
 
 // Training buffers for S samples (X, T given or allocated) and batch B.
 int train_buffers(Scratch &m, nb::Train &t, int S, int B, int iters)
 {
     int r = NB_OK;
-    for (float **f : {&t.P, &t.G, &t.M, &t.V})
+    for (float **f : {&t.P, &t.M, &t.V})
         if (!r) r = m.get(f, (size_t)nb::kMlpParams);
+    // the losses behind the gradient: one read for both
+    if (!r) r = m.get(&t.G, kLossAt + (size_t)std::max(iters, 1));
+    t.loss_hist = t.G + kLossAt;
     if (!r) r = m.get(&t.gpart, (size_t)nb::train_parts(B) * nb::kMlpParams);
     if (!r) r = m.get(&t.loss_part, (size_t)nb::train_parts(B));
-    if (!r) r = m.get(&t.loss_hist, (size_t)std::max(iters, 1));
     t.S = S;
     return r;
 }
@@ -811,6 +976,18 @@ int nb_create(const nb_params *p, nb_sim **out)
         fail(s, NB_E_HIP, "device allocation failed for %d bodies / %d cells", n, d.cap);
         return bail(NB_E_HIP);
     }
+    // two slots per worker; larger ones cross the bus faster (4M bodies' vertices:
+    // 512 KiB 3.7 ms, 1 MiB 3.15 ms), small systems do not fill them
+    s->slots = n < 65536 ? 4 : kMaxSlots;
+    s->slot_bytes = n < 65536 ? 256 << 10 : n < 524288 ? 512 << 10 : 1024 << 10;
+    ok = hipHostMalloc((void **)&s->slot, (size_t)s->slots * s->slot_bytes) == hipSuccess &&
+         hipHostMalloc((void **)&s->ctl_host, sizeof(nb::Ctl)) == hipSuccess;
+    for (int k = 0; ok && k < s->slots; ++k)
+        ok = hipEventCreateWithFlags(&s->slot_ev[k], hipEventDisableTiming) == hipSuccess;
+    if (!ok) {
+        fail(s, NB_E_HIP, "pinned host allocation of %zu bytes failed", (size_t)s->slots * s->slot_bytes);
+        return bail(NB_E_HIP);
+    }
     if (d.quad && ensure_learn(s) != NB_OK) return bail(NB_E_HIP);
     if (const int rs = init_scratch(s)) return bail(rs);
     // epoch 0 tags every slot as stale; the first bounding box moves to epoch 1
@@ -846,38 +1023,20 @@ int nb_set_state(nb_sim *s, const float *x, const float *y, const float *z, cons
     // nothing queued earlier may still read the buffers overwritten below
     drain(s);
     nb::Dev &d = s->d;
-    const size_t n = (size_t)d.n;
-    int r = NB_OK;
-    {
-        std::vector<float4> pm(n), vel(n), zero(n, make_float4(0.f, 0.f, 0.f, 0.f));
-        for (size_t i = 0; i < n; ++i) {
-            pm[i] = make_float4(x[i], y[i], z[i], m[i]);
-            vel[i] = make_float4(vx[i], vy[i], vz[i], 0.f);
-        }
-        r = upload(s, d.pm4, pm.data(), n * sizeof(float4));
-        if (!r) r = upload(s, d.vel4, vel.data(), n * sizeof(float4));
-        if (!r) r = upload(s, d.acc4, zero.data(), n * sizeof(float4));
-        if (r) return r;
-    }
-    if (d.fp64) {
-        std::vector<double4> p64(n);
-        for (size_t i = 0; i < n; ++i) p64[i] = make_double4(x[i], y[i], z[i], 0.0);
-        r = upload(s, d.pos64, p64.data(), n * sizeof(double4));
-        if (r) return r;
-    }
-    // sorted[] before the first tree: the identity
-    {
-        std::vector<int> ident((size_t)d.n);
-        for (int i = 0; i < d.n; ++i) ident[i] = i;
-        r = upload(s, d.sorted, ident.data(), (size_t)d.n * sizeof(int));
-        if (r) return r;
-    }
-    // keep the epoch running so that no slot of an earlier tree can look current
-    nb::Ctl cur;
-    r = read_ctl(s, &cur);
+    const float *const col[7] = {x, y, z, vx, vy, vz, m};
+    // records, accelerations of zero, the identity in sorted[] and a Ctl that
+    // starts over (but for the epoch, so that no slot of an earlier tree can look
+    // current), by the kernel that reads the columns
+    const int r = through_slots(
+        s, false, (size_t)d.n, slot_items(s, sizeof(float) * 7), sizeof(float) * 7,
+        [&](size_t first, size_t count, char *slot) {
+            return nb::launch_set_state(d, (int)first, (int)count, (const float *)slot, s->stream);
+        },
+        [&](size_t first, size_t count, char *slot) {
+            for (int k = 0; k < 7; ++k)
+                std::memcpy((float *)slot + k * count, col[k] + first, count * sizeof(float));
+        });
     if (r) return r;
-    nb::Ctl c = initial_ctl(s, cur.epoch);
-    HIP_TRY(s, hipMemcpyAsync(d.ctl, &c, sizeof c, hipMemcpyHostToDevice, s->stream));
     HIP_TRY(s, hipStreamSynchronize(s->stream));
     s->inter_before = 0;
     s->cell_inter_before = 0;
@@ -980,17 +1139,19 @@ int nb_copy_vertices(nb_sim *s, float *pos4, float *vel4)
     if (!s->have_state) return fail(s, NB_E_STATE, "nb_set_state has not been called");
     if (!pos4 && !vel4) return NB_OK;
     HIP_TRY(s, hipSetDevice(s->device));
-    const size_t n = (size_t)s->d.n, bytes = n * sizeof(float4);
-    // the staging buffer is taken once and reused by every later call (the
-    // renderer calls this after every step)
-    if (!s->vtx) HIP_TRY(s, dalloc(&s->vtx, 2 * n));
-    float4 *dp = pos4 ? s->vtx : nullptr, *dv = vel4 ? s->vtx + n : nullptr;
-    hipError_t e = nb::launch_copy_vertices(s->d, 0, (int)n, dp, dv, s->stream);
-    if (e == hipSuccess && dp) e = hipMemcpyAsync(pos4, dp, bytes, hipMemcpyDeviceToHost, s->stream);
-    if (e == hipSuccess && dv) e = hipMemcpyAsync(vel4, dv, bytes, hipMemcpyDeviceToHost, s->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
-    if (e != hipSuccess) return fail(s, NB_E_HIP, "copy_vertices: %s", hipGetErrorString(e));
-    return NB_OK;
+    const size_t bytes = (pos4 && vel4 ? 2 : 1) * sizeof(float4);
+    return through_slots(
+        s, true, (size_t)s->d.n, slot_items(s, bytes), bytes,
+        [&](size_t first, size_t count, char *slot) {
+            float4 *to = (float4 *)slot;
+            return nb::launch_copy_vertices(s->d, (int)first, (int)count, pos4 ? to : nullptr,
+                                            vel4 ? (pos4 ? to + count : to) : nullptr, s->stream);
+        },
+        [&](size_t first, size_t count, char *slot) {
+            const float *from = (const float *)slot;
+            if (pos4) std::memcpy(pos4 + 4 * first, from, count * sizeof(float4));
+            if (vel4) std::memcpy(vel4 + 4 * first, from + (pos4 ? 4 * count : 0), count * sizeof(float4));
+        });
 }
 
 int nb_copy_vertices_noalloc(nb_sim *s, float *pos4, float *vel4)
@@ -1026,36 +1187,15 @@ int nb_get_state(nb_sim *s, float *x, float *y, float *z, float *vx, float *vy, 
 {
     if (!s) return NB_E_ARG;
     HIP_TRY(s, hipSetDevice(s->device));
-    const size_t n = (size_t)s->d.n;
-    std::vector<float4> p, v;
-    int r = fetch(s, p, s->d.pm4, n);
-    if (!r) r = fetch(s, v, s->d.vel4, n);
-    if (r) return r;
-    for (size_t i = 0; i < n; ++i) {
-        if (x) x[i] = p[i].x;
-        if (y) y[i] = p[i].y;
-        if (z) z[i] = p[i].z;
-        if (vx) vx[i] = v[i].x;
-        if (vy) vy[i] = v[i].y;
-        if (vz) vz[i] = v[i].z;
-    }
-    return NB_OK;
+    const int r = receive_columns(s, s->d.pm4, {x, y, z});
+    return r ? r : receive_columns(s, s->d.vel4, {vx, vy, vz});
 }
 
 int nb_get_accel(nb_sim *s, float *ax, float *ay, float *az)
 {
     if (!s) return NB_E_ARG;
     HIP_TRY(s, hipSetDevice(s->device));
-    const size_t n = (size_t)s->d.n;
-    std::vector<float4> a;
-    int r = fetch(s, a, s->d.acc4, n);
-    if (r) return r;
-    for (size_t i = 0; i < n; ++i) {
-        if (ax) ax[i] = a[i].x;
-        if (ay) ay[i] = a[i].y;
-        if (az) az[i] = a[i].z;
-    }
-    return NB_OK;
+    return receive_columns(s, s->d.acc4, {ax, ay, az});
 }
 
 int nb_get_positions64(nb_sim *s, double *x, double *y, double *z)
@@ -1154,16 +1294,14 @@ int nb_get_cells(nb_sim *s, int32_t cap, int32_t *ncells, int32_t *count, float 
 // step counter is put back so the simulation's own stepping is unaffected.
 static int probe_pass(nb_sim *s)
 {
-    nb::Ctl c0;
-    int r = read_ctl(s, &c0);
-    if (r) return r;
+    HIP_TRY(s, nb::launch_step_mark(s->d, false, s->stream));
     for (int st = NB_STAGE_BBOX; st <= NB_STAGE_SORT; ++st) {
-        r = launch_stage(s, st);
+        const int r = launch_stage(s, st);
         if (r) return r;
     }
-    r = launch_force_method(s, force_method(s), 2);
+    const int r = launch_force_method(s, force_method(s), 2);
     if (r) return r;
-    HIP_TRY(s, hipMemcpyAsync(&s->d.ctl->step, &c0.step, sizeof(int), hipMemcpyHostToDevice, s->stream));
+    HIP_TRY(s, nb::launch_step_mark(s->d, true, s->stream));
     return check_device_error(s);
 }
 
@@ -1171,7 +1309,8 @@ static int direct_accel(nb_sim *s, const int32_t *idx, int32_t ns, std::vector<d
 {
     int r = ensure_check_buffers(s, ns);
     if (r) return r;
-    HIP_TRY(s, hipMemcpyAsync(s->chk_idx, idx, (size_t)ns * sizeof(int), hipMemcpyHostToDevice, s->stream));
+    r = send(s, s->chk_idx, idx, (size_t)ns * sizeof(int));
+    if (r) return r;
     hipError_t e = nb::launch_direct64(s->d, s->chk_idx, ns, s->chk_part, s->chk_out, nb::kDirectAcc, s->stream);
     if (e != hipSuccess) return fail(s, NB_E_HIP, "direct-sum launch: %s", hipGetErrorString(e));
     return fetch(s, out, (const double4 *)s->chk_out, (size_t)ns);
@@ -1184,15 +1323,7 @@ int nb_probe_accel(nb_sim *s, float *ax, float *ay, float *az)
     HIP_TRY(s, hipSetDevice(s->device));
     int r = probe_pass(s);
     if (r) return r;
-    std::vector<float4> a;
-    r = fetch(s, a, (const float4 *)s->d.probe, (size_t)s->d.n);
-    if (r) return r;
-    for (size_t i = 0; i < a.size(); ++i) {
-        if (ax) ax[i] = a[i].x;
-        if (ay) ay[i] = a[i].y;
-        if (az) az[i] = a[i].z;
-    }
-    return NB_OK;
+    return receive_columns(s, s->d.probe, {ax, ay, az});
 }
 
 int nb_direct_accel(nb_sim *s, const int32_t *idx, int32_t ns, double *out3)
@@ -1513,12 +1644,11 @@ int nb_mlp_forward(nb_sim *s, const float *x, int32_t n, float *y)
     int r = m.get(&xd, (size_t)n * nb::kFeat);
     if (!r) r = m.get(&yd, (size_t)n * nb::kOut);
     if (r) return r;
-    HIP_TRY(s, hipMemcpyAsync(xd, x, (size_t)n * nb::kFeat * sizeof(float), hipMemcpyHostToDevice, s->stream));
+    r = send(s, xd, x, (size_t)n * nb::kFeat * sizeof(float));
+    if (r) return r;
     hipError_t e = nb::launch_mlp_rows(s->L, xd, n, yd, s->stream);
     if (e != hipSuccess) return fail(s, NB_E_HIP, "network launch: %s", hipGetErrorString(e));
-    HIP_TRY(s, hipMemcpyAsync(y, yd, (size_t)n * nb::kOut * sizeof(float), hipMemcpyDeviceToHost, s->stream));
-    HIP_TRY(s, hipStreamSynchronize(s->stream));
-    return NB_OK;
+    return receive(s, y, yd, (size_t)n * nb::kOut * sizeof(float));
 }
 
 namespace {
@@ -1539,12 +1669,14 @@ int host_data_passes(nb_sim *s, const float *x, const float *t, int n, int iters
     if (r) return r;
     tr.X = xd;
     tr.T = td;
-    HIP_TRY(s, hipMemcpyAsync(xd, x, (size_t)n * nb::kFeat * sizeof(float), hipMemcpyHostToDevice, s->stream));
-    HIP_TRY(s, hipMemcpyAsync(td, t, (size_t)n * nb::kOut * sizeof(float), hipMemcpyHostToDevice, s->stream));
-    HIP_TRY(s, hipMemcpyAsync(tr.P, s->model.data(), (size_t)nb::kMlpParams * sizeof(float), hipMemcpyHostToDevice,
-                              s->stream));
-    HIP_TRY(s, hipMemsetAsync(tr.M, 0, (size_t)nb::kMlpParams * sizeof(float), s->stream));
-    HIP_TRY(s, hipMemsetAsync(tr.V, 0, (size_t)nb::kMlpParams * sizeof(float), s->stream));
+    r = send(s, xd, x, (size_t)n * nb::kFeat * sizeof(float));
+    if (!r) r = send(s, td, t, (size_t)n * nb::kOut * sizeof(float));
+    if (!r) r = send(s, tr.P, s->model.data(), (size_t)nb::kMlpParams * sizeof(float));
+    if (r) return r;
+    if (adam) {
+        HIP_TRY(s, hipMemsetAsync(tr.M, 0, (size_t)nb::kMlpParams * sizeof(float), s->stream));
+        HIP_TRY(s, hipMemsetAsync(tr.V, 0, (size_t)nb::kMlpParams * sizeof(float), s->stream));
+    }
     double p1 = 1.0, p2 = 1.0;
     for (int it = 0; it < iters; ++it) {
         p1 *= 0.9;
@@ -1553,10 +1685,12 @@ int host_data_passes(nb_sim *s, const float *x, const float *t, int n, int iters
                                              (float)(1.0 / (1.0 - p2)), s->stream);
         if (e != hipSuccess) return fail(s, NB_E_HIP, "training launch: %s", hipGetErrorString(e));
     }
-    if (loss) HIP_TRY(s, hipMemcpyAsync(loss, tr.loss_hist, sizeof(float), hipMemcpyDeviceToHost, s->stream));
-    HIP_TRY(s, hipMemcpyAsync(out, adam ? tr.P : tr.G, (size_t)nb::kMlpParams * sizeof(float), hipMemcpyDeviceToHost,
-                              s->stream));
-    HIP_TRY(s, hipStreamSynchronize(s->stream));
+    if (adam) return receive(s, out, tr.P, (size_t)nb::kMlpParams * sizeof(float));
+    std::vector<float> got;
+    r = fetch(s, got, (const float *)tr.G, kLossAt + 1);
+    if (r) return r;
+    std::copy(got.begin(), got.begin() + nb::kMlpParams, out);
+    if (loss) *loss = got.back();
     return NB_OK;
 }
 } // namespace
@@ -1616,8 +1750,8 @@ int nb_diagnostics(nb_sim *s, int32_t pe_samples, uint64_t seed, double *out)
     for (int b0 = 0; b0 < ns; b0 += batch) {
         const int nb_ = std::min(batch, ns - b0);
         std::vector<double4> res;
-        HIP_TRY(s, hipMemcpyAsync(s->chk_idx, idx.data() + b0, (size_t)nb_ * sizeof(int), hipMemcpyHostToDevice,
-                                  s->stream));
+        r = send(s, s->chk_idx, idx.data() + b0, (size_t)nb_ * sizeof(int));
+        if (r) return r;
         e = nb::launch_direct64(s->d, s->chk_idx, nb_, s->chk_part, s->chk_out,
                                 exact ? nb::kDirectPhiAfter : nb::kDirectPhi, s->stream);
         if (e != hipSuccess) return fail(s, NB_E_HIP, "direct-sum launch: %s", hipGetErrorString(e));

@@ -106,6 +106,7 @@ struct Tally {
 // a second launch finishes the box).
 struct Ctl {
     int step;            // reference _step, starts at -1 (java:167)
+    int step_mark;       // its value before a probe pass
     uint32_t epoch;      // tree generation: tags child slots
     int n_cells;         // cell allocation counter (reference _bottom)
     int max_depth;       // running maximum (reference _maxDepth, java:170)
@@ -214,6 +215,15 @@ constexpr int kMomentBlocks = 512;
 hipError_t launch_moments(const Dev &d, double *part, hipStream_t st);
 // bodies first .. first + count - 1 into pos[0 .. count) / vel[0 .. count) (either may be null)
 hipError_t launch_copy_vertices(const Dev &d, int first, int count, float4 *pos, float4 *vel, hipStream_t st);
+// bytes between device memory and pinned host memory (either 16-byte aligned)
+hipError_t launch_copy(void *dst, const void *src, size_t bytes, hipStream_t st);
+// keeps the step counter, or puts the kept one back
+hipError_t launch_step_mark(const Dev &d, bool back, hipStream_t st);
+// bodies first .. first + count - 1 from the columns x, y, z, vx, vy, vz, m of
+// `count` each (pinned host memory), and with body 0 a Ctl that starts over
+hipError_t launch_set_state(const Dev &d, int first, int count, const float *columns, hipStream_t st);
+// x, y, z of src[0 .. count) as three columns of `count` (pinned host memory)
+hipError_t launch_columns(const float4 *src, int count, float *columns, hipStream_t st);
 hipError_t launch_paths(const Dev &d, unsigned long long *paths3, int *depth, hipStream_t st);
 
 // ---- learned coarse-theta correction (nb_learned.hip) -----------------------

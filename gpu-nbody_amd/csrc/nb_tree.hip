@@ -10,6 +10,8 @@
 // reference's summarize are replaced by level launches.)
 #include "nb_device.h"
 
+#include <cstddef>
+
 namespace nb {
 
 __device__ __forceinline__ int dec_slot(unsigned long long w, uint32_t ep)
@@ -526,6 +528,60 @@ __global__ __launch_bounds__(256) void k_copy_vertices(Dev d, int first, int cou
     }
 }
 
+// Caller's columns to records and back, through pinned host memory that the
+// kernels read and write across the bus themselves (coalesced): a chunk needs no
+// copy of its own beside the launch.
+__global__ __launch_bounds__(256) void k_set_state(Dev d, int first, int count, const float *__restrict__ col)
+{
+    const int j = blockIdx.x * blockDim.x + threadIdx.x;
+    if (first == 0 && blockIdx.x == 0) {
+        // everything but the epoch; what does not start at zero
+        Ctl *c = d.ctl;
+        int *words = reinterpret_cast<int *>(c);
+        constexpr int epoch = (int)(offsetof(Ctl, epoch) / sizeof(int));
+        for (int i = threadIdx.x; i < (int)(sizeof(Ctl) / sizeof(int)); i += blockDim.x)
+            if (i != epoch) words[i] = 0;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            c->step = -1;     // GPUBarnesHutNBodySimulation.java:167
+            c->n_cells = 1;
+            c->max_depth = 1; // GPUBarnesHutNBodySimulation.java:170
+        }
+    }
+    if (j >= count) return;
+    const int i = first + j;
+    const float x = col[j], y = col[count + j], z = col[2 * count + j];
+    d.pm4[i] = make_float4(x, y, z, col[6 * count + j]);
+    d.vel4[i] = make_float4(col[3 * count + j], col[4 * count + j], col[5 * count + j], 0.0f);
+    d.acc4[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (d.fp64) d.pos64[i] = make_double4(x, y, z, 0.0);
+    d.sorted[i] = i; // before the first tree: the identity
+}
+
+__global__ __launch_bounds__(256) void k_copy(unsigned char *__restrict__ dst, const unsigned char *__restrict__ src,
+                                              size_t bytes)
+{
+    const size_t quads = bytes / 16, i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < quads) reinterpret_cast<uint4 *>(dst)[i] = reinterpret_cast<const uint4 *>(src)[i];
+    else if (i - quads < bytes % 16) dst[16 * quads + (i - quads)] = src[16 * quads + (i - quads)];
+}
+
+__global__ void k_step_mark(Ctl *c, bool back)
+{
+    if (back) c->step = c->step_mark;
+    else c->step_mark = c->step;
+}
+
+__global__ __launch_bounds__(256) void k_columns(const float4 *__restrict__ src, int count, float *__restrict__ col)
+{
+    const int j = blockIdx.x * blockDim.x + threadIdx.x;
+    if (j >= count) return;
+    const float4 q = src[j];
+    col[j] = q.x;
+    col[count + j] = q.y;
+    col[2 * count + j] = q.z;
+}
+
 // Leaf membership: descend the child slots along each body's own octants
 // until the slot that holds the body; record the octants. depth = -1 if the
 // descent does not end at the body.
@@ -606,6 +662,32 @@ hipError_t launch_copy_vertices(const Dev &d, int first, int count, float4 *pos,
 {
     if (first < 0 || count < 1 || first > d.n - count) return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_copy_vertices, dim3((count + 255) / 256), dim3(256), 0, st, d, first, count, pos, vel);
+    return hipGetLastError();
+}
+hipError_t launch_set_state(const Dev &d, int first, int count, const float *columns, hipStream_t st)
+{
+    if (first < 0 || count < 1 || first > d.n - count) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_set_state, dim3((count + 255) / 256), dim3(256), 0, st, d, first, count, columns);
+    return hipGetLastError();
+}
+hipError_t launch_copy(void *dst, const void *src, size_t bytes, hipStream_t st)
+{
+    if (bytes == 0) return hipSuccess;
+    // 16 bytes per thread; a caller's pointer that is not aligned to them would be a fault here
+    if (((uintptr_t)dst | (uintptr_t)src) % 16) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_copy, dim3((unsigned)((bytes / 16 + bytes % 16 + 255) / 256)), dim3(256), 0, st,
+                       static_cast<unsigned char *>(dst), static_cast<const unsigned char *>(src), bytes);
+    return hipGetLastError();
+}
+hipError_t launch_step_mark(const Dev &d, bool back, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_step_mark, dim3(1), dim3(1), 0, st, d.ctl, back);
+    return hipGetLastError();
+}
+hipError_t launch_columns(const float4 *src, int count, float *columns, hipStream_t st)
+{
+    if (count < 1) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_columns, dim3((count + 255) / 256), dim3(256), 0, st, src, count, columns);
     return hipGetLastError();
 }
 hipError_t launch_paths(const Dev &d, unsigned long long *paths3, int *depth, hipStream_t st)
