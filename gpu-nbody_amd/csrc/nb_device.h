@@ -34,19 +34,17 @@ __device__ __forceinline__ unsigned lane_write(unsigned old, unsigned v, int lan
     return (unsigned)amdgcn_writelane_i32((int)v, lane, (int)old);
 }
 
-// End of a round of K waves that took `take` entries off the top of the shared
-// stack of sp entries, this wave having opened npush cells (entry j in lane j
-// of `push`): after the barrier every wave knows the others' counts, the new
-// entries go behind those of the lower waves, and sp becomes the new count.
-// False when the tree is corrupt (some wave says so, or the stack would
-// overflow). Every wave of the block calls it; `pushed` holds K words.
-template <int K, class Entry>
-__device__ __forceinline__ bool end_round(Entry *stk, unsigned *pushed, int wv, int lane, int take, int npush, Entry push,
-                                          bool bad, int &sp)
+// After a round of K waves in which this one opened npush cells: a barrier, by
+// which the round's entries are read, then the cells that the lower waves and
+// that all opened. False when some wave says the tree is corrupt. Every wave of
+// the block calls it; `pushed` holds K words.
+template <int K>
+__device__ __forceinline__ bool count_round(unsigned *pushed, int wv, int lane, int npush, bool bad, unsigned &before,
+                                            unsigned &total)
 {
     if (lane == 0) pushed[wv] = (unsigned)npush | (bad ? kSplitBad : 0u);
-    __syncthreads(); // the entries of this round are read, the counts are in
-    unsigned before = 0, total = 0;
+    __syncthreads();
+    before = total = 0;
 #pragma unroll
     for (int w = 0; w < K; ++w) {
         const unsigned c = pushed[w];
@@ -54,7 +52,22 @@ __device__ __forceinline__ bool end_round(Entry *stk, unsigned *pushed, int wv, 
         total += c;
     }
     total = __builtin_amdgcn_readfirstlane(total);
-    if (total >= kSplitBad || sp - take + (int)total > split_stack<K>()) return false; // the same in every wave
+    return total < kSplitBad;
+}
+
+// End of a round of K waves that took `take` entries off the top of the shared
+// stack of sp entries, this wave having opened npush cells (entry j in lane j
+// of `push`): the new entries go behind those of the lower waves, and sp
+// becomes the new count. False when the tree is corrupt (some wave says so, or
+// the stack would overflow).
+template <int K, class Entry>
+__device__ __forceinline__ bool end_round(Entry *stk, unsigned *pushed, int wv, int lane, int take, int npush, Entry push,
+                                          bool bad, int &sp)
+{
+    unsigned before, total;
+    // the same in every wave
+    if (!count_round<K>(pushed, wv, lane, npush, bad, before, total) || sp - take + (int)total > split_stack<K>())
+        return false;
     if (lane < npush) stk[sp - take + (int)before + lane] = push;
     sp += (int)total - take;
     if (sp) __syncthreads();

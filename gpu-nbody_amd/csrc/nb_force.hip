@@ -197,18 +197,36 @@ template <> struct StackEntry<64> {
     using type = unsigned;
 };
 
-// The epilogue's per-wave sums overlay the stack.
+// K waves that share a group at vote width 64 walk breadth first until the queue
+// holds kFront cells; then each takes every K-th of them and walks their
+// subtrees by itself. The queue is a ring of kQueue entries; a wave's own stack
+// holds its share of it and 7 entries for each level below.
+constexpr int kFront = 256, kQueue = 512, kOwnStack = 576;
+template <int K> constexpr bool queue_fits()
+{
+    return kFront - 1 + 8 * K <= kQueue && (kFront - 1 + 8 * K + K - 1) / K + 7 * kMaxDepth + 8 <= kOwnStack;
+}
+
+// The epilogue's per-wave sums overlay the stacks.
 template <int G, int K> constexpr int force_lds()
 {
-    const int stack = split_stack<K>() * (int)sizeof(typename StackEntry<G>::type), red = K == 1 ? 0 : K * 3 * 64 * 8;
+    static_assert(K == 1 || G < 64 || queue_fits<K>(), "the queue and the stacks hold every tree of kMaxDepth levels");
+    const int entries = K == 1 ? kStack : G < 64 ? split_stack<K>() : kQueue + K * kOwnStack;
+    const int stack = entries * (int)sizeof(typename StackEntry<G>::type), red = K == 1 ? 0 : K * 3 * 64 * 8;
     return ((stack > red ? stack : red) + 15) & ~15;
 }
 
 // K waves share the group of 64 positions (K > 1: few groups, so that one
-// wave per group would leave the chip idle). They take the stack's top K
-// entries in rounds: wave w visits the w-th from the top, and after a barrier
-// pushes what it opened behind the lower waves' entries. The order depends on
-// nothing but the tree, and so do the sums. (Eight waves per SIMD by the
+// wave per group would leave the chip idle). With narrow votes they take the
+// stack's top K entries in rounds: wave w visits the w-th from the top, and
+// after a barrier pushes what it opened behind the lower waves' entries. At
+// width 64 they part after a first stretch of such rounds (kFront): a round
+// lasts as long as its slowest visit, and from there on no wave waits for
+// another (100,003 bodies, two spheres: 442 -> 377 us; 262,144: 980 -> 900; 65,536,
+// ball: 149 -> 134). Parting at 128 cells is faster for a uniform ball (177
+// against 195 us at 100,003 bodies) and slower where a few cells hold most of
+// the work (453 against 380). The order depends on nothing but the tree, and so
+// do the sums. (Eight waves per SIMD by the
 // attribute: the scalar registers would otherwise allow seven, 1.90 against
 // 2.19 ms at 1M Plummer bodies, theta 0.5, vote 64.)
 template <int G, int K>
@@ -304,43 +322,95 @@ __global__ __launch_bounds__(64 * K) __attribute__((amdgpu_waves_per_eu(8, 8))) 
         }
     } else {
         if (tid == 0) stk[0] = entry(0, 15u); // root cell 0 at depth 0
-        int sp = 1;                           // the same in every wave
         __syncthreads();
-        for (;;) {
-            const int take = sp > kSplitTop ? 1 : min(sp, K);
-            int npush = 0;
-            unsigned push = 0, pushf = 0; // entry j of this wave's children in lane j
-            if (wv < take) {
-                unsigned cur, fields = 15u;
-                take_entry(stk[sp - 1 - wv], cur, fields);
-                if ((cur >> 6) >= cap) { // the pool holds `cap` cells: corrupt
-                    bad = true;
-                } else {
-                    const uint64_t act = G < 64 ? field_lanes(fields) : kAllLanes;
-                    float px, py, pz;
-                    auto opened = [&](unsigned e, unsigned f = 15u) {
-                        push = lane_write(push, e, npush);
-                        if constexpr (G < 64) pushf = lane_write(pushf, f, npush);
-                        ++npush;
-                    };
-                    const float thr = dq_s[cur & 63u];
-                    int children;
-                    if constexpr (G < 64)
-                        children = visit_narrow<G, true>(cur, fields, act, thr, me, eps2, cchild, cdata, px, py, pz, bad, opened);
-                    else
-                        children = visit_wide<true>(cur, thr, me, eps2, cchild, cdata, px, py, pz, bad, opened);
-                    sx += (double)px;
-                    sy += (double)py;
-                    sz += (double)pz;
-                    inter += (G < 64 ? (unsigned long long)(unsigned)__popcll(act & vmask) : 1ull) *
-                             (unsigned)(children - 1);
+        if constexpr (G < 64) {
+            int sp = 1; // the same in every wave
+            for (;;) {
+                const int take = sp > kSplitTop ? 1 : min(sp, K);
+                int npush = 0;
+                unsigned push = 0, pushf = 0; // entry j of this wave's children in lane j
+                if (wv < take) {
+                    unsigned cur, fields;
+                    take_entry(stk[sp - 1 - wv], cur, fields);
+                    if ((cur >> 6) >= cap) { // the pool holds `cap` cells: corrupt
+                        bad = true;
+                    } else {
+                        const uint64_t act = field_lanes(fields);
+                        float px, py, pz;
+                        const int children = visit_narrow<G, true>(
+                            cur, fields, act, dq_s[cur & 63u], me, eps2, cchild, cdata, px, py, pz, bad,
+                            [&](unsigned e, unsigned f) {
+                                push = lane_write(push, e, npush);
+                                pushf = lane_write(pushf, f, npush);
+                                ++npush;
+                            });
+                        sx += (double)px;
+                        sy += (double)py;
+                        sz += (double)pz;
+                        inter += (unsigned long long)(unsigned)__popcll(act & vmask) * (unsigned)(children - 1);
+                    }
                 }
+                if (!end_round<K>(stk, pushed, wv, lane, take, npush, entry(push, pushf), bad, sp)) {
+                    bad = true;
+                    break;
+                }
+                if (sp == 0) break;
             }
-            if (!end_round<K>(stk, pushed, wv, lane, take, npush, entry(push, pushf), bad, sp)) {
-                bad = true;
-                break;
+        } else {
+            auto visit = [&](unsigned cur, auto &&opened) {
+                float px, py, pz;
+                const int children =
+                    visit_wide<false>(cur, dq_s[cur & 63u], me, eps2, cchild, cdata, px, py, pz, bad, opened);
+                sx += (double)px;
+                sy += (double)py;
+                sz += (double)pz;
+                inter += (unsigned)(children - 1);
+            };
+            // breadth first, a cell each, until the queue holds enough
+            int head = 0, tail = 1; // the same in every wave
+            while (tail > head && tail - head < kFront) {
+                const int take = min(tail - head, K);
+                int npush = 0;
+                unsigned push = 0; // entry j of this wave's children in lane j
+                if (wv < take) {
+                    const unsigned cur = __builtin_amdgcn_readfirstlane(stk[(head + wv) % kQueue]);
+                    if ((cur >> 6) >= cap) { // the pool holds `cap` cells: corrupt
+                        bad = true;
+                    } else {
+                        visit(cur, [&](unsigned e) {
+                            push = lane_write(push, e, npush);
+                            ++npush;
+                        });
+                    }
+                }
+                unsigned before, total;
+                if (!count_round<K>(pushed, wv, lane, npush, bad, before, total)) {
+                    bad = true;
+                    head = tail;
+                    break;
+                }
+                if (lane < npush) stk[(tail + (int)before + lane) % kQueue] = push;
+                head += take;
+                tail += (int)total;
+                __syncthreads();
             }
-            if (sp == 0) break;
+            // every K-th of them to a wave, whose subtrees it walks by itself
+            Entry *own = stk + kQueue + wv * kOwnStack;
+            int sp = (tail - head + K - 1 - wv) / K;
+            for (int i = lane; i < sp; i += 64) own[i] = stk[(head + wv + K * (sp - 1 - i)) % kQueue];
+            __builtin_amdgcn_wave_barrier();
+            while (sp > 0) {
+                --sp;
+                const unsigned cur = __builtin_amdgcn_readfirstlane(own[sp]);
+                if ((cur >> 6) >= cap) {
+                    bad = true;
+                    break;
+                }
+                visit(cur, [&](unsigned e) {
+                    own[sp] = e; // every lane, one address
+                    ++sp;
+                });
+            }
         }
         // the waves' sums in wave order
         __syncthreads();
@@ -376,15 +446,16 @@ __global__ __launch_bounds__(64 * K) __attribute__((amdgpu_waves_per_eu(8, 8))) 
 // Waves per group, by the number of groups. One wave per group leaves the
 // 1,024 SIMDs (8 waves each) short of waves below about 8,192 groups, and a
 // visit is a chain of a stack read and scalar loads; more waves shorten the
-// chain of visits but wait for each other every round (a fifth to a third of
-// the time once the chip is full). us of the force stage, 1 / 4 / 8 / 16 waves:
+// chain of visits but wait for each other. us of the force stage, 1 / 4 / 8 / 16 waves:
 //   16,384 bodies (256), ball, theta 0.5, vote 16          307 / 149 / 94 / 73
 //   32,768 bodies (512), disk, theta 1.22, vote 16         110 / 74 / 46 / 36
-//   65,536 bodies (1,024), ball, theta 0.5, vote 64        402 / 189 / 147 / 167
-//   100,003 bodies (1,563), two spheres, theta 0.4, 64     890 / 440 / 431 / 470
-//   131,072 bodies (2,048), Plummer, theta 1.22, vote 16   140 / 98 / 106 / 148
-//   262,144 bodies (4,096), two spheres, theta 0.4, 64     1156 / 913 / 1014 / 1216
-//   524,288 bodies (8,192), two spheres, theta 0.4, 64     1635 / 1740 / 1996 / 2452
+//   16,384 bodies (256), ball, theta 0.5, vote 64          272 / 113 / 71 / 56
+//   65,536 bodies (1,024), ball, theta 0.5, vote 64        397 / 172 / 134 / 152
+//   100,003 bodies (1,563), two spheres, theta 0.4, 64     895 / 411 / 380 / 428
+//   131,072 bodies (2,048), two spheres, theta 0.4, 64     934 / 471 / 471 / 550
+//   262,144 bodies (4,096), two spheres, theta 0.4, 64     1147 / 903 / 920 / 1113
+//   327,680 bodies (5,120), disk, theta 1.22, vote 64      138 / 133 / 162 / 263
+//   400,000 bodies (6,250), disk, theta 1.22, vote 64      152 / 160 / 198 / 304
 // Narrow votes split only where it gains most (three times and more). A wave
 // alone adds every body's terms in the order of its group's own depth-first
 // walk, bit for bit what a walk per group gives, and the reference's vote and
