@@ -968,7 +968,7 @@ int nb_create(const nb_params *p, nb_sim **out)
         for (int **a : {&d.kb_ipar, &d.kb_lpar, &d.kb_lo, &d.kb_own, &d.kb_ktop, &d.kb_obase})
             ok = ok && dalloc(a, (size_t)n) == hipSuccess;
         ok = ok && dalloc(&d.kb_scan, stiles) == hipSuccess && dalloc(&d.kb_tdep, stiles) == hipSuccess;
-        const size_t S = (size_t)nb::bucket_samples(n);
+        const size_t S = (size_t)nb::bucket_splitters(n);
         ok = ok && dalloc(&d.kb_spl, S) == hipSuccess && dalloc(&d.kb_bcnt, S + 1) == hipSuccess &&
              dalloc(&d.kb_bfill, S + 1) == hipSuccess && dalloc(&d.kb_bstart, S + 2) == hipSuccess;
     }

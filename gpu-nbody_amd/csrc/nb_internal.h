@@ -51,7 +51,7 @@
 //                                   (first sorted body), kb_own / kb_ktop /
 //                                   kb_obase (octree levels and first cell held)
 //            kb_scan, kb_tdep: per scan tile of the cell counts, its sum and depth
-//            kb_spl, kb_bcnt, kb_bfill, kb_bstart: the buckets of a warm build
+//            kb_spl, kb_bcnt, kb_bfill, kb_bstart: the buckets of a build
 //
 // Body records are 16-byte AoS: streaming kernels still read them with fully
 // coalesced 16-byte lanes, and the gathers of the tree stages touch one cache
@@ -163,7 +163,7 @@ struct Dev {
     unsigned long long *kb_deep;
     unsigned *kb_hist, *kb_offs, *kb_tot;
     int *kb_ipar, *kb_lpar, *kb_lo, *kb_own, *kb_ktop, *kb_obase, *kb_scan, *kb_tdep;
-    // warm builds: splitters (S = bucket_samples(n)), bucket counts, fill
+    // builds by buckets: splitters (S = bucket_splitters(n)), bucket counts, fill
     // counters (S + 1 each) and starts (S + 2)
     unsigned long long *kb_spl;
     unsigned *kb_bcnt, *kb_bfill, *kb_bstart;
@@ -181,6 +181,15 @@ constexpr int kKeyScanTile = 512;  // binary nodes per scan tile (at least)
 constexpr int kBucketT = 256;      // warm builds: one splitter per kBucketT bodies
 constexpr int kBucketCap = 512;    // buckets sorted in LDS up to this size
 inline int bucket_samples(int n) { return (n + kBucketT - 1) / kBucketT; }
+// first builds of up to kColdBodies bodies: splitters by sampling, one per
+// kColdT bodies (their buckets vary more in size, so they are smaller on average)
+constexpr int kColdBodies = 131072, kColdT = 128;
+inline int cold_samples(int n) { return n / kColdT; }
+inline int bucket_splitters(int n) // the most splitters of a build
+{
+    const int warm = bucket_samples(n), cold = n <= kColdBodies ? cold_samples(n) : 0;
+    return warm > cold ? warm : cold;
+}
 // The cells grouped by level: up to kBuildLevels bodies the build's last two
 // kernels scan the cell counts and group the cells themselves, by counters of
 // the levels in device memory; for more, two launches scan and launch_levels'

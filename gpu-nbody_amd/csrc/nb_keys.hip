@@ -64,6 +64,19 @@ __device__ __forceinline__ void key_descend(float &cx, float &cy, float &cz, flo
     r = rh;
 }
 
+// the key of a body at p: 21 levels of its octant path from the root cell
+__device__ __forceinline__ unsigned long long path_key(float cx, float cy, float cz, float r, float4 p)
+{
+    unsigned long long k = 0;
+#pragma unroll
+    for (int L = 0; L < kKeyLevels; ++L) {
+        const int o = key_octant(cx, cy, cz, p);
+        k = (k << 3) | (unsigned long long)o;
+        key_descend(cx, cy, cz, r, o);
+    }
+    return k;
+}
+
 // The level counters of the tree to be built, and no levels until it is there
 // (one block of at least kMaxDepth threads): a build that an error stops leaves
 // none to summarize.
@@ -88,16 +101,7 @@ __global__ __launch_bounds__(256) void k_keys(Dev d, const int *__restrict__ ord
     if (blockIdx.x == 0) clear_levels(d);
     if (i >= d.n || ctl->error) return;
     const int b = order ? order[i] : i;
-    const float4 p = d.pm4[b];
-    float cx = ctl->root[0], cy = ctl->root[1], cz = ctl->root[2], r = ctl->radius;
-    unsigned long long k = 0;
-#pragma unroll
-    for (int L = 0; L < kKeyLevels; ++L) {
-        const int o = key_octant(cx, cy, cz, p);
-        k = (k << 3) | (unsigned long long)o;
-        key_descend(cx, cy, cz, r, o);
-    }
-    key[i] = k;
+    key[i] = path_key(ctl->root[0], ctl->root[1], ctl->root[2], ctl->radius, d.pm4[b]);
     val[i] = b;
 }
 
@@ -281,8 +285,6 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_scatter(const unsigned long l
 // ---------------------------------------------------------------------------
 constexpr int kBsThreads = 256; // blocks of the bucket sort
 constexpr int kBsWaves = kBsThreads / 64;
-constexpr int kBsPerThread = kBucketCap / kBsThreads;
-static_assert(kBucketCap % kBsThreads == 0, "whole rows of the block");
 static_assert(kBsThreads == kRsBins, "a thread per digit");
 
 // the splitters of the next warm build alone (launch_bbox does it otherwise)
@@ -420,14 +422,7 @@ __global__ __launch_bounds__(256) void k_keys_warm(Dev d, const int *__restrict_
     for (int j = 0; j < kWarmPer; ++j) {
         const int i = first + j * 256 + t;
         const bool valid = i < n;
-        unsigned long long k = 0;
-        float cx = rx, cy = ry, cz = rz, r = rr;
-#pragma unroll
-        for (int L = 0; L < kKeyLevels; ++L) {
-            const int o = key_octant(cx, cy, cz, p[j]);
-            k = (k << 3) | (unsigned long long)o;
-            key_descend(cx, cy, cz, r, o);
-        }
+        const unsigned long long k = path_key(rx, ry, rz, rr, p[j]);
         int bk = valid ? bucket_in_window(ws, w0, k) : -1;
         const bool inwin = bk >= 0;
         if (valid && !inwin) {
@@ -597,6 +592,204 @@ __global__ __launch_bounds__(256) void k_bucket_scatter(const Ctl *ctl, const un
         kout[pos] = k[j];
         vout[pos] = v[j];
     }
+}
+
+// ---------------------------------------------------------------------------
+// First builds of up to kColdBodies bodies. There is no last order, so the
+// splitters come from a sample: one block sorts the keys of 1024 or 2048 bodies
+// spread over the indices and takes every (samples / (S + 1))-th (k_sample).
+// Blocks of kColdPer bodies then find each body's bucket among all S <= 1024
+// splitters in LDS, count the buckets in LDS and take their places in each
+// bucket with one atomic per bucket and block (k_keys_cold); the scan of the
+// counts gives the buckets' starts (k_cold_scatter), and the buckets are sorted
+// as in a warm build. Four launches where the radix sort takes 26: the first
+// build of 16,384 bodies takes 58 us instead of 187, of 100,003 87 instead of
+// 200.
+// A bucket has at least 2 samples to its name on average, so that one above
+// kColdCap = 8 times its size (Gamma(2) > 16: 2e-6) is rare.
+// ---------------------------------------------------------------------------
+constexpr int kColdCap = 1024; // bodies of a bucket sorted in LDS
+constexpr int kColdPer = 512;
+constexpr int kColdMax = kColdBodies / kColdT; // splitters
+constexpr int kSampleThreads = 1024;
+
+// The value of lane ^ STEP: DPP moves (quad_perm, row_half_mirror then the
+// reversed quads, row_ror) and the row swaps of permlane, which leave the LDS
+// unit alone.
+template <int CTRL> __device__ __forceinline__ unsigned dpp_u(unsigned v)
+{
+    return (unsigned)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xF, 0xF, false);
+}
+
+template <int STEP> __device__ __forceinline__ unsigned lane_xor(unsigned v)
+{
+    if constexpr (STEP == 1) return dpp_u<0xB1>(v);
+    if constexpr (STEP == 2) return dpp_u<0x4E>(v);
+    if constexpr (STEP == 4) return dpp_u<0x1B>(dpp_u<0x141>(v));
+    if constexpr (STEP == 8) return dpp_u<0x128>(v);
+    const bool high = (threadIdx.x & STEP) != 0;
+    if constexpr (STEP == 16) {
+        const auto s = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+        return high ? s[0] : s[1];
+    } else {
+        const auto s = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+        return high ? s[0] : s[1];
+    }
+}
+
+template <int STEP> __device__ __forceinline__ unsigned long long lane_xor64(unsigned long long v)
+{
+    return (unsigned long long)lane_xor<STEP>((unsigned)(v >> 32)) << 32 | lane_xor<STEP>((unsigned)v);
+}
+
+template <int R, class Other>
+__device__ __forceinline__ void keep(unsigned long long (&k)[R], bool smaller, const Other &other)
+{
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const unsigned long long o = other(r);
+        if ((o < k[r]) == smaller) k[r] = o;
+    }
+}
+
+// The index of sample i: multiples of the golden ratio modulo 1 spread evenly, and
+// unlike equal strides they keep no step with an order that has a period (a
+// lattice, row by row, of which equal strides may see one face).
+__device__ __forceinline__ int sample_index(int i, int n)
+{
+    return (int)(((unsigned long long)((unsigned)i * 0x9E3779B1u) * (unsigned)n) >> 32);
+}
+
+// R samples per thread, places R t .. R t + R - 1 of the bitonic sort: partners
+// `step` places apart are in the thread's registers, in its wave, or in LDS.
+template <int R> __global__ __launch_bounds__(kSampleThreads) void k_sample(Dev d, int S)
+{
+    constexpr int T = kSampleThreads, M = R * T;
+    static_assert(R == 1 || R == 2, "partners in a thread: places 0 and 1");
+    __shared__ unsigned long long sk[R][T];
+    const Ctl *ctl = d.ctl;
+    if (ctl->error) return;
+    const int t = threadIdx.x, n = d.n;
+    const float rx = ctl->root[0], ry = ctl->root[1], rz = ctl->root[2], rr = ctl->radius;
+    unsigned long long k[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) k[r] = path_key(rx, ry, rz, rr, d.pm4[sample_index(R * t + r, n)]);
+    for (int j = t; j <= S; j += T) d.kb_bcnt[j] = 0;
+    for (int size = 2; size <= M; size <<= 1) {
+        const bool up = (R * t & size) == 0;
+        for (int step = size >> 1; step >= R; step >>= 1) {
+            const bool smaller = ((R * t & step) == 0) == up;
+            const int lanes = step / R; // the same in every thread
+            switch (lanes) {
+            case 1: keep(k, smaller, [&](int r) { return lane_xor64<1>(k[r]); }); break;
+            case 2: keep(k, smaller, [&](int r) { return lane_xor64<2>(k[r]); }); break;
+            case 4: keep(k, smaller, [&](int r) { return lane_xor64<4>(k[r]); }); break;
+            case 8: keep(k, smaller, [&](int r) { return lane_xor64<8>(k[r]); }); break;
+            case 16: keep(k, smaller, [&](int r) { return lane_xor64<16>(k[r]); }); break;
+            case 32: keep(k, smaller, [&](int r) { return lane_xor64<32>(k[r]); }); break;
+            default:
+                __syncthreads();
+#pragma unroll
+                for (int r = 0; r < R; ++r) sk[r][t] = k[r];
+                __syncthreads();
+                keep(k, smaller, [&](int r) { return sk[r][t ^ lanes]; });
+            }
+        }
+        if constexpr (R == 2) {
+            const unsigned long long lo = min(k[0], k[1]), hi = max(k[0], k[1]);
+            k[0] = up ? lo : hi;
+            k[1] = up ? hi : lo;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < R; ++r) sk[r][t] = k[r];
+    __syncthreads();
+    for (int j = t; j < S; j += T) {
+        const int at = (int)((long long)(j + 1) * M / (S + 1));
+        d.kb_spl[j] = sk[at % R][at / R];
+    }
+}
+
+// (key, body) in the bodies' order, and where[i] = place in the bucket << 11 |
+// bucket (a place is below 2^17, a bucket at most 2^10)
+__global__ __launch_bounds__(256) void k_keys_cold(Dev d, int S, unsigned long long *__restrict__ key,
+                                                   int *__restrict__ where)
+{
+    __shared__ unsigned long long spl[kColdMax];
+    __shared__ unsigned h[kColdMax + 1];
+    const Ctl *ctl = d.ctl;
+    const int t = threadIdx.x, n = d.n, first = blockIdx.x * kColdPer;
+    if (blockIdx.x == 0) clear_levels(d);
+    if (__syncthreads_or(ctl->error)) return;
+    for (int j = t; j < S; j += 256) spl[j] = d.kb_spl[j];
+    for (int j = t; j <= S; j += 256) h[j] = 0;
+    __syncthreads();
+    const float rx = ctl->root[0], ry = ctl->root[1], rz = ctl->root[2], rr = ctl->radius;
+    constexpr int per = kColdPer / 256;
+    unsigned long long k[per];
+    int b[per];
+    unsigned at[per];
+#pragma unroll
+    for (int u = 0; u < per; ++u) {
+        const int i = first + u * 256 + t;
+        k[u] = path_key(rx, ry, rz, rr, d.pm4[min(i, n - 1)]);
+        if (i < n) key[i] = k[u];
+        b[u] = 0;
+    }
+    // b = the splitters <= k, all bodies of the thread at once
+#pragma unroll
+    for (int step = kColdMax; step > 0; step >>= 1) {
+#pragma unroll
+        for (int u = 0; u < per; ++u)
+            if (b[u] + step <= S && spl[b[u] + step - 1] <= k[u]) b[u] += step;
+    }
+#pragma unroll
+    for (int u = 0; u < per; ++u) {
+        if (first + u * 256 + t >= n) b[u] = -1;
+        else at[u] = atomicAdd(&h[b[u]], 1u);
+    }
+    __syncthreads();
+    for (int j = t; j <= S; j += 256)
+        if (h[j]) h[j] = atomicAdd(&d.kb_bcnt[j], h[j]);
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < per; ++u)
+        if (b[u] >= 0) where[first + u * 256 + t] = (int)((h[b[u]] + at[u]) << 11 | (unsigned)b[u]);
+}
+
+__global__ __launch_bounds__(256) void k_cold_scatter(const Ctl *ctl, int n, int S, const unsigned *__restrict__ bcnt,
+                                                      const unsigned long long *__restrict__ kin,
+                                                      const int *__restrict__ where,
+                                                      unsigned long long *__restrict__ kout, int *__restrict__ vout,
+                                                      unsigned *__restrict__ bstart)
+{
+    constexpr int per = (kColdMax + 1 + 255) / 256;
+    __shared__ unsigned starts[per * 256], wsum[4];
+    const int err = ctl->error;
+    const int t = threadIdx.x, i = blockIdx.x * 256 + t;
+    const unsigned long long k = i < n ? kin[i] : 0ull;
+    const int w = i < n ? where[i] : 0;
+    unsigned c[per], sum = 0;
+#pragma unroll
+    for (int q = 0; q < per; ++q) {
+        const int j = per * t + q;
+        c[q] = j <= S ? bcnt[j] : 0u;
+        sum += c[q];
+    }
+    unsigned run = scan256_total(sum, wsum);
+#pragma unroll
+    for (int q = 0; q < per; ++q) {
+        const int j = per * t + q;
+        starts[j] = run;
+        if (blockIdx.x == 0 && j <= S) bstart[j] = run;
+        run += c[q];
+    }
+    if (blockIdx.x == 0 && t == 0) bstart[S + 1] = (unsigned)n;
+    if (__syncthreads_or(err) || i >= n) return;
+    const unsigned pos = starts[w & 2047] + ((unsigned)w >> 11);
+    kout[pos] = k;
+    vout[pos] = i;
 }
 
 struct RankLds {
@@ -804,10 +997,10 @@ __device__ void order_long_run(const Dev &d, int i, int m, int *val, unsigned lo
 // A larger bucket goes through device memory by stable radix passes ((tkey,
 // tval) are free n-element buffers), and one thread orders each of its runs.
 constexpr int kCountStep = 4; // keys a count reads at once
-struct BucketLds {
-    unsigned long long sk[kBucketCap + kCountStep]; // past the bucket: ~0 (keys use 63 bits)
-    unsigned long long dw[kDeepWords][kBucketCap]; // deep words of the keys that have equals
-    int sv[kBucketCap];
+template <int CAP> struct BucketLds {
+    unsigned long long sk[CAP + kCountStep]; // past the bucket: ~0 (keys use 63 bits)
+    unsigned long long dw[kDeepWords][CAP]; // deep words of the keys that have equals
+    int sv[CAP];
     unsigned start[kRsBins + 1];
     unsigned cnt[kRsBins];
     unsigned wsum[kBsWaves];
@@ -816,10 +1009,10 @@ struct BucketLds {
 
 __device__ void sort_large_bucket(const Dev &d, unsigned long long *key, int *val, unsigned long long *deep,
                                   unsigned long long *tkey, int *tval, int *perm, int *tmp, int base, int m,
-                                  RankLds &R, unsigned long long *red)
+                                  bool warm, RankLds &R, unsigned long long *red)
 {
     const int t = threadIdx.x;
-    if (t == 0) atomicAdd(&d.ctl->large_buckets, 1);
+    if (warm && t == 0) atomicAdd(&d.ctl->large_buckets, 1);
     unsigned long long *k0 = key + base, *k1 = tkey + base;
     int *v0 = val + base, *v1 = tval + base;
     const int top = varying_top_bit(k0, m, red);
@@ -845,38 +1038,41 @@ __device__ void sort_large_bucket(const Dev &d, unsigned long long *key, int *va
     }
 }
 
+template <int CAP>
 __global__ __launch_bounds__(kBsThreads) void k_bucket_sort(Dev d, unsigned long long *__restrict__ key,
                                                             int *__restrict__ val,
                                                             unsigned long long *__restrict__ deep,
                                                             unsigned long long *__restrict__ tkey,
                                                             int *__restrict__ tval, int *__restrict__ perm,
                                                             int *__restrict__ tmp,
-                                                            const unsigned *__restrict__ bstart)
+                                                            const unsigned *__restrict__ bstart, bool warm)
 {
     __shared__ union {
-        BucketLds b;
+        BucketLds<CAP> b;
         struct {
             RankLds rank;
             unsigned long long red;
         } large;
     } lds;
+    constexpr int kPer = CAP / kBsThreads;
+    static_assert(CAP % kBsThreads == 0, "whole rows of the block");
     const Ctl *ctl = d.ctl;
     const int t = threadIdx.x, w = t >> 6;
     const int base = (int)bstart[blockIdx.x], m = (int)bstart[blockIdx.x + 1] - base;
     // the same decision in every wave: a bucket sorted at the same time may flag
     // an error, and a wave that left then would leave its keys out of the counts
     if (__syncthreads_or(ctl->error) || m <= 1) return;
-    if (m > kBucketCap) {
-        sort_large_bucket(d, key, val, deep, tkey, tval, perm, tmp, base, m, lds.large.rank, &lds.large.red);
+    if (m > CAP) {
+        sort_large_bucket(d, key, val, deep, tkey, tval, perm, tmp, base, m, warm, lds.large.rank, &lds.large.red);
         return;
     }
-    BucketLds &s = lds.b;
+    BucketLds<CAP> &s = lds.b;
     const size_t n = (size_t)d.n;
-    unsigned long long k[kBsPerThread], diff = 0;
-    int v[kBsPerThread];
+    unsigned long long k[kPer], diff = 0;
+    int v[kPer];
     const unsigned long long k0 = key[base];
 #pragma unroll
-    for (int r = 0; r < kBsPerThread; ++r) {
+    for (int r = 0; r < kPer; ++r) {
         const int i = r * kBsThreads + t;
         k[r] = i < m ? key[base + i] : k0;
         v[r] = i < m ? val[base + i] : 0;
@@ -890,9 +1086,9 @@ __global__ __launch_bounds__(kBsThreads) void k_bucket_sort(Dev d, unsigned long
     diff = s.diff[0] | s.diff[1] | s.diff[2] | s.diff[3];
     const int top = diff ? 63 - __clzll((long long)diff) : 0;
     const int shift = max(0, top - 7);
-    unsigned at[kBsPerThread];
+    unsigned at[kPer];
 #pragma unroll
-    for (int r = 0; r < kBsPerThread; ++r)
+    for (int r = 0; r < kPer; ++r)
         if (r * kBsThreads + t < m) at[r] = atomicAdd(&s.cnt[(unsigned)(k[r] >> shift) & 255u], 1u);
     __syncthreads();
     const unsigned mine = s.cnt[t];
@@ -900,7 +1096,7 @@ __global__ __launch_bounds__(kBsThreads) void k_bucket_sort(Dev d, unsigned long
     if (t == 0) s.start[kRsBins] = (unsigned)m;
     __syncthreads();
 #pragma unroll
-    for (int r = 0; r < kBsPerThread; ++r) {
+    for (int r = 0; r < kPer; ++r) {
         if (r * kBsThreads + t >= m) continue;
         const unsigned p = s.start[(unsigned)(k[r] >> shift) & 255u] + at[r];
         s.sk[p] = k[r];
@@ -910,9 +1106,9 @@ __global__ __launch_bounds__(kBsThreads) void k_bucket_sort(Dev d, unsigned long
     __syncthreads();
     // from here a thread's elements are the places i of the distributed order
     bool run = false;
-    int place[kBsPerThread];
+    int place[kPer];
 #pragma unroll
-    for (int r = 0; r < kBsPerThread; ++r) {
+    for (int r = 0; r < kPer; ++r) {
         const int i = r * kBsThreads + t;
         place[r] = -1;
         if (i >= m) continue;
@@ -937,7 +1133,7 @@ __global__ __launch_bounds__(kBsThreads) void k_bucket_sort(Dev d, unsigned long
     if (__syncthreads_or(run)) {
         const float rx = ctl->root[0], ry = ctl->root[1], rz = ctl->root[2], rr = ctl->radius;
 #pragma unroll
-        for (int r = 0; r < kBsPerThread; ++r) {
+        for (int r = 0; r < kPer; ++r) {
             if (place[r] < 0 || at[r] < 2) continue;
             unsigned long long w3[kDeepWords];
             deep_words(rx, ry, rz, rr, d.pm4[v[r]], w3);
@@ -946,7 +1142,7 @@ __global__ __launch_bounds__(kBsThreads) void k_bucket_sort(Dev d, unsigned long
         }
         __syncthreads();
 #pragma unroll
-        for (int r = 0; r < kBsPerThread; ++r) {
+        for (int r = 0; r < kPer; ++r) {
             if (place[r] < 0 || at[r] < 2) continue;
             const int i = r * kBsThreads + t;
             const unsigned dg = (unsigned)(k[r] >> shift) & 255u;
@@ -972,7 +1168,7 @@ __global__ __launch_bounds__(kBsThreads) void k_bucket_sort(Dev d, unsigned long
         }
     }
 #pragma unroll
-    for (int r = 0; r < kBsPerThread; ++r) {
+    for (int r = 0; r < kPer; ++r) {
         if (place[r] < 0) continue;
         key[base + place[r]] = k[r];
         val[base + place[r]] = v[r];
@@ -1591,8 +1787,18 @@ hipError_t launch_build_keys(const Dev &d, bool warm, bool staged, bool splitter
                                S, d.kb_bstart, d.kb_bfill);
         }
         // (the binary tree's arrays, written later, serve the runs of large buckets)
-        hipLaunchKernelGGL(k_bucket_sort, dim3(S + 1), dim3(kBsThreads), 0, st, d, ka, va, d.kb_deep, kb, vb, d.kb_ipar,
-                           d.kb_lpar, d.kb_bstart);
+        hipLaunchKernelGGL(k_bucket_sort<kBucketCap>, dim3(S + 1), dim3(kBsThreads), 0, st, d, ka, va, d.kb_deep, kb,
+                           vb, d.kb_ipar, d.kb_lpar, d.kb_bstart, true);
+    } else if (n <= kColdBodies) {
+        const int S = cold_samples(n);
+        const dim3 gc((n + kColdPer - 1) / kColdPer);
+        const dim3 one(1), ts(kSampleThreads);
+        if (n <= kColdBodies / 2) hipLaunchKernelGGL(k_sample<1>, one, ts, 0, st, d, S);
+        else hipLaunchKernelGGL(k_sample<2>, one, ts, 0, st, d, S);
+        hipLaunchKernelGGL(k_keys_cold, gc, b256, 0, st, d, S, kb, d.kb_lo);
+        hipLaunchKernelGGL(k_cold_scatter, g256, b256, 0, st, d.ctl, n, S, d.kb_bcnt, kb, d.kb_lo, ka, va, d.kb_bstart);
+        hipLaunchKernelGGL(k_bucket_sort<kColdCap>, dim3(S + 1), dim3(kBsThreads), 0, st, d, ka, va, d.kb_deep, kb, vb,
+                           d.kb_ipar, d.kb_lpar, d.kb_bstart, false);
     } else {
         const int ntiles = (n + kRsTile - 1) / kRsTile;
         hipLaunchKernelGGL(k_keys, g256, b256, 0, st, d, nullptr, ka, va);
