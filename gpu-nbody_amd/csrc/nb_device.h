@@ -74,6 +74,61 @@ __device__ __forceinline__ bool end_round(Entry *stk, unsigned *pushed, int wv, 
     return true;
 }
 
+// K waves that share a group and part: breadth first, a cell each per round,
+// until the queue holds FRONT cells; then each wave takes every K-th of them
+// and walks their subtrees by itself, depth first. The queue is a ring of
+// kQueue entries; a wave's own stack holds its share of it and 7 entries for
+// each level below. The order depends on the tree alone. stk: parted_stack
+// words, the root in the first (before a barrier); visit(entry, opened) calls
+// opened(entry) for what it opens and may set bad. Returns bad.
+constexpr int kQueue = 512, kOwnStack = 576;
+template <int K> constexpr int parted_stack() { return kQueue + K * kOwnStack; }
+
+template <int K, int FRONT, class Visit>
+__device__ __forceinline__ bool walk_parted(unsigned *stk, unsigned *pushed, int wv, int lane, unsigned cap, bool &bad,
+                                            Visit &&visit)
+{
+    static_assert(FRONT - 1 + 8 * K <= kQueue && (FRONT - 1 + 8 * K + K - 1) / K + 7 * kMaxDepth + 8 <= kOwnStack,
+                  "the queue and the stacks hold every tree of kMaxDepth levels");
+    int head = 0, tail = 1; // the same in every wave
+    while (tail > head && tail - head < FRONT) {
+        const int take = min(tail - head, K);
+        int npush = 0;
+        unsigned push = 0; // entry j of this wave's children in lane j
+        if (wv < take) {
+            const unsigned cur = __builtin_amdgcn_readfirstlane(stk[(head + wv) % kQueue]);
+            if ((cur >> 6) >= cap) { // the pool holds `cap` cells: corrupt
+                bad = true;
+            } else {
+                visit(cur, [&](unsigned e) {
+                    push = lane_write(push, e, npush);
+                    ++npush;
+                });
+            }
+        }
+        unsigned before, total;
+        if (!count_round<K>(pushed, wv, lane, npush, bad, before, total)) return true;
+        if (lane < npush) stk[(tail + (int)before + lane) % kQueue] = push;
+        head += take;
+        tail += (int)total;
+        __syncthreads();
+    }
+    unsigned *own = stk + kQueue + wv * kOwnStack;
+    int sp = (tail - head + K - 1 - wv) / K;
+    for (int i = lane; i < sp; i += 64) own[i] = stk[(head + wv + K * (sp - 1 - i)) % kQueue];
+    __builtin_amdgcn_wave_barrier();
+    while (sp > 0) {
+        --sp;
+        const unsigned cur = __builtin_amdgcn_readfirstlane(own[sp]);
+        if ((cur >> 6) >= cap) return true;
+        visit(cur, [&](unsigned e) {
+            own[sp] = e; // every lane, one address
+            ++sp;
+        });
+    }
+    return bad;
+}
+
 __device__ __forceinline__ void kahan_add(float &sum, float &comp, float x)
 {
     const float y = x - comp;

@@ -197,21 +197,10 @@ template <> struct StackEntry<64> {
     using type = unsigned;
 };
 
-// K waves that share a group at vote width 64 walk breadth first until the queue
-// holds kFront cells; then each takes every K-th of them and walks their
-// subtrees by itself. The queue is a ring of kQueue entries; a wave's own stack
-// holds its share of it and 7 entries for each level below.
-constexpr int kFront = 256, kQueue = 512, kOwnStack = 576;
-template <int K> constexpr bool queue_fits()
-{
-    return kFront - 1 + 8 * K <= kQueue && (kFront - 1 + 8 * K + K - 1) / K + 7 * kMaxDepth + 8 <= kOwnStack;
-}
-
 // The epilogue's per-wave sums overlay the stacks.
 template <int G, int K> constexpr int force_lds()
 {
-    static_assert(K == 1 || G < 64 || queue_fits<K>(), "the queue and the stacks hold every tree of kMaxDepth levels");
-    const int entries = K == 1 ? kStack : G < 64 ? split_stack<K>() : kQueue + K * kOwnStack;
+    const int entries = K == 1 ? kStack : G < 64 ? split_stack<K>() : parted_stack<K>();
     const int stack = entries * (int)sizeof(typename StackEntry<G>::type), red = K == 1 ? 0 : K * 3 * 64 * 8;
     return ((stack > red ? stack : red) + 15) & ~15;
 }
@@ -220,7 +209,7 @@ template <int G, int K> constexpr int force_lds()
 // wave per group would leave the chip idle). With narrow votes they take the
 // stack's top K entries in rounds: wave w visits the w-th from the top, and
 // after a barrier pushes what it opened behind the lower waves' entries. At
-// width 64 they part after a first stretch of such rounds (kFront): a round
+// width 64 they part after a first stretch of rounds (walk_parted): a round
 // lasts as long as its slowest visit, and from there on no wave waits for
 // another (100,003 bodies, two spheres: 442 -> 377 us; 262,144: 980 -> 900; 65,536,
 // ball: 149 -> 134). Parting at 128 cells is faster for a uniform ball (177
@@ -357,7 +346,7 @@ __global__ __launch_bounds__(64 * K) __attribute__((amdgpu_waves_per_eu(8, 8))) 
                 if (sp == 0) break;
             }
         } else {
-            auto visit = [&](unsigned cur, auto &&opened) {
+            bad = walk_parted<K, 256>(stk, pushed, wv, lane, cap, bad, [&](unsigned cur, auto &&opened) {
                 float px, py, pz;
                 const int children =
                     visit_wide<false>(cur, dq_s[cur & 63u], me, eps2, cchild, cdata, px, py, pz, bad, opened);
@@ -365,52 +354,7 @@ __global__ __launch_bounds__(64 * K) __attribute__((amdgpu_waves_per_eu(8, 8))) 
                 sy += (double)py;
                 sz += (double)pz;
                 inter += (unsigned)(children - 1);
-            };
-            // breadth first, a cell each, until the queue holds enough
-            int head = 0, tail = 1; // the same in every wave
-            while (tail > head && tail - head < kFront) {
-                const int take = min(tail - head, K);
-                int npush = 0;
-                unsigned push = 0; // entry j of this wave's children in lane j
-                if (wv < take) {
-                    const unsigned cur = __builtin_amdgcn_readfirstlane(stk[(head + wv) % kQueue]);
-                    if ((cur >> 6) >= cap) { // the pool holds `cap` cells: corrupt
-                        bad = true;
-                    } else {
-                        visit(cur, [&](unsigned e) {
-                            push = lane_write(push, e, npush);
-                            ++npush;
-                        });
-                    }
-                }
-                unsigned before, total;
-                if (!count_round<K>(pushed, wv, lane, npush, bad, before, total)) {
-                    bad = true;
-                    head = tail;
-                    break;
-                }
-                if (lane < npush) stk[(tail + (int)before + lane) % kQueue] = push;
-                head += take;
-                tail += (int)total;
-                __syncthreads();
-            }
-            // every K-th of them to a wave, whose subtrees it walks by itself
-            Entry *own = stk + kQueue + wv * kOwnStack;
-            int sp = (tail - head + K - 1 - wv) / K;
-            for (int i = lane; i < sp; i += 64) own[i] = stk[(head + wv + K * (sp - 1 - i)) % kQueue];
-            __builtin_amdgcn_wave_barrier();
-            while (sp > 0) {
-                --sp;
-                const unsigned cur = __builtin_amdgcn_readfirstlane(own[sp]);
-                if ((cur >> 6) >= cap) {
-                    bad = true;
-                    break;
-                }
-                visit(cur, [&](unsigned e) {
-                    own[sp] = e; // every lane, one address
-                    ++sp;
-                });
-            }
+            });
         }
         // the waves' sums in wave order
         __syncthreads();
@@ -473,11 +417,12 @@ template <int G> static void launch_force_g(const Dev &d, int mode, hipStream_t 
     const dim3 grid(groups);
     const int *cc = d.cchild;
     const float4 *cd = d.cdata;
-    switch (waves_per_group(groups, G < 64)) {
-    case 16: hipLaunchKernelGGL((k_force<G, 16>), grid, dim3(1024), 0, st, d, cc, cd, mode); break;
-    case 8: hipLaunchKernelGGL((k_force<G, 8>), grid, dim3(512), 0, st, d, cc, cd, mode); break;
-    case 4: hipLaunchKernelGGL((k_force<G, 4>), grid, dim3(256), 0, st, d, cc, cd, mode); break;
-    default: hipLaunchKernelGGL((k_force<G, 1>), grid, dim3(64), 0, st, d, cc, cd, mode); break;
+    const int k = waves_per_group(groups, G < 64);
+    if (k == 16) hipLaunchKernelGGL((k_force<G, 16>), grid, dim3(1024), 0, st, d, cc, cd, mode);
+    else if (k == 1) hipLaunchKernelGGL((k_force<G, 1>), grid, dim3(64), 0, st, d, cc, cd, mode);
+    else if constexpr (G == 64) {
+        if (k == 8) hipLaunchKernelGGL((k_force<G, 8>), grid, dim3(512), 0, st, d, cc, cd, mode);
+        else hipLaunchKernelGGL((k_force<G, 4>), grid, dim3(256), 0, st, d, cc, cd, mode);
     }
 }
 

@@ -219,7 +219,7 @@ template <int OUT, int K, bool REC> __device__ __forceinline__ void coarse_trave
     // learned step's 64 rows of BF16 features (64 x 24 x 2 bytes)
     constexpr int kRedBytes = K == 1 ? 0 : K * 64 * (kFeatOn ? 9 * 4 : 3 * 8);
     constexpr int kFeatBytes = OUT == kOutLearned ? 64 * kFeat * 2 : 0;
-    constexpr int kStackBytes = split_stack<K>() * 4;
+    constexpr int kStackBytes = (K == 1 ? kStack : parted_stack<K>()) * 4;
     constexpr int kLds = kStackBytes > kRedBytes ? (kStackBytes > kFeatBytes ? kStackBytes : kFeatBytes)
                                                  : (kRedBytes > kFeatBytes ? kRedBytes : kFeatBytes);
     struct WaveTotals {
@@ -422,29 +422,8 @@ template <int OUT, int K, bool REC> __device__ __forceinline__ void coarse_trave
         }
     } else {
         if (tid == 0) stk[0] = 0; // root cell 0 at depth 0
-        int sp = 1;               // the same in every wave
         __syncthreads();
-        for (;;) {
-            const int take = sp > kSplitTop ? 1 : min(sp, K);
-            int npush = 0;
-            unsigned push = 0; // entry j of this wave's children in lane j
-            if (wv < take) {
-                const unsigned cur = __builtin_amdgcn_readfirstlane(stk[sp - 1 - wv]);
-                if ((cur >> 6) >= cap) { // the pool holds `cap` cells: corrupt
-                    bad = true;
-                } else {
-                    visit(cur, [&](unsigned e) {
-                        push = lane_write(push, e, npush);
-                        ++npush;
-                    });
-                }
-            }
-            if (!end_round<K>(stk, pushed, wv, lane, take, npush, push, bad, sp)) {
-                bad = true;
-                break;
-            }
-            if (sp == 0) break;
-        }
+        bad = walk_parted<K, 64>(stk, pushed, wv, lane, cap, bad, visit);
         // the waves' sums in wave order
         __syncthreads();
         if (lane == 0) totals[wv] = WaveTotals{smb, nbod, nchild, nvisit};
@@ -789,17 +768,20 @@ hipError_t launch_group_order(const Dev &d, hipStream_t st)
 }
 
 // Waves per group, by the number of groups (see waves_per_group in
-// nb_force.hip). us of the force stage, 1 / 4 / 8 / 16 waves, coarse and
-// learned (theta_c 0.9, alpha 0.02):
-//   16,384 bodies (256 groups), Plummer      299 / 157 / 101 / 81     311 / 157 / 89 / 92
-//   40,960 (640), Plummer                    368 / 175 / 131 / 165    377 / 174 / 109 / 181
-//   65,536 (1,024), halo and disk            383 / 199 / 168 / 232    387 / 187 / 140 / 251
-//   131,072 (2,048), Plummer                 443 / 303 / 308 / 451    469 / 275 / 235 / 484
-//   262,144 (4,096), clusters                358 / 333 / 411 / 726    368 / 320 / 348 / 782
-//   524,288 (8,192), halo and disk           670 / 953 / 1105 / 1723  691 / 811 / 826 / 1803
+// nb_force.hip; the waves part at 64 cells: a group opens a few hundred, and
+// breadth first keeps every wave of a round busy, where rounds off the top of a
+// stack took 10 to 40 % longer). us of the force stage, 1 / 4 / 8 / 16 waves,
+// coarse and learned (theta_c 0.9, alpha 0.02):
+//   16,384 bodies (256 groups), Plummer      300 / 118 / 93 / 86      309 / 128 / 85 / 77
+//   40,960 (640), Plummer                    365 / 137 / 114 / 171    377 / 146 / 103 / 149
+//   65,536 (1,024), halo and disk            384 / 153 / 147 / 245    392 / 153 / 133 / 207
+//   100,003 (1,563), clusters                268 / 114 / 154 / 283    280 / 125 / 141 / 265
+//   262,144 (4,096), halo and disk           516 / 295 / 453 / 887    543 / 317 / 383 / 719
+//   524,288 (8,192), halo and disk           680 / 553 / 910 / 1859   720 / 614 / 764 / 1460
+//   700,001 (10,938), halo and disk          697 / 706 / 1202 / -     730 / 786 / 1019 / -
 static int coarse_waves_per_group(int groups)
 {
-    return groups <= 320 ? 16 : groups <= 1536 ? 8 : groups <= 5120 ? 4 : 1;
+    return groups <= 320 ? 16 : groups <= 1280 ? 8 : groups <= 9216 ? 4 : 1;
 }
 
 hipError_t launch_coarse(const Dev &d, const Learn &L, int out, const int *groups, int ngroups, float *xraw,

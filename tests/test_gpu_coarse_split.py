@@ -1,6 +1,6 @@
 """The coarse traversal on both sides of every number of bodies at which the
-number of waves per group changes (20,480, 98,304 and 327,680 bodies: 320, 1,536
-and 5,120 groups of 64), and its listed-group passes through training.
+number of waves per group changes (20,480, 81,920 and 589,824 bodies: 320, 1,280
+and 9,216 groups of 64), and its listed-group passes through training.
 
 The oracle takes the same opening decisions: equal interaction counts (through
 the features' exact counts and the counter), accelerations within 1e-5, as in
@@ -17,7 +17,7 @@ pytestmark = pytest.mark.gpu
 THETA_C, ALPHA, EPS = 0.9, 0.03, 0.02
 
 
-@pytest.mark.parametrize("n", [64, 65, 20_480, 20_481, 98_304, 98_331, 327_680, 327_699])
+@pytest.mark.parametrize("n", [64, 65, 20_480, 20_481, 81_920, 81_921, 98_331, 327_699, 589_824, 589_849])
 def test_coarse_at_split_edges(nb, oracle, n):
     from nbody_amd import universe as U
 
