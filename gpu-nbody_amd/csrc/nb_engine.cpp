@@ -376,12 +376,6 @@ int prepare_levels(nb_sim *s)
     return NB_OK;
 }
 
-// Device address of the force stage's opening table inside Ctl.
-const float *dq_plain_ptr(const nb_sim *s)
-{
-    return reinterpret_cast<const float *>(reinterpret_cast<const char *>(s->d.ctl) + offsetof(nb::Ctl, dq));
-}
-
 // The force method in effect: the configured mode, or plain theta after a
 // failed sampled check.
 int force_method(const nb_sim *s) { return s->fell_back ? NB_MODE_PLAIN : s->p.mode; }
@@ -1468,7 +1462,7 @@ int nb_train(nb_sim *s, const nb_train_params *tp_in, nb_train_report *rep)
     if (!r) r = m.get(&T, (size_t)S * nb::kOut);
     if (!r) r = m.get(&stats, (size_t)2 * (nb::kFeat + nb::kOut));
     if (!r) r = m.get(&frame, (size_t)2 * rows);
-    if (!r) r = m.get(&rec, (size_t)2 * rows);
+    if (!r) r = m.get(&rec, (size_t)2 * rows + nb::kPairCtl);
     if (!r) r = m.get(&afine, (size_t)rows);
     if (!r) r = m.get(&gdev, (size_t)G * tp.steps);
     if (r) return r;
@@ -1494,17 +1488,19 @@ int nb_train(nb_sim *s, const nb_train_params *tp_in, nb_train_report *rep)
     const auto t0 = std::chrono::steady_clock::now();
     for (int k = 0; k < tp.steps; ++k) {
         for (int st = NB_STAGE_BBOX; st <= NB_STAGE_SORT; ++st) {
+            // the last step's pairs read its cells
+            if (k > 0 && st == NB_STAGE_SUMMARIZE) HIP_TRY(s, hipStreamWaitEvent(s->stream, pairs_out, 0));
             r = launch_stage(s, st);
             if (r) return r;
         }
         // the pairs of this step's tree on the second stream, on copies of the
-        // bodies' records, beside the force pass that advances the bodies;
-        // the next step rebuilds the tree only when they are done
+        // bodies' records and the step's scalars, beside the force pass that
+        // advances the bodies and the next step's bounding box and build
         hipError_t e = nb::launch_pair_records(d, gdev + (size_t)k * G, G, rec, s->stream);
         if (e == hipSuccess) e = hipEventRecord(pairs_in, s->stream);
         if (e == hipSuccess) e = hipStreamWaitEvent(s->side, pairs_in, 0);
         if (e == hipSuccess)
-            e = nb::launch_pairs(d, s->L, dq_plain_ptr(s), gdev + (size_t)k * G, G, rec,
+            e = nb::launch_pairs(d, s->L, gdev + (size_t)k * G, G, rec,
                                  X + (size_t)k * rows * nb::kFeat, frame, afine, s->side);
         if (e == hipSuccess)
             e = nb::launch_make_target(frame, afine, rows, T + (size_t)k * rows * nb::kOut, s->side);
@@ -1513,8 +1509,8 @@ int nb_train(nb_sim *s, const nb_train_params *tp_in, nb_train_report *rep)
         // the bodies advance with plain theta
         r = launch_force_method(s, NB_MODE_PLAIN, 1);
         if (r) return r;
-        HIP_TRY(s, hipStreamWaitEvent(s->stream, pairs_out, 0));
     }
+    HIP_TRY(s, hipStreamWaitEvent(s->stream, pairs_out, 0));
     r = check_device_error(s);
     if (r) return r;
     const auto t1 = std::chrono::steady_clock::now();

@@ -282,18 +282,24 @@ struct Learn {
 // features and frames (of listed groups, or of all when `groups` is null),
 // accelerations of listed groups (training targets), or the body update with
 // the coarse acceleration alone.
-// kOutAccel opens cells with the force stage's table `dqtab` (the fine
-// traversal of the training targets); the others with the extent and
-// relative tests of the coarse traversal.
+// kOutAccel opens cells with the force stage's table (the fine traversal of the
+// training targets); the others with the extent and relative tests of the
+// coarse traversal.
 enum CoarseOut { kOutLearned = 0, kOutRaw = 1, kOutAccel = 2, kOutFinish = 3 };
 hipError_t launch_coarse(const Dev &d, const Learn &L, int out, const int *groups, int ngroups, float *xraw,
                          float4 *frame_out, int fmode, hipStream_t st);
-// a step's training pairs: the listed groups' records and accelerations
-// (rec: 2 * 64 per group), then kOutRaw and kOutAccel over the groups, which
-// read the bodies from rec only
+// a step's training pairs: the listed groups' records and accelerations (rec: 2
+// * 64 per group, then a PairCtl), then kOutRaw and kOutAccel over the groups,
+// which read the bodies and the step's scalars from rec only
+struct PairCtl {
+    float dq[kMaxDepth]; // Ctl's of the step
+    float radius;
+    int step;
+};
+constexpr size_t kPairCtl = (sizeof(PairCtl) + sizeof(float4) - 1) / sizeof(float4); // in records
 hipError_t launch_pair_records(const Dev &d, const int *groups, int ngroups, float4 *rec, hipStream_t st);
-hipError_t launch_pairs(const Dev &d, const Learn &L, const float *dqtab, const int *groups, int ngroups,
-                        const float4 *rec, float *xraw, float4 *frame_out, float4 *acc_out, hipStream_t st);
+hipError_t launch_pairs(const Dev &d, const Learn &L, const int *groups, int ngroups, const float4 *rec, float *xraw,
+                        float4 *frame_out, float4 *acc_out, hipStream_t st);
 // The network alone on raw FP32 features x[rows][24] -> residual y[rows][3]
 // (the same matrix-core code as the learned step)
 hipError_t launch_mlp_rows(const Learn &L, const float *xraw, int rows, float *y, hipStream_t st);

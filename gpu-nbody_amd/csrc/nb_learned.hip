@@ -202,15 +202,14 @@ __device__ __forceinline__ void mlp_wave(const uint16_t *fs, const Mlp &m, int l
 #define NB_COARSE_PARAMS                                                                                     \
     Dev d, Learn L, const int *__restrict__ cchild, const float4 *__restrict__ cdata,                        \
         const float4 *__restrict__ cqa, const float4 *__restrict__ cqb, const float2 *__restrict__ cmac,     \
-        const float *__restrict__ dqtab, const int *__restrict__ groups, int ngroups,                        \
+        const int *__restrict__ groups, int ngroups,                                                         \
         const float4 *__restrict__ rec, float *__restrict__ xraw, float4 *__restrict__ frame_out,            \
         float4 *__restrict__ acc_out, int fmode
 #define NB_COARSE_PASS \
-    d, L, cchild, cdata, cqa, cqb, cmac, dqtab, groups, ngroups, rec, xraw, frame_out, acc_out, fmode
+    d, L, cchild, cdata, cqa, cqb, cmac, groups, ngroups, rec, xraw, frame_out, acc_out, fmode
 
 // K waves share a vote group, as in k_force (nb_force.hip): one wave walks depth
-// first; K take the stack's top K entries in rounds, and their sums are added in
-// wave order.
+// first; K start breadth first and part, and their sums are added in wave order.
 template <int OUT, int K, bool REC> __device__ __forceinline__ void coarse_traverse(int gslot, NB_COARSE_PARAMS)
 {
     constexpr bool kFeatOn = OUT == kOutLearned || OUT == kOutRaw;
@@ -244,10 +243,12 @@ template <int OUT, int K, bool REC> __device__ __forceinline__ void coarse_trave
         if (tid == 0) flag_error(ctl, kErrDepth);
         return;
     }
+    // REC: the step's own scalars, as k_pair_records kept them
+    const PairCtl *pc = REC ? reinterpret_cast<const PairCtl *>(rec + 2 * 64 * (size_t)ngroups) : nullptr;
     if (kGeo)
-        for (int i = tid; i < kMaxDepth; i += 64 * K) dq_s[i] = dqtab[i];
-    const int step = ctl->step;
-    const float root_r = ctl->radius;
+        for (int i = tid; i < kMaxDepth; i += 64 * K) dq_s[i] = pc->dq[i];
+    const int step = REC ? pc->step : ctl->step;
+    const float root_r = REC ? pc->radius : ctl->radius;
 
     int g = gslot;
     if (groups) {
@@ -662,11 +663,21 @@ __global__ __launch_bounds__(64) void k_pairs(NB_COARSE_PARAMS)
         coarse_traverse<kOutRaw, 1, true>((int)blockIdx.x - ngroups, NB_COARSE_PASS);
 }
 
-// The records and accelerations of the listed groups' bodies, 64 slots a group
+// The records and accelerations of the listed groups' bodies, 64 slots a group,
+// and behind them the step's scalars: with both, the pairs read nothing that the
+// next step's bounding box and build write
 __global__ __launch_bounds__(256) void k_pair_records(Dev d, const int *__restrict__ groups, int slots,
                                                       float4 *__restrict__ rec)
 {
     const int i = blockIdx.x * 256 + threadIdx.x;
+    if (blockIdx.x == 0) {
+        PairCtl *pc = reinterpret_cast<PairCtl *>(rec + 2 * (size_t)slots);
+        if (threadIdx.x < kMaxDepth) pc->dq[threadIdx.x] = d.ctl->dq[threadIdx.x];
+        if (threadIdx.x == 0) {
+            pc->radius = d.ctl->radius;
+            pc->step = d.ctl->step;
+        }
+    }
     if (i >= slots) return;
     const int pos = groups[i >> 6] * 64 + (i & 63);
     if (pos < 0 || pos >= d.n) return;
@@ -791,12 +802,11 @@ hipError_t launch_coarse(const Dev &d, const Learn &L, int out, const int *group
 {
     const int waves = groups ? ngroups : (d.n + 63) / 64;
     if (waves <= 0) return hipSuccess;
-    const float *dqtab = nullptr;
     const float4 *rec = nullptr;
     float4 *acc_out = nullptr;
 #define NB_COARSE_ARGS                                                                             \
     d, L, (const int *)d.cchild, (const float4 *)d.cdata, (const float4 *)d.cqa, (const float4 *)d.cqb, \
-        (const float2 *)d.cmac, dqtab, groups, ngroups, rec, xraw, frame_out, acc_out, fmode
+        (const float2 *)d.cmac, groups, ngroups, rec, xraw, frame_out, acc_out, fmode
 #define NB_COARSE_LAUNCH(OUT)                                                                                  \
     switch (coarse_waves_per_group(waves)) {                                                                   \
     case 16: hipLaunchKernelGGL((k_coarse64<OUT, 16>), dim3(waves), dim3(1024), 0, st, NB_COARSE_ARGS); break; \
@@ -821,8 +831,8 @@ hipError_t launch_pair_records(const Dev &d, const int *groups, int ngroups, flo
     return hipGetLastError();
 }
 
-hipError_t launch_pairs(const Dev &d, const Learn &L, const float *dqtab, const int *groups, int ngroups,
-                        const float4 *rec, float *xraw, float4 *frame_out, float4 *acc_out, hipStream_t st)
+hipError_t launch_pairs(const Dev &d, const Learn &L, const int *groups, int ngroups, const float4 *rec,
+                        float *xraw, float4 *frame_out, float4 *acc_out, hipStream_t st)
 {
     if (ngroups <= 0) return hipSuccess;
     const int fmode = 0;
