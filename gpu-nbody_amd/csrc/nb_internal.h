@@ -265,7 +265,7 @@ constexpr int kW1Frag = 4 * 64 * 8, kW2Frag = 4 * 2 * 64 * 8, kW3Frag = 2 * 64 *
 // acceleration nearly cancels), which would otherwise dominate the squared loss
 constexpr float kClipZ = 8.0f;
 // training: rows of the batch per tile (one block), and the most blocks an iteration runs
-constexpr int kTrainTile = 64, kGradBlocks = 256;
+constexpr int kTrainTile = 32, kGradBlocks = 256;
 inline int train_parts(int batch)
 {
     const int tiles = (batch + kTrainTile - 1) / kTrainTile;

@@ -1007,27 +1007,31 @@ __device__ __forceinline__ int batch_row(uint64_t seed, int it, int r, int S)
 // The order of k is free as long as A and B agree, so a group of 16 k's is
 // taken as k = 4 g + s in step s = 0 .. 3.
 //
-// A wave takes 16 rows of the batch through the network in the transposed
-// form Z^T = W^T X^T, the rows being the columns: a lane's D registers (four
-// hidden units of one row) are then its B operands of the next layer, forward
-// and backward, and activations never leave the registers. The weights come
-// straight from the parameters (they sit in the caches: every wave reads the
-// same 24 KB). The weight gradients contract over the rows, which are spread
-// over the lanes: activations and their gradients go to LDS once, as [unit][row]
-// with rows of kTrainLd floats (a 16-byte read is conflict-free and holds four
-// steps of an operand), and after a barrier the block's four waves each take a
-// quarter of the gradient's tiles. A block loops over tiles of 64 rows and
-// keeps its gradient in accumulators; there are at most kGradBlocks blocks, so
-// the partial gradients stay within 6 MB. All sums have a fixed order.
+// The network runs in the transposed form Z^T = W^T X^T, the rows of the batch
+// being the columns: a lane's D registers are four hidden units of one row. A
+// block has 32 rows at a time, two waves for each 16, each of them with half of
+// every layer's units; a layer's activations go to LDS as [unit][row], where the
+// two waves take all of them as the next layer's B operands, forward and
+// backward. The weights come straight from the parameters (they sit in the
+// caches: every wave reads the same 24 KB). The weight gradients contract over
+// the rows, which are spread over the lanes: they read the same LDS rows, of
+// kTrainLd floats (a 16-byte read holds four steps of an operand), each of the
+// block's four waves a quarter of the gradient's tiles. A block loops over tiles
+// of 32 rows and keeps its gradient in accumulators; there are at most
+// kGradBlocks blocks, so the partial gradients stay within 6 MB. All sums have a
+// fixed order.
 //
-// Bound: latency (a batch of 4,096 rows is 64 blocks; about 300 matrix
-// instructions of 32 cycles per wave). An iteration of 4,096 rows takes 17.6 +
-// 4.8 us; as twelve launches that passed every layer's activations through
-// memory and re-read the batch for each row of weights it took 130 us.
+// Bound: the matrix unit of the CUs that have a block (a batch of 4,096 rows is
+// 128 blocks; about 150 matrix instructions of 32 cycles per wave) and the
+// latency of the layers. An iteration of 4,096 rows takes 11.8 + 4.7 us; with 64
+// rows per block, a wave having 16 of them with all units in its registers, 17.6
+// + 4.8 us (half as many CUs with twice the chain); as twelve launches that
+// passed every layer's activations through memory and re-read the batch for
+// each row of weights it took 130 us.
 // ---------------------------------------------------------------------------
-constexpr int kTrainRows = kTrainTile;     // rows per tile: four waves of 16
+constexpr int kTrainRows = kTrainTile;     // rows per tile: two waves for each 16
 constexpr int kTrainLd = kTrainRows + 4;   // LDS row length
-static_assert(kFeat == 24 && kHid == 64 && kOut == 3, "the tiling below");
+static_assert(kFeat == 24 && kHid == 64 && kOut == 3 && kTrainRows == 32, "the tiling below");
 
 __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c)
 {
@@ -1061,7 +1065,8 @@ __global__ __launch_bounds__(256) void k_train_grad(const float *__restrict__ P,
     const float sc = 2.0f / (3.0f * (float)B);
     const int ntiles = (B + kTrainRows - 1) / kTrainRows;
     for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-        const int rl = 16 * w + m, r = tile * kTrainRows + rl; // this lane's row (column of the products)
+        const int rl = 16 * (w & 1) + m, r = tile * kTrainRows + rl; // this lane's row (column of the products)
+        const int t0 = w & 2; // this wave's tiles of units: t0, t0 + 1
         const bool in = r < B;
         const size_t row = in ? (size_t)batch_row(seed, it, r, S) : 0;
         f32x4 x0 = z4, x1 = z4; // features 4 g .., and 16 + 4 g .. (g < 2)
@@ -1069,15 +1074,31 @@ __global__ __launch_bounds__(256) void k_train_grad(const float *__restrict__ P,
             x0 = *reinterpret_cast<const f32x4 *>(X + row * kFeat + 4 * g);
             if (g < 2) x1 = *reinterpret_cast<const f32x4 *>(X + row * kFeat + 16 + 4 * g);
         }
-        float t0 = 0.f, t1 = 0.f, t2 = 0.f;
+        float y0 = 0.f, y1 = 0.f, y2 = 0.f;
         if (in && g == 0) {
-            t0 = T[row * kOut];
-            t1 = T[row * kOut + 1];
-            t2 = T[row * kOut + 2];
+            y0 = T[row * kOut];
+            y1 = T[row * kOut + 1];
+            y2 = T[row * kOut + 2];
         }
-        f32x4 h1[4], p1[4], h2[4], p2[4]; // activations and their derivatives, units 16 t + 4 g + v
+        // this wave's units 16 (t0 + i) + 4 g + v into a layer's LDS rows, and all
+        // four tiles of the layer out of them
+        auto put = [&](float (*u)[kTrainLd], const f32x4 (&h)[2]) {
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) u[16 * (t0 + i) + 4 * g + v][rl] = h[i][v];
+            __syncthreads();
+        };
+        auto all = [&](float (*u)[kTrainLd], f32x4 (&h)[4]) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) h[t][v] = u[16 * t + 4 * g + v][rl];
+        };
+        f32x4 h[2], p1[2], p2[2], in4[4]; // activations, their derivatives; a layer's input
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int t = t0 + i;
             f32x4 z = *reinterpret_cast<const f32x4 *>(b1 + 16 * t + 4 * g);
 #pragma unroll
             for (int q = 0; q < 4; ++q) z = mfma4(W1[(4 * g + q) * kHid + 16 * t + m], x0[q], z);
@@ -1086,37 +1107,51 @@ __global__ __launch_bounds__(256) void k_train_grad(const float *__restrict__ P,
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
                 float d;
-                h1[t][v] = gelu_both(z[v], d);
-                p1[t][v] = d;
+                h[i][v] = gelu_both(z[v], d);
+                p1[i][v] = d;
             }
         }
+        __syncthreads(); // the last tile's gradients have been read
+        if (w < 2) {
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
+            for (int v = 0; v < 4; ++v) {
+                xs[4 * g + v][rl] = x0[v];
+                if (g < 2) xs[16 + 4 * g + v][rl] = x1[v];
+            }
+        }
+        put(h1s, h);
+        all(h1s, in4);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int t = t0 + i;
             f32x4 z = *reinterpret_cast<const f32x4 *>(b2 + 16 * t + 4 * g);
 #pragma unroll
             for (int rb = 0; rb < 4; ++rb)
 #pragma unroll
-                for (int q = 0; q < 4; ++q) z = mfma4(W2[(16 * rb + 4 * g + q) * kHid + 16 * t + m], h1[rb][q], z);
+                for (int q = 0; q < 4; ++q) z = mfma4(W2[(16 * rb + 4 * g + q) * kHid + 16 * t + m], in4[rb][q], z);
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
                 float d;
-                h2[t][v] = gelu_both(z[v], d);
-                p2[t][v] = d;
+                h[i][v] = gelu_both(z[v], d);
+                p2[i][v] = d;
             }
         }
-        // outputs 0 .. 2 of row r in lane m (g = 0)
+        put(h2s, h);
+        all(h2s, in4);
+        // outputs 0 .. 2 of row r in lane m (g = 0); both waves of the rows work
+        // them out
         f32x4 y = z4;
         if (g == 0) y = f32x4{b3[0], b3[1], b3[2], 0.f};
 #pragma unroll
         for (int rb = 0; rb < 4; ++rb)
 #pragma unroll
-            for (int q = 0; q < 4; ++q) y = mfma4(m < kOut ? W3[(16 * rb + 4 * g + q) * kOut + m] : 0.f, h2[rb][q], y);
+            for (int q = 0; q < 4; ++q) y = mfma4(m < kOut ? W3[(16 * rb + 4 * g + q) * kOut + m] : 0.f, in4[rb][q], y);
         float e0 = 0.f, e1 = 0.f, e2 = 0.f;
         if (in && g == 0) {
-            e0 = y[0] - t0;
-            e1 = y[1] - t1;
-            e2 = y[2] - t2;
-            loss += e0 * e0 + e1 * e1 + e2 * e2;
+            e0 = y[0] - y0;
+            e1 = y[1] - y1;
+            e2 = y[2] - y2;
+            if (w < 2) loss += e0 * e0 + e1 * e1 + e2 * e2;
         }
         e0 *= sc;
         e1 *= sc;
@@ -1124,35 +1159,23 @@ __global__ __launch_bounds__(256) void k_train_grad(const float *__restrict__ P,
         // output g's gradient of row r in lane (m, g)
         const float s0 = __shfl(e0, m), s1 = __shfl(e1, m), s2 = __shfl(e2, m);
         const float dy = g == 0 ? s0 : g == 1 ? s1 : g == 2 ? s2 : 0.f;
-        f32x4 d2[4], d1[4];
+        if (w < 2 && g < kOut) dys[g][rl] = dy;
 #pragma unroll
-        for (int t = 0; t < 4; ++t) d2[t] = mfma4(g < kOut ? W3[(16 * t + m) * kOut + g] : 0.f, dy, z4) * p2[t];
+        for (int i = 0; i < 2; ++i) h[i] = mfma4(g < kOut ? W3[(16 * (t0 + i) + m) * kOut + g] : 0.f, dy, z4) * p2[i];
+        put(d2s, h);
+        all(d2s, in4);
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
+        for (int i = 0; i < 2; ++i) {
             f32x4 z = z4;
 #pragma unroll
             for (int rb = 0; rb < 4; ++rb) {
-                const f32x4 a = *reinterpret_cast<const f32x4 *>(W2 + (16 * t + m) * kHid + 16 * rb + 4 * g);
+                const f32x4 a = *reinterpret_cast<const f32x4 *>(W2 + (16 * (t0 + i) + m) * kHid + 16 * rb + 4 * g);
 #pragma unroll
-                for (int q = 0; q < 4; ++q) z = mfma4(a[q], d2[rb][q], z);
+                for (int q = 0; q < 4; ++q) z = mfma4(a[q], in4[rb][q], z);
             }
-            d1[t] = z * p1[t];
+            h[i] = z * p1[i];
         }
-        __syncthreads(); // the last tile's gradients have been read
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            xs[4 * g + v][rl] = x0[v];
-            if (g < 2) xs[16 + 4 * g + v][rl] = x1[v];
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                h1s[16 * t + 4 * g + v][rl] = h1[t][v];
-                d1s[16 * t + 4 * g + v][rl] = d1[t][v];
-                h2s[16 * t + 4 * g + v][rl] = h2[t][v];
-                d2s[16 * t + 4 * g + v][rl] = d2[t][v];
-            }
-        }
-        if (g < kOut) dys[g][rl] = dy;
-        __syncthreads();
+        put(d1s, h);
 #pragma unroll
         for (int c = 0; c < kTrainRows / 16; ++c) {
             const int k0 = 16 * c + 4 * g; // this lane's rows of the chunk

@@ -1,5 +1,5 @@
 """The FP32 training kernels at the edges of their tiles: one row, part of a
-wave's 16 rows, one tile of 64 rows and its neighbours, as many tiles as blocks
+wave's 16 rows, one tile of 32 rows and its neighbours, as many tiles as blocks
 run (256) and one more, so that a block takes a second tile.
 
 Bars, as for the training kernels at other sizes: the loss within 1e-5 of the
@@ -14,7 +14,7 @@ from helpers import make_sim, random_model
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("rows", [1, 15, 16, 17, 63, 64, 65, 128, 16_384, 16_385, 16_449])
+@pytest.mark.parametrize("rows", [1, 15, 16, 17, 31, 32, 33, 64, 65, 128, 8192, 8193, 16_449])
 def test_gradient_at_tile_edges(nb, oracle, rows):
     from nbody_amd import universe as U
 
