@@ -456,7 +456,7 @@ def main():
     if os.path.exists(tpath):
         with open(tpath) as f:
             tj = json.load(f)
-        traffic = tj.get("bytes_per_launch", {}).get("k_coarse64" if mode == "learned" else "k_force64")
+        traffic = tj.get("bytes_per_launch", {}).get("k_coarse64" if mode == "learned" else "k_force")
         traffic_src = {"file": "profiles/force_traffic.json", "measured_on": tj.get("measured_on"),
                        "command": tj.get("command")}
 
@@ -481,7 +481,7 @@ def main():
             "softening": SOFTENING,
             "dt": DT,
             "vote_width": VOTE,
-            "precision": ("FP32 traversal (Kahan), FP64 summarize, FP64 positions" if mode == "plain" else
+            "precision": ("FP32 traversal (a visit's terms in FP32, their sums in FP64), FP64 summarize, FP64 positions" if mode == "plain" else
                           "FP32 traversal (three plain sums: bodies, monopoles, quadrupoles), FP64 summarize, FP64 positions"),
             "median_rel_force_err": round(main_r["err"]["median"], 8),
             "p90_rel_force_err": round(main_r["err"]["p90"], 8),
@@ -496,7 +496,7 @@ def main():
             "steps_per_s_median_of_3_runs": round(float(np.median(main_r["runs"])), 4),
         },
         "roofline": {
-            "kernel": "force traversal (" + ("k_coarse64, coarse traversal" if mode == "learned" else "k_force64") + ")",
+            "kernel": "force traversal (" + ("k_coarse64, coarse traversal" if mode == "learned" else "k_force") + ")",
             "bound": "valu",
             "engine": ("FP32 vector ALU; peak is MI355X FP32 157.3 TFLOP/s" +
                        ("; the BF16 matrix-core network in the kernel's epilogue is neither counted nor "
