@@ -2,9 +2,11 @@
 //
 // Replaces GPUBarnesHutNBodySimulation (the reference's host driver): device
 // selection, node-pool sizing, buffer allocation, the per-step launch order
-// and the error checks. One HIP stream per handle at default priority; a step
-// is six launches with no host synchronization between them, and nb_step
-// reads the device error word once at the end.
+// and the error checks. One HIP stream per handle at default priority (plus
+// one for sampled checks and training pairs and one for the group order); a
+// step's launches have no host synchronization between them, and nb_step reads
+// the device error word once at the end. Copies to and from the caller's arrays
+// go through pinned slots (through_slots).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -45,7 +47,7 @@ struct nb_sim {
     double4 *chk_part = nullptr, *chk_out = nullptr;
     int chk_cap = 0;
     // level sizes of an earlier tree (the last one read back): they size the
-    // grids of the summarize and sort launches, which read the current sizes
+    // grids of the summarize launches, which read the current sizes
     // on the device, so no step waits for them
     bool hint_valid = false;
     int hint_levels = 0;

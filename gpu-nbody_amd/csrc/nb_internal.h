@@ -151,7 +151,7 @@ struct Dev {
     int *sorted;
     float4 *probe;      // accelerations of a probe force pass (error checks)
     float *bbox_part; // 6 * kBBoxBlocks
-    int *gcost;       // per 64-body group: cost of its last coarse traversal (children tested)
+    int *gcost;       // per 64-body group: cost of its last coarse traversal (interactions + 3 per visited cell)
     int *gorder;      // the groups, most expensive first (the coarse traversal's launch order)
     // the key-sorted build (nb_keys.hip): octant-path keys and bodies (two
     // buffers each for the radix passes; the sorted result ends in [0]), the

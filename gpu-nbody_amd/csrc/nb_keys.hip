@@ -6,7 +6,7 @@
 // from the root with one FP32 recurrence (buildtree.cl:124-136), and a body
 // sits in the first level where no other body shares its path. So every body
 // works out its own path with that same recurrence, 3 bits per level, and the
-// bodies are radix-sorted by it. The cells are the path prefixes that at
+// bodies are sorted by it. The cells are the path prefixes that at
 // least two bodies share; from the sorted keys they follow without any
 // pointer chasing:
 //   * a binary radix tree over the sorted keys (Karras, "Maximizing
@@ -29,8 +29,8 @@
 //
 // Keys hold 21 levels in 63 bits (level 0 in the top bits). Bodies that share
 // all 21 (rare: 2 of 4M in the clustered benchmark universe) form runs of
-// equal keys; one thread per run extends its bodies' paths to 84 levels and
-// orders the run by them (in registers up to kMaxRun bodies, through global
+// equal keys; one thread per run, in the bucket sort or after the radix passes,
+// extends its bodies' paths to 84 levels and orders the run by them (in registers up to kMaxRun bodies, through global
 // memory beyond). Limit: cells on levels below kBuildLevelLimit (bodies at
 // most that deep); beyond it the build stops with a depth error, and a tree
 // of more cells than the pool holds stops it with a pool error.

@@ -59,8 +59,9 @@
 // with the matching order of k), and the three outputs return to their own
 // lanes by shuffles. The corrected acceleration then goes straight into the
 // body update, so the update overlaps with other waves' traversal. Training:
-// FP32 kernels for the forward pass, the backward pass and Adam, with
-// deterministic reductions.
+// forward, backward and weight gradients in one kernel on the FP32 matrix
+// instruction, the gradient's sum and Adam in a second, all sums in a fixed
+// order.
 #include "nb_device.h"
 
 namespace nb {
