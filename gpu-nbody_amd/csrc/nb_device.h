@@ -76,19 +76,24 @@ __device__ __forceinline__ bool end_round(Entry *stk, unsigned *pushed, int wv, 
 
 // K waves that share a group and part: breadth first, a cell each per round,
 // until the queue holds FRONT cells; then each wave takes every K-th of them
-// and walks their subtrees by itself, depth first. The queue is a ring of
-// kQueue entries; a wave's own stack holds its share of it and 7 entries for
+// and walks their subtrees by itself, depth first. After STRETCH visits, or
+// with nothing left, a wave waits for the others, and what all of them have
+// left is dealt out again, every K-th entry to one wave: the subtrees differ in
+// size, and without that the waves end far apart. The queue is a ring of kQueue
+// entries; a wave's own stack holds what it is dealt (at most kDealt entries:
+// with more left in all, the waves go on with what they have) and 7 entries for
 // each level below. The order depends on the tree alone. stk: parted_stack
 // words, the root in the first (before a barrier); visit(entry, opened) calls
 // opened(entry) for what it opens and may set bad. Returns bad.
-constexpr int kQueue = 512, kOwnStack = 576;
+constexpr int kQueue = 512, kOwnStack = 576, kDealt = 120;
 template <int K> constexpr int parted_stack() { return kQueue + K * kOwnStack; }
 
-template <int K, int FRONT, class Visit>
+template <int K, int FRONT, int STRETCH, class Visit>
 __device__ __forceinline__ bool walk_parted(unsigned *stk, unsigned *pushed, int wv, int lane, unsigned cap, bool &bad,
                                             Visit &&visit)
 {
-    static_assert(FRONT - 1 + 8 * K <= kQueue && (FRONT - 1 + 8 * K + K - 1) / K + 7 * kMaxDepth + 8 <= kOwnStack,
+    static_assert(FRONT - 1 + 8 * K <= kQueue && (FRONT - 1 + 8 * K + K - 1) / K <= kDealt && kDealt <= 128 &&
+                      kDealt + 7 * kMaxDepth + 8 <= kOwnStack && K * kOwnStack < (int)kSplitBad,
                   "the queue and the stacks hold every tree of kMaxDepth levels");
     int head = 0, tail = 1; // the same in every wave
     while (tail > head && tail - head < FRONT) {
@@ -117,16 +122,51 @@ __device__ __forceinline__ bool walk_parted(unsigned *stk, unsigned *pushed, int
     int sp = (tail - head + K - 1 - wv) / K;
     for (int i = lane; i < sp; i += 64) own[i] = stk[(head + wv + K * (sp - 1 - i)) % kQueue];
     __builtin_amdgcn_wave_barrier();
-    while (sp > 0) {
-        --sp;
-        const unsigned cur = __builtin_amdgcn_readfirstlane(own[sp]);
-        if ((cur >> 6) >= cap) return true;
-        visit(cur, [&](unsigned e) {
-            own[sp] = e; // every lane, one address
-            ++sp;
-        });
+    for (;;) {
+        for (int v = 0; v < STRETCH && sp > 0; ++v) {
+            --sp;
+            const unsigned cur = __builtin_amdgcn_readfirstlane(own[sp]);
+            if ((cur >> 6) >= cap) {
+                bad = true;
+                break;
+            }
+            visit(cur, [&](unsigned e) {
+                own[sp] = e; // every lane, one address
+                ++sp;
+            });
+        }
+        unsigned before, total;
+        if (!count_round<K>(pushed, wv, lane, sp, bad, before, total)) return true;
+        if (total == 0) return false;
+        const bool deal = total <= (unsigned)(K * kDealt); // the same in every wave
+        unsigned e[2];
+        if (deal) {
+            sp = ((int)total + K - 1 - wv) / K;
+#pragma unroll
+            for (int r = 0; r < 2; ++r) {
+                const int j = lane + 64 * r;
+                if (j >= sp) continue;
+                const unsigned at = wv + K * j; // place in the stacks one after the other
+                unsigned start = 0, from = 0, next = 0;
+#pragma unroll
+                for (int w = 0; w < K - 1; ++w) {
+                    next += pushed[w];
+                    if (at >= next) {
+                        start = next;
+                        from = w + 1;
+                    }
+                }
+                e[r] = stk[kQueue + from * kOwnStack + (at - start)];
+            }
+        }
+        __syncthreads(); // read by every wave: the stacks and the counts
+        if (deal) {
+#pragma unroll
+            for (int r = 0; r < 2; ++r)
+                if (lane + 64 * r < sp) own[lane + 64 * r] = e[r];
+            __builtin_amdgcn_wave_barrier();
+        }
     }
-    return bad;
 }
 
 __device__ __forceinline__ void kahan_add(float &sum, float &comp, float x)

@@ -210,11 +210,14 @@ template <int G, int K> constexpr int force_lds()
 // stack's top K entries in rounds: wave w visits the w-th from the top, and
 // after a barrier pushes what it opened behind the lower waves' entries. At
 // width 64 they part after a first stretch of rounds (walk_parted): a round
-// lasts as long as its slowest visit, and from there on no wave waits for
-// another (100,003 bodies, two spheres: 442 -> 377 us; 262,144: 980 -> 900; 65,536,
-// ball: 149 -> 134). Parting at 128 cells is faster for a uniform ball (177
-// against 195 us at 100,003 bodies) and slower where a few cells hold most of
-// the work (453 against 380). The order depends on nothing but the tree, and so
+// lasts as long as its slowest visit (taking turns to the end: 442 us at
+// 100,003 bodies, two spheres, 980 at 262,144). Parted waves stay even because
+// what they have left is dealt out anew every 8 visits, with four waves 16: 372
+// -> 331 us at 100,003 bodies and 873 -> 766 at 262,144 (two spheres), 128 -> 112
+// at 65,536 (ball), against parting at 256 cells, the best of 64 to 512, with no
+// dealing. Every 8 / 16 / 24 visits 331 / 345 / 368 us at 100,003 bodies, 777 / 766 /
+// 792 at 262,144. With dealing the first stretch can be short: parting at 256 /
+// 128 / 64 cells 355 / 352 / 345 us (8 waves, every 16). The order depends on nothing but the tree, and so
 // do the sums. (Eight waves per SIMD by the
 // attribute: the scalar registers would otherwise allow seven, 1.90 against
 // 2.19 ms at 1M Plummer bodies, theta 0.5, vote 64.)
@@ -346,7 +349,7 @@ __global__ __launch_bounds__(64 * K) __attribute__((amdgpu_waves_per_eu(8, 8))) 
                 if (sp == 0) break;
             }
         } else {
-            bad = walk_parted<K, 256>(stk, pushed, wv, lane, cap, bad, [&](unsigned cur, auto &&opened) {
+            bad = walk_parted<K, 8 * K, K == 4 ? 16 : 8>(stk, pushed, wv, lane, cap, bad, [&](unsigned cur, auto &&opened) {
                 float px, py, pz;
                 const int children =
                     visit_wide<false>(cur, dq_s[cur & 63u], me, eps2, cchild, cdata, px, py, pz, bad, opened);
@@ -393,13 +396,17 @@ __global__ __launch_bounds__(64 * K) __attribute__((amdgpu_waves_per_eu(8, 8))) 
 // chain of visits but wait for each other. us of the force stage, 1 / 4 / 8 / 16 waves:
 //   16,384 bodies (256), ball, theta 0.5, vote 16          307 / 149 / 94 / 73
 //   32,768 bodies (512), disk, theta 1.22, vote 16         110 / 74 / 46 / 36
-//   16,384 bodies (256), ball, theta 0.5, vote 64          272 / 113 / 71 / 56
-//   65,536 bodies (1,024), ball, theta 0.5, vote 64        397 / 172 / 134 / 152
-//   100,003 bodies (1,563), two spheres, theta 0.4, 64     895 / 411 / 380 / 428
-//   131,072 bodies (2,048), two spheres, theta 0.4, 64     934 / 471 / 471 / 550
-//   262,144 bodies (4,096), two spheres, theta 0.4, 64     1147 / 903 / 920 / 1113
-//   327,680 bodies (5,120), disk, theta 1.22, vote 64      138 / 133 / 162 / 263
-//   400,000 bodies (6,250), disk, theta 1.22, vote 64      152 / 160 / 198 / 304
+//   16,384 bodies (256), ball, theta 0.5, vote 64          272 / 94 / 60 / 45
+//   32,768 bodies (512), two spheres, theta 0.4, vote 64   659 / 226 / 151 / 132
+//   40,960 bodies (640), two spheres, theta 0.4, 64        685 / 240 / 169 / 178
+//   40,960 bodies (640), disk, theta 1.22, vote 64         96 / 42 / 37 / 46
+//   100,003 bodies (1,563), two spheres, theta 0.4, 64     919 / 380 / 354 / 381
+//   131,072 bodies (2,048), two spheres, theta 0.4, 64     952 / 427 / 414 / 489
+//   131,072 bodies (2,048), disk, theta 1.22, vote 64      110 / 63 / 76 / 105
+//   262,144 bodies (4,096), two spheres, theta 0.4, 64     1132 / 783 / 832 / 996
+//   400,000 bodies (6,250), two spheres, theta 0.4, 64     1267 / 1161 / 1194 / 1486
+//   400,000 bodies (6,250), disk, theta 1.22, vote 64      157 / 149 / 196 / 294
+//   524,288 bodies (8,192), disk, theta 1.22, vote 64      173 / 190 / 247 / 378
 // Narrow votes split only where it gains most (three times and more). A wave
 // alone adds every body's terms in the order of its group's own depth-first
 // walk, bit for bit what a walk per group gives, and the reference's vote and
@@ -408,7 +415,7 @@ __global__ __launch_bounds__(64 * K) __attribute__((amdgpu_waves_per_eu(8, 8))) 
 static int waves_per_group(int groups, bool narrow)
 {
     if (narrow) return groups <= 640 ? 16 : 1;
-    return groups <= 640 ? 16 : groups <= 1792 ? 8 : groups <= 5120 ? 4 : 1;
+    return groups <= 576 ? 16 : groups <= 1792 ? 8 : groups <= 6400 ? 4 : 1;
 }
 
 template <int G> static void launch_force_g(const Dev &d, int mode, hipStream_t st)

@@ -425,7 +425,7 @@ template <int OUT, int K, bool REC> __device__ __forceinline__ void coarse_trave
     } else {
         if (tid == 0) stk[0] = 0; // root cell 0 at depth 0
         __syncthreads();
-        bad = walk_parted<K, 64>(stk, pushed, wv, lane, cap, bad, visit);
+        bad = walk_parted<K, 64, 32>(stk, pushed, wv, lane, cap, bad, visit);
         // the waves' sums in wave order
         __syncthreads();
         if (lane == 0) totals[wv] = WaveTotals{smb, nbod, nchild, nvisit};
