@@ -1744,7 +1744,10 @@ int nb_diagnostics(nb_sim *s, int32_t pe_samples, uint64_t seed, double *out)
     const int batch = std::min(ns, 65536);
     r = ensure_check_buffers(s, batch);
     if (r) return r;
-    double pe = 0.0;
+    // summed in runs of 64 and the runs in extended precision: n terms one after
+    // the other would be the largest rounding error of the whole potential (131,072
+    // bodies 7.6e-15 against 5e-16; every term in extended precision takes 0.15 ms more)
+    long double pe = 0.0L;
     for (int b0 = 0; b0 < ns; b0 += batch) {
         const int nb_ = std::min(batch, ns - b0);
         std::vector<double4> res;
@@ -1755,12 +1758,17 @@ int nb_diagnostics(nb_sim *s, int32_t pe_samples, uint64_t seed, double *out)
         if (e != hipSuccess) return fail(s, NB_E_HIP, "direct-sum launch: %s", hipGetErrorString(e));
         r = fetch(s, res, (const double4 *)s->chk_out, (size_t)nb_);
         if (r) return r;
-        for (int i = 0; i < nb_; ++i) pe += (double)pm[idx[b0 + i]].w * res[i].w;
+        for (int i = 0; i < nb_; i += 256) {
+            double run[4] = {};
+            const int end = std::min(nb_, i + 256);
+            for (int k = i; k < end; ++k) run[k & 3] += (double)pm[idx[b0 + k]].w * res[k].w;
+            for (double q : run) pe += q;
+        }
     }
     // every pair once, or the sampled bodies' pairs, scaled and halved
-    pe *= exact ? -1.0 : -0.5 * (double)n / (double)ns;
+    pe *= exact ? -1.0L : -0.5L * n / ns;
     out[0] = sum[4];
-    out[1] = pe;
+    out[1] = (double)pe;
     out[2] = sum[1];
     out[3] = sum[2];
     out[4] = sum[3];
