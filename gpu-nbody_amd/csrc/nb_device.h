@@ -184,6 +184,19 @@ __device__ __forceinline__ void flag_error(Ctl *ctl, int code)
                                          __ATOMIC_RELAXED, AGENT);
 }
 
+// One decision for all waves of a block on the device error word: `err` as
+// thread 0 read it, behind a barrier. Another block, or a kernel on another
+// stream, may set the word between two waves' reads, and a wave that left by
+// itself would owe the others what it should have put into LDS. Called once per
+// kernel, by every thread.
+__device__ __forceinline__ bool block_stops(int err)
+{
+    __shared__ int stop;
+    if (threadIdx.x == 0) stop = err;
+    __syncthreads();
+    return __builtin_amdgcn_readfirstlane(stop) != 0;
+}
+
 // Splitter j of a warm build (j < S = bucket_samples(n)): the key at position
 // j * kBucketT of the last tree's sorted keys, so non-decreasing (a decrease
 // means the buffer does not hold them and stops the build with an error), and

@@ -340,7 +340,7 @@ constexpr int kWinBodies = 256 * kWinPer;
 constexpr int kWin = 128;
 
 // ws[0 .. kWin]: spl[w0 - 1 .. w0 + kWin - 1], 0 below the first splitter
-// and ~0 past the last (keys use 63 bits); block-wide, ends with a barrier
+// and ~0 past the last (keys use 63 bits); block-wide, before a barrier
 __device__ __forceinline__ void load_window(const unsigned long long *__restrict__ spl, int S, int w0,
                                             unsigned long long *ws)
 {
@@ -349,7 +349,6 @@ __device__ __forceinline__ void load_window(const unsigned long long *__restrict
         const int j = w0 - 1 + t;
         ws[t] = j < 0 ? 0ull : (j >= S ? ~0ull : spl[j]);
     }
-    __syncthreads();
 }
 
 // bucket of k if it is one of w0 .. w0 + kWin - 1, else -1
@@ -385,8 +384,8 @@ __global__ __launch_bounds__(256) void k_keys_warm(Dev d, const int *__restrict_
     const int t = threadIdx.x, first = blockIdx.x * kWarmBodies;
     const int n = d.n;
     const Ctl *ctl = d.ctl;
+    const int err = ctl->error;
     if (blockIdx.x == 0) clear_levels(d);
-    if (ctl->error) return;
     const int w0 = first / kBucketT + 1 - kWin / 4;
     if (t < kWin) h[t] = 0;
     int b[kWarmPer];
@@ -398,6 +397,7 @@ __global__ __launch_bounds__(256) void k_keys_warm(Dev d, const int *__restrict_
         p[j] = staged ? staged[ic] : d.pm4[b[j]];
     }
     load_window(spl, S, w0, ws);
+    if (block_stops(err)) return;
     const float rx = ctl->root[0], ry = ctl->root[1], rz = ctl->root[2], rr = ctl->radius;
 #pragma unroll
     for (int j = 0; j < kWarmPer; ++j) {
@@ -436,7 +436,7 @@ __global__ __launch_bounds__(1024) void k_bucket_scan(const Ctl *ctl, const unsi
     __shared__ unsigned c[kBsChunk + kBsChunk / kBsPer];
     __shared__ unsigned wsum[16];
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    if (ctl->error) return;
+    if (block_stops(ctl->error)) return;
     const int nb = S + 1;
     unsigned carry = 0;
     for (int c0 = 0; c0 < nb; c0 += kBsChunk) {
@@ -648,7 +648,7 @@ template <int R> __global__ __launch_bounds__(kSampleThreads) void k_sample(Dev 
     static_assert(R == 1 || R == 2, "partners in a thread: places 0 and 1");
     __shared__ unsigned long long sk[R][T];
     const Ctl *ctl = d.ctl;
-    if (ctl->error) return;
+    if (block_stops(ctl->error)) return;
     const int t = threadIdx.x, n = d.n;
     const float rx = ctl->root[0], ry = ctl->root[1], rz = ctl->root[2], rr = ctl->radius;
     unsigned long long k[R];
@@ -1320,8 +1320,10 @@ __device__ __forceinline__ int2 bintree_node(const Dev &d, const K &ka, const un
         t = (t + 1) >> 1;
         if (delta_above(ka, deep, n, i, ki, i + (s + t) * dir, dn, ln)) s += t;
     } while (t > 1);
-    const int g = i + s * dir + min(dir, 0);
     const int lo = min(i, j), hi = max(i, j);
+    // of keys in order the split lies inside the range; the bounds keep the
+    // links below inside their arrays whatever the keys are
+    const int g = max(lo, min(i + s * dir + min(dir, 0), hi - 1));
     if (lo == g) o.lparent[g] = i;
     else o.iparent[g] = i;
     if (hi == g + 1) o.lparent[g + 1] = i;
@@ -1353,15 +1355,17 @@ __global__ __launch_bounds__(kBtThreads) void k_bintree(Dev d, const unsigned lo
     __shared__ int wsum[SCAN ? kBtThreads / 64 : 1], wdep[SCAN ? kBtThreads / 64 : 1];
     __shared__ int h[SCAN ? kMaxDepth : 1];
     const int n = d.n, t = threadIdx.x, lane = t & 63, w = t >> 6;
-    Ctl *ctl = d.ctl;
-    if (ctl->error) return; // block-uniform
+    const int err = d.ctl->error;
     const int base = (int)blockIdx.x * kBtThreads - kBtHalo;
     if (SCAN && t < kMaxDepth) h[t] = 0;
     for (int u = t; u < kBtSpan; u += kBtThreads) {
         const int g = base + u;
         ks[u] = g >= 0 && g < n ? key[g] : 0ull;
     }
-    __syncthreads();
+    // one decision for the block: bintree_node of another block may flag a depth
+    // error meanwhile, and a window without the keys of waves that left would be
+    // searched as if it were in order
+    if (block_stops(err)) return;
     const int i = (int)blockIdx.x * kBtThreads + t;
     int2 node = make_int2(0, 0); // cells held, level of the first
     if (i < n - 1) node = bintree_node(d, KeysAny{ks, key, base}, deep, n, i, o);
@@ -1440,7 +1444,7 @@ __global__ __launch_bounds__(256) void k_scan_tiles(const Ctl *ctl, const int *_
                                                     int *__restrict__ sums, int *__restrict__ tdepth)
 {
     __shared__ int wsum[4], wdep[4];
-    if (ctl->error) return;
+    const int err = ctl->error;
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
     const int i0 = blockIdx.x * kScanTile + t * kScanPer;
     const int4 v = load4(in, i0, m), kt = load4(ktop, i0, m);
@@ -1460,7 +1464,7 @@ __global__ __launch_bounds__(256) void k_scan_tiles(const Ctl *ctl, const int *_
         if (lane >= o) x += y;
     }
     if (lane == 63) wsum[w] = x;
-    __syncthreads();
+    if (block_stops(err)) return;
     int run = x - acc;
     for (int ww = 0; ww < w; ++ww) run += wsum[ww];
     const int4 e = make_int4(run, run + v.x, run + v.x + v.y, run + v.x + v.y + v.z);
@@ -1485,7 +1489,7 @@ __global__ __launch_bounds__(1024) void k_scan_sums(Dev d, int *__restrict__ sum
     __shared__ int s[1024];
     __shared__ int wdep[16];
     Ctl *ctl = d.ctl;
-    if (ctl->error) return;
+    const int err = ctl->error;
     const int t = threadIdx.x;
     const int per = (ntiles + 1023) / 1024;
     int acc = 0, dep = 0;
@@ -1500,7 +1504,7 @@ __global__ __launch_bounds__(1024) void k_scan_sums(Dev d, int *__restrict__ sum
     for (int o = 32; o > 0; o >>= 1) dep = max(dep, __shfl_xor(dep, o));
     if ((t & 63) == 0) wdep[t >> 6] = dep;
     s[t] = acc;
-    __syncthreads();
+    if (block_stops(err)) return;
     for (int st = 1; st < 1024; st <<= 1) {
         const int u = t >= st ? s[t - st] : 0;
         __syncthreads();

@@ -125,8 +125,9 @@ template <int T, bool ONE> __global__ __launch_bounds__(T) void k_bbox(Dev d, in
 {
     __shared__ float part[T / 64][6];
     // a device error stops the pipeline until the host has seen it: the steps
-    // that were already queued behind it change nothing
-    if (d.ctl->error) return;
+    // that were already queued behind it change nothing (no box, by the thread
+    // that writes it; every wave has given it its part)
+    const int err = d.ctl->error;
     const int n = d.n;
     // seeded with body 0 as the reference does (boundingbox.cl:44-58)
     const float4 b0 = d.pm4[0];
@@ -151,7 +152,7 @@ template <int T, bool ONE> __global__ __launch_bounds__(T) void k_bbox(Dev d, in
     }
     for (int j = blockIdx.x * T + threadIdx.x; j <= S; j += gridDim.x * T) make_splitter(d, j, S);
     block_minmax<T>(v, part);
-    if (threadIdx.x == 0) {
+    if (threadIdx.x == 0 && !err) {
         if (ONE) {
             finish_box(d, v);
         } else {
@@ -165,7 +166,7 @@ template <int T, bool ONE> __global__ __launch_bounds__(T) void k_bbox(Dev d, in
 __global__ __launch_bounds__(256) void k_bbox_final(Dev d, int blocks)
 {
     __shared__ float part[4][6];
-    if (d.ctl->error) return;
+    const int err = d.ctl->error;
     float w[6] = {d.bbox_part[0], d.bbox_part[1], d.bbox_part[2], d.bbox_part[3], d.bbox_part[4],
                   d.bbox_part[5]};
     for (int b = threadIdx.x; b < blocks; b += blockDim.x) {
@@ -174,7 +175,7 @@ __global__ __launch_bounds__(256) void k_bbox_final(Dev d, int blocks)
         w[3] = fmaxf(w[3], q[3]); w[4] = fmaxf(w[4], q[4]); w[5] = fmaxf(w[5], q[5]);
     }
     block_minmax<256>(w, part);
-    if (threadIdx.x == 0) finish_box(d, w);
+    if (threadIdx.x == 0 && !err) finish_box(d, w);
 }
 
 // ---------------------------------------------------------------------------
