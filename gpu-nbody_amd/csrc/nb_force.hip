@@ -249,7 +249,11 @@ __global__ __launch_bounds__(64 * K) __attribute__((amdgpu_waves_per_eu(8, 8))) 
     const int wv = K == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = d.n;
     Ctl *ctl = d.ctl;
-    if (ctl->error) return;
+    // several waves decide together, at the barrier before their walk: one that
+    // left by itself would leave its count of a round unwritten, which the
+    // others add up, and they stop when the sum is zero
+    const int err = ctl->error;
+    if (K == 1 && err) return;
     if (ctl->max_depth > kMaxDepth) { // calculateforce.cl:69-73
         if (tid == 0) flag_error(ctl, kErrDepth);
         return;
@@ -314,7 +318,7 @@ __global__ __launch_bounds__(64 * K) __attribute__((amdgpu_waves_per_eu(8, 8))) 
         }
     } else {
         if (tid == 0) stk[0] = entry(0, 15u); // root cell 0 at depth 0
-        __syncthreads();
+        if (block_stops(err)) return;
         if constexpr (G < 64) {
             int sp = 1; // the same in every wave
             for (;;) {

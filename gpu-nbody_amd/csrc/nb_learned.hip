@@ -239,7 +239,8 @@ template <int OUT, int K, bool REC> __device__ __forceinline__ void coarse_trave
     const int wv = K == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = d.n;
     Ctl *ctl = d.ctl;
-    if (ctl->error) return;
+    const int err = ctl->error; // several waves decide together, as in k_force
+    if (K == 1 && err) return;
     if (ctl->max_depth > kMaxDepth) {
         if (tid == 0) flag_error(ctl, kErrDepth);
         return;
@@ -424,7 +425,7 @@ template <int OUT, int K, bool REC> __device__ __forceinline__ void coarse_trave
         }
     } else {
         if (tid == 0) stk[0] = 0; // root cell 0 at depth 0
-        __syncthreads();
+        if (block_stops(err)) return;
         bad = walk_parted<K, 64, 32>(stk, pushed, wv, lane, cap, bad, visit);
         // the waves' sums in wave order
         __syncthreads();

@@ -15,7 +15,7 @@ import re
 import pytest
 
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "gpu-nbody_amd", "csrc")
-FILES = ["nb_keys.hip", "nb_tree.hip"]
+FILES = ["nb_force.hip", "nb_keys.hip", "nb_learned.hip", "nb_tree.hip"]
 BARRIERS = {"__syncthreads", "__syncthreads_or"}
 
 
@@ -70,4 +70,4 @@ def test_blocks_decide_together(name):
 
 def test_kernels_are_found():
     names = {f for name in FILES for f, _ in _functions(_source(name))}
-    assert {"k_bintree", "k_bucket_sort", "k_link", "k_bbox", "k_scan_sums"} <= names
+    assert {"k_force", "coarse_traverse", "k_bintree", "k_bucket_sort", "k_link", "k_bbox", "k_scan_sums"} <= names
