@@ -1019,6 +1019,15 @@ int nb_set_state(nb_sim *s, const float *x, const float *y, const float *z, cons
     // nothing queued earlier may still read the buffers overwritten below
     drain(s);
     nb::Dev &d = s->d;
+    // from the first piece on nothing of the old state holds, sorted[] least of
+    // all: a copy that fails halfway leaves a handle without a state
+    s->have_state = false;
+    s->hint_valid = false; // the first step reads its level sizes back
+    s->ord_ready = false;  // the launch order of the coarse traversal belongs to the old bodies
+    s->keys_warm = false;  // and so does sorted[]: the next build sorts from scratch
+    s->staged = false;
+    s->splitters = false;
+    s->sort_pending = false;
     const float *const col[7] = {x, y, z, vx, vy, vz, m};
     // records, accelerations of zero, the identity in sorted[] and a Ctl that
     // starts over (but for the epoch, so that no slot of an earlier tree can look
@@ -1036,12 +1045,6 @@ int nb_set_state(nb_sim *s, const float *x, const float *y, const float *z, cons
     HIP_TRY(s, hipStreamSynchronize(s->stream));
     s->inter_before = 0;
     s->cell_inter_before = 0;
-    s->hint_valid = false; // the first step reads its level sizes back
-    s->ord_ready = false;  // the launch order of the coarse traversal belongs to the old bodies
-    s->keys_warm = false;  // and so does sorted[]: the next build sorts from scratch
-    s->staged = false;
-    s->splitters = false;
-    s->sort_pending = false;
     reset_control(s);
     s->have_state = true;
     s->err.clear();
@@ -1812,6 +1815,7 @@ int nb_restore_state(nb_sim *s, const double *x, const double *y, const double *
     }
     int r = nb_set_state(s, fx.data(), fy.data(), fz.data(), vx, vy, vz, mass);
     if (r) return r;
+    s->have_state = false; // until all of it is there
     nb::Dev &d = s->d;
     {
         std::vector<float4> acc(n);
@@ -1828,7 +1832,7 @@ int nb_restore_state(nb_sim *s, const double *x, const double *y, const double *
     HIP_TRY(s, hipMemcpyAsync(&d.ctl->step, &step, sizeof(int), hipMemcpyHostToDevice, s->stream));
     HIP_TRY(s, hipMemcpyAsync(&d.ctl->max_depth, &max_depth, sizeof(int), hipMemcpyHostToDevice, s->stream));
     HIP_TRY(s, hipStreamSynchronize(s->stream));
-    s->hint_valid = false;
+    s->have_state = true;
     return NB_OK;
 }
 
