@@ -177,6 +177,28 @@ template <class T> hipError_t dalloc(T **p, size_t count)
     return hipMalloc((void **)p, count * sizeof(T) + 64);
 }
 
+// Device memory for a handle: what earlier calls' Scratch left with it goes back
+// when it is in the way. A failure is taken out of the runtime's last error, which
+// the next launch would report as its own.
+hipError_t alloc_for(nb_sim *s, void **p, size_t bytes)
+{
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipSuccess) return e;
+    (void)hipGetLastError();
+    if (s->kept.empty()) return e;
+    for (const auto &b : s->kept) (void)hipFree(b.first);
+    s->kept.clear();
+    s->kept_bytes = 0;
+    e = hipMalloc(p, bytes);
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e;
+}
+
+template <class T> hipError_t alloc_for(nb_sim *s, T **p, size_t count)
+{
+    return alloc_for(s, (void **)p, count * sizeof(T) + 64);
+}
+
 nb::Ctl initial_ctl(const nb_sim *s, uint32_t epoch)
 {
     nb::Ctl c{};
@@ -491,16 +513,16 @@ int ensure_quad(nb_sim *s)
 {
     nb::Dev &d = s->d;
     const size_t cap = (size_t)d.cap;
-    if (!d.cq64) HIP_TRY(s, dalloc(&d.cq64, 8 * cap));
-    if (!d.cqa) HIP_TRY(s, dalloc(&d.cqa, 8 * cap));
-    if (!d.cqb) HIP_TRY(s, dalloc(&d.cqb, 8 * cap));
-    if (!d.cmac) HIP_TRY(s, dalloc(&d.cmac, 8 * cap));
+    if (!d.cq64) HIP_TRY(s, alloc_for(s, &d.cq64, 8 * cap));
+    if (!d.cqa) HIP_TRY(s, alloc_for(s, &d.cqa, 8 * cap));
+    if (!d.cqb) HIP_TRY(s, alloc_for(s, &d.cqb, 8 * cap));
+    if (!d.cmac) HIP_TRY(s, alloc_for(s, &d.cmac, 8 * cap));
     return NB_OK;
 }
 
 int ensure_learn(nb_sim *s)
 {
-    if (!s->mlpbuf) HIP_TRY(s, hipMalloc(&s->mlpbuf, nb::kMlpBufBytes));
+    if (!s->mlpbuf) HIP_TRY(s, alloc_for(s, &s->mlpbuf, nb::kMlpBufBytes));
     return ensure_quad(s);
 }
 
@@ -685,20 +707,20 @@ int ensure_check_buffers(nb_sim *s, int ns)
     s->chk_idx = nullptr;
     s->chk_part = s->chk_out = nullptr;
     s->chk_cap = 0;
-    HIP_TRY(s, hipMalloc((void **)&s->chk_idx, (size_t)ns * sizeof(int)));
-    HIP_TRY(s, hipMalloc((void **)&s->chk_part, (size_t)ns * 64 * sizeof(double4)));
-    HIP_TRY(s, hipMalloc((void **)&s->chk_out, (size_t)ns * sizeof(double4)));
+    HIP_TRY(s, alloc_for(s, &s->chk_idx, (size_t)ns));
+    HIP_TRY(s, alloc_for(s, &s->chk_part, (size_t)ns * 64));
+    HIP_TRY(s, alloc_for(s, &s->chk_out, (size_t)ns));
     if (s->chk_acc) (void)hipFree(s->chk_acc);
     s->chk_acc = nullptr;
-    HIP_TRY(s, hipMalloc((void **)&s->chk_acc, (size_t)ns * sizeof(float4)));
+    HIP_TRY(s, alloc_for(s, &s->chk_acc, (size_t)ns));
     s->chk_cap = ns;
     return NB_OK;
 }
 
-// Device allocations that live for one API call; freed after the stream drains.
-// Device memory of one call. The blocks stay with the handle for its next call
-// (a gradient of 4096 rows spent half its time on hipMalloc and hipFree), up to
-// kKeepBytes; more is freed.
+// Device memory of one call. When it ends the handle's streams are drained and
+// the blocks stay with the handle for its next call (a gradient of 4096 rows spent
+// half its time on hipMalloc and hipFree), up to kKeepBytes; more is freed, and
+// what is kept is freed when another allocation finds no room (alloc_for).
 struct Scratch {
     nb_sim *s;
     std::vector<std::pair<void *, size_t>> blocks;
@@ -719,6 +741,8 @@ struct Scratch {
     {
         const size_t bytes = (count * sizeof(T) + 64 + 255) & ~(size_t)255;
         *p = nullptr;
+        blocks.reserve(blocks.size() + 1);
+        s->kept.reserve(s->kept.size() + blocks.size() + 1); // the destructor does not allocate
         auto best = s->kept.end();
         for (auto it = s->kept.begin(); it != s->kept.end(); ++it)
             if (it->second >= bytes && it->second <= 2 * bytes && (best == s->kept.end() || it->second < best->second))
@@ -730,14 +754,7 @@ struct Scratch {
             s->kept.erase(best);
             return NB_OK;
         }
-        hipError_t e = hipMalloc((void **)p, bytes);
-        if (e != hipSuccess) {
-            // what is kept may be in the way
-            for (const auto &b : s->kept) (void)hipFree(b.first);
-            s->kept.clear();
-            s->kept_bytes = 0;
-            e = hipMalloc((void **)p, bytes);
-        }
+        const hipError_t e = alloc_for(s, (void **)p, bytes);
         if (e != hipSuccess) return fail(s, NB_E_HIP, "hipMalloc(%zu): %s", count * sizeof(T), hipGetErrorString(e));
         blocks.push_back({*p, bytes});
         return NB_OK;
@@ -1246,8 +1263,8 @@ int nb_get_paths(nb_sim *s, uint64_t *paths3, int32_t *depth)
     const size_t n = (size_t)s->d.n;
     unsigned long long *dp = nullptr;
     int *dd = nullptr;
-    HIP_TRY(s, hipMalloc((void **)&dp, 3 * n * sizeof(unsigned long long)));
-    hipError_t e = hipMalloc((void **)&dd, n * sizeof(int));
+    HIP_TRY(s, alloc_for(s, &dp, 3 * n));
+    hipError_t e = alloc_for(s, &dd, n);
     if (e == hipSuccess) e = nb::launch_paths(s->d, dp, dd, s->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(paths3, dp, 3 * n * 8, hipMemcpyDeviceToHost, s->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(depth, dd, n * sizeof(int), hipMemcpyDeviceToHost, s->stream);

@@ -49,6 +49,14 @@ struct Pool {
 
 Pool device, pinned;
 std::atomic<int> fail_state{0}; // which set-state launch from now on fails (0: none)
+// as the runtime keeps it: the last failure, until it is asked for; a launch asks
+thread_local hipError_t last_error = hipSuccess;
+
+hipError_t kept(hipError_t e)
+{
+    if (e != hipSuccess) last_error = e;
+    return e;
+}
 
 } // namespace
 
@@ -61,9 +69,15 @@ long long host_device_used() { return (long long)device.used; }
 long long host_pinned_used() { return (long long)pinned.used; }
 void host_fail_state_launch(int nth) { fail_state = nth; }
 
-hipError_t hipMalloc(void **p, size_t bytes) { return device.get(p, bytes); }
+hipError_t hipGetLastError()
+{
+    const hipError_t e = last_error;
+    last_error = hipSuccess;
+    return e;
+}
+hipError_t hipMalloc(void **p, size_t bytes) { return kept(device.get(p, bytes)); }
 hipError_t hipFree(void *p) { return device.give_back(p); }
-hipError_t hipHostMalloc(void **p, size_t bytes, unsigned) { return pinned.get(p, bytes); }
+hipError_t hipHostMalloc(void **p, size_t bytes, unsigned) { return kept(pinned.get(p, bytes)); }
 hipError_t hipHostFree(void *p) { return pinned.give_back(p); }
 hipError_t hipMemcpyAsync(void *dst, const void *src, size_t bytes, hipMemcpyKind, hipStream_t)
 {
@@ -136,13 +150,13 @@ hipError_t launch_set_state(const Dev &d, int first, int count, const float *c, 
         d.sorted[i] = i;
     }
     if (first == 0) d.ctl->step = -1;
-    return hipSuccess;
+    return hipGetLastError();
 }
 hipError_t launch_copy(void *dst, const void *src, size_t bytes, hipStream_t)
 {
     if (((uintptr_t)dst | (uintptr_t)src) % 16) return hipErrorInvalidValue;
     memcpy(dst, src, bytes);
-    return hipSuccess;
+    return hipGetLastError();
 }
 hipError_t launch_columns(const float4 *src, int count, float *col, hipStream_t)
 {
@@ -151,7 +165,7 @@ hipError_t launch_columns(const float4 *src, int count, float *col, hipStream_t)
         col[count + j] = src[j].y;
         col[2 * count + j] = src[j].z;
     }
-    return hipSuccess;
+    return hipGetLastError();
 }
 hipError_t launch_copy_vertices(const Dev &d, int first, int count, float4 *pos, float4 *vel, hipStream_t)
 {
@@ -160,47 +174,51 @@ hipError_t launch_copy_vertices(const Dev &d, int first, int count, float4 *pos,
         if (pos) pos[j] = make_float4(p.x, p.y, p.z, 1.0f);
         if (vel) vel[j] = make_float4(v.x, v.y, v.z, 1.0f);
     }
-    return hipSuccess;
+    return hipGetLastError();
 }
 
-hipError_t launch_bbox(const Dev &, int, bool, hipStream_t) { return hipSuccess; }
-hipError_t launch_build_keys(const Dev &, bool, bool, bool, hipStream_t) { return hipSuccess; }
-hipError_t launch_levels(const Dev &, hipStream_t) { return hipSuccess; }
-hipError_t launch_summarize_level(const Dev &, int, int, hipStream_t) { return hipSuccess; }
-hipError_t launch_summarize_block(const Dev &, int, int, hipStream_t) { return hipSuccess; }
-hipError_t launch_force(const Dev &, int, int, hipStream_t) { return hipSuccess; }
-hipError_t launch_integrate(const Dev &, hipStream_t) { return hipSuccess; }
-hipError_t launch_step_mark(const Dev &, bool, hipStream_t) { return hipSuccess; }
-hipError_t launch_paths(const Dev &, unsigned long long *, int *, hipStream_t) { return hipSuccess; }
+hipError_t launch_bbox(const Dev &, int, bool, hipStream_t) { return hipGetLastError(); }
+hipError_t launch_build_keys(const Dev &d, bool, bool, bool, hipStream_t)
+{
+    for (int i = 0; i < d.n; ++i) d.kb_val[0][i] = i; // the order is an order
+    return hipGetLastError();
+}
+hipError_t launch_levels(const Dev &, hipStream_t) { return hipGetLastError(); }
+hipError_t launch_summarize_level(const Dev &, int, int, hipStream_t) { return hipGetLastError(); }
+hipError_t launch_summarize_block(const Dev &, int, int, hipStream_t) { return hipGetLastError(); }
+hipError_t launch_force(const Dev &, int, int, hipStream_t) { return hipGetLastError(); }
+hipError_t launch_integrate(const Dev &, hipStream_t) { return hipGetLastError(); }
+hipError_t launch_step_mark(const Dev &, bool, hipStream_t) { return hipGetLastError(); }
+hipError_t launch_paths(const Dev &, unsigned long long *, int *, hipStream_t) { return hipGetLastError(); }
 hipError_t launch_moments(const Dev &, double *part, hipStream_t)
 {
     memset(part, 0, sizeof(double) * 11 * kMomentBlocks);
-    return hipSuccess;
+    return hipGetLastError();
 }
 hipError_t launch_direct64(const Dev &, const int *, int ns, double4 *, double4 *out, DirectSum, hipStream_t)
 {
     memset(out, 0, sizeof(double4) * (size_t)ns);
-    return hipSuccess;
+    return hipGetLastError();
 }
-hipError_t launch_gather_acc(const Dev &, const int *, int, float4 *, hipStream_t) { return hipSuccess; }
-hipError_t launch_group_order(const Dev &, hipStream_t) { return hipSuccess; }
+hipError_t launch_gather_acc(const Dev &, const int *, int, float4 *, hipStream_t) { return hipGetLastError(); }
+hipError_t launch_group_order(const Dev &, hipStream_t) { return hipGetLastError(); }
 hipError_t launch_coarse(const Dev &, const Learn &, int, const int *, int, float *, float4 *, int, hipStream_t)
 {
-    return hipSuccess;
+    return hipGetLastError();
 }
-hipError_t launch_pair_records(const Dev &, const int *, int, float4 *, hipStream_t) { return hipSuccess; }
+hipError_t launch_pair_records(const Dev &, const int *, int, float4 *, hipStream_t) { return hipGetLastError(); }
 hipError_t launch_pairs(const Dev &, const Learn &, const int *, int, const float4 *, float *, float4 *, float4 *,
                         hipStream_t)
 {
-    return hipSuccess;
+    return hipGetLastError();
 }
-hipError_t launch_make_target(const float4 *, const float4 *, int, float *, hipStream_t) { return hipSuccess; }
-hipError_t launch_standardize(float *, int, int, float *, float *, hipStream_t) { return hipSuccess; }
-hipError_t launch_mlp_rows(const Learn &, const float *, int, float *, hipStream_t) { return hipSuccess; }
+hipError_t launch_make_target(const float4 *, const float4 *, int, float *, hipStream_t) { return hipGetLastError(); }
+hipError_t launch_standardize(float *, int, int, float *, float *, hipStream_t) { return hipGetLastError(); }
+hipError_t launch_mlp_rows(const Learn &, const float *, int, float *, hipStream_t) { return hipGetLastError(); }
 hipError_t launch_train_iter(const Train &, int, int, uint64_t, bool, float, float, float, float, float, float,
                              hipStream_t)
 {
-    return hipSuccess;
+    return hipGetLastError();
 }
 
 } // namespace nb

@@ -73,3 +73,78 @@ def test_failed_state_is_no_state(host, nth):
         assert np.array_equal(got, put)
     sim.close()
     assert host.host_device_used() == 0 and host.host_pinned_used() == 0
+
+
+_ROWS = 4096
+_CALLS = {
+    # what leaves scratch with the handle, then what needs room
+    "direct": ("gradient", lambda sim: sim.direct_accel(np.arange(1024, dtype=np.int32))),
+    "paths": ("gradient", lambda sim: sim.paths()),
+    "features": ("diagnostics", lambda sim: sim.coarse_features()),
+    "model": ("diagnostics", lambda sim: sim.set_model(_model())),
+    "gradient": ("forward", lambda sim: sim.mlp_loss_grad(*_pairs(20 * _ROWS))),
+}
+
+
+def _model():
+    from helpers import random_model
+
+    return random_model(3)
+
+
+def _pairs(rows):
+    g = np.random.default_rng(rows)
+    return g.normal(size=(rows, 24)).astype(np.float32), g.normal(size=(rows, 3)).astype(np.float32)
+
+
+def _before(sim, kind):
+    """What the call that leaves scratch also takes for good."""
+    if kind == "diagnostics":
+        sim.direct_accel(np.arange(16, dtype=np.int32))  # the check buffers
+    else:
+        sim.set_model(_model())
+
+
+def _leave_scratch(sim, kind):
+    if kind == "diagnostics":
+        sim.diagnostics(pe_samples=16)
+    elif kind == "gradient":
+        sim.mlp_loss_grad(*_pairs(_ROWS))
+    else:
+        sim.mlp_forward(_pairs(_ROWS)[0])
+
+
+@pytest.mark.parametrize("what", list(_CALLS))
+def test_kept_scratch_makes_room(host, what):
+    """What one call left with the handle goes back when another finds no room: a
+    call fits wherever it would fit if nothing had been kept, and the launches
+    after it do not see the failed attempt."""
+    from nbody_amd import NbError, _lib
+
+    kind, call = _CALLS[what]
+    lo, hi = 0, 1 << 28  # by halves, the least room that the call needs with nothing kept
+    while hi - lo > 64:
+        room = (lo + hi) // 2
+        fresh = _sim(_state(20_000))
+        _before(fresh, kind)
+        host.host_device_room(room)
+        try:
+            call(fresh)
+            hi = room
+        except NbError as e:
+            assert e.code == _lib.NB_E_HIP
+            lo = room
+        host.host_device_room(-1)
+        fresh.close()
+    sim = _sim(_state(20_000))
+    _before(sim, kind)
+    fixed = host.host_device_used()
+    _leave_scratch(sim, kind)
+    left = host.host_device_used() - fixed
+    assert left > 0
+    host.host_device_room(hi - left)
+    call(sim)
+    host.host_device_room(-1)
+    sim.steps(1)
+    sim.close()
+    assert host.host_device_used() == 0
