@@ -177,6 +177,15 @@ template <class T> hipError_t dalloc(T **p, size_t count)
     return hipMalloc((void **)p, count * sizeof(T) + 64);
 }
 
+// The start of a call: the handle's device, and nothing left in the runtime's last
+// error, which launches report as their own (an allocation of the program's that
+// failed earlier, say).
+hipError_t set_device(const nb_sim *s)
+{
+    (void)hipGetLastError();
+    return hipSetDevice(s->device);
+}
+
 // Device memory for a handle: what earlier calls' Scratch left with it goes back
 // when it is in the way. A failure is taken out of the runtime's last error, which
 // the next launch would report as its own.
@@ -1032,7 +1041,7 @@ int nb_set_state(nb_sim *s, const float *x, const float *y, const float *z, cons
 {
     if (!s) return NB_E_ARG;
     if (!x || !y || !z || !vx || !vy || !vz || !m) return fail(s, NB_E_ARG, "null state array");
-    HIP_TRY(s, hipSetDevice(s->device));
+    HIP_TRY(s, set_device(s));
     // nothing queued earlier may still read the buffers overwritten below
     drain(s);
     nb::Dev &d = s->d;
@@ -1072,7 +1081,7 @@ int nb_run_stage(nb_sim *s, int32_t stage)
 {
     if (!s) return NB_E_ARG;
     if (!s->have_state) return fail(s, NB_E_STATE, "nb_set_state has not been called");
-    HIP_TRY(s, hipSetDevice(s->device));
+    HIP_TRY(s, set_device(s));
     int r = launch_stage(s, stage);
     if (r) return r;
     return check_device_error(s);
@@ -1085,7 +1094,7 @@ int nb_step(nb_sim *s, int32_t nsteps)
     if (!s) return NB_E_ARG;
     if (nsteps < 0) return fail(s, NB_E_ARG, "negative step count");
     if (!s->have_state) return fail(s, NB_E_STATE, "nb_set_state has not been called");
-    HIP_TRY(s, hipSetDevice(s->device));
+    HIP_TRY(s, set_device(s));
     if (force_method(s) == NB_MODE_LEARNED && !s->have_model)
         return fail(s, NB_E_MODEL, "learned mode without a model (nb_train or nb_set_model)");
     const int r = step_loop(s, nsteps);
@@ -1154,7 +1163,7 @@ int nb_copy_vertices(nb_sim *s, float *pos4, float *vel4)
     if (!s) return NB_E_ARG;
     if (!s->have_state) return fail(s, NB_E_STATE, "nb_set_state has not been called");
     if (!pos4 && !vel4) return NB_OK;
-    HIP_TRY(s, hipSetDevice(s->device));
+    HIP_TRY(s, set_device(s));
     const size_t bytes = (pos4 && vel4 ? 2 : 1) * sizeof(float4);
     return through_slots(
         s, true, (size_t)s->d.n, slot_items(s, bytes), bytes,
@@ -1175,7 +1184,7 @@ int nb_copy_vertices_noalloc(nb_sim *s, float *pos4, float *vel4)
     if (!s) return NB_E_ARG;
     if (!s->have_state) return fail(s, NB_E_STATE, "nb_set_state has not been called");
     if (!pos4 && !vel4) return NB_OK;
-    HIP_TRY(s, hipSetDevice(s->device));
+    HIP_TRY(s, set_device(s));
     float4 *stage = scratch_ptr(s->device);
     if (!stage) return fail(s, NB_E_STATE, "no staging address for device %d", s->device);
     const int n = s->d.n;
@@ -1202,7 +1211,7 @@ int32_t nb_num_bodies(const nb_sim *s) { return s ? s->d.n : 0; }
 int nb_get_state(nb_sim *s, float *x, float *y, float *z, float *vx, float *vy, float *vz)
 {
     if (!s) return NB_E_ARG;
-    HIP_TRY(s, hipSetDevice(s->device));
+    HIP_TRY(s, set_device(s));
     const int r = receive_columns(s, s->d.pm4, {x, y, z});
     return r ? r : receive_columns(s, s->d.vel4, {vx, vy, vz});
 }
@@ -1210,7 +1219,7 @@ int nb_get_state(nb_sim *s, float *x, float *y, float *z, float *vx, float *vy, 
 int nb_get_accel(nb_sim *s, float *ax, float *ay, float *az)
 {
     if (!s) return NB_E_ARG;
-    HIP_TRY(s, hipSetDevice(s->device));
+    HIP_TRY(s, set_device(s));
     return receive_columns(s, s->d.acc4, {ax, ay, az});
 }
 
@@ -1218,7 +1227,7 @@ int nb_get_positions64(nb_sim *s, double *x, double *y, double *z)
 {
     if (!s) return NB_E_ARG;
     if (!s->d.fp64) return fail(s, NB_E_STATE, "NB_FP64_POSITIONS is not set");
-    HIP_TRY(s, hipSetDevice(s->device));
+    HIP_TRY(s, set_device(s));
     const size_t n = (size_t)s->d.n;
     std::vector<double4> p;
     int r = fetch(s, p, s->d.pos64, n);
@@ -1234,7 +1243,7 @@ int nb_get_positions64(nb_sim *s, double *x, double *y, double *z)
 int nb_get_root(nb_sim *s, float *out4)
 {
     if (!s || !out4) return NB_E_ARG;
-    HIP_TRY(s, hipSetDevice(s->device));
+    HIP_TRY(s, set_device(s));
     nb::Ctl c;
     int r = read_ctl(s, &c);
     if (r) return r;
@@ -1248,7 +1257,7 @@ int nb_get_root(nb_sim *s, float *out4)
 int nb_get_sorted(nb_sim *s, int32_t *sorted)
 {
     if (!s || !sorted) return NB_E_ARG;
-    HIP_TRY(s, hipSetDevice(s->device));
+    HIP_TRY(s, set_device(s));
     HIP_TRY(s, hipMemcpyAsync(sorted, s->d.sorted, (size_t)s->d.n * sizeof(int), hipMemcpyDeviceToHost,
                               s->stream));
     HIP_TRY(s, hipStreamSynchronize(s->stream));
@@ -1259,7 +1268,7 @@ int nb_get_paths(nb_sim *s, uint64_t *paths3, int32_t *depth)
 {
     if (!s || !paths3 || !depth) return NB_E_ARG;
     if (!s->have_state) return fail(s, NB_E_STATE, "nb_set_state has not been called");
-    HIP_TRY(s, hipSetDevice(s->device));
+    HIP_TRY(s, set_device(s));
     const size_t n = (size_t)s->d.n;
     unsigned long long *dp = nullptr;
     int *dd = nullptr;
@@ -1279,7 +1288,7 @@ int nb_get_cells(nb_sim *s, int32_t cap, int32_t *ncells, int32_t *count, float 
                  float *m)
 {
     if (!s || !ncells) return NB_E_ARG;
-    HIP_TRY(s, hipSetDevice(s->device));
+    HIP_TRY(s, set_device(s));
     nb::Ctl c;
     int r = read_ctl(s, &c);
     if (r) return r;
@@ -1336,7 +1345,7 @@ int nb_probe_accel(nb_sim *s, float *ax, float *ay, float *az)
 {
     if (!s) return NB_E_ARG;
     if (!s->have_state) return fail(s, NB_E_STATE, "nb_set_state has not been called");
-    HIP_TRY(s, hipSetDevice(s->device));
+    HIP_TRY(s, set_device(s));
     int r = probe_pass(s);
     if (r) return r;
     return receive_columns(s, s->d.probe, {ax, ay, az});
@@ -1349,7 +1358,7 @@ int nb_direct_accel(nb_sim *s, const int32_t *idx, int32_t ns, double *out3)
     for (int i = 0; i < ns; ++i)
         if (idx[i] < 0 || idx[i] >= s->d.n) return fail(s, NB_E_ARG, "sample index %d out of range", idx[i]);
     if (ns == 0) return NB_OK;
-    HIP_TRY(s, hipSetDevice(s->device));
+    HIP_TRY(s, set_device(s));
     std::vector<double4> out;
     int r = direct_accel(s, idx, ns, out);
     if (r) return r;
@@ -1365,7 +1374,7 @@ int nb_force_error(nb_sim *s, int32_t nsamples, uint64_t seed, double *stats4)
 {
     if (!s || !stats4 || nsamples < 1) return NB_E_ARG;
     if (!s->have_state) return fail(s, NB_E_STATE, "nb_set_state has not been called");
-    HIP_TRY(s, hipSetDevice(s->device));
+    HIP_TRY(s, set_device(s));
     const int n = s->d.n;
     const int ns = std::min(nsamples, n);
     // ns distinct bodies: partial Fisher-Yates shuffle driven by splitmix64
@@ -1429,7 +1438,7 @@ int nb_set_model(nb_sim *s, const float *model, int32_t count)
 {
     if (!s || !model) return NB_E_ARG;
     if (count != NB_MODEL_FLOATS) return fail(s, NB_E_MODEL, "model blob has %d floats, expected %d", count, NB_MODEL_FLOATS);
-    HIP_TRY(s, hipSetDevice(s->device));
+    HIP_TRY(s, set_device(s));
     return install_model(s, model);
 }
 
@@ -1463,7 +1472,7 @@ int nb_train(nb_sim *s, const nb_train_params *tp_in, nb_train_report *rep)
     if (S64 > (1LL << 26)) return fail(s, NB_E_ARG, "%lld training samples exceed 2^26", S64);
     const int S = (int)S64;
     const int B = std::min(tp.batch, S);
-    HIP_TRY(s, hipSetDevice(s->device));
+    HIP_TRY(s, set_device(s));
     int r = ensure_learn(s);
     if (r) return r;
     const int saved_quad = d.quad;
@@ -1595,7 +1604,7 @@ int nb_coarse_features(nb_sim *s, float *feat, float *acc3, float *e2)
     if (!s) return NB_E_ARG;
     if (!s->have_state) return fail(s, NB_E_STATE, "nb_set_state has not been called");
     if (s->p.vote_width != 64) return fail(s, NB_E_ARG, "the coarse traversal needs vote width 64");
-    HIP_TRY(s, hipSetDevice(s->device));
+    HIP_TRY(s, set_device(s));
     nb::Dev &d = s->d;
     int r = ensure_quad(s);
     if (r) return r;
@@ -1656,7 +1665,7 @@ int nb_mlp_forward(nb_sim *s, const float *x, int32_t n, float *y)
     if (!s || n < 0 || (n > 0 && (!x || !y))) return NB_E_ARG;
     if (!s->have_model) return fail(s, NB_E_MODEL, "no model installed");
     if (n == 0) return NB_OK;
-    HIP_TRY(s, hipSetDevice(s->device));
+    HIP_TRY(s, set_device(s));
     Scratch m(s);
     float *xd = nullptr, *yd = nullptr;
     int r = m.get(&xd, (size_t)n * nb::kFeat);
@@ -1677,7 +1686,7 @@ int host_data_passes(nb_sim *s, const float *x, const float *t, int n, int iters
 {
     if (!s || !x || !t || n < 1 || iters < 1) return NB_E_ARG;
     if (!s->have_model) return fail(s, NB_E_MODEL, "no model installed");
-    HIP_TRY(s, hipSetDevice(s->device));
+    HIP_TRY(s, set_device(s));
     Scratch m(s);
     nb::Train tr{};
     float *xd = nullptr, *td = nullptr;
@@ -1731,7 +1740,7 @@ int nb_diagnostics(nb_sim *s, int32_t pe_samples, uint64_t seed, double *out)
 {
     if (!s || !out) return NB_E_ARG;
     if (!s->have_state) return fail(s, NB_E_STATE, "nb_set_state has not been called");
-    HIP_TRY(s, hipSetDevice(s->device));
+    HIP_TRY(s, set_device(s));
     const int n = s->d.n;
     Scratch m(s);
     double *mp = nullptr;
@@ -1806,7 +1815,7 @@ int nb_diagnostics(nb_sim *s, int32_t pe_samples, uint64_t seed, double *out)
 int nb_get_masses(nb_sim *s, float *mass)
 {
     if (!s || !mass) return NB_E_ARG;
-    HIP_TRY(s, hipSetDevice(s->device));
+    HIP_TRY(s, set_device(s));
     std::vector<float4> p;
     int r = fetch(s, p, (const float4 *)s->d.pm4, (size_t)s->d.n);
     if (r) return r;
@@ -1822,7 +1831,7 @@ int nb_restore_state(nb_sim *s, const double *x, const double *y, const double *
     if (!x || !y || !z || !vx || !vy || !vz || !ax || !ay || !az || !mass)
         return fail(s, NB_E_ARG, "null state array");
     if (step < -1 || max_depth < 1 || max_depth > NB_MAX_DEPTH) return fail(s, NB_E_ARG, "invalid step or depth");
-    HIP_TRY(s, hipSetDevice(s->device));
+    HIP_TRY(s, set_device(s));
     const size_t n = (size_t)s->d.n;
     std::vector<float> fx(n), fy(n), fz(n);
     for (size_t i = 0; i < n; ++i) {
@@ -1856,7 +1865,7 @@ int nb_restore_state(nb_sim *s, const double *x, const double *y, const double *
 int nb_get_counters(nb_sim *s, nb_counters *out)
 {
     if (!s || !out) return NB_E_ARG;
-    HIP_TRY(s, hipSetDevice(s->device));
+    HIP_TRY(s, set_device(s));
     nb::Ctl c;
     int r = read_ctl(s, &c);
     if (r) return r;

@@ -148,3 +148,23 @@ def test_kept_scratch_makes_room(host, what):
     sim.steps(1)
     sim.close()
     assert host.host_device_used() == 0
+
+
+@pytest.mark.parametrize("call", ["state", "accel", "masses", "positions64", "vertices", "set_state", "step", "root"])
+def test_an_earlier_failure_is_not_this_calls(host, call):
+    """A handle that could not be created leaves an error with the runtime; calls
+    on another handle do not report it as theirs."""
+    from nbody_amd import NbError, _lib
+
+    st = _state(1000)
+    sim = _sim(st, flags=_lib.NB_FP64_POSITIONS)
+    host.host_device_room(1 << 20)
+    with pytest.raises(NbError) as e:
+        _sim(_state(100_000))
+    assert e.value.code == _lib.NB_E_HIP
+    host.host_device_room(-1)
+    out = np.zeros((1000, 4), np.float32)
+    {"state": sim.state, "accel": sim.accel, "masses": sim.masses, "positions64": sim.positions64,
+     "vertices": lambda: sim.copy_vertices(out, None), "set_state": lambda: sim.set_state(*st),
+     "step": sim.step, "root": sim.root}[call]()
+    sim.close()
