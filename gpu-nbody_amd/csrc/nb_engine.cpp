@@ -18,6 +18,7 @@
 #include <cstdio>
 #include <cstring>
 #include <mutex>
+#include <new>
 #include <string>
 #include <thread>
 #include <vector>
@@ -85,9 +86,10 @@ struct nb_sim {
     bool staged = false;    // d.bnode holds pm4 in d.sorted order (the last fused update wrote it)
     bool splitters = false; // the last bounding box worked out the next warm build's splitters
     bool sort_pending = false; // d.kb_val[0] holds the order of a build the sort stage has not taken yet
-    // pinned staging of the copies to and from the caller's arrays (through_slots),
-    // and a pinned copy of Ctl
-    char *slot = nullptr;
+    // staging of the copies to and from the caller's arrays (through_slots), pinned,
+    // and a pinned copy of Ctl; with no pinned memory to be had, ordinary memory
+    // (no copy of Ctl) and the device side of the slots in device memory
+    char *slot = nullptr, *dev_slot = nullptr;
     int slots = 0;
     size_t slot_bytes = 0;
     hipEvent_t slot_ev[kMaxSlots] = {};
@@ -222,9 +224,12 @@ nb::Ctl initial_ctl(const nb_sim *s, uint32_t epoch)
 
 int read_ctl(nb_sim *s, nb::Ctl *out)
 {
-    HIP_TRY(s, nb::launch_copy(s->ctl_host, s->d.ctl, sizeof(nb::Ctl), s->stream));
+    if (s->ctl_host)
+        HIP_TRY(s, nb::launch_copy(s->ctl_host, s->d.ctl, sizeof(nb::Ctl), s->stream));
+    else
+        HIP_TRY(s, hipMemcpyAsync(out, s->d.ctl, sizeof(nb::Ctl), hipMemcpyDeviceToHost, s->stream));
     HIP_TRY(s, hipStreamSynchronize(s->stream));
-    *out = *s->ctl_host;
+    if (s->ctl_host) *out = *s->ctl_host;
     return NB_OK;
 }
 
@@ -241,6 +246,9 @@ int read_ctl(nb_sim *s, nb::Ctl *out)
 // several workers, which take chunks as they come free. New state of 16,384
 // bodies 446 -> 48 us, of 1M 12.7 -> 0.80 ms; vertices of 1000 bodies 55 -> 17
 // us, of 4M 7.5 -> 3.1 ms (43 GB/s).
+//
+// A handle that got no pinned memory has two slots in ordinary memory and, for the
+// kernel, two in device memory, and the runtime copies between the two.
 constexpr size_t kWorkerBytes = (size_t)4 << 20; // one worker more for each of these (helpers for 1 MiB cost more than they copy)
 
 // How a transfer's chunks are cut: `per` items of `bytes` each fill a slot.
@@ -263,13 +271,18 @@ int through_slots(nb_sim *s, bool out, size_t items, size_t per, size_t bytes, c
         for (int turn = 0; e == hipSuccess && bad.load() == (int)hipSuccess; ++turn) {
             const int k = 2 * worker + (turn & 1), other = 2 * worker + (~turn & 1);
             char *const slot = s->slot + (size_t)k * s->slot_bytes;
+            char *const dev_slot = s->dev_slot ? s->dev_slot + (size_t)k * s->slot_bytes : slot;
             const size_t c = next.fetch_add(1), first = c * per;
             if (c < chunks) {
                 const size_t count = std::min(per, items - first);
                 if (s->slot_busy[k]) e = hipEventSynchronize(s->slot_ev[k]);
                 s->slot_busy[k] = false;
                 if (e == hipSuccess && !out) host(first, count, slot);
-                if (e == hipSuccess) e = issue(first, count, slot);
+                if (e == hipSuccess && !out && s->dev_slot)
+                    e = hipMemcpyAsync(dev_slot, slot, count * bytes, hipMemcpyHostToDevice, s->stream);
+                if (e == hipSuccess) e = issue(first, count, dev_slot);
+                if (e == hipSuccess && out && s->dev_slot)
+                    e = hipMemcpyAsync(slot, dev_slot, count * bytes, hipMemcpyDeviceToHost, s->stream);
                 if (e == hipSuccess) e = hipEventRecord(s->slot_ev[k], s->stream);
                 s->slot_busy[k] = true;
             }
@@ -691,7 +704,12 @@ void free_all(nb_sim *s)
     if (s->chk_host) (void)hipHostFree(s->chk_host);
     for (auto &e : s->slot_ev)
         if (e) (void)hipEventDestroy(e);
-    if (s->slot) (void)hipHostFree(s->slot);
+    if (s->dev_slot) {
+        (void)hipFree(s->dev_slot);
+        delete[] s->slot;
+    } else if (s->slot) {
+        (void)hipHostFree(s->slot);
+    }
     if (s->ctl_host) (void)hipHostFree(s->ctl_host);
     for (const auto &b : s->kept) (void)hipFree(b.first);
     if (s->side) (void)hipStreamDestroy(s->side);
@@ -1002,12 +1020,21 @@ int nb_create(const nb_params *p, nb_sim **out)
     // 512 KiB 3.7 ms, 1 MiB 3.15 ms), small systems do not fill them
     s->slots = n < 65536 ? 4 : kMaxSlots;
     s->slot_bytes = n < 65536 ? 256 << 10 : n < 524288 ? 512 << 10 : 1024 << 10;
-    ok = hipHostMalloc((void **)&s->slot, (size_t)s->slots * s->slot_bytes) == hipSuccess &&
-         hipHostMalloc((void **)&s->ctl_host, sizeof(nb::Ctl)) == hipSuccess;
+    if (hipHostMalloc((void **)&s->ctl_host, sizeof(nb::Ctl)) != hipSuccess ||
+        hipHostMalloc((void **)&s->slot, (size_t)s->slots * s->slot_bytes) != hipSuccess) {
+        // the handle does without: slower copies, the same results
+        (void)hipGetLastError();
+        if (s->ctl_host) (void)hipHostFree(s->ctl_host);
+        s->ctl_host = nullptr;
+        s->slot = nullptr;
+        s->slots = 2;
+        ok = dalloc(&s->dev_slot, s->slots * s->slot_bytes) == hipSuccess &&
+             (s->slot = new (std::nothrow) char[s->slots * s->slot_bytes]) != nullptr;
+    }
     for (int k = 0; ok && k < s->slots; ++k)
         ok = hipEventCreateWithFlags(&s->slot_ev[k], hipEventDisableTiming) == hipSuccess;
     if (!ok) {
-        fail(s, NB_E_HIP, "pinned host allocation of %zu bytes failed", (size_t)s->slots * s->slot_bytes);
+        fail(s, NB_E_HIP, "allocation of %zu bytes for copies failed", (size_t)s->slots * s->slot_bytes);
         return bail(NB_E_HIP);
     }
     if (d.quad && ensure_learn(s) != NB_OK) return bail(NB_E_HIP);

@@ -125,8 +125,9 @@ int nb_run_stage(nb_sim *sim, int32_t stage);
  * n_bodies float4 (x, y, z, 1) into pos4 and (vx, vy, vz, 1) into vel4
  * (either may be NULL). Replaces the CL-GL shared VBOs of initGLBuffers
  * (java:229-246): the caller uploads them into its own VBOs. Staged through
- * pinned host memory that the handle holds; large systems are copied by
- * several threads, which end before the call returns. */
+ * pinned host memory that the handle holds (ordinary memory when nb_create got
+ * none pinned); large systems are copied by several threads, which end before
+ * the call returns. */
 int nb_copy_vertices(nb_sim *sim, float *pos4, float *vel4);
 
 /* No counterpart in the reference. For callers that cannot allocate device

@@ -168,3 +168,30 @@ def test_an_earlier_failure_is_not_this_calls(host, call):
      "vertices": lambda: sim.copy_vertices(out, None), "set_state": lambda: sim.set_state(*st),
      "step": sim.step, "root": sim.root}[call]()
     sim.close()
+
+
+@pytest.mark.parametrize("n", [1, 8193, 20_000, 70_001, 600_001])
+@pytest.mark.parametrize("pinned", [0, 1 << 13])
+def test_a_handle_without_pinned_memory(host, n, pinned):
+    """No pinned memory at all, or too little for the slots: the handle is created
+    and its copies (pieces of 256 KiB, 512 KiB and 1 MiB) are the same."""
+    from nbody_amd import _lib
+
+    st = _state(n)
+    host.host_pinned_room(pinned)
+    sim = _sim(_state(n, 2), flags=_lib.NB_FP64_POSITIONS)
+    sim.steps(1)
+    sim.set_state(*st)
+    assert sim.counters().step == -1
+    for got, put in zip(sim.state(), st):
+        assert np.array_equal(got, put)
+    assert np.array_equal(sim.positions64(), np.stack(st[:3], 1).astype(np.float64))
+    assert np.array_equal(sim.masses(), st[6]) and not sim.accel().any()
+    pos, vel = np.full((n, 4), 7, np.float32), np.full((n, 4), 7, np.float32)
+    sim.copy_vertices(pos, vel)
+    one = np.ones(n, np.float32)
+    assert np.array_equal(pos, np.stack([*st[:3], one], 1)) and np.array_equal(vel, np.stack([*st[3:6], one], 1))
+    sim.steps(2)
+    assert host.host_pinned_used() == 0
+    sim.close()
+    assert host.host_device_used() == 0
