@@ -751,7 +751,7 @@ int ensure_check_buffers(nb_sim *s, int ns)
 struct Scratch {
     nb_sim *s;
     std::vector<std::pair<void *, size_t>> blocks;
-    explicit Scratch(nb_sim *sim) : s(sim) {}
+    explicit Scratch(nb_sim *sim) : s(sim) { blocks.reserve(16); }
     ~Scratch()
     {
         drain(s); // the training pairs' stream too, when a launch failed halfway
@@ -768,7 +768,6 @@ struct Scratch {
     {
         const size_t bytes = (count * sizeof(T) + 64 + 255) & ~(size_t)255;
         *p = nullptr;
-        blocks.reserve(blocks.size() + 1);
         s->kept.reserve(s->kept.size() + blocks.size() + 1); // the destructor does not allocate
         auto best = s->kept.end();
         for (auto it = s->kept.begin(); it != s->kept.end(); ++it)
