@@ -42,10 +42,12 @@ __device__ __forceinline__ bool cell_live(const Dev &d, int c, uint32_t ep, int 
 // ---------------------------------------------------------------------------
 // Stage 1: bounding box (boundingbox.cl:20-199): min/max per block (wave64
 // shuffle reduction), then the root, the opening table and the per-step
-// counters. Up to kBoxOne bodies one block of 1024 threads does it all: it
-// reads 512 KiB in about the time of one launch, which it saves (16,384
-// bodies: 9.1 us of two launches -> 6.7 us). More bodies take two launches,
-// one partial per block and one block that combines them; the launch boundary
+// counters. Up to kBoxOne bodies one block of 1024 threads does it all and saves
+// a launch; beyond, its reads take longer than that. us of a whole step (disk,
+// vote 16), two launches / one block: 4,096 bodies 110.5 / 107.8, 16,384 125.3 /
+// 123.9, 20,480 132.9 / 132.4, 24,576 133.8 / 133.4, 32,768 137.9 / 138.6; of the
+// stage alone at 65,536 10.2 / 16.8. More bodies take two launches, one
+// partial per block and one block that combines them; the launch boundary
 // orders the two, where the reference's last-block hand-off
 // (boundingbox.cl:133-196) needs an agent-scope release per block: on MI355X
 // an L2 write-back each, which cost about 40 us per step at 4M bodies against
@@ -54,7 +56,7 @@ __device__ __forceinline__ bool cell_live(const Dev &d, int c, uint32_t ep, int 
 // The splitters of a warm build (S >= 0: there are S) go with the box: neither
 // needs the other, and alone they were a launch of 4.6 us.
 // ---------------------------------------------------------------------------
-constexpr int kBoxOne = 32768;
+constexpr int kBoxOne = 24576;
 constexpr int kBoxOneThreads = 1024;
 
 __device__ __forceinline__ float wave_min(float v)
