@@ -85,6 +85,7 @@ struct nb_sim {
     bool keys_warm = false; // d.sorted holds the last tree's body order (the build starts from it)
     bool staged = false;    // d.bnode holds pm4 in d.sorted order (the last fused update wrote it)
     bool splitters = false; // the last bounding box worked out the next warm build's splitters
+    bool grouped = false; // the build since the last bounding box has grouped the cells by level
     bool sort_pending = false; // d.kb_val[0] holds the order of a build the sort stage has not taken yet
     // staging of the copies to and from the caller's arrays (through_slots), pinned,
     // and a pinned copy of Ctl; with no pinned memory to be had, ordinary memory
@@ -400,12 +401,13 @@ int hint_cells(const nb_sim *s, int level)
 // first larger level, and from the top down to the first larger level.
 constexpr int kTailCells = 2 * nb::kTailThreads / 8;
 
-// The live cells grouped by level, if the build has not done it. Without level sizes of an earlier tree (the
+// The live cells grouped by level, if the build has not done it (after a bounding
+// box without a build the root is the only one). Without level sizes of an earlier tree (the
 // first step of a state) it reads this tree's back, the only host wait inside
 // a step; later steps size their launches from the last sizes read.
 int prepare_levels(nb_sim *s)
 {
-    const hipError_t e = nb::build_levels(s->d.n) ? hipSuccess : nb::launch_levels(s->d, s->stream);
+    const hipError_t e = s->grouped ? hipSuccess : nb::launch_levels(s->d, s->stream);
     if (e != hipSuccess) return fail(s, NB_E_HIP, "level grouping launch: %s", hipGetErrorString(e));
     if (!s->hint_valid) {
         nb::Ctl c;
@@ -490,11 +492,13 @@ int launch_stage(nb_sim *s, int stage, bool whole_step = false)
     case NB_STAGE_BBOX:
         e = nb::launch_bbox(d, s->bbox_blocks, s->keys_warm, s->stream);
         s->splitters = s->keys_warm;
+        s->grouped = false;
         break;
     case NB_STAGE_BUILD:
         e = nb::launch_build_keys(d, s->keys_warm, s->keys_warm && s->staged, s->splitters, s->stream);
         s->splitters = false; // the build replaces the keys they were taken from
         s->sort_pending = e == hipSuccess;
+        s->grouped = e == hipSuccess && nb::build_levels(d.n);
         break;
     case NB_STAGE_SUMMARIZE: {
         int r = prepare_levels(s);
@@ -1079,6 +1083,7 @@ int nb_set_state(nb_sim *s, const float *x, const float *y, const float *z, cons
     s->keys_warm = false;  // and so does sorted[]: the next build sorts from scratch
     s->staged = false;
     s->splitters = false;
+    s->grouped = false;
     s->sort_pending = false;
     const float *const col[7] = {x, y, z, vx, vy, vz, m};
     // records, accelerations of zero, the identity in sorted[] and a Ctl that
