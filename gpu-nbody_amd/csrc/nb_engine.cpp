@@ -330,8 +330,20 @@ int receive(nb_sim *s, void *dst, const void *src, size_t bytes)
         [&](size_t first, size_t count, char *slot) { std::memcpy((char *)dst + first, slot, count); });
 }
 
+// Above kSendThrough the runtime's own copy is the faster one for plain bytes (it
+// needs no weaving and no second pass): network rows in and out on a handle of
+// 2,048 bodies, through slots / the runtime, 0.4 MB 49 / 47 us, 0.8 MB 95 / 63,
+// 1.6 MB 136 / 103, 6.3 MB 381 / 281, 25 MB 1,347 / 913; of 100,003 bodies 44 /
+// 47, 65 / 61, 124 / 96, 321 / 239, 1,085 / 877. It is done with the caller's
+// memory when it returns.
+constexpr size_t kSendThrough = (size_t)512 << 10;
+
 int send(nb_sim *s, void *dst, const void *src, size_t bytes)
 {
+    if (bytes >= kSendThrough) {
+        HIP_TRY(s, hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s->stream));
+        return NB_OK;
+    }
     return through_slots(
         s, false, bytes, s->slot_bytes, 1,
         [&](size_t first, size_t count, char *slot) {
