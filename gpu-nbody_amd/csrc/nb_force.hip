@@ -216,7 +216,7 @@ template <int G, int K> constexpr int force_lds()
 // -> 331 us at 100,003 bodies and 873 -> 766 at 262,144 (two spheres), 128 -> 112
 // at 65,536 (ball), against parting at 256 cells, the best of 64 to 512, with no
 // dealing. Every 8 / 16 / 24 visits 331 / 345 / 368 us at 100,003 bodies, 777 / 766 /
-// 792 at 262,144. With dealing the first stretch can be short: parting at 256 /
+// 792 at 262,144 (a series on another card than that of waves_per_group). With dealing the first stretch can be short: parting at 256 /
 // 128 / 64 cells 355 / 352 / 345 us (8 waves, every 16). The order depends on nothing but the tree, and so
 // do the sums. (Eight waves per SIMD by the
 // attribute: the scalar registers would otherwise allow seven, 1.90 against
@@ -397,25 +397,39 @@ __global__ __launch_bounds__(64 * K) __attribute__((amdgpu_waves_per_eu(8, 8))) 
 // Waves per group, by the number of groups. One wave per group leaves the
 // 1,024 SIMDs (8 waves each) short of waves below about 8,192 groups, and a
 // visit is a chain of a stack read and scalar loads; more waves shorten the
-// chain of visits but wait for each other. us of the force stage, 1 / 4 / 8 / 16 waves:
-//   16,384 bodies (256), ball, theta 0.5, vote 16          307 / 149 / 94 / 73
-//   32,768 bodies (512), disk, theta 1.22, vote 16         110 / 74 / 46 / 36
-//   16,384 bodies (256), ball, theta 0.5, vote 64          272 / 94 / 60 / 45
-//   32,768 bodies (512), two spheres, theta 0.4, vote 64   659 / 226 / 151 / 132
-//   40,960 bodies (640), two spheres, theta 0.4, 64        685 / 240 / 169 / 178
-//   40,960 bodies (640), disk, theta 1.22, vote 64         96 / 42 / 37 / 46
-//   100,003 bodies (1,563), two spheres, theta 0.4, 64     919 / 380 / 354 / 381
-//   131,072 bodies (2,048), two spheres, theta 0.4, 64     952 / 427 / 414 / 489
-//   131,072 bodies (2,048), disk, theta 1.22, vote 64      110 / 63 / 76 / 105
-//   262,144 bodies (4,096), two spheres, theta 0.4, 64     1132 / 783 / 832 / 996
-//   400,000 bodies (6,250), two spheres, theta 0.4, 64     1267 / 1161 / 1194 / 1486
-//   400,000 bodies (6,250), disk, theta 1.22, vote 64      157 / 149 / 196 / 294
-//   524,288 bodies (8,192), disk, theta 1.22, vote 64      173 / 190 / 247 / 378
-// Narrow votes split only where it gains most (three times and more). A wave
-// alone adds every body's terms in the order of its group's own depth-first
-// walk, bit for bit what a walk per group gives, and the reference's vote and
-// time step can make a run chaotic: a rotating disk (dt 0.025) carries a
-// last-bit difference to 1e-3 of the velocities in 20 steps.
+// chain of visits but wait for each other. us of the force stage, 1 / 4 / 8 / 16
+// waves (one series on one card):
+//   vote 64
+//   16,384 bodies (256 groups), ball, theta 0.5      282 / 97 / 63 / 46
+//   32,768 (512), two spheres, theta 0.4             654 / 228 / 144 / 118
+//   40,960 (640), two spheres                        710 / 244 / 157 / 171
+//   40,960 (640), disk, theta 1.22                   99 / 43 / 38 / 47
+//   100,003 (1,563), two spheres                     862 / 345 / 323 / 360
+//   131,072 (2,048), two spheres                     930 / 439 / 404 / 476
+//   131,072 (2,048), disk                            111 / 63 / 76 / 101
+//   262,144 (4,096), two spheres                     1125 / 750 / 762 / 944
+//   400,000 (6,250), two spheres                     1319 / 1121 / 1154 / 1454
+//   400,000 (6,250), disk                            150 / 146 / 191 / 285
+//   524,288 (8,192), two spheres                     1600 / 1437 / 1499 / 1909
+//   524,288 (8,192), disk                            170 / 182 / 245 / 374
+//   vote 16 (32 alike)
+//   16,384 (256), ball, theta 0.5                    391 / 194 / 102 / 74
+//   32,768 (512), disk, theta 1.22                   136 / 61 / 43 / 40
+//   40,960 (640), ball                               514 / 255 / 144 / 146
+//   65,536 (1,024), ball                             537 / 300 / 175 / 190
+//   65,536 (1,024), disk                             140 / 73 / 55 / 72
+//   100,003 (1,563), ball                            599 / 390 / 264 / 289
+//   262,144 (4,096), ball                            764 / 832 / 591 / 700
+//   400,000 (6,250), ball                            928 / 1215 / 897 / 1072
+// The narrow line is no crossing: 8 waves would be the faster up to 4,096 groups.
+// From 641 groups on a wave alone keeps, at that price, the order of its group's own
+// depth-first walk, and so every body's sum bit for bit as a walk per group gives
+// it; below, where a step gains three times and more, the order is given up. The
+// sums of both orders are equally far from 64 bits (16,384 bodies, ball: rms 4.9e-8
+// and 4.8e-8 of the acceleration; 32,768, disk: 8.7e-8 and 8.4e-8), but a run may
+// grow their difference: a rotating disk at the reference's vote and time step (0.025)
+// to 2e-5 of the velocities in 20 steps at 1,000 and 16,384 bodies, 6e-5 at 32,768
+// and 65,536, 3e-4 at 262,144 (the body that differs most).
 static int waves_per_group(int groups, bool narrow)
 {
     if (narrow) return groups <= 640 ? 16 : 1;

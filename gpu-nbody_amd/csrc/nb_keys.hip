@@ -29,9 +29,10 @@
 //
 // Keys hold 21 levels in 63 bits (level 0 in the top bits). Bodies that share
 // all 21 (rare: 2 of 4M in the clustered benchmark universe) form runs of
-// equal keys; one thread per run, in the bucket sort or after the radix passes,
-// extends its bodies' paths to 84 levels and orders the run by them (in registers up to kMaxRun bodies, through global
-// memory beyond). Limit: cells on levels below kBuildLevelLimit (bodies at
+// equal keys, which are ordered by their paths extended to 84 levels: in a bucket
+// that fits LDS every body counts the smaller ones of its run; in a larger bucket
+// and after the radix passes one thread orders a run (after the passes in
+// registers up to kMaxRun bodies, else through global memory). Limit: cells on levels below kBuildLevelLimit (bodies at
 // most that deep); beyond it the build stops with a depth error, and a tree
 // of more cells than the pool holds stops it with a pool error.
 #include "nb_device.h"
@@ -969,8 +970,8 @@ __device__ void order_long_run(const Dev &d, int i, int m, int *val, unsigned lo
 // dependent LDS accesses in all, where radix passes over every varying digit
 // took some 30 of each per pass (one wave per bucket, 5 or 6 passes):
 // bound by that latency, not by bandwidth or the adds. One launch instead of
-// three (buckets, large buckets, runs): 16,384 bodies 29 -> 6.3 us, 1M 42 ->
-// 24 us, 4M 85 -> 58 us.
+// three (buckets, large buckets, runs): 16,384 bodies 29 -> 6.0 us, 1M 42 ->
+// 22 us, 4M 85 -> 58 us.
 // Keys that meet an equal key get their levels 21 .. 83 here too, and their
 // place among the equals by counting the smaller of those.
 //
