@@ -2,7 +2,7 @@
 // (nb_engine.cpp) without a GPU: device and pinned memory are host memory with
 // limits that a test sets, streams and events do nothing because every launch is
 // done when it returns, and the launches that move bodies move them. The others
-// only count. Linked with nb_engine.cpp into a library of its own.
+// do nothing. Linked with nb_engine.cpp into a library of its own.
 #include <hip/hip_runtime.h>
 
 #include <atomic>
